@@ -1,6 +1,6 @@
 """The work that is timed: what a program that uses `deep_ep` has it do, through `EPBuffer` and its helpers.
 
-A case is a dict of plain values.  Four kinds:
+A case is a dict of plain values.  Three kinds:
 
   serve   inference on one GPU's share: dispatch of a batch, combine of the experts' outputs.  `sync`: the host reads the
           counts (exact output sizes); without it outputs have worst-case sizes; `graph`: the two calls are captured once
