@@ -58,8 +58,11 @@ struct EpLayoutArgs {
                                   //   (EP_LAYOUT_FOLDED), or ints that ep_layout_scan replaces by the exclusive prefix
                                   //   over the workgroups (EP_LAYOUT_SCANNED)
     int* col_total;               // [cnt_stride]  column totals (written by ep_layout_scan)
-    int cnt_stride;               // El + R rounded up to a multiple of 8 columns
-    int* slot_map;                // [T, K]  expanded slot of (t, j) if its expert is local, else -1
+    int cnt_stride;               // count_experts + R rounded up to a multiple of 8 columns
+    int count_experts, count_lo;  // experts that get count columns and ranks: [count_lo, count_lo + count_experts)
+                                  //   (this partition's; on a send side that ships ranks: all of them)
+    int* slot_map;                // [T, K]  expanded slot of (t, j) if its expert is local, else -1; on a send side that
+                                  //   ships ranks: entries of the same expert before (t, j), -1 without an expert
     int* tok_row;                 // [T]  token -> its row of the receive stream (written for received tokens only)
     // handle tensors (device)
     int* dst_buffer_slot_idx;     // [T, K]
@@ -80,6 +83,10 @@ struct EpLayoutArgs {
     int* recv_src_metadata;       // [rows_cap, K+2]  (receive side: written here, there is no slot_map)
     int rows_cap;                 // rows the metadata tensor holds
     int connected;                // the peers are arenas of their own (a node), not this arena again
+    int64_t count_box_off;        // byte offset in every arena of the count box [R sources][El]: entries per expert; 0: the
+                                  //   send side ships neither counts nor ranks (the receive side counts and ranks itself)
+    const int* count_box;         // this partition's count box (receive side)
+    const int* rank_box;          // [R * max_tokens, K]  per packed row: what its source ranked (receive side)
 };
 
 // One receive-stream row per wave: copy (or quantise) it into every expanded slot it owns.
@@ -127,6 +134,7 @@ struct EpScatterArgs {
     int region_by_source;
     int num_ranks;
     int pack_sf_off;              // byte offset of the scales inside a packed row (pack mode)
+    int64_t rank_box_off;         // byte offset in every arena of the rank box [R * max_tokens, K] (pack mode; 0: none is kept)
     int vecs_per_lane;            // verbatim kernel: 16-byte vectors a lane moves per task (1..4)
     int rows_are_tokens;          // cached expand: every token was received, so row i of the receive stream is token i
 };

@@ -4,9 +4,10 @@
 // Kernels (all HBM-bound, no MFMA):
 //   ep_layout_count / ep_layout_assign (/ ep_layout_scan)  stable counting sort of the (token, slot)
 //       entries by destination partition and by local expert -> every handle tensor; with several
-//       partitions once on the send side (slots in the destinations' regions) and once on the receive
-//       side (slots of the rows that arrived).  Two launches up to a few hundred workgroups (the
+//       partitions once on the send side (slots in the destinations' regions) and, where the send sides
+//       ship no ranks, once on the receive side (slots of the rows that arrived).  Two launches up to a few hundred workgroups (the
 //       assignment sums the histograms of the workgroups before it itself), three beyond.
+//   ep_layout_place                                        receive side of a node out of the shipped counts and ranks
 //   ep_scatter_copy / ep_scatter_quant                     token (or receive-stream row) -> its expanded slots
 //   ep_scatter_copy_pack / ep_scatter_quant_pack           token -> one packed row per destination partition
 //   ep_sf_transpose                                        scale rows -> scale columns
@@ -215,10 +216,10 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_count(
         if (j >= K) j -= K;
     }
     __syncthreads();
-    // one row of the count matrix: this partition's experts, then the partitions, then zero fill.  For the scan kernel
+    // one row of the count matrix: the counted experts, then the partitions, then zero fill.  For the scan kernel
     // the counts are ints; the slot assignment that sums the rows itself takes them as 16-bit halves (a count is at
     // most EP_TOKENS_PER_BLOCK * EP_MAX_TOPK = 4096), eight columns a 16-byte load and two columns an add.
-    const int El = a.experts_per_rank, lo = a.rank_idx * El;
+    const int El = a.count_experts, lo = a.count_lo;
     if (a.scan_mode == EP_LAYOUT_FOLDED) {
         unsigned* row = (unsigned*)a.blk_cnt + (int64_t)blockIdx.x * (a.cnt_stride >> 1);
         auto count_of = [&](int i) -> unsigned { return i < El ? s_ecnt[lo + i] : (i < El + R ? s_rcnt[i - El] : 0); };
@@ -307,10 +308,10 @@ extern "C" __global__ __launch_bounds__(EP_SCAN_THREADS) void ep_layout_scan(EpL
 template <bool FOLD, bool RECV>
 __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
     extern __shared__ int smem[];
-    const int E = a.num_experts, R = a.num_ranks, K = a.num_topk, El = a.experts_per_rank, A = a.expert_alignment;
+    const int E = a.num_experts, R = a.num_ranks, K = a.num_topk, El = a.count_experts, A = a.expert_alignment;
     const int NW = EP_LAYOUT_THREADS / WAVE;
     const int b = blockIdx.x;
-    int* s_tot = smem;                     // [El + R] totals of the local experts, then of the partitions
+    int* s_tot = smem;                     // [El + R] totals of the counted experts, then of the partitions
     int* s_we = s_tot + El + R;            // [NW][E] per-wave counts, then running slot counters
     int* s_wr = s_we + NW * E;             // [NW][R]
     int* s_tmp = s_wr + NW * R;            // [NW + 1]
@@ -318,8 +319,8 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
     short* s_rk = s_key + EP_TOKENS_PER_BLOCK * K;
     int* s_psum = (int*)(s_rk + EP_TOKENS_PER_BLOCK * K);      // [R + NW]  (receive side)
     const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
-    const int lo = a.rank_idx * El;
-    const int ncols = El + R;              // column c < El: local expert lo + c; else partition c - El
+    const int lo = a.count_lo;
+    const int ncols = El + R;              // column c < El: expert lo + c; else partition c - El
 
     // The launch has one workgroup more than blocks of tokens.  It ranks nothing: it gets the totals like the others
     // (a single block: it counts that block's ids once more) and publishes them (handle tensors, inboxes, the host count
@@ -607,6 +608,16 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
                 if (a.cumulative_stats != nullptr) atomicAdd(&a.cumulative_stats[e], c);
                 if (a.notify_host) a.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
             }
+            if (!RECV && a.send_only) {
+                // slots are the receivers' business: ranks count from 0, and the receivers get the counts they need
+                // to place them (a partition that is not connected to a node ships nothing)
+                if (publisher && a.count_box_off != 0) {
+                    const int r = e / a.experts_per_rank;
+                    ((int*)(a.peer_arenas[r] + a.count_box_off))[a.rank_idx * a.experts_per_rank + (e - r * a.experts_per_rank)] = c;
+                }
+                s_start[e] = 0;
+                continue;
+            }
             s_start[e] = run;
             run += align_up(c, A);
         }
@@ -692,10 +703,8 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
             } else {
                 a.dst_buffer_slot_idx[g] = rslot;
                 a.dst_gsge_idx[g] = -1;             // every copy is local: no transport descriptors
-                if (!a.send_only) {
-                    a.slot_map[g] = eslot;
-                    if (mr == a.rank_idx) a.tok_row[b * EP_TOKENS_PER_BLOCK + tok] = rslot;
-                }
+                if (a.slot_map != nullptr) a.slot_map[g] = eslot;
+                if (!a.send_only && mr == a.rank_idx) a.tok_row[b * EP_TOKENS_PER_BLOCK + tok] = rslot;
             }
         }
         // the running counters of a wave are touched by that wave only and the LDS operations of a wave
@@ -729,6 +738,139 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
 extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_fold(EpLayoutArgs a) { layout_assign_body<true, false>(a); }
 extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_recv(EpLayoutArgs a) { layout_assign_body<false, true>(a); }
 extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_fold_recv(EpLayoutArgs a) { layout_assign_body<true, true>(a); }
+
+// ------------------------------------------------------------------------------------------------
+// Receive side of a node whose send sides ship ranks: nothing is counted or ranked here.  An entry's slot is
+//   first slot of its expert + entries of the same expert from the sources before its own + its rank inside its source,
+// the first two out of the count box [R][El] that the sources filled, the last out of the rank box beside the packed
+// rows: the order of the receive stream (sources in turn, a source's tokens ascending) makes that the lexicographic
+// (row, j) rank of the general receive side above.  Same outputs; two dependent trips to memory (counts, then ids and
+// ranks) where the general form has a histogram launch, a trip for its rows and a ranking.
+// Bound by those trips and the launch.  Workgroup 0 publishes (handle tensors, host count page), the others place 128 rows each.
+// Eight partitions of 64 / 2048 tokens, a partition: count 7.4 + assign 14.0 -> 5.7 us / 6.1 + 11.3 -> 5.5 us (the send side,
+// which now counts all experts, 11.2 -> 10.7 / 17.0 -> 16.9 us); all phases of the node 543 -> 397 / 1522 -> 1436 us.
+// ------------------------------------------------------------------------------------------------
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_place(EpLayoutArgs a) {
+    extern __shared__ int smem[];
+    constexpr int NW = EP_LAYOUT_THREADS / WAVE;
+    const int E = a.num_experts, R = a.num_ranks, K = a.num_topk, El = a.experts_per_rank, A = a.expert_alignment;
+    int* s_box = smem;                     // [E]  counts per source and local expert, then the first slot of each pair
+    int* s_tot = s_box + E;                // [El]
+    int* s_tmp = s_tot + El;               // [NW]
+    int* s_psum = s_tmp + NW;              // [R + NW]
+    int* s_pr = s_psum + R + NW;           // [EP_TOKENS_PER_BLOCK]  packed row of this workgroup's rows
+    int* s_at = s_pr + EP_TOKENS_PER_BLOCK;                    // [EP_TOKENS_PER_BLOCK]  their source's place in s_box
+    signed char* s_local = (signed char*)(s_at + EP_TOKENS_PER_BLOCK);     // [EP_TOKENS_PER_BLOCK * K]  entry is local
+    const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
+    const bool publisher = blockIdx.x == 0;
+    const int b = (int)blockIdx.x - 1, lo = a.rank_idx * El;
+    for (int i = tid; i < E; i += EP_LAYOUT_THREADS) s_box[i] = a.count_box[i];
+    const int num_rows = recv_scan_sources(a, s_psum);          // (its barriers cover s_box)
+    if (!publisher && b * EP_TOKENS_PER_BLOCK >= num_rows) return;
+
+    // counts -> entries of the sources before, totals; then the aligned scan over the experts
+    for (int e = tid; e < El; e += EP_LAYOUT_THREADS) {
+        int run = 0;
+        for (int s = 0; s < R; ++s) {
+            const int c = s_box[s * El + e];
+            s_box[s * El + e] = run;
+            run += c;
+        }
+        s_tot[e] = run;
+    }
+    __syncthreads();
+    const int per = (El + EP_LAYOUT_THREADS - 1) / EP_LAYOUT_THREADS;
+    const int e0 = min(El, tid * per), e1 = min(El, e0 + per);
+    int mine = 0;
+    for (int e = e0; e < e1; ++e) mine += align_up(s_tot[e], A);
+    const int incl = wave_inclusive_sum(mine);
+    if (lane == WAVE - 1) s_tmp[w] = incl;
+    __syncthreads();
+    int run = incl - mine, grand = 0;
+    for (int i = 0; i < NW; ++i) {
+        if (i < w) run += s_tmp[i];
+        grand += s_tmp[i];
+    }
+    for (int e = e0; e < e1; ++e) {
+        const int c = s_tot[e];
+        if (publisher) {
+            a.unaligned_expert[e] = c;
+            a.psum_expert[e] = run + c;
+            if (a.cumulative_stats != nullptr) atomicAdd(&a.cumulative_stats[e], c);
+            if (a.notify_host) a.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
+        }
+        s_tot[e] = run;
+        run += align_up(c, A);
+    }
+    if (publisher) {
+        for (int r = tid; r < R; r += EP_LAYOUT_THREADS) {
+            const int upto = s_psum[r], from = r ? s_psum[r - 1] : 0;
+            a.psum_rank[r] = upto;
+            if (a.notify_host) a.host_page[EP_HOST_RANK_OFF + r] = upto - from;
+        }
+        if (a.notify_host) {
+            __threadfence_system();
+            __syncthreads();
+            if (tid == 0) {
+                a.host_page[1] = num_rows;
+                a.host_page[2] = grand;
+                __threadfence_system();
+                __hip_atomic_store(&a.host_page[0], a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+        return;
+    }
+    const int first = b * EP_TOKENS_PER_BLOCK;
+    const int nrow = min(EP_TOKENS_PER_BLOCK, num_rows - first), n = nrow * K;
+    int src = 0;
+    if (tid < nrow) {
+        const int64_t pr = recv_packed_row(s_psum, R, a.max_tokens, first + tid);
+        s_pr[tid] = (int)pr;
+        s_at[tid] = (int)pr / a.max_tokens * El;
+        src = *(const int*)(a.packed_base + pr * a.packed_row_bytes + a.src_off);
+    }
+    __syncthreads();
+
+    // the entries of this workgroup's rows, four a thread in flight (an entry past the end re-reads the last one);
+    // row and position of an entry are carried along instead of divided out
+    const int row_step = EP_LAYOUT_THREADS / K, pos_step = EP_LAYOUT_THREADS - row_step * K;
+    int row = tid / K, pos = tid - row * K;
+    for (int i0 = tid; i0 < n; i0 += 4 * EP_LAYOUT_THREADS) {
+        int64_t id[4];
+        int rank[4], rows[4], js[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const bool in = row < nrow;
+            rows[u] = in ? row : nrow - 1;
+            js[u] = in ? pos : K - 1;
+            const int64_t pr = s_pr[rows[u]];
+            id[u] = ((const int64_t*)(a.packed_base + pr * a.packed_row_bytes + a.idx_off))[js[u]];
+            rank[u] = a.rank_box[pr * K + js[u]];
+            row += row_step;
+            pos += pos_step;
+            if (pos >= K) { pos -= K; ++row; }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (i0 + u * EP_LAYOUT_THREADS >= n) break;
+            const bool local = id[u] >= lo && id[u] < lo + El;
+            const int le = local ? (int)id[u] - lo : 0;
+            const int slot = local ? s_tot[le] + s_box[s_at[rows[u]] + le] + rank[u] : -1;
+            s_local[rows[u] * K + js[u]] = local;
+            if (first + rows[u] < a.rows_cap) a.recv_src_metadata[(int64_t)(first + rows[u]) * (K + 2) + js[u]] = slot;
+        }
+    }
+    __syncthreads();
+    // the two trailing columns: source token and last local selection (dispatch_copy_epilogue.hpp:514-522)
+    if (tid < nrow && first + tid < a.rows_cap) {
+        int master = -1;
+        for (int j = 0; j < K; ++j)
+            if (s_local[tid * K + j]) master = j;
+        int* m = a.recv_src_metadata + (int64_t)(first + tid) * (K + 2);
+        m[K] = src;
+        m[K + 1] = master;
+    }
+}
 
 // ------------------------------------------------------------------------------------------------
 // Scatter (dispatch copy epilogue): a wave task is one column part of one row (a token, or a row of the receive stream).
@@ -840,10 +982,13 @@ __device__ __forceinline__ bool scatter_row_prologue(const EpScatterArgs& a, int
         c.src_row = t;
         if (part == 0) {
             const float w = (a.topk_weights != nullptr && lane < K) ? a.topk_weights[(int64_t)t * K + lane] : 0.0f;
+            const int rank = (a.rank_box_off != 0 && lane < K) ? a.slot_map[(int64_t)t * K + lane] : 0;
             for (int j = 0; j < K; ++j) {
                 const int g = readlane(myslot, j);
                 if (g < 0) continue;
-                char* row = out_rows_of<PACK>(a, c, j) + (int64_t)g * a.out_row_bytes;
+                char* rows = out_rows_of<PACK>(a, c, j);
+                char* row = rows + (int64_t)g * a.out_row_bytes;
+                if (a.rank_box_off != 0 && lane < K) ((int*)(rows - a.buffer_off + a.rank_box_off))[(int64_t)g * K + lane] = rank;
                 if (lane < K) {
                     if (a.with_metadata) ((int64_t*)(row + a.idx_off))[lane] = e;
                     ((float*)(row + a.w_off))[lane] = w;

@@ -111,7 +111,7 @@ int64_t combine_buffer_size(int ranks, int max_tokens, int hidden, int topk) {
 // ---- code object ------------------------------------------------------------------------------
 struct Kernels {
     hipModule_t module = nullptr;
-    hipFunction_t layout_count, layout_scan, layout_assign[2][2];      // [sums the counts itself][receive side]
+    hipFunction_t layout_count, layout_scan, layout_place, layout_assign[2][2];      // [sums the counts itself][receive side]
     hipFunction_t scatter_copy, scatter_quant, scatter_quant_sw, sf_transpose;
     hipFunction_t scatter_copy_pack, scatter_quant_pack, scatter_quant_sw_pack;
     hipFunction_t combine[3][5];     // [mode][generic, k2, k4, k6, k8]
@@ -178,6 +178,7 @@ void load_kernels(const char* dir) {
     auto get = [&](hipFunction_t& fn, const char* name) { HIP_CHECK(hipModuleGetFunction(&fn, m, name)); };
     get(g_k.layout_count, "ep_layout_count");
     get(g_k.layout_scan, "ep_layout_scan");
+    get(g_k.layout_place, "ep_layout_place");
     get(g_k.layout_assign[0][0], "ep_layout_assign");
     get(g_k.layout_assign[1][0], "ep_layout_assign_fold");
     get(g_k.layout_assign[0][1], "ep_layout_assign_recv");
@@ -256,6 +257,7 @@ struct ep_buffer {
         int* slot_map = nullptr;
         int* tok_row = nullptr;
         bool notified = false;
+        bool ships_ranks = false;   // more than one partition: the send sides leave counts and ranks in the receivers' boxes
         bool recv_done = false;     // more than one partition: the receive-side layout has been enqueued
     } last;
 
@@ -278,33 +280,33 @@ unsigned layout_count_lds(int E, int R, int K) {
     return (unsigned)(E + R + R + EP_LAYOUT_THREADS / 64) * sizeof(int) + layout_key_bytes(K);
 }
 // (cnt_stride > 0: the assignment sums the count rows itself and needs two rows of ints where the partial sums meet)
-unsigned layout_assign_lds(int E, int R, int K, int cnt_stride) {
+unsigned layout_assign_lds(int E, int R, int K, int count_experts, int cnt_stride) {
     const unsigned nw = EP_LAYOUT_THREADS / 64;
-    return (unsigned)(E / R + R + nw * (E + R) + nw + 1 + R + nw + 2 * cnt_stride) * sizeof(int) + layout_key_bytes(K);
+    return (unsigned)(count_experts + R + nw * (E + R) + nw + 1 + R + nw + 2 * cnt_stride) * sizeof(int) + layout_key_bytes(K);
 }
 
 // The layout pass: per-block histograms, then the slot assignment.  One block needs no histogram pass; up
 // to g_fold_max_blocks blocks the assignment kernel sums the histograms of the blocks before it itself;
 // beyond that a scan kernel turns them into prefixes first.
 void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
-    const int E = la.num_experts, R = la.num_ranks, K = la.num_topk;
+    const int E = la.num_experts, R = la.num_ranks, K = la.num_topk, C = la.count_experts;
     // (the few shapes with more count columns than the summing instance has threads for, or whose LDS would not hold
     //  the rows where its sums meet, take the scan kernel at any size)
     // (what the summing costs is rows a thread: blocks x column groups of 8 / threads.  The limit is quoted in blocks at
     //  the headline's 264 columns, 33 groups; narrower rows, as the 40 columns of an EP32 partition, sum that many more)
     const bool fold = (int64_t)num_blocks * (la.cnt_stride / 8) <= (int64_t)g_fold_max_blocks * 33 and
-                      la.cnt_stride <= 8 * EP_LAYOUT_THREADS and layout_assign_lds(E, R, K, la.cnt_stride) <= 64 * 1024;
+                      la.cnt_stride <= 8 * EP_LAYOUT_THREADS and layout_assign_lds(E, R, K, C, la.cnt_stride) <= 64 * 1024;
     // a few blocks of one partition (send side): the slot assignment counts the ids of all blocks itself, a launch less
     // (two histograms of El + R ints and a byte a token on top of its LDS)
     const unsigned recount_extra = (unsigned)(2 * (E / R + R)) * sizeof(int) + (unsigned)num_blocks * EP_TOKENS_PER_BLOCK;
     const bool recount = R == 1 and not la.recv_mode and not la.send_only and num_blocks >= 2 and
                          (int64_t)num_blocks * K <= std::min(g_recount_limit.load(), 2 * EP_RECOUNT_DEPTH) and
-                         layout_assign_lds(E, R, K, 0) + recount_extra <= 64 * 1024;
+                         layout_assign_lds(E, R, K, C, 0) + recount_extra <= 64 * 1024;
     la.scan_mode = num_blocks == 1 ? EP_LAYOUT_SINGLE
                    : recount       ? EP_LAYOUT_RECOUNTED
                    : fold          ? EP_LAYOUT_FOLDED
                                    : EP_LAYOUT_SCANNED;
-    const unsigned smem_assign = layout_assign_lds(E, R, K, la.scan_mode == EP_LAYOUT_FOLDED ? la.cnt_stride : 0) +
+    const unsigned smem_assign = layout_assign_lds(E, R, K, C, la.scan_mode == EP_LAYOUT_FOLDED ? la.cnt_stride : 0) +
                                  (la.scan_mode == EP_LAYOUT_RECOUNTED ? recount_extra : 0u);
     EP_HOST_ASSERT(smem_assign <= 64 * 1024);
     if (la.scan_mode == EP_LAYOUT_FOLDED or la.scan_mode == EP_LAYOUT_SCANNED)
@@ -314,6 +316,37 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
     // (one workgroup more than blocks: it publishes the totals and ranks nothing)
     launch(g_k.layout_assign[la.scan_mode == EP_LAYOUT_FOLDED][la.recv_mode != 0], (unsigned)num_blocks + 1u, EP_LAYOUT_THREADS,
            smem_assign, stream, la);
+}
+
+unsigned layout_place_lds(int E, int R, int K) {
+    const unsigned nw = EP_LAYOUT_THREADS / 64;
+    return (unsigned)(E + E / R + nw + R + nw + 2 * EP_TOKENS_PER_BLOCK) * sizeof(int) + EP_TOKENS_PER_BLOCK * K;
+}
+
+// Boxes of a connected partition's workspace, behind its header, at the same place in every arena of the node: counts
+// per source and local expert [R][El], then per packed row the ranks of its entries inside their source [R * max_tokens][K].
+struct RankBoxes {
+    int64_t count_off = 0, rank_off = 0, end = EP_WS_HEADER_BYTES;
+    bool used = false;
+};
+// Every partition of a node comes to the same answer: only what all of them agree on goes in.  Without room for the boxes
+// beside the send side's scratch of max_tokens tokens (32 partitions of 16384 tokens at top-6 fit), or for the counters
+// of all experts in LDS, the receive side counts and ranks itself.
+RankBoxes rank_boxes(const ep_buffer* b, int max_tokens, int K, int E) {
+    RankBoxes x;
+    const int R = b->num_ranks;
+    if (R == 1 or not b->connected) return x;
+    auto a256 = [](int64_t n) { return align_up(std::max<int64_t>(n, 1), 256); };
+    const int64_t W = align_up(E + R, 8), blocks = std::max<int64_t>(1, ceil_div(max_tokens, EP_TOKENS_PER_BLOCK));
+    const int64_t counts = a256(4 * (int64_t)E), ranks = a256(4 * (int64_t)R * max_tokens * K);
+    const int64_t scratch = a256(4 * W) + a256(4 * blocks * W) + a256(4 * (int64_t)max_tokens * K);
+    if (EP_WS_HEADER_BYTES + counts + ranks + scratch > b->workspace_bytes) return x;
+    if (layout_assign_lds(E, R, K, E, 0) > 64 * 1024 or layout_place_lds(E, R, K) > 64 * 1024) return x;
+    x.count_off = EP_WS_HEADER_BYTES;
+    x.rank_off = x.count_off + counts;
+    x.end = x.rank_off + ranks;
+    x.used = true;
+    return x;
 }
 
 void write_peer_table(ep_buffer* b, const std::vector<char*>& arenas) {
@@ -667,6 +700,8 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         EP_HOST_ASSERT(unaligned.dtype == EP_DTYPE_I32);
         EP_HOST_ASSERT(a.dst_buffer_slot_idx.dtype == EP_DTYPE_I32 and a.dst_gsge_idx.dtype == EP_DTYPE_I32);
 
+        const RankBoxes boxes = cached_mode ? RankBoxes{} : rank_boxes(b, a.num_max_tokens_per_rank, num_topk, a.num_experts);
+        int* rank_map = nullptr;
         // geometry of the packed rows of the partition-major regions (only materialised when R > 1)
         const PackedToken pk = packed_token(hidden * packed_elem, packed_sf * 2, num_topk, not cached_mode);
         auto launch_pack = [&]() {
@@ -708,6 +743,8 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
             sa.region_by_source = b->connected ? 1 : 0;
             sa.num_ranks = num_ranks;
             sa.pack_sf_off = pk.sf_off;
+            sa.slot_map = rank_map;
+            sa.rank_box_off = boxes.used ? boxes.rank_off : 0;
             sa.vecs_per_lane = 1;
             sa.num_parts = (int)std::max<int64_t>(1, a.fused_fp8_quant ? ceil_div(hidden, 512) : ceil_div(sa.copy_bytes, 1024));
             sa.num_row_blocks = (int)ceil_div((int64_t)num_tokens * sa.num_parts, EP_ROWS_PER_BLOCK);
@@ -734,20 +771,22 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         const int E = a.num_experts, R = num_ranks, K = num_topk;
         const int num_blocks = std::max<int>(1, (int)ceil_div(num_tokens, EP_TOKENS_PER_BLOCK));
         int* ws = (int*)b->workspace();
-        int64_t off = EP_WS_HEADER_BYTES / sizeof(int);
+        int64_t off = boxes.end / sizeof(int);
         auto carve = [&](int64_t n) {
             int* p = ws + off;
             off += align_up(std::max<int64_t>(n, 1), 64);
             return p;
         };
         EpLayoutArgs la{};
-        la.cnt_stride = (int)align_up(E / R + R, 8);
+        la.count_experts = boxes.used ? E : E / R;
+        la.count_lo = boxes.used ? 0 : b->rank_idx * (E / R);
+        la.count_box_off = boxes.used ? boxes.count_off : 0;
+        la.cnt_stride = (int)align_up(la.count_experts + R, 8);
         la.col_total = carve(la.cnt_stride);
         la.blk_cnt = carve((int64_t)num_blocks * la.cnt_stride);
-        if (R == 1) {
-            la.slot_map = carve((int64_t)num_tokens * K);
-            la.tok_row = carve(num_tokens);
-        }
+        if (R == 1 or boxes.used) la.slot_map = carve((int64_t)num_tokens * K);
+        if (R == 1) la.tok_row = carve(num_tokens);
+        rank_map = la.slot_map;
         if (b->is_static and off * (int64_t)sizeof(int) > b->workspace_bytes)
             throw EpError{format("Assertion exception (%s:%d): the layout scratch of %d tokens x top-%d over %d experts (%lld bytes) "
                                  "exceeds the library's static scratch of %lld bytes", __FILE_NAME__, __LINE__, num_tokens, K, E,
@@ -792,6 +831,7 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         b->last.max_tokens = a.num_max_tokens_per_rank;
         b->last.slot_map = la.slot_map;
         b->last.tok_row = la.tok_row;
+        b->last.ships_ranks = boxes.used;
         b->last.notified = do_cpu_sync and R == 1;
         b->last.recv_done = false;
     });
@@ -854,10 +894,19 @@ int ep_dispatch_recv_launch(ep_buffer_t* b, const ep_dispatch_recv_args_t* pa) {
             off += align_up(std::max<int64_t>(n, 1), 64);
             return p;
         };
+        const RankBoxes boxes = rank_boxes(b, a.num_max_tokens_per_rank, K, E);
+        EP_HOST_ASSERT(boxes.used == b->last.ships_ranks and "the node is connected as it was at the dispatch launch");
         EpLayoutArgs la{};
+        la.count_experts = El;
+        la.count_lo = b->rank_idx * El;
         la.cnt_stride = (int)align_up(E / R + R, 8);
-        la.col_total = carve(la.cnt_stride);
-        la.blk_cnt = carve((int64_t)num_blocks * la.cnt_stride);
+        if (boxes.used) {
+            la.count_box = (const int*)(b->workspace() + boxes.count_off);
+            la.rank_box = (const int*)(b->workspace() + boxes.rank_off);
+        } else {
+            la.col_total = carve(la.cnt_stride);
+            la.blk_cnt = carve((int64_t)num_blocks * la.cnt_stride);
+        }
         EP_HOST_ASSERT(off * (int64_t)sizeof(int) <= b->workspace_bytes and "layout scratch of the receive stream fits the workspace");
         la.recv_mode = 1;
         la.num_tokens = (int)rows_bound;
@@ -885,7 +934,10 @@ int ep_dispatch_recv_launch(ep_buffer_t* b, const ep_dispatch_recv_args_t* pa) {
         la.src_off = pk.src_off;
         la.recv_src_metadata = (int*)meta.data;
         la.rows_cap = (int)std::min<int64_t>(meta.size[0], INT32_MAX);
-        launch_layout(la, num_blocks, a.stream);
+        if (boxes.used)
+            launch(g_k.layout_place, (unsigned)num_blocks + 1u, EP_LAYOUT_THREADS, layout_place_lds(E, R, K), a.stream, la);
+        else
+            launch_layout(la, num_blocks, a.stream);
         b->last.recv_done = true;
         b->last.notified = a.do_cpu_sync != 0;
     });

@@ -195,6 +195,43 @@ def test_node_dispatch_combine(R, max_tokens, H, E, K, A, masked, mode, do_cpu_s
         b.destroy()
 
 
+@pytest.mark.parametrize('R,max_tokens,Ts,E,K', [
+    (2, 128, [128, 127], 16, 8),            # one block of tokens a partition, receive streams of one block and a row
+    (4, 129, [129, 1, 128, 0], 8, 3),       # sources of one and of no token
+    (2, 600, [600, 511], 12, 1),            # a single selection: several blocks on both sides
+    (16, 300, [300 - 9 * r for r in range(16)], 2048, 4),   # more count columns than the send side sums itself
+    (3, 2500, [2500, 2049, 2304], 384, 7),  # more entries a workgroup than one round of four a thread
+    (2, 70000, [300, 129], 40, 32),         # the rank box does not fit the workspace: counted and ranked on arrival
+])
+def test_node_receive_layout(R, max_tokens, Ts, E, K):
+    """Slots out of the shipped counts and ranks, or counted on arrival: the handles of the oracle either way."""
+    H, A = 32, 8
+    bufs = make_node(R, max_tokens, H, K, False)
+    xs = [make_tokens(T, H, seed=r) if T else torch.empty((0, H), dtype=torch.bfloat16) for r, T in enumerate(Ts)]
+    routing = [make_routing(T, E, K, seed=r + 3, masked=0.1) if T else (torch.empty((0, K), dtype=torch.int64),
+                                                                        torch.empty((0, K), dtype=torch.float32))
+               for r, T in enumerate(Ts)]
+    topks, ws = [t.clone() for t, _ in routing], [w for _, w in routing]
+    if K > 2:
+        topks[0][0, 1] = topks[0][0, 0]         # an expert selected twice
+    rows = [bf16_bits(x).view(np.uint8).reshape(x.size(0), H * 2) for x in xs]
+    _, want = oracle_dispatch(rows, [None] * R, [t.numpy() for t in topks], [w.numpy() for w in ws], E, R, A, max_tokens)
+    for _ in range(2):                          # the second time over what the first left in the boxes
+        outs = dispatch_all(bufs, [x.to(DEV) for x in xs], [t.to(DEV) for t in topks], [w.to(DEV) for w in ws],
+                            num_experts=E, num_max_tokens_per_rank=max_tokens, expert_alignment=A, do_expand=True,
+                            do_zero_padding=True)
+        torch.cuda.synchronize()
+        for r, (rx, _, rw, handle) in enumerate(outs):
+            lay = want[r]['lay']
+            for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert',
+                         'num_unaligned_recv_tokens_per_expert', 'recv_src_metadata'):
+                assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (r, name)
+            assert np.array_equal(rx.view(torch.uint8).cpu().numpy().reshape(rx.size(0), H * 2), want[r]['x'])
+            assert np.array_equal(rw.cpu().numpy().view(np.uint32), want[r]['w'].view(np.uint32))
+    for b in bufs:
+        b.destroy()
+
+
 def test_node_reproduces_the_reference_dispatch_vectors():
     """tests/golden/dispatch_golden_w2.npz: inputs of both ranks and what refs.dispatch gave each of them
     (received rows in source order, local expert ids, weights, source tokens, per-source counts)."""
