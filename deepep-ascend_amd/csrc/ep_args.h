@@ -43,6 +43,14 @@
 #define EP_HOST_RANK_OFF 16
 #define EP_HOST_EXPERT_OFF (16 + EP_MAX_RANKS)
 #define EP_HOST_PAGE_INTS (16 + EP_MAX_RANKS + EP_MAX_EXPERTS)
+// Behind it, with several partitions: two slots (dispatches alternate) that the send sides of a node fill:
+//   [source][El] entries per local expert, then per source the rows it sent here, then per source its sequence number
+//   (written last, release at system scope)
+#define EP_HOST_BOX_ROWS_OFF EP_MAX_EXPERTS
+#define EP_HOST_BOX_SEQ_OFF (EP_HOST_BOX_ROWS_OFF + EP_MAX_RANKS)
+#define EP_HOST_BOX_INTS (EP_HOST_BOX_SEQ_OFF + EP_MAX_RANKS)
+// Workspace of a connected partition, behind the header: device address of every partition's host boxes.
+#define EP_WS_HOST_BOXES_BYTES (8 * EP_MAX_RANKS)
 
 struct EpLayoutArgs {
     const int64_t* topk_idx;      // [T, K]
@@ -85,6 +93,8 @@ struct EpLayoutArgs {
     int connected;                // the peers are arenas of their own (a node), not this arena again
     int64_t count_box_off;        // byte offset in every arena of the count box [R sources][El]: entries per expert; 0: the
                                   //   send side ships neither counts nor ranks (the receive side counts and ranks itself)
+    int* const* host_boxes;       // [R] slot of this dispatch in every partition's host boxes (send side), or null: the
+    int64_t host_box_slot;        //   hosts of the node get their counts straight from the send sides; offset of the slot
     const int* count_box;         // this partition's count box (receive side)
     const int* rank_box;          // [R * max_tokens, K]  per packed row: what its source ranked (receive side)
 };

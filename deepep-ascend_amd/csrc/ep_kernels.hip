@@ -612,8 +612,9 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
                 // slots are the receivers' business: ranks count from 0, and the receivers get the counts they need
                 // to place them (a partition that is not connected to a node ships nothing)
                 if (publisher && a.count_box_off != 0) {
-                    const int r = e / a.experts_per_rank;
-                    ((int*)(a.peer_arenas[r] + a.count_box_off))[a.rank_idx * a.experts_per_rank + (e - r * a.experts_per_rank)] = c;
+                    const int r = e / a.experts_per_rank, at = a.rank_idx * a.experts_per_rank + (e - r * a.experts_per_rank);
+                    ((int*)(a.peer_arenas[r] + a.count_box_off))[at] = c;
+                    if (a.host_boxes != nullptr) a.host_boxes[r][a.host_box_slot + at] = c;
                 }
                 s_start[e] = 0;
                 continue;
@@ -629,6 +630,18 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
         for (int r = tid; r < R; r += blockDim.x)
             if (a.connected || r == a.rank_idx)
                 ((int*)(a.peer_arenas[r] + EP_WS_INBOX_OFF))[a.rank_idx] = min(s_tot[El + r], a.max_tokens);
+        if (a.host_boxes != nullptr) {
+            // the hosts' copies: a receiver's host then sizes its outputs without waiting for its receive side, which
+            // in a stream of phases comes behind the copies of the partitions before it (eight partitions of 2048 tokens:
+            // 18-21 us of idle GPU a partition, all phases 1436 -> 1384 us)
+            for (int r = tid; r < R; r += blockDim.x)
+                a.host_boxes[r][a.host_box_slot + EP_HOST_BOX_ROWS_OFF + a.rank_idx] = min(s_tot[El + r], a.max_tokens);
+            __threadfence_system();
+            __syncthreads();
+            for (int r = tid; r < R; r += blockDim.x)
+                __hip_atomic_store(&a.host_boxes[r][a.host_box_slot + EP_HOST_BOX_SEQ_OFF + a.rank_idx], a.seq, __ATOMIC_RELEASE,
+                                   __HIP_MEMORY_SCOPE_SYSTEM);
+        }
     }
     if (publisher && !a.send_only) {
         // one partition: the receive stream is this partition's own routed tokens; several: the rows counted

@@ -258,6 +258,9 @@ struct ep_buffer {
         int* tok_row = nullptr;
         bool notified = false;
         bool ships_ranks = false;   // more than one partition: the send sides leave counts and ranks in the receivers' boxes
+        bool notifies_peers = false;// ... and their counts in the receivers' host boxes
+        bool host_boxes = false;    // this partition's host counts come from its host boxes, filled by the send sides
+        int send_seq = 0;           // the sequence number the sources left there
         bool recv_done = false;     // more than one partition: the receive-side layout has been enqueued
     } last;
 
@@ -328,6 +331,7 @@ unsigned layout_place_lds(int E, int R, int K) {
 struct RankBoxes {
     int64_t count_off = 0, rank_off = 0, end = EP_WS_HEADER_BYTES;
     bool used = false;
+    static constexpr int64_t kBegin = EP_WS_HEADER_BYTES + EP_WS_HOST_BOXES_BYTES;
 };
 // Every partition of a node comes to the same answer: only what all of them agree on goes in.  Without room for the boxes
 // beside the send side's scratch of max_tokens tokens (32 partitions of 16384 tokens at top-6 fit), or for the counters
@@ -336,13 +340,14 @@ RankBoxes rank_boxes(const ep_buffer* b, int max_tokens, int K, int E) {
     RankBoxes x;
     const int R = b->num_ranks;
     if (R == 1 or not b->connected) return x;
+    x.end = RankBoxes::kBegin;
     auto a256 = [](int64_t n) { return align_up(std::max<int64_t>(n, 1), 256); };
     const int64_t W = align_up(E + R, 8), blocks = std::max<int64_t>(1, ceil_div(max_tokens, EP_TOKENS_PER_BLOCK));
     const int64_t counts = a256(4 * (int64_t)E), ranks = a256(4 * (int64_t)R * max_tokens * K);
     const int64_t scratch = a256(4 * W) + a256(4 * blocks * W) + a256(4 * (int64_t)max_tokens * K);
-    if (EP_WS_HEADER_BYTES + counts + ranks + scratch > b->workspace_bytes) return x;
+    if (RankBoxes::kBegin + counts + ranks + scratch > b->workspace_bytes) return x;
     if (layout_assign_lds(E, R, K, E, 0) > 64 * 1024 or layout_place_lds(E, R, K) > 64 * 1024) return x;
-    x.count_off = EP_WS_HEADER_BYTES;
+    x.count_off = RankBoxes::kBegin;
     x.rank_off = x.count_off + counts;
     x.end = x.rank_off + ranks;
     x.used = true;
@@ -507,8 +512,9 @@ int ep_buffer_create(int rank_idx, int num_ranks, int64_t num_bytes, int64_t num
             const int64_t total = kWorkspaceBytes + num_bytes + num_lb_bytes;
             HIP_CHECK(hipMalloc((void**)&b->arena, (size_t)total));
             HIP_CHECK(hipMemset(b->arena, 0, (size_t)total));
-            HIP_CHECK(hipHostMalloc((void**)&b->host_page, EP_HOST_PAGE_INTS * sizeof(int), hipHostMallocMapped));
-            memset(b->host_page, 0, EP_HOST_PAGE_INTS * sizeof(int));
+            const size_t page_bytes = (EP_HOST_PAGE_INTS + (num_ranks > 1 ? 2 * EP_HOST_BOX_INTS : 0)) * sizeof(int);
+            HIP_CHECK(hipHostMalloc((void**)&b->host_page, page_bytes, hipHostMallocMapped));
+            memset(b->host_page, 0, page_bytes);
             HIP_CHECK(hipHostGetDevicePointer((void**)&b->host_page_dev, b->host_page, 0));
             write_peer_table(b, std::vector<char*>(num_ranks, b->arena));    // not connected: every peer is this arena
             HIP_CHECK(hipDeviceSynchronize());
@@ -534,8 +540,12 @@ int ep_buffer_connect(ep_buffer_t** bufs, int n) {
             arenas[i] = bufs[i]->arena;
         }
         HIP_CHECK(hipDeviceSynchronize());
+        std::vector<int*> boxes(EP_MAX_RANKS, nullptr);
+        for (int i = 0; i < n; ++i) boxes[i] = bufs[i]->host_page_dev + EP_HOST_PAGE_INTS;
         for (int i = 0; i < n; ++i) {
             write_peer_table(bufs[i], arenas);
+            HIP_CHECK(hipMemcpy(bufs[i]->arena + EP_WS_HEADER_BYTES, boxes.data(), EP_WS_HOST_BOXES_BYTES, hipMemcpyHostToDevice));
+            memset(bufs[i]->host_page + EP_HOST_PAGE_INTS, 0, 2 * EP_HOST_BOX_INTS * sizeof(int));     // (a former node's counts)
             bufs[i]->connected = true;
             bufs[i]->peers.assign(bufs, bufs + n);
         }
@@ -808,8 +818,15 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         la.max_tokens = a.num_max_tokens_per_rank;
         la.experts_per_rank = num_experts_per_rank;
         la.num_blocks = num_blocks;
-        la.seq = R == 1 ? ++b->seq : 0;
+        la.seq = R == 1 ? ++b->seq : (int)b->num_sends;
         la.notify_host = do_cpu_sync and R == 1 ? 1 : 0;
+        // a node in this process: the counts go to every receiver's host as well (arenas that were only mapped here
+        // have no host pages this process knows: their counts come from the receive side)
+        const bool notify_peers = boxes.used and do_cpu_sync and not b->peers.empty();
+        if (notify_peers) {
+            la.host_boxes = (int* const*)(b->workspace() + EP_WS_HEADER_BYTES);
+            la.host_box_slot = (b->num_sends & 1) * EP_HOST_BOX_INTS;
+        }
         la.dst_buffer_slot_idx = (int*)a.dst_buffer_slot_idx.data;
         la.dst_gsge_idx = (int*)a.dst_gsge_idx.data;
         la.psum_rank = (int*)psum_rank.data;
@@ -832,6 +849,8 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         b->last.slot_map = la.slot_map;
         b->last.tok_row = la.tok_row;
         b->last.ships_ranks = boxes.used;
+        b->last.notifies_peers = notify_peers;
+        b->last.host_boxes = false;
         b->last.notified = do_cpu_sync and R == 1;
         b->last.recv_done = false;
     });
@@ -888,13 +907,13 @@ int ep_dispatch_recv_launch(ep_buffer_t* b, const ep_dispatch_recv_args_t* pa) {
 
         const int num_blocks = std::max<int>(1, (int)ceil_div(rows_bound, EP_TOKENS_PER_BLOCK));
         int* ws = (int*)b->workspace();
-        int64_t off = EP_WS_HEADER_BYTES / sizeof(int);
+        const RankBoxes boxes = rank_boxes(b, a.num_max_tokens_per_rank, K, E);
+        int64_t off = boxes.end / sizeof(int);
         auto carve = [&](int64_t n) {
             int* p = ws + off;
             off += align_up(std::max<int64_t>(n, 1), 64);
             return p;
         };
-        const RankBoxes boxes = rank_boxes(b, a.num_max_tokens_per_rank, K, E);
         EP_HOST_ASSERT(boxes.used == b->last.ships_ranks and "the node is connected as it was at the dispatch launch");
         EpLayoutArgs la{};
         la.count_experts = El;
@@ -918,8 +937,11 @@ int ep_dispatch_recv_launch(ep_buffer_t* b, const ep_dispatch_recv_args_t* pa) {
         la.max_tokens = a.num_max_tokens_per_rank;
         la.experts_per_rank = El;
         la.num_blocks = num_blocks;
+        // every source has left its counts with this partition's host (or will, before this launch runs)
+        bool told = boxes.used and not b->peers.empty();
+        for (const ep_buffer* p : b->peers) told = told and p->last.valid and p->last.notifies_peers and p->num_sends == b->num_sends;
         la.seq = ++b->seq;
-        la.notify_host = a.do_cpu_sync ? 1 : 0;
+        la.notify_host = a.do_cpu_sync and not told ? 1 : 0;
         la.psum_rank = (int*)psum_rank.data;
         la.psum_expert = (int*)psum_expert.data;
         la.unaligned_expert = (int*)unaligned.data;
@@ -940,6 +962,8 @@ int ep_dispatch_recv_launch(ep_buffer_t* b, const ep_dispatch_recv_args_t* pa) {
             launch_layout(la, num_blocks, a.stream);
         b->last.recv_done = true;
         b->last.notified = a.do_cpu_sync != 0;
+        b->last.host_boxes = a.do_cpu_sync != 0 and told;
+        b->last.send_seq = (int)b->num_sends;
     });
 }
 
@@ -950,6 +974,28 @@ int ep_dispatch_wait_counts(ep_buffer_t* b, int* num_recv_tokens, int* num_expan
         EP_HOST_ASSERT(b->last.notified and "the last dispatch was launched with do_cpu_sync (nothing else publishes the counts)");
         const auto deadline = std::chrono::steady_clock::now() + std::chrono::seconds(b->cpu_timeout_secs);
         volatile int* page = b->host_page;
+        if (b->last.host_boxes) {
+            // sum what the sources left here; the host does not wait for this partition's own receive side
+            const int R = b->num_ranks, El = b->last.num_experts / R;
+            volatile int* box = page + EP_HOST_PAGE_INTS + (b->last.send_seq & 1) * EP_HOST_BOX_INTS;
+            int rows = 0, expanded = 0;
+            for (int s = 0; s < R; ++s) {
+                while (__atomic_load_n(&box[EP_HOST_BOX_SEQ_OFF + s], __ATOMIC_ACQUIRE) != b->last.send_seq) {
+                    if (std::chrono::steady_clock::now() >= deadline) EP_HOST_UNREACHABLE("reduction timeout");
+                }
+                rows += box[EP_HOST_BOX_ROWS_OFF + s];
+            }
+            for (int e = 0; e < El; ++e) {
+                int count = 0;
+                for (int s = 0; s < R; ++s) count += box[s * El + e];
+                const int aligned = (int)align_up(count, b->last.alignment);
+                if (per_expert != nullptr) per_expert[e] = aligned;
+                expanded += aligned;
+            }
+            if (num_recv_tokens != nullptr) *num_recv_tokens = rows;
+            if (num_expanded_tokens != nullptr) *num_expanded_tokens = expanded;
+            return;
+        }
         while (__atomic_load_n(&page[0], __ATOMIC_ACQUIRE) != b->seq) {
             if (std::chrono::steady_clock::now() >= deadline) EP_HOST_UNREACHABLE("reduction timeout");
         }

@@ -216,13 +216,22 @@ def test_node_receive_layout(R, max_tokens, Ts, E, K):
         topks[0][0, 1] = topks[0][0, 0]         # an expert selected twice
     rows = [bf16_bits(x).view(np.uint8).reshape(x.size(0), H * 2) for x in xs]
     _, want = oracle_dispatch(rows, [None] * R, [t.numpy() for t in topks], [w.numpy() for w in ws], E, R, A, max_tokens)
-    for _ in range(2):                          # the second time over what the first left in the boxes
-        outs = dispatch_all(bufs, [x.to(DEV) for x in xs], [t.to(DEV) for t in topks], [w.to(DEV) for w in ws],
-                            num_experts=E, num_max_tokens_per_rank=max_tokens, expert_alignment=A, do_expand=True,
-                            do_zero_padding=True)
+    # again and again over what the last pass left in the boxes; the hosts get their counts from the send sides unless
+    # one of these does not publish any (the last pass)
+    for unsynced in (None, None, None, 1):
+        events = [bufs[r].dispatch(xs[r].to(DEV), topk_idx=topks[r].to(DEV), topk_weights=ws[r].to(DEV), num_experts=E,
+                                   num_max_tokens_per_rank=max_tokens, expert_alignment=A, do_expand=True,
+                                   do_zero_padding=True, do_cpu_sync=r != unsynced, async_with_compute_stream=True,
+                                   defer_epilogue=True) for r in range(R)]
+        outs = [ev.current_stream_wait() for ev in events]
         torch.cuda.synchronize()
         for r, (rx, _, rw, handle) in enumerate(outs):
             lay = want[r]['lay']
+            if r == unsynced:
+                assert np.array_equal(handle.recv_src_metadata.cpu().numpy()[:lay['num_recv_tokens']], lay['recv_src_metadata'])
+                continue
+            assert handle.num_recv_tokens == lay['num_recv_tokens']
+            assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
             for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert',
                          'num_unaligned_recv_tokens_per_expert', 'recv_src_metadata'):
                 assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (r, name)
