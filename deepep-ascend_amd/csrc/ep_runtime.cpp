@@ -115,6 +115,7 @@ struct Kernels {
     hipFunction_t scatter_copy, scatter_quant, scatter_quant_sw, sf_transpose;
     hipFunction_t scatter_copy_pack, scatter_quant_pack, scatter_quant_sw_pack;
     hipFunction_t combine[3][5];     // [mode][generic, k2, k4, k6, k8]
+    hipFunction_t combine_odd[3];    // single partition, small launches: k3, k5, k7
     hipFunction_t fp8_selftest, quant_rows;
     int device = -1;
 };
@@ -195,6 +196,9 @@ void load_kernels(const char* dir) {
     for (int mode = 0; mode < 3; ++mode)
         for (int k = 0; k < 5; ++k)
             get(g_k.combine[mode][k], (std::string("ep_combine") + modes[mode] + ks[k]).c_str());
+    get(g_k.combine_odd[0], "ep_combine_k3");
+    get(g_k.combine_odd[1], "ep_combine_k5");
+    get(g_k.combine_odd[2], "ep_combine_k7");
     get(g_k.fp8_selftest, "ep_fp8_selftest");
     get(g_k.quant_rows, "ep_quant_rows");
     g_k.module = m;
@@ -1328,7 +1332,12 @@ int ep_combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase) {
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROWS_PER_BLOCK);
             const unsigned grid = (unsigned)ca.num_row_blocks + (unsigned)ceil_div(num_combined_tokens, EP_ROW_THREADS);
             if (grid == 0) return;
-            launch(g_k.combine[EP_COMBINE_FUSED][kidx], grid, EP_ROW_THREADS, combine_lds_cap(K + (ca.bias_0 != nullptr) + (ca.bias_1 != nullptr), kidx != 0, ca.num_row_blocks, hidden), a.stream, ca);
+            // odd top-k: a launch of less than a row block a CU waits for its trips to memory and takes the unrolled kernel;
+            // at 765 blocks the two are level (top-3 / 5 / 7: 9.5 / 11.2 / 13.0 us against 9.6 / 11.3 / 13.1 of the general
+            // one), beyond, the general one's shorter bursts win (1787 blocks: 14.9 / 19.7 / 23.8 us against 16.5 / 20.4 / 25.0)
+            const bool odd = ca.num_row_blocks < 256 and (K == 3 or K == 5 or K == 7);
+            const unsigned cap = combine_lds_cap(K + (ca.bias_0 != nullptr) + (ca.bias_1 != nullptr), kidx != 0, ca.num_row_blocks, hidden);
+            launch(odd ? g_k.combine_odd[(K - 3) / 2] : g_k.combine[EP_COMBINE_FUSED][kidx], grid, EP_ROW_THREADS, cap, a.stream, ca);
         } else {
             check_peers(b, [&](const ep_buffer& p) { return p.num_partials >= b->num_partials; },
                         "its owner-side reduce (phase 0) comes before any token-side reduce");

@@ -530,3 +530,25 @@ def test_gpu_quantiser_helper_matches_the_oracle(T, H):
     back = de.utils.math.per_token_cast_back(vq, vs).float()
     ref = wide[:, :H].float()
     assert ((back - ref).abs() <= 0.07 * ref.abs().amax(dim=1, keepdim=True) + 1e-6).all()
+
+
+@pytest.mark.parametrize('T,H,K', [(1, 8, 3), (61, 1032, 3), (129, 5120, 5), (33, 7168, 7), (64, 1016, 7)])
+def test_odd_topk_combine_of_small_launches(T, H, K):
+    """The unrolled kernels of top-3, 5 and 7: missing selections, biases, both sides of a 1024-channel part."""
+    E, A = 16, 1
+    topk, w = make_routing(T, E, K, seed=T, masked=0.3)
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
+    buf = _buffer(T, H, K)
+    _, _, rw, handle, _ = buf.dispatch(make_tokens(T, H).to(DEV), topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E,
+                                       num_max_tokens_per_rank=T, expert_alignment=A, do_expand=True)
+    y = make_tokens(max(1, lay['num_expanded_tokens']), H, seed=5)[:lay['num_expanded_tokens']]
+    for nbias in (0, 1, 2):
+        bias = [make_tokens(T, H, seed=6 + b) for b in range(nbias)]
+        gpu = [b.to(DEV) for b in bias]
+        cx, cw, _ = buf.combine(y.to(DEV), handle, topk_weights=rw, bias=None if nbias == 0 else gpu[0] if nbias == 1 else tuple(gpu))
+        ox, ow = O.combine_fast(y, rw.cpu(), lay['recv_src_metadata'], T, K, *bias)
+        assert np.array_equal(bf16_bits(cx), bf16_bits(ox)), nbias
+        assert torch.equal(cw.cpu(), w)
+    cx, _, _ = buf.combine(y.to(DEV), handle, topk_weights=rw, apply_weights=True)
+    assert np.array_equal(bf16_bits(cx), bf16_bits(O.combine_weighted(y, rw.cpu(), lay['recv_src_metadata'], T, K)))
+    buf.destroy()
