@@ -10,6 +10,7 @@
 //   ep_layout_place                                        receive side of a node out of the shipped counts and ranks
 //   ep_scatter_copy / ep_scatter_quant                     token (or receive-stream row) -> its expanded slots
 //   ep_scatter_copy_pack / ep_scatter_quant_pack           token -> one packed row per destination partition
+//   ep_dispatch_small_*                                    layout and copy (or pack) of a decode-size dispatch in one launch
 //   ep_sf_transpose                                        scale rows -> scale columns
 //   ep_quant_rows                                          the quantiser alone (rows in place)
 //   ep_combine_k<K> / ep_combine_generic                   K-way gather + fp32 reduce back to token order
@@ -958,6 +959,24 @@ __device__ __forceinline__ char* out_sf_of(const EpScatterArgs& a, char* rows) {
     return PACK ? rows + a.pack_sf_off : (char*)a.recv_sf;
 }
 
+// Part 0 of a packed row's task: the metadata of the row and its ranks, in every destination.  Lane j < K holds the
+// expert id, the gate weight and the rank of entry (t, j).
+__device__ __forceinline__ void pack_row_metadata(const EpScatterArgs& a, const RowCtx& c, int64_t e, float w, int rank) {
+    const int lane = lane_id(), K = a.num_topk;
+    for (int j = 0; j < K; ++j) {
+        const int g = readlane(c.myslot, j);
+        if (g < 0) continue;
+        char* rows = out_rows_of<true>(a, c, j);
+        char* row = rows + (int64_t)g * a.out_row_bytes;
+        if (a.rank_box_off != 0 && lane < K) ((int*)(rows - a.buffer_off + a.rank_box_off))[(int64_t)g * K + lane] = rank;
+        if (lane < K) {
+            if (a.with_metadata) ((int64_t*)(row + a.idx_off))[lane] = e;
+            ((float*)(row + a.w_off))[lane] = w;
+        }
+        if (a.with_metadata && lane == 0) *(int*)(row + a.src_off) = a.rank_idx * a.max_tokens + c.t;
+    }
+}
+
 // A wave task is (row, column part).  Resolves the row's token, its source row and its destination
 // rows; the task of part 0 also writes the row's small items.  Three modes:
 //   EP_SCATTER_EXPAND  rows are tokens (non-cached: slots from the slot map) or rows of the receive stream
@@ -996,18 +1015,7 @@ __device__ __forceinline__ bool scatter_row_prologue(const EpScatterArgs& a, int
         if (part == 0) {
             const float w = (a.topk_weights != nullptr && lane < K) ? a.topk_weights[(int64_t)t * K + lane] : 0.0f;
             const int rank = (a.rank_box_off != 0 && lane < K) ? a.slot_map[(int64_t)t * K + lane] : 0;
-            for (int j = 0; j < K; ++j) {
-                const int g = readlane(myslot, j);
-                if (g < 0) continue;
-                char* rows = out_rows_of<PACK>(a, c, j);
-                char* row = rows + (int64_t)g * a.out_row_bytes;
-                if (a.rank_box_off != 0 && lane < K) ((int*)(rows - a.buffer_off + a.rank_box_off))[(int64_t)g * K + lane] = rank;
-                if (lane < K) {
-                    if (a.with_metadata) ((int64_t*)(row + a.idx_off))[lane] = e;
-                    ((float*)(row + a.w_off))[lane] = w;
-                }
-                if (a.with_metadata && lane == 0) *(int*)(row + a.src_off) = a.rank_idx * a.max_tokens + t;
-            }
+            pack_row_metadata(a, c, e, w, rank);
         }
         return true;
     }
@@ -1083,11 +1091,8 @@ __device__ __forceinline__ void zero_span(char* base, int64_t nbytes, int part, 
     for (int64_t o = head + body + tid * 2; o < nbytes; o += nthreads * 2) *(unsigned short*)(base + o) = 0;
 }
 
-__device__ __forceinline__ void zero_padding_rows(const EpScatterArgs& a) {
-    const int pb = blockIdx.x - a.num_row_blocks;
-    const int e = pb / a.pad_blocks_per_expert, part = pb % a.pad_blocks_per_expert;
-    if (e >= a.num_local_experts) return;
-    const int end = a.psum_expert[e];
+// (end: one past the expert's last row)
+__device__ __forceinline__ void zero_padding_piece(const EpScatterArgs& a, int end, int part) {
     const int rows = min(align_up(end, a.expert_alignment), a.num_out_rows) - end;     // never past the outputs
     if (end < 0 || rows <= 0) return;
     zero_span((char*)a.recv_x + (int64_t)end * a.out_row_bytes, (int64_t)rows * a.out_row_bytes, part,
@@ -1096,6 +1101,41 @@ __device__ __forceinline__ void zero_padding_rows(const EpScatterArgs& a) {
         zero_span((char*)a.recv_sf + (int64_t)end * a.out_sf_row_bytes, (int64_t)rows * a.out_sf_row_bytes, 0, 1);
     if (a.recv_topk_weights != nullptr && part == a.pad_blocks_per_expert - 1)
         zero_span((char*)(a.recv_topk_weights + end), (int64_t)rows * 4, 0, 1);
+}
+__device__ __forceinline__ void zero_padding_rows(const EpScatterArgs& a) {
+    const int pb = blockIdx.x - a.num_row_blocks;
+    const int e = pb / a.pad_blocks_per_expert, part = pb % a.pad_blocks_per_expert;
+    if (e < a.num_local_experts) zero_padding_piece(a, a.psum_expert[e], part);
+}
+
+// The stores of a verbatim task: d[u] = vector (part * vecs_per_lane + u) * 64 + lane of the row; part 0 also carries the
+// scale packs of pre-quantised rows.
+template <bool PACK>
+__device__ __forceinline__ void copy_row_out(const EpScatterArgs& a, const RowCtx& c, int part, const u32x4 (&d)[4]) {
+    const int lane = lane_id(), K = a.num_topk, U = a.vecs_per_lane;
+    const int nvec = (int)(a.copy_bytes >> 4);
+    for (int j = 0; j < K; ++j) {
+        const int s = readlane(c.myslot, j);
+        if (s < 0) continue;
+        u32x4* row = (u32x4*)(out_rows_of<PACK>(a, c, j) + (int64_t)s * a.out_row_bytes);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int v = (part * U + u) * WAVE + lane;
+            if (u < U && v < nvec) stream_store<EP_SCATTER_ST_POL>(row + v, d[u]);
+        }
+    }
+    if (part == 0 && a.recv_sf != nullptr) {
+        const int P = a.num_sf_packs;
+        const char* sfrow = (const char*)a.sf + c.src_row * a.sf_token_stride_bytes;
+        for (int p = lane; p < P; p += WAVE) {
+            const unsigned short val = *(const unsigned short*)(sfrow + (int64_t)p * a.sf_pack_stride_bytes);
+            for (int j = 0; j < K; ++j) {
+                const int s = readlane(c.myslot, j);
+                if (s < 0) continue;
+                ((unsigned short*)(out_sf_of<PACK>(a, out_rows_of<PACK>(a, c, j)) + (int64_t)s * a.out_sf_row_bytes))[p] = val;
+            }
+        }
+    }
 }
 
 // Verbatim rows: BF16 payload, or FP8 payload with its 2-byte scale packs.  A task moves 1 KiB of
@@ -1111,7 +1151,6 @@ __device__ __forceinline__ void scatter_copy_body(const EpScatterArgs& a) {
     const int task = blockIdx.x * EP_ROWS_PER_BLOCK + wave_id();
     const int i = task / a.num_parts, part = task - i * a.num_parts;
     if (i >= a.num_rows_bound) return;
-    const int K = a.num_topk;
     const int nvec = (int)(a.copy_bytes >> 4);
     // a task moves vecs_per_lane KiB of the row: 1 where a row fans out to several slots, more where
     // nearly every row has a single destination and the set-up above would outweigh the copy
@@ -1139,28 +1178,7 @@ __device__ __forceinline__ void scatter_copy_body(const EpScatterArgs& a) {
                 d[u] = __builtin_nontemporal_load((const u32x4*)((const char*)a.x + c.src_row * a.x_row_bytes) + v);
         }
     }
-    for (int j = 0; j < K; ++j) {
-        const int s = readlane(c.myslot, j);
-        if (s < 0) continue;
-        u32x4* row = (u32x4*)(out_rows_of<PACK>(a, c, j) + (int64_t)s * a.out_row_bytes);
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int v = (part * U + u) * WAVE + lane;
-            if (u < U && v < nvec) stream_store<EP_SCATTER_ST_POL>(row + v, d[u]);
-        }
-    }
-    if (part == 0 && a.recv_sf != nullptr) {
-        const int P = a.num_sf_packs;
-        const char* sfrow = (const char*)a.sf + c.src_row * a.sf_token_stride_bytes;
-        for (int p = lane; p < P; p += WAVE) {
-            const unsigned short val = *(const unsigned short*)(sfrow + (int64_t)p * a.sf_pack_stride_bytes);
-            for (int j = 0; j < K; ++j) {
-                const int s = readlane(c.myslot, j);
-                if (s < 0) continue;
-                ((unsigned short*)(out_sf_of<PACK>(a, out_rows_of<PACK>(a, c, j)) + (int64_t)s * a.out_sf_row_bytes))[p] = val;
-            }
-        }
-    }
+    copy_row_out<PACK>(a, c, part, d);
 }
 
 // Fused BF16 -> e4m3fn quantisation (deep_ep/utils/math.py:30-38) + scatter.  A task owns 512
@@ -1173,31 +1191,11 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_scatter_copy_pac
     scatter_copy_body<true>(a);
 }
 
-// (LOADS = false exists for the benchmarks' calibration code object only: the same tasks and stores with a
-// made-up payload in place of the row of x.)
-template <bool HW, bool PACK, bool LOADS = true>
-__device__ __forceinline__ void scatter_quant_body(const EpScatterArgs& a) {
-    if ((int)blockIdx.x >= a.num_row_blocks) {
-        zero_padding_rows(a);
-        return;
-    }
-    const int lane = lane_id();
-    const int task = blockIdx.x * EP_ROWS_PER_BLOCK + wave_id();
-    const int i = task / a.num_parts, part = task - i * a.num_parts;
-    if (i >= a.num_rows_bound) return;
-    const int K = a.num_topk;
-    const int nvec = a.hidden >> 3;                      // 16-byte vectors of 8 BF16
-    const int v = part * WAVE + lane;
-    const bool live = v < nvec;
-    u32x4 d = {0u, 0u, 0u, 0u};
-    // the payload is fetched while the prologue looks up the slots wherever the source row is known up front
-    const int64_t guess = scatter_guess_source_row<PACK>(a, i);
-    if (live && LOADS && guess >= 0) d = __builtin_nontemporal_load((const u32x4*)((const char*)a.x + guess * a.x_row_bytes) + v);
-    RowCtx c;
-    if (!scatter_row_prologue<PACK>(a, i, part, c)) return;
-    if (live && LOADS && c.src_row != guess)
-        d = __builtin_nontemporal_load((const u32x4*)((const char*)a.x + c.src_row * a.x_row_bytes) + v);
-    if (!LOADS) d = u32x4{0x3f803f80u + (unsigned)v, 0x40004000u, 0xbf80bf80u, 0x3f003f00u};
+// Quantises the 8 channels a lane holds (vector v of the row; a 128-channel group is one DPP row of 16 lanes) and stores
+// them, and the group's scale, into every destination of the row.
+template <bool HW, bool PACK>
+__device__ __forceinline__ void quant_row_out(const EpScatterArgs& a, const RowCtx& c, int v, bool live, const u32x4& d) {
+    const int lane = lane_id(), K = a.num_topk;
     float f[8] = {bf16_lo(d.x), bf16_hi(d.x), bf16_lo(d.y), bf16_hi(d.y),
                   bf16_lo(d.z), bf16_hi(d.z), bf16_lo(d.w), bf16_hi(d.w)};
     unsigned mbits = 0u;
@@ -1220,6 +1218,33 @@ __device__ __forceinline__ void scatter_quant_body(const EpScatterArgs& a) {
     }
 }
 
+// (LOADS = false exists for the benchmarks' calibration code object only: the same tasks and stores with a
+// made-up payload in place of the row of x.)
+template <bool HW, bool PACK, bool LOADS = true>
+__device__ __forceinline__ void scatter_quant_body(const EpScatterArgs& a) {
+    if ((int)blockIdx.x >= a.num_row_blocks) {
+        zero_padding_rows(a);
+        return;
+    }
+    const int lane = lane_id();
+    const int task = blockIdx.x * EP_ROWS_PER_BLOCK + wave_id();
+    const int i = task / a.num_parts, part = task - i * a.num_parts;
+    if (i >= a.num_rows_bound) return;
+    const int nvec = a.hidden >> 3;                      // 16-byte vectors of 8 BF16
+    const int v = part * WAVE + lane;
+    const bool live = v < nvec;
+    u32x4 d = {0u, 0u, 0u, 0u};
+    // the payload is fetched while the prologue looks up the slots wherever the source row is known up front
+    const int64_t guess = scatter_guess_source_row<PACK>(a, i);
+    if (live && LOADS && guess >= 0) d = __builtin_nontemporal_load((const u32x4*)((const char*)a.x + guess * a.x_row_bytes) + v);
+    RowCtx c;
+    if (!scatter_row_prologue<PACK>(a, i, part, c)) return;
+    if (live && LOADS && c.src_row != guess)
+        d = __builtin_nontemporal_load((const u32x4*)((const char*)a.x + c.src_row * a.x_row_bytes) + v);
+    if (!LOADS) d = u32x4{0x3f803f80u + (unsigned)v, 0x40004000u, 0xbf80bf80u, 0x3f003f00u};
+    quant_row_out<HW, PACK>(a, c, v, live, d);
+}
+
 extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_scatter_quant(EpScatterArgs a) {
     scatter_quant_body<true, false>(a);
 }
@@ -1232,6 +1257,217 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_scatter_quant_pa
 extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_scatter_quant_sw_pack(EpScatterArgs a) {
     scatter_quant_body<false, true>(a);
 }
+
+// ------------------------------------------------------------------------------------------------
+// A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES entries in one launch.  Instead of a slot
+// assignment in front of the copy (a launch that one or two workgroups of the chip work at, bound by its own dependent
+// phases), every workgroup stages all ids in LDS, counts them per expert, and its waves rank the one token each of
+// them copies: the number of earlier entries with the same expert, sixteen compare-and-count steps an expert at most.
+// The payload is fetched before the ids are looked at.  Workgroup 0 publishes what the assignment's publishing workgroup
+// does, the next ones copy (or, with several partitions, pack) as the kernels above, the last zero the padding.
+// Bound by the launch, two trips to memory and the phases in LDS between them.  Assignment + copy -> this kernel (us): 32 tokens,
+// top-8 of 256, FP8 8.8 + 6.2 -> 10.1; 61 tokens x 5120, top-6 of 160, BF16 7.5 + 4.2 -> 8.2; 128 tokens, top-8, 230 MB of
+// padding 10.0 + 31.2 -> 35.3; one of eight partitions of 64 tokens 11.2 + 5.6 -> 10.7.
+// ------------------------------------------------------------------------------------------------
+template <bool QUANT, bool HW, bool PACK>
+__device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
+    extern __shared__ int smem[];
+    constexpr int NW = EP_ROW_THREADS / WAVE, CH = EP_SMALL_ENTRIES / WAVE, PER = EP_SMALL_ENTRIES / EP_ROW_THREADS;
+    const EpLayoutArgs& l = a.l;
+    const EpScatterArgs& s = a.s;
+    const int E = l.num_experts, R = l.num_ranks, K = l.num_topk, A = l.expert_alignment, El = l.experts_per_rank;
+    int* s_cnt = smem;                                  // [E] entries per expert
+    int* s_start = s_cnt + E;                           // [E] first slot of each expert (one partition)
+    unsigned* s_tok = (unsigned*)(s_start + E);         // [R][EP_TOKENS_PER_BLOCK / 32] tokens that go to a partition, a bit each
+    int* s_tmp = (int*)(s_tok + R * (EP_TOKENS_PER_BLOCK / 32));       // [NW]
+    short* s_key = (short*)(s_tmp + NW);                // [EP_SMALL_ENTRIES] expert of every entry, -1: none
+    constexpr int TW = EP_TOKENS_PER_BLOCK / 32;
+    const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
+    const int n = l.num_tokens * K;
+    const bool publisher = blockIdx.x == 0;
+    const int rb = (int)blockIdx.x - 1;
+    const bool copies = !publisher && rb < s.num_row_blocks;
+
+    // ids, then the payload of this wave's task, all in flight together
+    int64_t id[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) id[u] = l.topk_idx[min(tid + u * EP_ROW_THREADS, n - 1)];
+    const int task = copies ? rb * EP_ROWS_PER_BLOCK + w : 0;
+    const int t = task / s.num_parts, part = task - t * s.num_parts;
+    const bool works = copies && t < s.num_rows_bound;
+    const int nvec = QUANT ? s.hidden >> 3 : (int)(s.copy_bytes >> 4);
+    const int v = part * WAVE + lane;
+    const bool live = works && v < nvec;
+    u32x4 d[4];
+    d[0] = u32x4{0u, 0u, 0u, 0u};
+    if (live) d[0] = __builtin_nontemporal_load((const u32x4*)((const char*)s.x + (int64_t)t * s.x_row_bytes) + v);
+    float gate = 0.0f;
+    if (works && part == 0 && lane < K && s.topk_weights != nullptr) gate = s.topk_weights[(int64_t)t * K + lane];
+
+    for (int i = tid; i < E; i += EP_ROW_THREADS) s_cnt[i] = 0;
+    for (int i = tid; i < R * TW; i += EP_ROW_THREADS) s_tok[i] = 0u;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * EP_ROW_THREADS;
+        const bool valid = i < n && id[u] >= 0 && id[u] < E;
+        const int e = valid ? (int)id[u] : -1;
+        s_key[i] = (short)e;
+        if (valid) {
+            const int tok = i / K;
+            atomicAdd(&s_cnt[e], 1);
+            atomicOr(&s_tok[(PACK ? e / El : 0) * TW + (tok >> 5)], 1u << (tok & 31));
+        }
+    }
+    __syncthreads();
+    int grand = 0;
+    if (!PACK) {
+        // aligned exclusive scan over the experts
+        const int per = (E + EP_ROW_THREADS - 1) / EP_ROW_THREADS;
+        const int e0 = min(E, tid * per), e1 = min(E, e0 + per);
+        int mine = 0;
+        for (int e = e0; e < e1; ++e) mine += align_up(s_cnt[e], A);
+        const int incl = wave_inclusive_sum(mine);
+        if (lane == WAVE - 1) s_tmp[w] = incl;
+        __syncthreads();
+        int run = incl - mine;
+        for (int i = 0; i < NW; ++i) {
+            if (i < w) run += s_tmp[i];
+            grand += s_tmp[i];
+        }
+        for (int e = e0; e < e1; ++e) {
+            s_start[e] = run;
+            run += align_up(s_cnt[e], A);
+        }
+        __syncthreads();
+    }
+    auto tokens_to = [&](int r, int before) -> int {     // tokens below `before` that go to partition r
+        int c = 0;
+        for (int q = 0; q < TW; ++q) {
+            const int bits = min(max(before - 32 * q, 0), 32);
+            c += __popc(bits == 32 ? s_tok[r * TW + q] : s_tok[r * TW + q] & ((1u << bits) - 1u));
+        }
+        return c;
+    };
+
+    if (publisher) {
+        for (int e = tid; e < E; e += EP_ROW_THREADS) {
+            const int c = s_cnt[e];
+            if (PACK) {
+                const int r = e / El, at = l.rank_idx * El + (e - r * El);
+                if (l.count_box_off != 0) ((int*)(l.peer_arenas[r] + l.count_box_off))[at] = c;
+                if (l.host_boxes != nullptr) l.host_boxes[r][l.host_box_slot + at] = c;
+            } else {
+                l.unaligned_expert[e] = c;
+                l.psum_expert[e] = s_start[e] + c;
+                if (l.cumulative_stats != nullptr) atomicAdd(&l.cumulative_stats[e], c);
+                if (l.notify_host) l.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
+            }
+        }
+        for (int r = tid; r < R; r += EP_ROW_THREADS) {
+            const int rows = min(tokens_to(r, EP_TOKENS_PER_BLOCK), l.max_tokens);
+            if (PACK) {
+                if (l.connected || r == l.rank_idx) ((int*)(l.peer_arenas[r] + EP_WS_INBOX_OFF))[l.rank_idx] = rows;
+                if (l.host_boxes != nullptr) l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_ROWS_OFF + l.rank_idx] = rows;
+            } else {
+                l.psum_rank[r] = rows;
+                if (l.notify_host) l.host_page[EP_HOST_RANK_OFF + r] = rows;
+            }
+        }
+        if (PACK ? l.host_boxes != nullptr : l.notify_host != 0) {
+            __threadfence_system();
+            __syncthreads();
+            if (PACK) {
+                for (int r = tid; r < R; r += EP_ROW_THREADS)
+                    __hip_atomic_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_SEQ_OFF + l.rank_idx], l.seq,
+                                       __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            } else if (tid == 0) {
+                l.host_page[1] = tokens_to(0, EP_TOKENS_PER_BLOCK);
+                l.host_page[2] = grand;
+                __threadfence_system();
+                __hip_atomic_store(&l.host_page[0], l.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+        }
+        return;
+    }
+    if (!copies) {
+        const int pieces = s.num_local_experts * s.pad_blocks_per_expert;
+        for (int p = rb - s.num_row_blocks; p < pieces; p += a.num_pad_blocks) {
+            const int e = p / s.pad_blocks_per_expert;
+            zero_padding_piece(s, s_start[e] + s_cnt[e], p - e * s.pad_blocks_per_expert);
+        }
+        return;
+    }
+    if (!works) return;
+
+    // ---- rank of the token's entries: earlier entries with the same expert ----
+    const int e = lane < K ? s_key[t * K + lane] : -1;
+    const int before = t * K, chunks = (before + WAVE - 1) / WAVE;
+    int key[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int i = c * WAVE + lane;
+        key[c] = i < before ? s_key[i] : -2;            // (-2 equals no expert and no missing selection)
+    }
+    int rank = 0;
+    for (int j = 0; j < K; ++j) {
+        const int ej = readlane(e, j);
+        if (ej < 0) continue;
+        // (the same expert twice in one token: the earlier one counts too)
+        int c0 = __popcll(__ballot(e == ej) & ((1ull << j) - 1ull));
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            if (c >= chunks) break;
+            c0 += __popcll(__ballot(key[c] == ej));
+        }
+        if (lane == j) rank = c0;
+    }
+    // ---- masters: the last entry of the token for a partition; its slot there ----
+    const int r = e < 0 ? -1 : PACK ? e / El : 0;
+    bool master = r >= 0;
+    for (int jj = 1; jj < K; ++jj) {
+        const int rj = readlane(r, jj);
+        if (lane < jj && rj == r) master = false;
+    }
+    const int rslot = master ? tokens_to(r, t) : -1;
+    if (part == 0 && lane < K) {
+        l.dst_buffer_slot_idx[(int64_t)t * K + lane] = rslot;
+        l.dst_gsge_idx[(int64_t)t * K + lane] = -1;     // every copy is local: no transport descriptors
+    }
+    RowCtx c;
+    c.t = t;
+    c.src_row = t;
+    c.mybase = 0;
+    c.myslot = -1;
+    if (PACK) {
+        if (master && rslot < s.max_tokens) {
+            c.myslot = (s.region_by_source ? s.rank_idx : r) * s.max_tokens + rslot;
+            c.mybase = (uint64_t)(s.peer_arenas[r] + s.buffer_off);
+        }
+        if (part == 0) pack_row_metadata(s, c, (lane < K && e >= 0) ? e : (lane < K ? l.topk_idx[(int64_t)t * K + lane] : 0), gate, e >= 0 ? rank : -1);
+    } else {
+        const uint64_t vm = __ballot(e >= 0);
+        if (vm == 0) return;                            // a token nobody receives
+        const int slot = e >= 0 ? s_start[e] + rank : -1;
+        if (part == 0) {
+            const int last = 63 - __builtin_clzll(vm);
+            const int row = readlane(rslot, last);
+            // [slot_0 .. slot_{K-1}, src_token_global_idx, last local j]  (dispatch_copy_epilogue.hpp:514-522)
+            const int mv = lane < K ? slot : (lane == K ? s.rank_idx * s.max_tokens + t : last);
+            if (lane < K + 2 && row >= 0 && row < s.num_meta_rows) s.recv_src_metadata[(int64_t)row * (K + 2) + lane] = mv;
+        }
+        c.myslot = slot < s.num_out_rows ? slot : -1;
+        if (part == 0 && s.recv_topk_weights != nullptr && c.myslot >= 0) s.recv_topk_weights[c.myslot] = gate;
+    }
+    if (QUANT) quant_row_out<HW, PACK>(s, c, v, live, d[0]);
+    else copy_row_out<PACK>(s, c, part, d);
+}
+extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_copy(EpSmallArgs a) { dispatch_small_body<false, true, false>(a); }
+extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_quant(EpSmallArgs a) { dispatch_small_body<true, true, false>(a); }
+extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_quant_sw(EpSmallArgs a) { dispatch_small_body<true, false, false>(a); }
+extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_copy_pack(EpSmallArgs a) { dispatch_small_body<false, true, true>(a); }
+extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_quant_pack(EpSmallArgs a) { dispatch_small_body<true, true, true>(a); }
+extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_quant_sw_pack(EpSmallArgs a) { dispatch_small_body<true, false, true>(a); }
 
 // The quantiser alone (deep_ep/utils/math.py:30-38, what a caller runs before a dispatch of pre-quantised rows):
 // the arithmetic of the fused kernel above, rows written in place of being scattered.

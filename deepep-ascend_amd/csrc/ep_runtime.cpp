@@ -114,6 +114,7 @@ struct Kernels {
     hipFunction_t layout_count, layout_scan, layout_place, layout_assign[2][2];      // [sums the counts itself][receive side]
     hipFunction_t scatter_copy, scatter_quant, scatter_quant_sw, sf_transpose;
     hipFunction_t scatter_copy_pack, scatter_quant_pack, scatter_quant_sw_pack;
+    hipFunction_t small[2][3];       // [packs][copy, quant, quant_sw]
     hipFunction_t combine[3][5];     // [mode][generic, k2, k4, k6, k8]
     hipFunction_t combine_odd[3];    // single partition, small launches: k3, k5, k7
     hipFunction_t fp8_selftest, quant_rows;
@@ -190,6 +191,11 @@ void load_kernels(const char* dir) {
     get(g_k.scatter_copy_pack, "ep_scatter_copy_pack");
     get(g_k.scatter_quant_pack, "ep_scatter_quant_pack");
     get(g_k.scatter_quant_sw_pack, "ep_scatter_quant_sw_pack");
+    const char* small_names[3] = {"copy", "quant", "quant_sw"};
+    for (int i = 0; i < 3; ++i) {
+        get(g_k.small[0][i], (std::string("ep_dispatch_small_") + small_names[i]).c_str());
+        get(g_k.small[1][i], (std::string("ep_dispatch_small_") + small_names[i] + "_pack").c_str());
+    }
     get(g_k.sf_transpose, "ep_sf_transpose");
     const char* modes[3] = {"", "_partial", "_final"};
     const char* ks[5] = {"_generic", "_k2", "_k4", "_k6", "_k8"};
@@ -265,6 +271,10 @@ struct ep_buffer {
         bool notifies_peers = false;// ... and their counts in the receivers' host boxes
         bool host_boxes = false;    // this partition's host counts come from its host boxes, filled by the send sides
         int send_seq = 0;           // the sequence number the sources left there
+        bool layout_pending = false;// the layout is left to the copy launch (pending, on pending_stream)
+        EpLayoutArgs pending{};
+        void* pending_stream = nullptr;
+        bool copied = false;        // the copy launch has used it up: the workspace holds no layout to copy by again
         bool recv_done = false;     // more than one partition: the receive-side layout has been enqueued
     } last;
 
@@ -323,6 +333,24 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
     // (one workgroup more than blocks: it publishes the totals and ranks nothing)
     launch(g_k.layout_assign[la.scan_mode == EP_LAYOUT_FOLDED][la.recv_mode != 0], (unsigned)num_blocks + 1u, EP_LAYOUT_THREADS,
            smem_assign, stream, la);
+}
+
+// Decode sizes: layout and copy in one launch.
+unsigned small_lds(int E, int R) {
+    return (unsigned)(2 * E + R * (EP_TOKENS_PER_BLOCK / 32) + EP_ROW_THREADS / 64) * sizeof(int) + EP_SMALL_ENTRIES * sizeof(short);
+}
+constexpr unsigned kSmallPadBlocks = 2048;
+bool small_dispatch(int num_tokens, int K) {
+    return num_tokens > 0 and num_tokens <= EP_TOKENS_PER_BLOCK and num_tokens * K <= EP_SMALL_ENTRIES;
+}
+void launch_small(const EpLayoutArgs& la, const EpScatterArgs& sa, bool pack, bool quantise, int num_pad_blocks, void* stream) {
+    EpSmallArgs args{};
+    args.l = la;
+    args.s = sa;
+    args.num_pad_blocks = num_pad_blocks;
+    EP_HOST_ASSERT(sa.vecs_per_lane == 1);
+    launch(g_k.small[pack][quantise ? (g_fp8_hw ? 1 : 2) : 0], 1u + (unsigned)sa.num_row_blocks + (unsigned)num_pad_blocks, EP_ROW_THREADS,
+           small_lds(la.num_experts, la.num_ranks), stream, args);
 }
 
 unsigned layout_place_lds(int E, int R, int K) {
@@ -619,7 +647,7 @@ int ep_buffer_print_memory_usage(ep_buffer_t* b) {
 }
 
 // ---- dispatch ---------------------------------------------------------------------------------
-int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
+static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool epilogue_follows) {
     return guarded([&] {
         EP_HOST_ASSERT(pa != nullptr);
         check_buffer(b);
@@ -716,6 +744,7 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
 
         const RankBoxes boxes = cached_mode ? RankBoxes{} : rank_boxes(b, a.num_max_tokens_per_rank, num_topk, a.num_experts);
         int* rank_map = nullptr;
+        const EpLayoutArgs* small_layout = nullptr;     // the pack launch works out the layout as well
         // geometry of the packed rows of the partition-major regions (only materialised when R > 1)
         const PackedToken pk = packed_token(hidden * packed_elem, packed_sf * 2, num_topk, not cached_mode);
         auto launch_pack = [&]() {
@@ -763,6 +792,10 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
             sa.num_parts = (int)std::max<int64_t>(1, a.fused_fp8_quant ? ceil_div(hidden, 512) : ceil_div(sa.copy_bytes, 1024));
             sa.num_row_blocks = (int)ceil_div((int64_t)num_tokens * sa.num_parts, EP_ROWS_PER_BLOCK);
             if (sa.num_row_blocks == 0) return;
+            if (small_layout != nullptr) {
+                launch_small(*small_layout, sa, true, a.fused_fp8_quant != 0, 0, a.stream);
+                return;
+            }
             hipFunction_t fn = a.fused_fp8_quant ? (g_fp8_hw ? g_k.scatter_quant_pack : g_k.scatter_quant_sw_pack)
                                                  : g_k.scatter_copy_pack;
             launch(fn, (unsigned)sa.num_row_blocks, EP_ROW_THREADS, 0, a.stream, sa);
@@ -776,7 +809,7 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         }
         if (cached_mode) {
             // the cached handle already holds the whole layout: only the packed regions are refreshed
-            b->last.valid = false;
+            b->last.valid = b->last.layout_pending = false;
             if (num_ranks > 1) launch_pack();
             return;
         }
@@ -839,7 +872,17 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         la.cumulative_stats = (int*)a.cumulative_local_expert_recv_stats.data;
         la.host_page = b->host_page_dev;
 
-        launch_layout(la, num_blocks, a.stream);
+        const bool small = small_dispatch(num_tokens, K);
+        b->last.layout_pending = b->last.copied = false;
+        if (small and num_ranks > 1) {
+            small_layout = &la;
+        } else if (small and epilogue_follows) {
+            b->last.layout_pending = true;
+            b->last.pending = la;
+            b->last.pending_stream = a.stream;
+        } else {
+            launch_layout(la, num_blocks, a.stream);
+        }
 
         if (num_ranks > 1) launch_pack();
 
@@ -859,6 +902,9 @@ int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) {
         b->last.recv_done = false;
     });
 }
+
+int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) { return dispatch_launch(b, pa, false); }
+int ep_dispatch_begin(ep_buffer_t* b, const ep_dispatch_args_t* pa) { return dispatch_launch(b, pa, true); }
 
 int64_t ep_dispatch_stamp(ep_buffer_t* b) {
     return (b == nullptr || b->destroyed || !b->last.valid) ? 0 : b->last.stamp;
@@ -975,6 +1021,7 @@ int ep_dispatch_wait_counts(ep_buffer_t* b, int* num_recv_tokens, int* num_expan
     return guarded([&] {
         EP_HOST_ASSERT(b != nullptr and not b->destroyed);
         EP_HOST_ASSERT(b->last.valid);
+        EP_HOST_ASSERT(not b->last.layout_pending and "the copy epilogue of an ep_dispatch_begin comes before the counts");
         EP_HOST_ASSERT(b->last.notified and "the last dispatch was launched with do_cpu_sync (nothing else publishes the counts)");
         const auto deadline = std::chrono::steady_clock::now() + std::chrono::seconds(b->cpu_timeout_secs);
         volatile int* page = b->host_page;
@@ -1190,9 +1237,17 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
         // expert at alignment 128 and 32 or 64 give the same time; one per 4 KiB chunk, 223 a expert, is 10-20 %
         // slower: every workgroup first waits for the expert's row count)
         sa.pad_blocks_per_expert = std::max(1, std::min(EP_MAX_PAD_BLOCKS_PER_EXPERT, a.expert_alignment / 8));
-        const unsigned pad_blocks = a.do_zero_padding ? (unsigned)(El * sa.pad_blocks_per_expert) : 0u;
+        const unsigned pad_blocks = a.do_zero_padding and a.expert_alignment > 1 ? (unsigned)(El * sa.pad_blocks_per_expert) : 0u;
         const unsigned grid = (unsigned)sa.num_row_blocks + pad_blocks;
-        if (grid > 0) {
+        const bool pending = not cached_mode and b->last.layout_pending;
+        b->last.layout_pending = false;
+        EP_HOST_ASSERT((cached_mode or not b->last.copied) and "an ep_dispatch_begin has one copy epilogue");
+        const bool whole = pending and b->last.pending_stream == a.stream and sa.num_row_blocks > 0;
+        if (pending and not whole) launch_layout(b->last.pending, 1, b->last.pending_stream);
+        if (whole) {
+            b->last.copied = true;
+            launch_small(b->last.pending, sa, false, quantise_here, (int)std::min(pad_blocks, kSmallPadBlocks), a.stream);
+        } else if (grid > 0) {
             hipFunction_t fn = quantise_here ? (g_fp8_hw ? g_k.scatter_quant : g_k.scatter_quant_sw) : g_k.scatter_copy;
             launch(fn, grid, EP_ROW_THREADS, 0, a.stream, sa);
         }
@@ -1420,7 +1475,7 @@ extern "C" int ep_dispatch_static_launch(const ep_dispatch_args_t* d, const ep_d
     ep_buffer* v = nullptr;
     rc = guarded([&] { v = static_view_of_current_device(); });
     if (rc != 0) return rc;
-    rc = ep_dispatch_launch(v, d);
+    rc = ep_dispatch_begin(v, d);
     if (rc != 0) return rc;
     ep_dispatch_epilogue_args_t ee = *e;
     ee.dispatch_stamp = v->last.stamp;

@@ -384,7 +384,9 @@ public:
         a.do_cpu_sync = do_cpu_sync ? 1 : 0;
         a.fused_fp8_quant = fused_fp8_quant ? 1 : 0;
         a.stream = current_stream();
-        check(ep_dispatch_launch(buf_, &a));
+        // (the copy follows at once, unless it is deferred or the output sizes are waited for first)
+        const bool copy_follows = num_ranks_ == 1 && !defer_epilogue && !(do_cpu_sync && exact_sync_sizes_);
+        check(copy_follows ? ep_dispatch_begin(buf_, &a) : ep_dispatch_launch(buf_, &a));
         // the epilogue below belongs to this launch: the library refuses it once a later dispatch has taken over
         // the buffer's workspace
         s.stamp = ep_dispatch_stamp(buf_);

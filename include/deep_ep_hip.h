@@ -147,6 +147,11 @@ typedef struct ep_dispatch_args {
  * partition this is the send side (dst_buffer_slot_idx, dst_gsge_idx, packed rows, inbox counts)
  * and ep_dispatch_recv_launch writes the other handle tensors. */
 int ep_dispatch_launch(ep_buffer_t* buf, const ep_dispatch_args_t* args);
+/* The same for a caller whose next call on this buffer is this dispatch's ep_dispatch_epilogue_launch: the library may
+ * then leave the layout to the copy launch (one partition, at most 128 tokens and 1024 (token, slot) entries: one
+ * launch instead of two; the handle tensors are complete behind the epilogue).  Counts can be waited for after the
+ * epilogue only. */
+int ep_dispatch_begin(ep_buffer_t* buf, const ep_dispatch_args_t* args);
 
 typedef struct ep_dispatch_recv_args {
     /* handle tensors, written here (csrc/buffers/ep.hpp:205-246) */

@@ -1,0 +1,90 @@
+"""Dispatches of decode size, layout and copy in one launch: handles and rows of the oracle at the edges of what that
+launch takes, in every payload form, with and without a host sync, and the calls around it that it must not change."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import bf16_bits, make_routing, make_tokens
+from oracle import ep_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = 'cuda'
+
+CASES = [
+    # T, H, E, K, A, masked, zipf
+    (1, 128, 1, 1, 1, 0.0, None),
+    (1, 16, 40, 32, 3, 0.2, None),
+    (32, 128, 2048, 32, 1, 0.1, None),      # every entry of the limit, the largest expert count
+    (33, 128, 64, 32, 4, 0.0, None),        # one entry row beyond it: two launches
+    (128, 528, 24, 8, 128, 0.3, None),      # every entry of the limit, both sides of a 512-channel part
+    (128, 1040, 256, 8, 16, 0.1, 1.2),      # hot and empty experts
+    (127, 2064, 8, 3, 8, 0.5, None),
+    (129, 256, 16, 2, 64, 0.0, None),       # one token beyond it
+    (64, 256, 300, 16, 1, 0.0, None),       # more experts than threads
+]
+
+
+@pytest.mark.parametrize('T,H,E,K,A,masked,zipf', CASES)
+@pytest.mark.parametrize('mode', ['bf16', 'fused', 'pair'])
+def test_small_dispatch(T, H, E, K, A, masked, zipf, mode):
+    import deep_ep
+    x = make_tokens(T, H, seed=T + H, outliers=True)
+    topk, w = make_routing(T, E, K, seed=T + K, masked=masked, zipf=zipf)
+    if T > 2 and K > 1:
+        topk[2], w[2] = -1, 0.0             # a token that nobody receives
+        topk[0, 1] = topk[0, 0]             # an expert selected twice
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
+    n, ne = lay['num_recv_tokens'], lay['num_expanded_tokens']
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T + 5, hidden=H, num_topk=K, use_fp8_dispatch=mode != 'bf16',
+                           explicitly_destroy=True)
+    q, s = O.quantise(x)
+    xin = x.to(DEV) if mode != 'pair' else (q.view(torch.float8_e4m3fn).to(DEV), s.view(torch.int16).to(DEV))
+    ex, es, ew = O.rank_share_dispatch(bf16_bits(x) if mode == 'bf16' else q.numpy(), None if mode == 'bf16' else s.numpy().view(np.uint32),
+                                       w.numpy(), lay)
+    stats = torch.zeros(E, dtype=torch.int32, device=DEV)
+    for k, sync in enumerate((True, False, True)):
+        recv, _, rw, handle, _ = buf.dispatch(xin, topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E,
+                                              num_max_tokens_per_rank=T + 5, expert_alignment=A, do_expand=True, do_zero_padding=True,
+                                              do_cpu_sync=sync, fused_fp8_quant=mode == 'fused', cumulative_local_expert_recv_stats=stats)
+        torch.cuda.synchronize()
+        for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
+                     'dst_buffer_slot_idx', 'dst_gsge_idx'):
+            assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
+        meta = lay['recv_src_metadata'].copy()
+        assert np.array_equal(handle.recv_src_metadata.cpu().numpy()[:n], meta)
+        assert np.array_equal(stats.cpu().numpy(), (k + 1) * lay['num_unaligned_recv_tokens_per_expert'])
+        if sync:
+            assert handle.num_recv_tokens == n and handle.num_expanded_tokens == ne
+            assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
+        rows, sf = recv if isinstance(recv, tuple) else (recv, None)
+        got = bf16_bits(rows) if mode == 'bf16' else rows.view(torch.uint8).cpu().numpy()
+        assert np.array_equal(got[:ne], ex)
+        if sf is not None:
+            assert np.array_equal(np.ascontiguousarray(sf.cpu().numpy()).view(np.uint32).reshape(sf.size(0), -1)[:ne], es)
+        assert np.array_equal(rw.cpu().numpy().view(np.uint32)[:ne], ew.view(np.uint32))
+    buf.destroy()
+
+
+def test_small_dispatch_deferred_exact_and_replayed():
+    """The same handles from the calls that keep the two launches (a deferred epilogue, exact sizes), and a cached
+    dispatch behind the single launch."""
+    import deep_ep
+    T, H, E, K, A = 50, 256, 16, 4, 8
+    x = make_tokens(T, H, seed=1).to(DEV)
+    topk, w = make_routing(T, E, K, seed=2, masked=0.2)
+    args = dict(topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E, num_max_tokens_per_rank=T, expert_alignment=A,
+                do_expand=True, do_zero_padding=True)
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    r0, _, w0, h0, _ = buf.dispatch(x, **args)
+    deferred = buf.dispatch(x, async_with_compute_stream=True, defer_epilogue=True, **args)
+    r1, _, w1, h1 = deferred.current_stream_wait()
+    buf.set_exact_sync_sizes(True)
+    r2, _, w2, h2, _ = buf.dispatch(x, **args)
+    buf.set_exact_sync_sizes(False)
+    r3, _, w3, _, _ = buf.dispatch(x, topk_weights=w.to(DEV), handle=h0, do_expand=True, do_zero_padding=True)
+    torch.cuda.synchronize()
+    for r, ww, h in ((r1, w1, h1), (r2, w2, h2), (r3, w3, h0)):
+        assert torch.equal(r.view(torch.int16), r0.view(torch.int16)) and torch.equal(ww, w0)
+        assert torch.equal(h.recv_src_metadata, h0.recv_src_metadata)
+        assert torch.equal(h.dst_buffer_slot_idx, h0.dst_buffer_slot_idx)
+    buf.destroy()
