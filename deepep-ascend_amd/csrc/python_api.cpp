@@ -94,6 +94,18 @@ py::object new_event() {
 at::Tensor alloc(at::IntArrayRef shape, at::ScalarType dtype, const at::Device& dev) {
     return at::Tensor(at::detail::empty_cuda(shape, dtype, dev, std::nullopt));
 }
+// A view of `base` without the dispatcher (a narrow() through it costs 1.2 us, and a synchronised dispatch makes seven).
+at::Tensor view_of(const at::Tensor& base, at::IntArrayRef sizes, at::IntArrayRef strides, int64_t offset) {
+    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(base.storage()), base.key_set(),
+                                                            base.dtype());
+    t.unsafeGetTensorImpl()->set_storage_offset(base.storage_offset() + offset);
+    t.unsafeGetTensorImpl()->set_sizes_and_strides(sizes, strides);
+    return t;
+}
+// The first rows of a contiguous tensor.
+at::Tensor first_rows(const at::Tensor& t, int64_t rows) {
+    return t.dim() == 1 ? view_of(t, {rows}, {1}, 0) : view_of(t, {rows, t.size(1)}, {t.size(1), 1}, 0);
+}
 at::Tensor empty_i32(std::initializer_list<int64_t> shape, const at::Device& dev) { return alloc(shape, at::kInt, dev); }
 
 // What a dispatch call keeps until its copy epilogue has been enqueued (the descriptors hold raw pointers:
@@ -172,7 +184,7 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
         counts_from_host = true;
         alloc_recv = num_recv;
         alloc_expanded = num_expanded;
-        if (have_meta) meta = meta.narrow(0, 0, num_recv);
+        if (have_meta) meta = first_rows(meta, num_recv);
     } else if (s.do_cpu_sync) {
         // Exact sizes come from the host count page, but waiting for it here would leave the GPU idle between the
         // layout kernels and the copy.  Allocate for this call's upper bound, enqueue the copy, and read the counts
@@ -201,7 +213,7 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
             // scale rows go to a staging tensor, a tiled kernel of the library turns them into columns
             sf_staging = alloc({alloc_expanded, sf_cols}, sf_type, dev);
             sf_storage = alloc({sf_cols * alloc_expanded}, sf_type, dev);
-            recv_sf = sf_storage->as_strided({alloc_expanded, sf_cols}, {1, alloc_expanded});
+            recv_sf = view_of(*sf_storage, {alloc_expanded, sf_cols}, {1, alloc_expanded}, 0);
         } else {
             recv_sf = alloc({alloc_expanded, sf_cols}, sf_type, dev);
         }
@@ -245,22 +257,22 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
         counts_from_host = true;
         if (num_recv > alloc_recv || num_expanded > alloc_expanded)
             throw EpPyError("Assertion exception (python_api.cpp): received counts exceed this call's bound");
-        recv_x = recv_x.narrow(0, 0, num_expanded);
+        recv_x = first_rows(recv_x, num_expanded);
         if (recv_sf.has_value() && s.use_col_major_sf)
-            recv_sf = sf_storage->as_strided({(int64_t)num_expanded, sf_cols}, {1, (int64_t)num_expanded});
+            recv_sf = view_of(*sf_storage, {(int64_t)num_expanded, sf_cols}, {1, (int64_t)num_expanded}, 0);
         else if (recv_sf.has_value())
-            recv_sf = recv_sf->narrow(0, 0, num_expanded);
-        if (recv_w.has_value()) recv_w = recv_w->narrow(0, 0, num_expanded);
-        meta = meta.narrow(0, 0, num_recv);
+            recv_sf = first_rows(*recv_sf, num_expanded);
+        if (recv_w.has_value()) recv_w = first_rows(*recv_w, num_expanded);
+        meta = first_rows(meta, num_recv);
     }
 
     py::object list_obj;
     if (s.cached_mode) {
         list_obj = s.cached_list;
     } else {
-        py::list l;
+        py::list l(counts_from_host ? El : 0);
         if (counts_from_host)
-            for (int i = 0; i < El; ++i) l.append(per_expert[(size_t)i]);
+            for (int i = 0; i < El; ++i) PyList_SET_ITEM(l.ptr(), i, py::int_(per_expert[(size_t)i]).release().ptr());
         list_obj = std::move(l);
     }
     return py::make_tuple(recv_x, recv_sf, recv_w, num_recv, num_expanded, list_obj, s.psum_rank, s.psum_expert,
@@ -360,9 +372,9 @@ public:
             // the three count vectors share one allocation (each starts on a multiple of 64 bytes)
             const int64_t r16 = (num_ranks_ + 15) / 16 * 16, e16 = (s.num_local_experts + 15) / 16 * 16;
             at::Tensor counts = empty_i32({r16 + 2 * e16}, dev);
-            s.psum_rank = counts.narrow(0, 0, num_ranks_);
-            s.psum_expert = counts.narrow(0, r16, s.num_local_experts);
-            s.unaligned = counts.narrow(0, r16 + e16, s.num_local_experts);
+            s.psum_rank = view_of(counts, {(int64_t)num_ranks_}, {1}, 0);
+            s.psum_expert = view_of(counts, {(int64_t)s.num_local_experts}, {1}, r16);
+            s.unaligned = view_of(counts, {(int64_t)s.num_local_experts}, {1}, r16 + e16);
             s.dst_slot = empty_i32({s.num_tokens, s.num_topk}, dev);
             s.dst_gsge = empty_i32({s.num_tokens, s.num_topk}, dev);
         }
@@ -467,6 +479,10 @@ private:
 PYBIND11_MODULE(_native, m) {
     m.doc() = "compiled binding of the EP dispatch/combine calls over the C ABI of libdeep_ep_hip.so";
     py::register_exception<EpPyError>(m, "EPException", PyExc_RuntimeError);
+    m.def("current_stream_key", []() {
+        const auto stream = c10::hip::getCurrentHIPStream();
+        return py::make_tuple((int64_t)stream.id(), (int)stream.device_index(), (int)stream.unwrap().device_type());
+    }, "(stream_id, device_index, device_type) of the current stream");
     py::class_<NativeBuffer>(m, "Buffer")
         .def(py::init<uintptr_t, int, int>())
         .def("set_connected", &NativeBuffer::set_connected)
