@@ -28,6 +28,8 @@
 #define EP_COMBINE_PARTIAL 1    // owner side: per received row, partial into the combine buffer
 #define EP_COMBINE_FINAL 2      // token side: biases + partials of the masters into combined_x
 
+#define EP_COMBINE_LONG_PART 2048
+
 // Host-visible count page (pinned, mapped).  Written once per non-cached dispatch.
 //   [0] ready sequence number (written last, release at system scope)
 //   [1] number of received tokens   [2] number of expanded tokens (aligned)
@@ -202,7 +204,7 @@ struct EpCombineArgs {
     // owner-side reduce: the partial of a row goes to the combine buffer of the partition its token came from
     char* const* peer_arenas;
     int64_t buffer_off;
-    int whole_rows;               // owner-side reduce: a task is a whole row (num_parts == 1), not a 1024-channel part
+    int long_parts;               // owner-side reduce: a task is EP_COMBINE_LONG_PART channels of a row, not 1024
 };
 
 // Caller-side quantiser: rows of BF16 -> rows of e4m3fn bytes + one fp32 scale per row and 128 channels.

@@ -1728,9 +1728,10 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
         if (MODE == EP_COMBINE_PARTIAL && (group < 0 || group >= a.num_groups)) return;
     }
     const int nvalid = __popcll(__ballot(myslot >= 0));
-    // Owner side with whole rows per task: a received row mostly has a single slot among this partition's few
-    // experts, and its partial is then that row verbatim: up to 16 vectors a lane in flight, no arithmetic.
-    const bool verbatim = MODE == EP_COMBINE_PARTIAL && a.whole_rows && nvalid == 1;
+    // Owner side with long parts (32 / 16 / 4 partitions of 4096 / 4096 / 8192 tokens, top-6: 157 / 152 / 227 us with a wave a
+    // row, 136 / 136 / 199 so): a received row mostly has one or two slots among this partition's few experts, and one
+    // slot's partial is that row verbatim: 4 vectors a lane and slot in flight, the second slot's behind the first's.
+    const bool verbatim = MODE == EP_COMBINE_PARTIAL && a.long_parts && nvalid == 1;
     const int nvec = a.hidden >> 3;
     const int64_t yvec = a.y_row_bytes >> 4;
     const u32x4* y = (const u32x4*)a.y;
@@ -1782,27 +1783,39 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
     u32x4* out = (u32x4*)out_row;
     const bool has0 = a.bias_0 != nullptr, has1 = a.bias_1 != nullptr;
     const bool weighted = MODE == EP_COMBINE_FUSED && a.weighted;
-    if (verbatim) {
-        const int s1 = readlane(myslot, __builtin_ctzll(__ballot(myslot >= 0)));
-        const u32x4* src = y + (int64_t)s1 * yvec;
-        // (the loop counter is the same in every lane: a row shorter than the wave still gets its weights)
-        for (int v0 = 0; v0 < nvec; v0 += 16 * WAVE) {
-            const int vb = v0 + lane;
-            u32x4 d[16];
+    constexpr int LONG = EP_COMBINE_LONG_PART / (8 * WAVE);       // vectors a lane of a long part
+    const bool long_parts = MODE == EP_COMBINE_PARTIAL && a.long_parts;
+    if (long_parts && nvalid >= 1 && nvalid <= 2) {
+        const uint64_t vm = __ballot(myslot >= 0);
+        const u32x4* src0 = y + (int64_t)readlane(myslot, __builtin_ctzll(vm)) * yvec;
+        const u32x4* src1 = y + (int64_t)readlane(myslot, 63 - __builtin_clzll(vm)) * yvec;
+        // (a lane past the end of the row re-reads the last vector and stores nothing)
+        const int vb = part * LONG * WAVE + lane;
+        u32x4 d0[LONG], d1[LONG];
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                if (vb + u * WAVE < nvec) d[u] = __builtin_nontemporal_load(src + vb + u * WAVE);
-            if (v0 == 0 && lane < K && a.expanded_weights != nullptr) ((float*)(out_row + (a.hidden << 1)))[lane] = myw;
+        for (int u = 0; u < LONG; ++u) d0[u] = __builtin_nontemporal_load(src0 + min(vb + u * WAVE, nvec - 1));
+        if (verbatim) {
+            if (part == 0 && lane < K && a.expanded_weights != nullptr) ((float*)(out_row + (a.hidden << 1)))[lane] = myw;
 #pragma unroll
-            for (int u = 0; u < 16; ++u)
-                if (vb + u * WAVE < nvec) stream_store<EP_COMBINE_ST_POL>(out + vb + u * WAVE, d[u]);
+            for (int u = 0; u < LONG; ++u)
+                if (vb + u * WAVE < nvec) stream_store<EP_COMBINE_ST_POL>(out + vb + u * WAVE, d0[u]);
+            return;
+        }
+#pragma unroll
+        for (int u = 0; u < LONG; ++u) d1[u] = __builtin_nontemporal_load(src1 + min(vb + u * WAVE, nvec - 1));
+#pragma unroll
+        for (int u = 0; u < LONG; ++u) {
+            float f[8], g[8];
+            unpack8(d0[u], f);
+            unpack8(d1[u], g);
+            for (int q = 0; q < 8; ++q) f[q] = f[q] + g[q];
+            if (vb + u * WAVE < nvec) stream_store<EP_COMBINE_ST_POL>(out + vb + u * WAVE, pack8(f));
         }
         return;
     }
-    // a task is one 1024-channel part of its row, or (owner side, whole rows) all of them in turn
-    const bool whole = MODE == EP_COMBINE_PARTIAL && a.whole_rows;
-    const int part_end = whole ? (nvec + 2 * WAVE - 1) / (2 * WAVE) : part + 1;
-    for (int cp = whole ? 0 : part; cp < part_end; ++cp) {
+    // a task is one 1024-channel part of its row, or (owner side, long parts) several in turn
+    const int part_end = long_parts ? min((part + 1) * (LONG / 2), (nvec + 2 * WAVE - 1) / (2 * WAVE)) : part + 1;
+    for (int cp = long_parts ? part * (LONG / 2) : part; cp < part_end; ++cp) {
     const int v0 = cp * 2 * WAVE + lane, v1 = v0 + WAVE;
     const bool live0 = v0 < nvec, live1 = v1 < nvec;
     // the gate weights are scattered 4-byte loads: only the task that carries them back (part 0) or multiplies

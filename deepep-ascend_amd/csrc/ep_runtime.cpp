@@ -1352,11 +1352,14 @@ int ep_combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase) {
             ca.peer_arenas = b->peer_table();
             ca.buffer_off = b->workspace_bytes;
             ca.out_row_bytes = combine_token;
-            // a received row mostly has one slot among a partition's few experts: whole rows per wave task once
-            // there are enough rows to fill the machine that way (a few thousand rows are spread part by part)
-            if (ca.num_rows_bound >= 16384) {
-                ca.whole_rows = 1;
-                ca.num_parts = 1;
+            // With few slots a row (less than two selections a partition) the rows are short of loads in flight, and from
+            // about 16384 of them on there are enough tasks to give each 2048 channels.  us a launch with 1024 / 2048 / whole
+            // rows, top-6 unless noted: 16 partitions, 21k rows 140 / 135 / 151; 8 partitions, 22k (top-8) 166 / 163 / 174;
+            // 4 partitions, 27k 200 / 201 / 228; against them 2 partitions, 33k (top-8) 399 / 418 / 466.  At 9k rows of 8
+            // partitions the forms are level (68.6 / 68.6 us).
+            if (ca.num_rows_bound >= 16384 and K < 2 * R) {
+                ca.long_parts = 1;
+                ca.num_parts = (int)std::max<int64_t>(1, ceil_div(hidden, EP_COMBINE_LONG_PART));
             }
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROWS_PER_BLOCK);
             if (ca.num_row_blocks == 0) return;

@@ -558,3 +558,38 @@ def test_owner_side_whole_rows_shorter_than_a_wave_carry_all_their_weights():
         assert torch.equal(cw.cpu(), ow) and torch.equal(cw.cpu(), ws[s]), s
     for b in bufs:
         b.destroy()
+
+
+@pytest.mark.parametrize('H,K', [(64, 7), (512, 6), (2048, 6), (2056, 6), (4104, 3), (7168, 6)])
+def test_owner_side_long_parts(H, K):
+    """From 16384 metadata rows on and with few slots a row, a task of the owner-side reduce is 2048 channels: rows of
+    one, two and more slots, on both sides of a part."""
+    R, max_tokens, E, A = 4, 4100, 16, 4
+    bufs = make_node(R, max_tokens, H, K, False)
+    Ts = [70 - r for r in range(R)]
+    xs = [make_tokens(T, H, seed=70 + r) for r, T in enumerate(Ts)]
+    routing = [make_routing(T, E, K, seed=80 + r, masked=0.3) for r, T in enumerate(Ts)]
+    topks, ws = [t for t, _ in routing], [w for _, w in routing]
+    rows = [bf16_bits(x).view(np.uint8).reshape(x.size(0), -1) for x in xs]
+    _, want = oracle_dispatch(rows, [None] * R, [t.numpy() for t in topks], [w.numpy() for w in ws], E, R, A, max_tokens)
+    outs = dispatch_all(bufs, [x.to(DEV) for x in xs], [t.to(DEV) for t in topks], [w.to(DEV) for w in ws],
+                        num_experts=E, num_max_tokens_per_rank=max_tokens, expert_alignment=A, do_expand=True, do_cpu_sync=False)
+    slots = np.concatenate([(o['lay']['recv_src_metadata'][:, :K] >= 0).sum(axis=1) for o in want])
+    assert all((slots == n).any() for n in (1, 2, 3))
+    g = torch.Generator().manual_seed(9)
+    ys = [torch.randn((outs[r][0].size(0), H), generator=g).to(torch.bfloat16) for r in range(R)]
+    for b in bufs:
+        b.runtime.buffer_tensor().fill_(0x5A)
+    res = combine_all(bufs, [y.to(DEV) for y in ys], [o[3] for o in outs], [o[2] for o in outs], [None] * R)
+    parts, wvecs = {}, {}
+    for r in range(R):
+        ne = want[r]['lay']['num_expanded_tokens']
+        p, wv = O.combine_partial(ys[r][:ne], torch.from_numpy(want[r]['w']), want[r]['lay']['recv_src_metadata'], R, r, max_tokens)
+        parts.update(p)
+        wvecs.update(wv)
+    for s in range(R):
+        ox, ow = O.combine_final(topks[s].numpy(), E, R, s, max_tokens, lambda k: parts[k], lambda k: wvecs[k], None, None, H, True)
+        assert np.array_equal(bf16_bits(res[s][0]), bf16_bits(ox)), s
+        assert torch.equal(res[s][1].cpu(), ow)
+    for b in bufs:
+        b.destroy()
