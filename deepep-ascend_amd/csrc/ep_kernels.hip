@@ -1416,10 +1416,8 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
         // (the same expert twice in one token: the earlier one counts too)
         int c0 = __popcll(__ballot(e == ej) & ((1ull << j) - 1ull));
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            if (c >= chunks) break;
-            c0 += __popcll(__ballot(key[c] == ej));
-        }
+        for (int c = 0; c < CH; ++c)                    // (a break would keep the loop from being unrolled: 10.7 -> 10.1 us)
+            if (c < chunks) c0 += __popcll(__ballot(key[c] == ej));
         if (lane == j) rank = c0;
     }
     // ---- masters: the last entry of the token for a partition; its slot there ----
