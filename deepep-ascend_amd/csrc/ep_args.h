@@ -148,6 +148,7 @@ struct EpScatterArgs {
     int pack_sf_off;              // byte offset of the scales inside a packed row (pack mode)
     int64_t rank_box_off;         // byte offset in every arena of the rank box [R * max_tokens, K] (pack mode; 0: none is kept)
     int vecs_per_lane;            // verbatim kernel: 16-byte vectors a lane moves per task (1..4)
+    int sf_pairs;                 // verbatim kernel: scale packs move two at a time (even count, 4-byte aligned rows on both sides)
     int rows_are_tokens;          // cached expand: every token was received, so row i of the receive stream is token i
 };
 

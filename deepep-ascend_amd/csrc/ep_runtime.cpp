@@ -353,6 +353,12 @@ void launch_small(const EpLayoutArgs& la, const EpScatterArgs& sa, bool pack, bo
            small_lds(la.num_experts, la.num_ranks), stream, args);
 }
 
+// Scale packs (2 bytes) can move two at a time: packs side by side, rows that start on 4 bytes where they are read and written.
+int sf_pairs(const EpScatterArgs& sa, const void* out) {
+    return sa.sf != nullptr and out != nullptr and sa.num_sf_packs % 2 == 0 and sa.sf_pack_stride_bytes == 2 and
+           sa.sf_token_stride_bytes % 4 == 0 and sa.out_sf_row_bytes % 4 == 0 and (((uintptr_t)sa.sf | (uintptr_t)out) & 3) == 0;
+}
+
 unsigned layout_place_lds(int E, int R, int K) {
     const unsigned nw = EP_LAYOUT_THREADS / 64;
     return (unsigned)(E + E / R + nw + R + nw + 2 * EP_TOKENS_PER_BLOCK) * sizeof(int) + EP_TOKENS_PER_BLOCK * K;
@@ -786,6 +792,7 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
             sa.region_by_source = b->connected ? 1 : 0;
             sa.num_ranks = num_ranks;
             sa.pack_sf_off = pk.sf_off;
+            sa.sf_pairs = sf_pairs(sa, sa.recv_sf);
             sa.slot_map = rank_map;
             sa.rank_box_off = boxes.used ? boxes.rank_off : 0;
             sa.vecs_per_lane = 1;
@@ -1223,6 +1230,7 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
             sa.w_off = pk.w_off;
             quantise_here = false;
         }
+        sa.sf_pairs = quantise_here ? 0 : sf_pairs(sa, sa.recv_sf);
         // a wave task covers 1 KiB of a verbatim row (4 KiB of a packed row, which mostly has one destination
         // among this partition's few experts), or 512 channels of a row being quantised
         sa.vecs_per_lane = sa.mode == EP_SCATTER_REGION ? 4 : 1;

@@ -552,3 +552,30 @@ def test_odd_topk_combine_of_small_launches(T, H, K):
     cx, _, _ = buf.combine(y.to(DEV), handle, topk_weights=rw, apply_weights=True)
     assert np.array_equal(bf16_bits(cx), bf16_bits(O.combine_weighted(y, rw.cpu(), lay['recv_src_metadata'], T, K)))
     buf.destroy()
+
+
+@pytest.mark.parametrize('packs', [1, 2, 63, 64, 128, 130, 258])
+@pytest.mark.parametrize('alignment', [1, 2, 8])
+def test_scale_packs_of_any_count_and_stride(packs, alignment):
+    """2-byte scale packs two at a time or one (odd counts, rows that start off 4 bytes, columns), more than a wave's
+    worth of pairs, and their columns with 16-byte, 4-byte and single stores, up to and beyond the widest rows in one go."""
+    T, H, E, K = 73, 4096, 5, 3
+    topk, w = make_routing(T, E, K, seed=alignment, masked=0.2)
+    g = torch.Generator().manual_seed(packs)
+    xq = torch.randint(0, 255, (T, H), generator=g, dtype=torch.uint8)
+    sf = torch.randint(-32768, 32767, (T, packs), generator=g, dtype=torch.int16)
+    forms = {'rows': sf.to(DEV), 'columns': sf.to(DEV).t().contiguous().t()}
+    wide = torch.zeros((T, packs + 2), dtype=torch.int16, device=DEV)
+    forms['shifted rows'] = wide[:, 1:1 + packs].copy_(forms['rows'])
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, alignment, T)
+    ex, es, _ = O.rank_share_dispatch(xq.numpy(), sf.numpy().view(np.uint8).reshape(T, -1), w.numpy(), lay)
+    n = lay['num_expanded_tokens']
+    buf = _buffer(T, H, K, fp8=True)
+    for name, s in forms.items():
+        for col_major in (False, True):
+            (rx, rsf), _, _, _, _ = buf.dispatch((xq.view(torch.float8_e4m3fn).to(DEV), s), topk_idx=topk.to(DEV),
+                                                 topk_weights=w.to(DEV), num_experts=E, expert_alignment=alignment, do_expand=True,
+                                                 do_zero_padding=True, use_tma_aligned_col_major_sf=col_major)
+            assert np.array_equal(rsf.cpu().numpy(), es.view(np.int16).reshape(n, packs)), (name, col_major)
+            assert np.array_equal(rx.view(torch.uint8).cpu().numpy(), ex), (name, col_major)
+    buf.destroy()
