@@ -1526,11 +1526,8 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_quant_rows(EpQua
 // (csrc/buffers/ep.hpp:379-381); writing columns straight from the copy kernel was measured and is
 // slower, since every 4-byte scale then lands in a cache line of its own.
 template <typename E>
-__device__ __forceinline__ void sf_transpose_body(const EpSfTransposeArgs& a, unsigned (*tile)[EP_SF_TILE + 1]) {
-    int n = a.num_rows;
-    if (a.counted) n = min(n, align_up(a.psum_expert[a.num_local_experts - 1], a.expert_alignment));
+__device__ __forceinline__ void sf_transpose_body(const EpSfTransposeArgs& a, int n, unsigned (*tile)[EP_SF_TILE + 1]) {
     const int r0 = blockIdx.x * EP_SF_TILE;
-    if (r0 >= n) return;
     const int tx = threadIdx.x % EP_SF_TILE, ty = threadIdx.x / EP_SF_TILE;
     constexpr int STEP = EP_LAYOUT_THREADS / EP_SF_TILE;
     const E* src = (const E*)a.src;
@@ -1545,49 +1542,78 @@ __device__ __forceinline__ void sf_transpose_body(const EpSfTransposeArgs& a, un
     }
 }
 
-// 2-byte packs, two at a time: a thread reads two adjacent columns of a row as one 32-bit word and writes two
-// adjacent rows of a column as one.  Needs an even column count (rows of the source start on 4 bytes) and an even
-// row count (columns of the destination do); half the steps of the element-wise form.
-__device__ __forceinline__ void sf_transpose_pairs(const EpSfTransposeArgs& a, int n, unsigned short (*tile)[EP_SF_TILE + 2]) {
-    const int r0 = blockIdx.x * EP_SF_TILE;
-    constexpr int HALF = EP_SF_TILE / 2;
-    const int tx = threadIdx.x % HALF, ty = threadIdx.x / HALF;
-    constexpr int STEP = EP_LAYOUT_THREADS / HALF;
-    const unsigned* src = (const unsigned*)a.src;
-    unsigned* dst = (unsigned*)a.dst;
-    const int cols2 = a.num_cols >> 1, n2 = n >> 1;
-    for (int c0 = 0; c0 < a.num_cols; c0 += EP_SF_TILE) {
-        for (int rr = ty; rr < EP_SF_TILE; rr += STEP) {
-            const int c = c0 + 2 * tx;
-            if (r0 + rr < n && c < a.num_cols) {
-                const unsigned v = src[(int64_t)(r0 + rr) * cols2 + (c >> 1)];
-                tile[rr][2 * tx] = (unsigned short)v;
-                tile[rr][2 * tx + 1] = (unsigned short)(v >> 16);
-            }
-        }
-        __syncthreads();
-        for (int cc = ty; cc < EP_SF_TILE; cc += STEP) {
-            const int r = r0 + 2 * tx;
-            if (c0 + cc < a.num_cols && r < n)
-                dst[(int64_t)(c0 + cc) * n2 + (r >> 1)] = (unsigned)tile[2 * tx][cc] | ((unsigned)tile[2 * tx + 1][cc] << 16);
-        }
-        __syncthreads();
+// Rows of at most EP_SF_WIDE_ROW_BYTES from a 16-byte aligned source.  The 64 rows of a workgroup are one contiguous piece
+// of it: the piece goes to LDS in 16-byte loads, all of a thread's in flight, and leaves as V adjacent rows of a column a
+// store: 16 bytes where columns start on 16 bytes (128 or 256 bytes a column and workgroup), else 4, else one element.
+// 52 thousand rows of 112 2-byte packs: 11.2 us with pairs of packs and two barriers per 64 columns, 7.7 us so (fetching the
+// rows before the row count is known, to save its trip, measured 8.4: the workgroups beyond the rows then fetch as well).
+template <typename E, int V>
+__device__ __forceinline__ void sf_columns_out(const EpSfTransposeArgs& a, int n, int rows, int pitch, const unsigned char* lds) {
+    typedef E vec_t __attribute__((ext_vector_type(V)));
+    constexpr int GROUPS = EP_SF_TILE / V;
+    const int r0 = blockIdx.x * EP_SF_TILE, rr = threadIdx.x % GROUPS * V;
+    for (int c = threadIdx.x / GROUPS; c < a.num_cols; c += EP_LAYOUT_THREADS / GROUPS) {
+        E* out = (E*)a.dst + (int64_t)c * n + r0 + rr;
+        vec_t x;
+#pragma unroll
+        for (int q = 0; q < V; ++q) x[q] = *(const E*)(lds + (rr + q) * pitch + c * (int)sizeof(E));
+        if (rr + V <= rows) *(vec_t*)out = x;
+        else
+            for (int q = 0; q < V; ++q)
+                if (rr + q < rows) out[q] = x[q];
     }
+}
+template <typename E>
+__device__ __forceinline__ void sf_transpose_wide(const EpSfTransposeArgs& a, int n, unsigned char* lds) {
+    constexpr int VEC = 16 / (int)sizeof(E), MAXV = EP_SF_TILE * EP_SF_WIDE_ROW_BYTES / 16 / EP_LAYOUT_THREADS;
+    const int cols = a.num_cols, r0 = blockIdx.x * EP_SF_TILE, rows = min(EP_SF_TILE, n - r0);
+    // rows of an odd number of words: the rows that neighbouring lanes read spread over the banks
+    const int pitch = ((cols * (int)sizeof(E) + 3) / 4 | 1) * 4;
+    const int count = rows * cols, nvec = count / VEC;
+    const E* src = (const E*)a.src + (int64_t)r0 * cols;
+    u32x4 v[MAXV];
+#pragma unroll
+    for (int u = 0; u < MAXV; ++u) {
+        const int i = threadIdx.x + u * EP_LAYOUT_THREADS;
+        if (i < nvec) v[u] = ((const u32x4*)src)[i];
+    }
+#pragma unroll
+    for (int u = 0; u < MAXV; ++u) {
+        const int i = threadIdx.x + u * EP_LAYOUT_THREADS;
+        if (i >= nvec) break;
+        int r = i * VEC / cols, c = i * VEC - r * cols;
+        E x[VEC];
+        __builtin_memcpy(x, &v[u], 16);
+#pragma unroll
+        for (int q = 0; q < VEC; ++q) {
+            *(E*)(lds + r * pitch + c * (int)sizeof(E)) = x[q];
+            if (++c == cols) { c = 0; ++r; }
+        }
+    }
+    if ((int)threadIdx.x < count - nvec * VEC) {            // the last, partial vector
+        const int i = nvec * VEC + threadIdx.x, r = i / cols;
+        *(E*)(lds + r * pitch + (i - r * cols) * (int)sizeof(E)) = src[i];
+    }
+    __syncthreads();
+    const int step = n * (int)sizeof(E) | (int)((uintptr_t)a.dst & 15);
+    if ((step & 15) == 0) sf_columns_out<E, VEC>(a, n, rows, pitch, lds);
+    else if ((step & 3) == 0) sf_columns_out<E, 4 / (int)sizeof(E)>(a, n, rows, pitch, lds);
+    else sf_columns_out<E, 1>(a, n, rows, pitch, lds);
 }
 
 extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_sf_transpose(EpSfTransposeArgs a) {
-    __shared__ unsigned tile[EP_SF_TILE][EP_SF_TILE + 1];
-    if (a.elem_bytes == 4) {
-        sf_transpose_body<unsigned>(a, tile);
-        return;
-    }
+    __shared__ __align__(16) unsigned char lds[EP_SF_TILE * (EP_SF_WIDE_ROW_BYTES + 4)];
     int n = a.num_rows;
     if (a.counted) n = min(n, align_up(a.psum_expert[a.num_local_experts - 1], a.expert_alignment));
-    if ((n & 1) == 0 && (a.num_cols & 1) == 0 && (((uintptr_t)a.src | (uintptr_t)a.dst) & 3) == 0) {
-        if ((int)blockIdx.x * EP_SF_TILE < n) sf_transpose_pairs(a, n, (unsigned short (*)[EP_SF_TILE + 2])tile);
-        return;
+    if ((int)blockIdx.x * EP_SF_TILE >= n) return;
+    const bool wide = a.num_cols * a.elem_bytes <= EP_SF_WIDE_ROW_BYTES && ((uintptr_t)a.src & 15) == 0;
+    if (a.elem_bytes == 4) {
+        if (wide) sf_transpose_wide<unsigned>(a, n, lds);
+        else sf_transpose_body<unsigned>(a, n, (unsigned (*)[EP_SF_TILE + 1])lds);
+    } else {
+        if (wide) sf_transpose_wide<unsigned short>(a, n, lds);
+        else sf_transpose_body<unsigned short>(a, n, (unsigned (*)[EP_SF_TILE + 1])lds);
     }
-    sf_transpose_body<unsigned short>(a, tile);
 }
 
 // ------------------------------------------------------------------------------------------------

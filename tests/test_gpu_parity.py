@@ -579,3 +579,21 @@ def test_scale_packs_of_any_count_and_stride(packs, alignment):
             assert np.array_equal(rsf.cpu().numpy(), es.view(np.int16).reshape(n, packs)), (name, col_major)
             assert np.array_equal(rx.view(torch.uint8).cpu().numpy(), ex), (name, col_major)
     buf.destroy()
+
+
+@pytest.mark.parametrize('H', [8, 128, 520, 8192, 8200])
+def test_column_major_scales_of_the_fused_quantiser(H):
+    """4-byte scales as columns: one column, a partial group, rows as wide as one go takes and one column wider."""
+    T, E, K = 130, 6, 2
+    topk, w = make_routing(T, E, K, seed=H)
+    x = make_tokens(T, H, seed=H)
+    buf = _buffer(T, H, K, fp8=True)
+    for alignment in (1, 4):
+        lay = O.rank_share_layout(topk.numpy(), E, 1, 0, alignment, T)
+        q, s = O.quantise(x)
+        _, es, _ = O.rank_share_dispatch(q.numpy(), s.numpy().view(np.uint32), w.numpy(), lay)
+        (_, rsf), _, _, _, _ = buf.dispatch(x.to(DEV), topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E,
+                                            expert_alignment=alignment, do_expand=True, do_zero_padding=True,
+                                            use_tma_aligned_col_major_sf=True, fused_fp8_quant=True)
+        assert np.array_equal(np.ascontiguousarray(rsf.cpu().numpy()).view(np.uint32), es)
+    buf.destroy()
