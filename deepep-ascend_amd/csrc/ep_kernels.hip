@@ -366,20 +366,20 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
             // (token and position of an id are carried along from load to load instead of divided out)
             const int tok_step = EP_LAYOUT_THREADS / K, pos_step = EP_LAYOUT_THREADS - tok_step * K;
             int tok = tid / K, pos = tid - tok * K;
-            // all ids at once, in up to three goes of eight a thread (as many as there are blocks to read: the same in
+            // all ids at once, in up to four goes of eight a thread (as many as there are blocks to read: the same in
             // every thread, so that a short launch neither asks for nor looks at the rest)
-            constexpr int GO = EP_RECOUNT_DEPTH / 3;
-            const int goes = (n_all + GO * EP_LAYOUT_THREADS - 1) / (GO * EP_LAYOUT_THREADS);      // 1..3 (the host's limit)
-            int64_t v[3][GO];
+            constexpr int GOES = 4, GO = EP_RECOUNT_DEPTH / GOES;
+            const int goes = (n_all + GO * EP_LAYOUT_THREADS - 1) / (GO * EP_LAYOUT_THREADS);      // 1..4 (the host's limit)
+            int64_t v[GOES][GO];
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
+            for (int c = 0; c < GOES; ++c) {
                 if (c >= goes) break;
 #pragma unroll
                 for (int u = 0; u < GO; ++u) v[c][u] = a.topk_idx[min((int64_t)tid + (c * GO + u) * EP_LAYOUT_THREADS, key_total - 1)];
             }
             __builtin_amdgcn_sched_barrier(0);      // (every id is asked for before the first is looked at)
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
+            for (int c = 0; c < GOES; ++c) {
                 if (c >= goes) break;
 #pragma unroll
                 for (int u = 0; u < GO; ++u) {

@@ -278,7 +278,7 @@ def set_layout_fold_max_blocks(num_blocks: int) -> None:
 
 
 def set_layout_recount_limit(blocks_times_topk: int) -> None:
-    """Tuning: with one partition and few layout blocks (blocks x top-k up to this limit, at most 48; 0: never) the slot
+    """Tuning: with one partition and few layout blocks (blocks x top-k up to this limit, at most 64; 0: never) the slot
     assignment counts the ids of all blocks itself and the histogram kernel is not launched.  Results do not depend on it."""
     _ep_set_recount(int(blocks_times_topk))
 

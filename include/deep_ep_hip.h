@@ -178,7 +178,7 @@ int64_t ep_dispatch_stamp(ep_buffer_t* buf);
  * not depend on it. */
 void ep_set_layout_fold_max_blocks(int num_blocks);
 
-/* Tuning: with one partition and few layout blocks (blocks x top-k up to this limit; default and most 48, 0 turns it
+/* Tuning: with one partition and few layout blocks (blocks x top-k up to this limit; default and most 64, 0 turns it
  * off) the histogram kernel is not launched: every workgroup of the slot assignment counts the ids of all blocks itself.
  * Results do not depend on it. */
 void ep_set_layout_recount_limit(int blocks_times_topk);

@@ -88,3 +88,22 @@ def test_small_dispatch_deferred_exact_and_replayed():
         assert torch.equal(h.recv_src_metadata, h0.recv_src_metadata)
         assert torch.equal(h.dst_buffer_slot_idx, h0.dst_buffer_slot_idx)
     buf.destroy()
+
+
+@pytest.mark.parametrize('T,E,K', [(1021, 64, 7), (1024, 256, 8), (1025, 256, 8), (257, 48, 21), (900, 16, 6)])
+def test_ids_of_all_blocks_counted_in_place(T, E, K):
+    """Around the most blocks x top-k (64) for which no histogram kernel runs: every workgroup reads all ids itself."""
+    import deep_ep
+    H, A = 64, 4
+    x = make_tokens(T, H, seed=T).to(DEV)
+    topk, w = make_routing(T, E, K, seed=K, masked=0.1)
+    topk[5] = -1
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    deep_ep._C.set_layout_recount_limit(64)             # (another test may have left a lower one)
+    _, _, _, handle, _ = buf.dispatch(x, topk_idx=topk.to(DEV), num_experts=E, expert_alignment=A, do_expand=True)
+    torch.cuda.synchronize()
+    for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
+                 'dst_buffer_slot_idx', 'recv_src_metadata'):
+        assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
+    buf.destroy()
