@@ -1287,8 +1287,8 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_scatter_quant_sw
 // The payload is fetched before the ids are looked at.  Workgroup 0 publishes what the assignment's publishing workgroup
 // does, the next ones copy (or, with several partitions, pack) as the kernels above, the last zero the padding.
 // Bound by the launch, two trips to memory and the phases in LDS between them.  Assignment + copy -> this kernel (us): 32 tokens,
-// top-8 of 256, FP8 8.8 + 6.2 -> 10.1; 61 tokens x 5120, top-6 of 160, BF16 7.5 + 4.2 -> 8.2; 128 tokens, top-8, 230 MB of
-// padding 10.0 + 31.2 -> 35.3; one of eight partitions of 64 tokens 11.2 + 5.6 -> 10.7.
+// top-8 of 256, FP8 8.8 + 6.2 -> 9.0; 61 tokens x 5120, top-6 of 160, BF16 7.5 + 4.2 -> 8.2; 128 tokens, top-8, 230 MB of
+// padding 10.0 + 31.2 -> 35.3; one of eight partitions of 64 tokens 11.2 + 5.6 -> 10.1.
 // ------------------------------------------------------------------------------------------------
 template <bool QUANT, bool HW, bool PACK>
 __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
@@ -1438,8 +1438,11 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
         // (the same expert twice in one token: the earlier one counts too)
         int c0 = __popcll(__ballot(e == ej) & ((1ull << j) - 1ull));
 #pragma unroll
-        for (int c = 0; c < CH; ++c)                    // (a break would keep the loop from being unrolled: 10.7 -> 10.1 us)
-            if (c < chunks) c0 += __popcll(__ballot(key[c] == ej));
+        for (int c = 0; c < CH; c += 4)                 // (four chunks a branch; a break would keep the loop from being unrolled)
+            if (c < chunks) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) c0 += __popcll(__ballot(key[c + q] == ej));
+            }
         if (lane == j) rank = c0;
     }
     // ---- masters: the last entry of the token for a partition; its slot there ----
