@@ -38,9 +38,13 @@
 // Fixed header of every arena's workspace; the layout scratch is carved behind it.
 //   [0, 4*EP_MAX_RANKS)                    inbox: rows each source partition put into this partition's regions
 //   [EP_WS_PEERS_OFF, +8*EP_MAX_RANKS)     arena base of every partition of the node (own arena when not connected)
+//   [EP_WS_HOST_BOXES_OFF, header end)     device address of every partition's host boxes (nodes of at most
+//                                          EP_HOST_BOXES_MAX_RANKS partitions; the hosts of larger ones read their own pages)
 #define EP_WS_INBOX_OFF 0
 #define EP_WS_PEERS_OFF 1024
+#define EP_WS_HOST_BOXES_OFF 3072
 #define EP_WS_HEADER_BYTES 4096
+#define EP_HOST_BOXES_MAX_RANKS ((EP_WS_HEADER_BYTES - EP_WS_HOST_BOXES_OFF) / 8)
 
 #define EP_HOST_RANK_OFF 16
 #define EP_HOST_EXPERT_OFF (16 + EP_MAX_RANKS)
@@ -51,8 +55,6 @@
 #define EP_HOST_BOX_ROWS_OFF EP_MAX_EXPERTS
 #define EP_HOST_BOX_SEQ_OFF (EP_HOST_BOX_ROWS_OFF + EP_MAX_RANKS)
 #define EP_HOST_BOX_INTS (EP_HOST_BOX_SEQ_OFF + EP_MAX_RANKS)
-// Workspace of a connected partition, behind the header: device address of every partition's host boxes.
-#define EP_WS_HOST_BOXES_BYTES (8 * EP_MAX_RANKS)
 
 struct EpLayoutArgs {
     const int64_t* topk_idx;      // [T, K]

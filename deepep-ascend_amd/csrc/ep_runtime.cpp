@@ -370,7 +370,6 @@ unsigned layout_place_lds(int E, int R, int K) {
 struct RankBoxes {
     int64_t count_off = 0, rank_off = 0, end = EP_WS_HEADER_BYTES;
     bool used = false;
-    static constexpr int64_t kBegin = EP_WS_HEADER_BYTES + EP_WS_HOST_BOXES_BYTES;
 };
 // Every partition of a node comes to the same answer: only what all of them agree on goes in.  Without room for the boxes
 // beside the send side's scratch of max_tokens tokens (32 partitions of 16384 tokens at top-6 fit), or for the counters
@@ -379,14 +378,13 @@ RankBoxes rank_boxes(const ep_buffer* b, int max_tokens, int K, int E) {
     RankBoxes x;
     const int R = b->num_ranks;
     if (R == 1 or not b->connected) return x;
-    x.end = RankBoxes::kBegin;
     auto a256 = [](int64_t n) { return align_up(std::max<int64_t>(n, 1), 256); };
     const int64_t W = align_up(E + R, 8), blocks = std::max<int64_t>(1, ceil_div(max_tokens, EP_TOKENS_PER_BLOCK));
     const int64_t counts = a256(4 * (int64_t)E), ranks = a256(4 * (int64_t)R * max_tokens * K);
     const int64_t scratch = a256(4 * W) + a256(4 * blocks * W) + a256(4 * (int64_t)max_tokens * K);
-    if (RankBoxes::kBegin + counts + ranks + scratch > b->workspace_bytes) return x;
+    if (EP_WS_HEADER_BYTES + counts + ranks + scratch > b->workspace_bytes) return x;
     if (layout_assign_lds(E, R, K, E, 0) > 64 * 1024 or layout_place_lds(E, R, K) > 64 * 1024) return x;
-    x.count_off = RankBoxes::kBegin;
+    x.count_off = EP_WS_HEADER_BYTES;
     x.rank_off = x.count_off + counts;
     x.end = x.rank_off + ranks;
     x.used = true;
@@ -579,11 +577,11 @@ int ep_buffer_connect(ep_buffer_t** bufs, int n) {
             arenas[i] = bufs[i]->arena;
         }
         HIP_CHECK(hipDeviceSynchronize());
-        std::vector<int*> boxes(EP_MAX_RANKS, nullptr);
-        for (int i = 0; i < n; ++i) boxes[i] = bufs[i]->host_page_dev + EP_HOST_PAGE_INTS;
+        std::vector<int*> boxes(EP_HOST_BOXES_MAX_RANKS, nullptr);
+        for (int i = 0; i < std::min(n, EP_HOST_BOXES_MAX_RANKS); ++i) boxes[i] = bufs[i]->host_page_dev + EP_HOST_PAGE_INTS;
         for (int i = 0; i < n; ++i) {
             write_peer_table(bufs[i], arenas);
-            HIP_CHECK(hipMemcpy(bufs[i]->arena + EP_WS_HEADER_BYTES, boxes.data(), EP_WS_HOST_BOXES_BYTES, hipMemcpyHostToDevice));
+            HIP_CHECK(hipMemcpy(bufs[i]->arena + EP_WS_HOST_BOXES_OFF, boxes.data(), sizeof(int*) * boxes.size(), hipMemcpyHostToDevice));
             memset(bufs[i]->host_page + EP_HOST_PAGE_INTS, 0, 2 * EP_HOST_BOX_INTS * sizeof(int));     // (a former node's counts)
             bufs[i]->connected = true;
             bufs[i]->peers.assign(bufs, bufs + n);
@@ -867,9 +865,9 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
         la.notify_host = do_cpu_sync and R == 1 ? 1 : 0;
         // a node in this process: the counts go to every receiver's host as well (arenas that were only mapped here
         // have no host pages this process knows: their counts come from the receive side)
-        const bool notify_peers = boxes.used and do_cpu_sync and not b->peers.empty();
+        const bool notify_peers = boxes.used and do_cpu_sync and not b->peers.empty() and R <= EP_HOST_BOXES_MAX_RANKS;
         if (notify_peers) {
-            la.host_boxes = (int* const*)(b->workspace() + EP_WS_HEADER_BYTES);
+            la.host_boxes = (int* const*)(b->workspace() + EP_WS_HOST_BOXES_OFF);
             la.host_box_slot = (b->num_sends & 1) * EP_HOST_BOX_INTS;
         }
         la.dst_buffer_slot_idx = (int*)a.dst_buffer_slot_idx.data;
