@@ -271,9 +271,8 @@ struct ep_buffer {
         bool notifies_peers = false;// ... and their counts in the receivers' host boxes
         bool host_boxes = false;    // this partition's host counts come from its host boxes, filled by the send sides
         int send_seq = 0;           // the sequence number the sources left there
-        bool layout_pending = false;// the layout is left to the copy launch (pending, on pending_stream)
+        bool layout_pending = false;// the layout is left to the copy launch, whatever stream that comes on
         EpLayoutArgs pending{};
-        void* pending_stream = nullptr;
         bool copied = false;        // the copy launch has used it up: the workspace holds no layout to copy by again
         bool recv_done = false;     // more than one partition: the receive-side layout has been enqueued
     } last;
@@ -885,7 +884,6 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
         } else if (small and epilogue_follows) {
             b->last.layout_pending = true;
             b->last.pending = la;
-            b->last.pending_stream = a.stream;
         } else {
             launch_layout(la, num_blocks, a.stream);
         }
@@ -1249,9 +1247,10 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
         const bool pending = not cached_mode and b->last.layout_pending;
         b->last.layout_pending = false;
         EP_HOST_ASSERT((cached_mode or not b->last.copied) and "an ep_dispatch_begin has one copy epilogue");
-        const bool whole = pending and b->last.pending_stream == a.stream and sa.num_row_blocks > 0;
-        if (pending and not whole) launch_layout(b->last.pending, 1, b->last.pending_stream);
-        if (whole) {
+        if (pending) {
+            // (one partition, tokens and metadata rows at hand: there are row workgroups.  The layout runs on this call's
+            // stream, whichever the begin came on: a caller who changes streams has ordered this one behind the begin)
+            EP_HOST_ASSERT(sa.num_row_blocks > 0);
             b->last.copied = true;
             launch_small(b->last.pending, sa, false, quantise_here, (int)std::min(pad_blocks, kSmallPadBlocks), a.stream);
         } else if (grid > 0) {

@@ -149,8 +149,10 @@ typedef struct ep_dispatch_args {
 int ep_dispatch_launch(ep_buffer_t* buf, const ep_dispatch_args_t* args);
 /* The same for a caller whose next call on this buffer is this dispatch's ep_dispatch_epilogue_launch: the library may
  * then leave the layout to the copy launch (one partition, at most 128 tokens and 1024 (token, slot) entries: one
- * launch instead of two; the handle tensors are complete behind the epilogue).  Counts can be waited for after the
- * epilogue only. */
+ * launch instead of two).  Everything this call would have enqueued is then enqueued by the epilogue, on the epilogue's
+ * stream: the handle tensors, the running statistics and the host counts are complete behind the epilogue only, and the
+ * inputs have to stay until then.  An epilogue on another stream is ordered behind what the begin is ordered behind by
+ * the caller, as after ep_dispatch_launch (an event recorded after the begin, waited for on the other stream). */
 int ep_dispatch_begin(ep_buffer_t* buf, const ep_dispatch_args_t* args);
 
 typedef struct ep_dispatch_recv_args {

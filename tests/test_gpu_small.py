@@ -1,5 +1,7 @@
 """Dispatches of decode size, layout and copy in one launch: handles and rows of the oracle at the edges of what that
 launch takes, in every payload form, with and without a host sync, and the calls around it that it must not change."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -106,4 +108,77 @@ def test_ids_of_all_blocks_counted_in_place(T, E, K):
     for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
                  'dst_buffer_slot_idx', 'recv_src_metadata'):
         assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
+    buf.destroy()
+
+
+class AbiDispatch:
+    """One BF16 dispatch through the C ABI: descriptors and outputs of the two calls it is made of."""
+
+    def __init__(self, C, buf, T, H, E, K, A, x, topk, w):
+        n_recv, n_exp = ctypes.c_int(), ctypes.c_int()
+        C._check(C._ep_worst(None, T, K, E, A, ctypes.byref(n_recv), ctypes.byref(n_exp)))
+        i32 = dict(dtype=torch.int32, device=DEV)
+        self.C, self.buf = C, buf
+        self.keep = (x, topk, w)
+        self.psum_expert = torch.full((E,), -7, **i32)
+        self.counts = [torch.full((1,), -7, **i32), torch.full((E,), -7, **i32), torch.full((T, K), -7, **i32)]
+        self.dst_slot = torch.full((T, K), -7, **i32)
+        self.meta = torch.full((T, K + 2), -7, **i32)
+        self.rows = torch.full((n_exp.value, H), 77, dtype=torch.int16, device=DEV).view(torch.bfloat16)
+        self.gates = torch.full((n_exp.value,), -7.0, device=DEV)
+        self.a, self.e = C._DispatchArgs(), C._DispatchEpilogueArgs()
+        for f in (self.a, self.e):
+            f.x, f.topk_weights = C._desc(x), C._desc(w)
+            f.psum_num_recv_tokens_per_rank, f.psum_num_recv_tokens_per_expert = C._desc(self.counts[0]), C._desc(self.psum_expert)
+            f.num_max_tokens_per_rank, f.num_experts, f.expert_alignment = T, E, A
+        self.a.topk_idx, self.a.num_unaligned_recv_tokens_per_expert = C._desc(topk), C._desc(self.counts[1])
+        self.a.dst_buffer_slot_idx, self.a.dst_gsge_idx = C._desc(self.dst_slot), C._desc(self.counts[2])
+        self.e.recv_x, self.e.recv_topk_weights, self.e.recv_src_metadata = C._desc(self.rows), C._desc(self.gates), C._desc(self.meta)
+        self.e.num_topk, self.e.do_zero_padding = K, 1
+        torch.cuda.synchronize()
+
+    def begin(self, stream):
+        self.a.stream = stream.cuda_stream
+        self.C._check(self.C._ep_dispatch_begin(self.buf.runtime._h, ctypes.byref(self.a)))
+        self.e.dispatch_stamp = self.C._ep_stamp(self.buf.runtime._h)
+
+    def epilogue(self, stream):
+        self.e.stream = stream.cuda_stream
+        self.C._check(self.C._ep_dispatch_epi(self.buf.runtime._h, ctypes.byref(self.e)))
+
+    def check(self, x, topk, w, E, A):
+        T = x.size(0)
+        lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
+        n, ne = lay['num_recv_tokens'], lay['num_expanded_tokens']
+        ex, _, ew = O.rank_share_dispatch(bf16_bits(x), None, w.numpy(), lay)
+        assert np.array_equal(self.psum_expert.cpu().numpy(), lay['psum_num_recv_tokens_per_expert'])
+        assert np.array_equal(self.dst_slot.cpu().numpy(), lay['dst_buffer_slot_idx'])
+        assert np.array_equal(self.meta.cpu().numpy()[:n], lay['recv_src_metadata'])
+        assert np.array_equal(bf16_bits(self.rows)[:ne], ex)
+        assert np.array_equal(self.gates.cpu().numpy().view(np.uint32)[:ne], ew.view(np.uint32))
+
+
+def test_begin_and_epilogue_on_two_streams():
+    """The epilogue of an ep_dispatch_begin on another stream, ordered behind the begin by an event only: the ids arrive
+    late on the first stream, and every pass routes differently, so that a layout of the pass before would show."""
+    import deep_ep
+    C = deep_ep._C
+    T, H, E, K, A = 96, 256, 16, 4, 8
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    x = make_tokens(T, H, seed=4)
+    first, second = torch.cuda.Stream(), torch.cuda.Stream()
+    for seed in range(4):
+        topk, w = make_routing(T, E, K, seed=20 + seed, masked=0.1 * seed)
+        source, late = topk.to(DEV), torch.full_like(topk, -1).to(DEV)
+        d = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), late, w.to(DEV))
+        with torch.cuda.stream(first):
+            for _ in range(4):
+                junk = torch.randn((1024, 1024), device=DEV) @ torch.randn((1024, 1024), device=DEV)
+            late.copy_(source)
+        d.begin(first)
+        second.wait_event(first.record_event())
+        d.epilogue(second)
+        torch.cuda.synchronize()
+        del junk
+        d.check(x, topk, w, E, A)
     buf.destroy()
