@@ -1244,15 +1244,15 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
         sa.pad_blocks_per_expert = std::max(1, std::min(EP_MAX_PAD_BLOCKS_PER_EXPERT, a.expert_alignment / 8));
         const unsigned pad_blocks = a.do_zero_padding and a.expert_alignment > 1 ? (unsigned)(El * sa.pad_blocks_per_expert) : 0u;
         const unsigned grid = (unsigned)sa.num_row_blocks + pad_blocks;
-        const bool pending = not cached_mode and b->last.layout_pending;
-        b->last.layout_pending = false;
+        const bool pending = not cached_mode and b->last.layout_pending;      // (a cached epilogue in between leaves it waiting)
         EP_HOST_ASSERT((cached_mode or not b->last.copied) and "an ep_dispatch_begin has one copy epilogue");
         if (pending) {
             // (one partition, tokens and metadata rows at hand: there are row workgroups.  The layout runs on this call's
             // stream, whichever the begin came on: a caller who changes streams has ordered this one behind the begin)
             EP_HOST_ASSERT(sa.num_row_blocks > 0);
-            b->last.copied = true;
             launch_small(b->last.pending, sa, false, quantise_here, (int)std::min(pad_blocks, kSmallPadBlocks), a.stream);
+            b->last.layout_pending = false;
+            b->last.copied = true;
         } else if (grid > 0) {
             hipFunction_t fn = quantise_here ? (g_fp8_hw ? g_k.scatter_quant : g_k.scatter_quant_sw) : g_k.scatter_copy;
             launch(fn, grid, EP_ROW_THREADS, 0, a.stream, sa);

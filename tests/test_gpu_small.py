@@ -182,3 +182,30 @@ def test_begin_and_epilogue_on_two_streams():
         del junk
         d.check(x, topk, w, E, A)
     buf.destroy()
+
+
+def test_cached_epilogue_between_begin_and_its_epilogue():
+    """A replay of another handle between the two calls leaves the waiting layout where it is."""
+    import deep_ep
+    C = deep_ep._C
+    T, H, E, K, A = 96, 256, 16, 4, 8
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    x = make_tokens(T, H, seed=6)
+    stream = torch.cuda.current_stream()
+    old_topk, old_w = make_routing(T, E, K, seed=40)
+    old = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), old_topk.to(DEV), old_w.to(DEV))
+    old.begin(stream)
+    old.epilogue(stream)
+    topk, w = make_routing(T, E, K, seed=41, masked=0.2)
+    d = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), topk.to(DEV), w.to(DEV))
+    d.begin(stream)
+    old.rows.zero_()
+    old.e.cached_mode = 1
+    old.epilogue(stream)
+    d.epilogue(stream)
+    torch.cuda.synchronize()
+    old.check(x, old_topk, old_w, E, A)
+    d.check(x, topk, w, E, A)
+    with pytest.raises(C.EPException, match='one copy epilogue'):
+        d.epilogue(stream)
+    buf.destroy()
