@@ -1250,6 +1250,9 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
             // (one partition, tokens and metadata rows at hand: there are row workgroups.  The layout runs on this call's
             // stream, whichever the begin came on: a caller who changes streams has ordered this one behind the begin)
             EP_HOST_ASSERT(sa.num_row_blocks > 0);
+            // the one launch sizes its LDS by the begin's experts and pads by the epilogue's
+            EP_HOST_ASSERT(a.num_experts == b->last.num_experts and a.expert_alignment == b->last.alignment and
+                           "the copy epilogue has the experts and the alignment of its ep_dispatch_begin");
             launch_small(b->last.pending, sa, false, quantise_here, (int)std::min(pad_blocks, kSmallPadBlocks), a.stream);
             b->last.layout_pending = false;
             b->last.copied = true;

@@ -209,3 +209,30 @@ def test_cached_epilogue_between_begin_and_its_epilogue():
     with pytest.raises(C.EPException, match='one copy epilogue'):
         d.epilogue(stream)
     buf.destroy()
+
+
+@pytest.mark.parametrize('field,value', [('experts', 64), ('experts', 8), ('alignment', 16)])
+def test_epilogue_of_other_experts_or_alignment_is_refused(field, value):
+    """The one launch counts in LDS sized by the begin's experts: an epilogue that names others is refused on the host,
+    and the right one still runs."""
+    import deep_ep
+    C = deep_ep._C
+    T, H, E, K, A = 64, 128, 16, 4, 8
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    x = make_tokens(T, H, seed=7)
+    topk, w = make_routing(T, E, K, seed=42, masked=0.2)
+    d = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), topk.to(DEV), w.to(DEV))
+    stream = torch.cuda.current_stream()
+    d.begin(stream)
+    if field == 'experts':
+        other = torch.zeros(value, dtype=torch.int32, device=DEV)
+        d.e.num_experts, d.e.psum_num_recv_tokens_per_expert = value, C._desc(other)
+    else:
+        d.e.expert_alignment = value
+    with pytest.raises(C.EPException, match='of its ep_dispatch_begin'):
+        d.epilogue(stream)
+    d.e.num_experts, d.e.expert_alignment, d.e.psum_num_recv_tokens_per_expert = E, A, C._desc(d.psum_expert)
+    d.epilogue(stream)
+    torch.cuda.synchronize()
+    d.check(x, topk, w, E, A)
+    buf.destroy()
