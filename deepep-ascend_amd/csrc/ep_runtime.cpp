@@ -806,16 +806,20 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
             launch(fn, (unsigned)sa.num_row_blocks, EP_ROW_THREADS, 0, a.stream, sa);
         };
 
-        if (num_ranks > 1) {
-            // the rows about to be packed overwrite what the peers received last time
+        // the rows about to be packed overwrite what the peers received last time
+        if (num_ranks > 1)
             check_peers(b, [&](const ep_buffer& p) { return p.num_expands >= b->num_sends; },
                         "has not run the copy epilogue of the previous dispatch yet");
-            ++b->num_sends;
-        }
+        // (counted once everything is enqueued: a dispatch that is refused on the way is none to the peers, whose receive
+        //  sides would otherwise take the counts of the one before for its)
+        const int64_t send = b->num_sends + 1;
         if (cached_mode) {
             // the cached handle already holds the whole layout: only the packed regions are refreshed
             b->last.valid = b->last.layout_pending = false;
-            if (num_ranks > 1) launch_pack();
+            if (num_ranks > 1) {
+                launch_pack();
+                b->num_sends = send;
+            }
             return;
         }
 
@@ -860,14 +864,14 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
         la.max_tokens = a.num_max_tokens_per_rank;
         la.experts_per_rank = num_experts_per_rank;
         la.num_blocks = num_blocks;
-        la.seq = R == 1 ? ++b->seq : (int)b->num_sends;
+        la.seq = R == 1 ? ++b->seq : (int)send;
         la.notify_host = do_cpu_sync and R == 1 ? 1 : 0;
         // a node in this process: the counts go to every receiver's host as well (arenas that were only mapped here
         // have no host pages this process knows: their counts come from the receive side)
         const bool notify_peers = boxes.used and do_cpu_sync and not b->peers.empty() and R <= EP_HOST_BOXES_MAX_RANKS;
         if (notify_peers) {
             la.host_boxes = (int* const*)(b->workspace() + EP_WS_HOST_BOXES_OFF);
-            la.host_box_slot = (b->num_sends & 1) * EP_HOST_BOX_INTS;
+            la.host_box_slot = (send & 1) * EP_HOST_BOX_INTS;
         }
         la.dst_buffer_slot_idx = (int*)a.dst_buffer_slot_idx.data;
         la.dst_gsge_idx = (int*)a.dst_gsge_idx.data;
@@ -888,7 +892,10 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
             launch_layout(la, num_blocks, a.stream);
         }
 
-        if (num_ranks > 1) launch_pack();
+        if (num_ranks > 1) {
+            launch_pack();
+            b->num_sends = send;
+        }
 
         b->last.valid = true;
         b->last.stamp = ++b->launch_stamp;

@@ -241,6 +241,48 @@ def test_node_receive_layout(R, max_tokens, Ts, E, K):
         b.destroy()
 
 
+def test_a_refused_dispatch_counts_for_nothing():
+    """A dispatch that a partition refuses on the way (its layout scratch does not fit): the partition dispatches again and
+    everything arrives; the receive sides of the others are refused until it has, instead of waiting for host counts that
+    nobody sends."""
+    import deep_ep
+    R, E, K, H, A, T, most = 2, 2048, 1, 16, 4, 64, 524288
+    node = deep_ep.LocalNode(R)
+    bufs = [deep_ep.EPBuffer(node.group(r), num_max_tokens_per_rank=most, hidden=H, num_topk=K, num_cpu_timeout_secs=5,
+                             explicitly_destroy=True) for r in range(R)]
+    kw = dict(num_experts=E, expert_alignment=A, do_expand=True, do_zero_padding=True, async_with_compute_stream=True,
+              defer_epilogue=True)
+    xs = [make_tokens(T, H, seed=r) for r in range(R)]
+
+    def send(r, seed):
+        topk, w = make_routing(T, E, K, seed=seed + r)
+        return topk, w, bufs[r].dispatch(xs[r].to(DEV), topk_idx=topk.to(DEV), topk_weights=w.to(DEV),
+                                         num_max_tokens_per_rank=T, **kw)
+
+    def refused(r):
+        with pytest.raises(deep_ep._C.EPException, match='workspace_bytes'):
+            bufs[r].dispatch(torch.zeros((most, H), dtype=torch.bfloat16, device=DEV), num_max_tokens_per_rank=most,
+                             topk_idx=torch.zeros((most, K), dtype=torch.int64, device=DEV), **kw)
+
+    for seed in (10, 20):
+        if seed == 20:
+            refused(1)
+        sent = [send(r, seed) for r in range(R)]
+        outs = [s[2].current_stream_wait() for s in sent]
+        torch.cuda.synchronize()
+        rows = [bf16_bits(x).view(np.uint8).reshape(T, H * 2) for x in xs]
+        _, want = oracle_dispatch(rows, [None] * R, [s[0].numpy() for s in sent], [s[1].numpy() for s in sent], E, R, A, T)
+        for r, (rx, _, _, handle) in enumerate(outs):
+            assert handle.num_recv_tokens_per_expert_list == want[r]['lay']['num_recv_tokens_per_expert_list']
+            assert np.array_equal(rx.view(torch.uint8).cpu().numpy().reshape(rx.size(0), H * 2), want[r]['x'])
+    alone = send(0, 30)[2]
+    refused(1)
+    with pytest.raises(deep_ep._C.EPException, match='comes before any receive side'):
+        alone.current_stream_wait()
+    for b in bufs:
+        b.destroy()
+
+
 def test_node_reproduces_the_reference_dispatch_vectors():
     """tests/golden/dispatch_golden_w2.npz: inputs of both ranks and what refs.dispatch gave each of them
     (received rows in source order, local expert ids, weights, source tokens, per-source counts)."""
