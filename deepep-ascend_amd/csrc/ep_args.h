@@ -20,6 +20,12 @@
 #define EP_LAYOUT_RECOUNTED 3     // no kernel in front: every workgroup counts the ids of all (few) blocks itself
 #define EP_RECOUNT_DEPTH 32       // ids a thread of the slot assignment holds in flight for that (blocks x top-k <= 2 x this)
 
+// Instances of the slot assignment: one partition; of several, the send side (dst_buffer_slot_idx, dst_gsge_idx, the peers'
+// inboxes and boxes) and the receive side
+#define EP_LAYOUT_SIDE_SINGLE 0
+#define EP_LAYOUT_SIDE_SEND 1
+#define EP_LAYOUT_SIDE_RECV 2
+
 #define EP_SCATTER_EXPAND 0
 #define EP_SCATTER_PACK 1
 #define EP_SCATTER_REGION 2
@@ -85,7 +91,6 @@ struct EpLayoutArgs {
     int* cumulative_stats;        // [El] or null
     int* host_page;               // device view of the mapped host page
     // partitioned path (more than one partition)
-    int send_only;                // send side: only dst_buffer_slot_idx / dst_gsge_idx and the peers' inboxes are written
     int recv_mode;                // receive side: the entries are the rows that arrived in this partition's regions
     char* const* peer_arenas;     // [R] arena bases (send side: whose inbox gets this partition's row counts)
     const int* inbox;             // [R] rows per source (receive side)

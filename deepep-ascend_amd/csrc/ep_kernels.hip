@@ -304,12 +304,16 @@ extern "C" __global__ __launch_bounds__(EP_SCAN_THREADS) void ep_layout_scan(EpL
 #define EP_KEY_MASTER 0x4000          // flag in a staged key: the entry is the master of its partition (ids < 2048)
 #define EP_LAYOUT_MAX_COLS_PER_THREAD ((EP_MAX_EXPERTS + EP_MAX_RANKS + EP_LAYOUT_THREADS - 1) / EP_LAYOUT_THREADS)
 
-// Four instances.  FOLD: for EP_LAYOUT_FOLDED (the other modes run one without the summing code).  RECV: for the
-// receive side of a node (a.recv_mode).
-template <bool FOLD, bool RECV>
+// Six instances.  FOLD: for EP_LAYOUT_FOLDED (the other modes run one without the summing code).  SIDE: one partition, or
+// the send or the receive side of several.  (With the send side's shipping of counts in the instance of one partition, which
+// never runs it, that instance took 11.0 instead of 10.2 us at 129 tokens and 12.1 instead of 11.6 at 1024, top-8 of 256.)
+enum LayoutSide { SIDE_SINGLE = EP_LAYOUT_SIDE_SINGLE, SIDE_SEND = EP_LAYOUT_SIDE_SEND, SIDE_RECV = EP_LAYOUT_SIDE_RECV };
+template <bool FOLD, LayoutSide SIDE>
 __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
+    constexpr bool RECV = SIDE == SIDE_RECV, SEND = SIDE == SIDE_SEND;
     extern __shared__ int smem[];
-    const int E = a.num_experts, R = a.num_ranks, K = a.num_topk, El = a.count_experts, A = a.expert_alignment;
+    const int E = a.num_experts, R = a.num_ranks, K = a.num_topk, A = a.expert_alignment;
+    const int El = RECV ? a.experts_per_rank : a.count_experts;
     const int NW = EP_LAYOUT_THREADS / WAVE;
     const int b = blockIdx.x;
     int* s_tot = smem;                     // [El + R] totals of the counted experts, then of the partitions
@@ -320,7 +324,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
     short* s_rk = s_key + EP_TOKENS_PER_BLOCK * K;
     int* s_psum = (int*)(s_rk + EP_TOKENS_PER_BLOCK * K);      // [R + NW]  (receive side)
     const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
-    const int lo = a.count_lo;
+    const int lo = RECV ? a.rank_idx * El : a.count_lo;
     const int ncols = El + R;              // column c < El: expert lo + c; else partition c - El
 
     // The launch has one workgroup more than blocks of tokens.  It ranks nothing: it gets the totals like the others
@@ -351,7 +355,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
     // go: a histogram of all of them (the totals), one of the blocks before its own, its own block's ids staged on the
     // way.  With one partition the master of a token is its last valid position: the partition's column counts the
     // tokens that have a valid id at all (flags in LDS, counted by ballot).
-    const bool recount = !FOLD && !RECV && a.scan_mode == EP_LAYOUT_RECOUNTED;
+    const bool recount = !FOLD && SIDE == SIDE_SINGLE && a.scan_mode == EP_LAYOUT_RECOUNTED;
     if (recount) {
         int* s_rpre = s_psum + R + NW;                         // [ncols]
         int* s_rtot = s_rpre + ncols;                          // [ncols]
@@ -603,13 +607,13 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
         int run = wave_off + incl - mine;
         for (int e = e0; e < e1; ++e) {
             const int c = s_tot[e];
-            if (publisher && !a.send_only) {
+            if (publisher && !SEND) {
                 a.unaligned_expert[e] = c;
                 a.psum_expert[e] = run + c;
                 if (a.cumulative_stats != nullptr) atomicAdd(&a.cumulative_stats[e], c);
                 if (a.notify_host) a.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
             }
-            if (!RECV && a.send_only) {
+            if (SEND) {
                 // slots are the receivers' business: ranks count from 0, and the receivers get the counts they need
                 // to place them (a partition that is not connected to a node ships nothing)
                 if (publisher && a.count_box_off != 0) {
@@ -624,7 +628,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
             run += align_up(c, A);
         }
     }
-    if (publisher && a.send_only) {
+    if (publisher && SEND) {
         // rows this partition sends to every partition, left in the receivers' inboxes: the count half of
         // the reference's cross-rank reduction (impls/ep/dispatch.hpp:469-545)
         // (a partition that is not connected to a node only has its own inbox)
@@ -644,7 +648,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
                                    __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
-    if (publisher && !a.send_only) {
+    if (publisher && !SEND) {
         // one partition: the receive stream is this partition's own routed tokens; several: the rows counted
         // in the inbox (csrc/buffers/ep.hpp:205-246 names the tensors)
         const int n_recv = RECV ? num_rows : s_tot[El + a.rank_idx];
@@ -717,8 +721,8 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
             } else {
                 a.dst_buffer_slot_idx[g] = rslot;
                 a.dst_gsge_idx[g] = -1;             // every copy is local: no transport descriptors
-                if (a.slot_map != nullptr) a.slot_map[g] = eslot;
-                if (!a.send_only && mr == a.rank_idx) a.tok_row[b * EP_TOKENS_PER_BLOCK + tok] = rslot;
+                if (!SEND || a.slot_map != nullptr) a.slot_map[g] = eslot;
+                if (!SEND && mr == a.rank_idx) a.tok_row[b * EP_TOKENS_PER_BLOCK + tok] = rslot;
             }
         }
         // the running counters of a wave are touched by that wave only and the LDS operations of a wave
@@ -748,10 +752,12 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
     }
 }
 
-extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign(EpLayoutArgs a) { layout_assign_body<false, false>(a); }
-extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_fold(EpLayoutArgs a) { layout_assign_body<true, false>(a); }
-extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_recv(EpLayoutArgs a) { layout_assign_body<false, true>(a); }
-extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_fold_recv(EpLayoutArgs a) { layout_assign_body<true, true>(a); }
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign(EpLayoutArgs a) { layout_assign_body<false, SIDE_SINGLE>(a); }
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_send(EpLayoutArgs a) { layout_assign_body<false, SIDE_SEND>(a); }
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_recv(EpLayoutArgs a) { layout_assign_body<false, SIDE_RECV>(a); }
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_fold(EpLayoutArgs a) { layout_assign_body<true, SIDE_SINGLE>(a); }
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_fold_send(EpLayoutArgs a) { layout_assign_body<true, SIDE_SEND>(a); }
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_fold_recv(EpLayoutArgs a) { layout_assign_body<true, SIDE_RECV>(a); }
 
 // ------------------------------------------------------------------------------------------------
 // Receive side of a node whose send sides ship ranks: nothing is counted or ranked here.  An entry's slot is

@@ -111,7 +111,7 @@ int64_t combine_buffer_size(int ranks, int max_tokens, int hidden, int topk) {
 // ---- code object ------------------------------------------------------------------------------
 struct Kernels {
     hipModule_t module = nullptr;
-    hipFunction_t layout_count, layout_scan, layout_place, layout_assign[2][2];      // [sums the counts itself][receive side]
+    hipFunction_t layout_count, layout_scan, layout_place, layout_assign[2][3];      // [sums the counts itself][EP_LAYOUT_SIDE_*]
     hipFunction_t scatter_copy, scatter_quant, scatter_quant_sw, sf_transpose;
     hipFunction_t scatter_copy_pack, scatter_quant_pack, scatter_quant_sw_pack;
     hipFunction_t small[2][3];       // [packs][copy, quant, quant_sw]
@@ -181,10 +181,11 @@ void load_kernels(const char* dir) {
     get(g_k.layout_count, "ep_layout_count");
     get(g_k.layout_scan, "ep_layout_scan");
     get(g_k.layout_place, "ep_layout_place");
-    get(g_k.layout_assign[0][0], "ep_layout_assign");
-    get(g_k.layout_assign[1][0], "ep_layout_assign_fold");
-    get(g_k.layout_assign[0][1], "ep_layout_assign_recv");
-    get(g_k.layout_assign[1][1], "ep_layout_assign_fold_recv");
+    const char* sides[3] = {"", "_send", "_recv"};      // EP_LAYOUT_SIDE_*
+    for (int side = 0; side < 3; ++side) {
+        get(g_k.layout_assign[0][side], (std::string("ep_layout_assign") + sides[side]).c_str());
+        get(g_k.layout_assign[1][side], (std::string("ep_layout_assign_fold") + sides[side]).c_str());
+    }
     get(g_k.scatter_copy, "ep_scatter_copy");
     get(g_k.scatter_quant, "ep_scatter_quant");
     get(g_k.scatter_quant_sw, "ep_scatter_quant_sw");
@@ -316,7 +317,8 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
     // (two histograms of El + R ints and a byte a token on top of its LDS).  The limit: at 64 blocks x top-k a thread holds 32
     // ids; 1021 tokens at top-7 (56) take 14.4 us in one launch against 4.6 + 10.6 us and the gap between two.
     const unsigned recount_extra = (unsigned)(2 * (E / R + R)) * sizeof(int) + (unsigned)num_blocks * EP_TOKENS_PER_BLOCK;
-    const bool recount = R == 1 and not la.recv_mode and not la.send_only and num_blocks >= 2 and
+    const int side = la.recv_mode ? EP_LAYOUT_SIDE_RECV : R > 1 ? EP_LAYOUT_SIDE_SEND : EP_LAYOUT_SIDE_SINGLE;
+    const bool recount = side == EP_LAYOUT_SIDE_SINGLE and num_blocks >= 2 and
                          (int64_t)num_blocks * K <= std::min(g_recount_limit.load(), 2 * EP_RECOUNT_DEPTH) and
                          layout_assign_lds(E, R, K, C, 0) + recount_extra <= 64 * 1024;
     la.scan_mode = num_blocks == 1 ? EP_LAYOUT_SINGLE
@@ -331,7 +333,7 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
     if (la.scan_mode == EP_LAYOUT_SCANNED)
         launch(g_k.layout_scan, (unsigned)ceil_div(la.cnt_stride, 16), EP_SCAN_THREADS, 0, stream, la);
     // (one workgroup more than blocks: it publishes the totals and ranks nothing)
-    launch(g_k.layout_assign[la.scan_mode == EP_LAYOUT_FOLDED][la.recv_mode != 0], (unsigned)num_blocks + 1u, EP_LAYOUT_THREADS,
+    launch(g_k.layout_assign[la.scan_mode == EP_LAYOUT_FOLDED][side], (unsigned)num_blocks + 1u, EP_LAYOUT_THREADS,
            smem_assign, stream, la);
 }
 
@@ -850,7 +852,6 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
         EP_HOST_ASSERT(off * (int64_t)sizeof(int) <= b->workspace_bytes);
         // more than one partition: this launch is the send side only (slots in the destinations' regions, row
         // counts into their inboxes); the receive side is ep_dispatch_recv_launch
-        la.send_only = R > 1 ? 1 : 0;
         la.peer_arenas = b->peer_table();
         la.connected = b->connected ? 1 : 0;
 

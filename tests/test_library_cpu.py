@@ -50,7 +50,8 @@ def test_code_object_is_built_for_gfx950(de):
 
 def test_code_object_has_every_instance_of_the_slot_assignment(de):
     blob = open(os.path.join(os.path.dirname(LIB), 'ep_kernels.hsaco'), 'rb').read()
-    for k in (b'ep_layout_assign_fold', b'ep_layout_assign_recv', b'ep_layout_assign_fold_recv'):
+    for k in (b'ep_layout_assign_fold', b'ep_layout_assign_send', b'ep_layout_assign_fold_send', b'ep_layout_assign_recv',
+              b'ep_layout_assign_fold_recv'):
         assert k in blob, k
 
 
