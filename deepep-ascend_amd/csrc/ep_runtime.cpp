@@ -153,7 +153,7 @@ unsigned combine_lds_cap(int num_topk, bool specialised, int num_row_blocks, int
     if (share <= 1024u) return 0;
     return std::min(64u * 1024u, share - 1024u);       // n of them fit a CU, n + 1 do not
 }
-std::atomic<int> g_recount_limit{2 * EP_RECOUNT_DEPTH};   // blocks x top-k up to which one partition's slot assignment counts all ids itself
+std::atomic<int> g_recount_limit{-1};     // blocks x top-k up to which one partition's slot assignment counts all ids itself; negative: recount_pays
 std::atomic<int> g_fold_max_blocks{256};    // up to this many layout workgroups the slot assignment sums the block counts itself
 
 std::string library_dir() {
@@ -302,6 +302,18 @@ unsigned layout_assign_lds(int E, int R, int K, int count_experts, int cnt_strid
     return (unsigned)(count_experts + R + nw * (E + R) + nw + 1 + R + nw + 2 * cnt_stride) * sizeof(int) + layout_key_bytes(K);
 }
 
+// Where one launch that counts the ids of all blocks in every workgroup beats a histogram launch in front of the slot
+// assignment.  It saves a launch; each further block is more ids to every workgroup, and one more of these.  us of a replayed
+// dispatch of 16 channels, 256 experts, two launches / one: top-1, 16 blocks 12.8 / 11.6, 24 12.9 / 13.9, 64 14.4 / 21.9; top-2,
+// 12 13.0 / 12.5, 16 13.0 / 13.1, 32 13.6 / 17.8; top-3, 10 14.4 / 13.4, 16 14.6 / 15.6; top-4, 8 14.5 / 13.3, 16 14.8 / 17.0; top-6, 8
+// 16.1 / 15.7, 10 16.3 / 17.3; top-8, 6 17.5 / 16.7, 8 17.6 / 18.3; top-12, 4 21.1 / 18.9; top-32, 2 37.3 / 31.5.  To a host that waits for
+// the counts the saved launch is worth more (wall clock, 8 blocks, top-7 24.3 / 23.7, top-8 25.3 / 25.0).
+bool recount_pays(int num_blocks, int K, bool host_waits) {
+    const int most = 2 * EP_RECOUNT_DEPTH;
+    const int limit = K > 8 ? most : std::min(8 * K, host_waits ? most : 48);
+    return num_blocks <= 16 and num_blocks * K <= std::max(limit, 32);
+}
+
 // The layout pass: per-block histograms, then the slot assignment.  One block needs no histogram pass; up
 // to g_fold_max_blocks blocks the assignment kernel sums the histograms of the blocks before it itself;
 // beyond that a scan kernel turns them into prefixes first.
@@ -314,12 +326,12 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
     const bool fold = (int64_t)num_blocks * (la.cnt_stride / 8) <= (int64_t)g_fold_max_blocks * 33 and
                       la.cnt_stride <= 8 * EP_LAYOUT_THREADS and layout_assign_lds(E, R, K, C, la.cnt_stride) <= 64 * 1024;
     // a few blocks of one partition (send side): the slot assignment counts the ids of all blocks itself, a launch less
-    // (two histograms of El + R ints and a byte a token on top of its LDS).  The limit: at 64 blocks x top-k a thread holds 32
-    // ids; 1021 tokens at top-7 (56) take 14.4 us in one launch against 4.6 + 10.6 us and the gap between two.
+    // (two histograms of El + R ints and a byte a token on top of its LDS; at 64 blocks x top-k a thread holds 32 ids)
     const unsigned recount_extra = (unsigned)(2 * (E / R + R)) * sizeof(int) + (unsigned)num_blocks * EP_TOKENS_PER_BLOCK;
     const int side = la.recv_mode ? EP_LAYOUT_SIDE_RECV : R > 1 ? EP_LAYOUT_SIDE_SEND : EP_LAYOUT_SIDE_SINGLE;
+    const int limit = g_recount_limit.load();
     const bool recount = side == EP_LAYOUT_SIDE_SINGLE and num_blocks >= 2 and
-                         (int64_t)num_blocks * K <= std::min(g_recount_limit.load(), 2 * EP_RECOUNT_DEPTH) and
+                         (limit < 0 ? recount_pays(num_blocks, K, la.notify_host != 0) : num_blocks <= std::min(limit, 2 * EP_RECOUNT_DEPTH) / K) and
                          layout_assign_lds(E, R, K, C, 0) + recount_extra <= 64 * 1024;
     la.scan_mode = num_blocks == 1 ? EP_LAYOUT_SINGLE
                    : recount       ? EP_LAYOUT_RECOUNTED

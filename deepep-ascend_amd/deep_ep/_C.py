@@ -279,8 +279,9 @@ def set_layout_fold_max_blocks(num_blocks: int) -> None:
 
 
 def set_layout_recount_limit(blocks_times_topk: int) -> None:
-    """Tuning: with one partition and few layout blocks (blocks x top-k up to this limit, at most 64; 0: never) the slot
-    assignment counts the ids of all blocks itself and the histogram kernel is not launched.  Results do not depend on it."""
+    """Tuning: with one partition and few layout blocks of 128 tokens the slot assignment counts the ids of all blocks
+    itself and the histogram kernel is not launched.  Negative (default): the library's own rule by blocks and top-k; else
+    blocks x top-k up to this limit (at most 64; 0: never).  Results do not depend on it."""
     _ep_set_recount(int(blocks_times_topk))
 
 

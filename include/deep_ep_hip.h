@@ -180,9 +180,9 @@ int64_t ep_dispatch_stamp(ep_buffer_t* buf);
  * not depend on it. */
 void ep_set_layout_fold_max_blocks(int num_blocks);
 
-/* Tuning: with one partition and few layout blocks (blocks x top-k up to this limit; default and most 64, 0 turns it
- * off) the histogram kernel is not launched: every workgroup of the slot assignment counts the ids of all blocks itself.
- * Results do not depend on it. */
+/* Tuning: with one partition and few layout blocks of 128 tokens the histogram kernel is not launched: every workgroup of
+ * the slot assignment counts the ids of all blocks itself.  Negative (default): the library's own rule by blocks and
+ * top-k; else blocks x top-k up to this limit (at most 64; 0 turns it off).  Results do not depend on it. */
 void ep_set_layout_recount_limit(int blocks_times_topk);
 
 /* Tuning: workgroups (of 4 waves) of the single-partition combine kernel that a compute unit holds at once;

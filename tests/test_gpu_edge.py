@@ -268,8 +268,9 @@ def test_layout_paths_agree(T, E, K, R, rank):
     topk, w = make_routing(T, E, K, seed=T + 1, masked=0.1)
     lay = O.rank_share_layout(topk.numpy(), E, R, rank, A, T)
     try:
-        # fold_max 0: every multi-block layout takes the scan kernel; recount limit 0: the histogram kernel always runs
-        for fold_max, recount in ((256, 48), (256, 0), (0, 0)):
+        # fold_max 0: every multi-block layout takes the scan kernel; recount limit 0: the histogram kernel always runs, 64: never
+        # where the one launch can hold the ids
+        for fold_max, recount in ((256, 64), (256, 0), (0, 0)):
             deep_ep._C.set_layout_fold_max_blocks(fold_max)
             deep_ep._C.set_layout_recount_limit(recount)
             buf = _buffer(T, H, K, R, rank)
@@ -282,7 +283,7 @@ def test_layout_paths_agree(T, E, K, R, rank):
             buf.destroy()
     finally:
         deep_ep._C.set_layout_fold_max_blocks(256)
-        deep_ep._C.set_layout_recount_limit(48)
+        deep_ep._C.set_layout_recount_limit(-1)
 
 
 @pytest.mark.parametrize('fused', [False, True])

@@ -92,9 +92,11 @@ def test_small_dispatch_deferred_exact_and_replayed():
     buf.destroy()
 
 
-@pytest.mark.parametrize('T,E,K', [(1021, 64, 7), (1024, 256, 8), (1025, 256, 8), (257, 48, 21), (900, 16, 6)])
+@pytest.mark.parametrize('T,E,K', [(1021, 64, 7), (1024, 256, 8), (1025, 256, 8), (257, 48, 21), (900, 16, 6), (8192, 8, 1), (2048, 32, 2),
+                                   (2049, 32, 2), (1281, 64, 5)])
 def test_ids_of_all_blocks_counted_in_place(T, E, K):
-    """Around the most blocks x top-k (64) for which no histogram kernel runs: every workgroup reads all ids itself."""
+    """Around the most blocks x top-k (64) for which the histogram kernel can be left out (every workgroup then reads all ids
+    itself), and around the library's own limits: the same handles whichever launches run."""
     import deep_ep
     H, A = 64, 4
     x = make_tokens(T, H, seed=T).to(DEV)
@@ -102,12 +104,18 @@ def test_ids_of_all_blocks_counted_in_place(T, E, K):
     topk[5] = -1
     lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
     buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
-    deep_ep._C.set_layout_recount_limit(64)             # (another test may have left a lower one)
-    _, _, _, handle, _ = buf.dispatch(x, topk_idx=topk.to(DEV), num_experts=E, expert_alignment=A, do_expand=True)
-    torch.cuda.synchronize()
-    for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
-                 'dst_buffer_slot_idx', 'recv_src_metadata'):
-        assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
+    try:
+        for limit, sync in ((64, True), (-1, True), (-1, False)):
+            deep_ep._C.set_layout_recount_limit(limit)
+            _, _, _, handle, _ = buf.dispatch(x, topk_idx=topk.to(DEV), num_experts=E, expert_alignment=A, do_expand=True,
+                                              do_cpu_sync=sync)
+            torch.cuda.synchronize()
+            for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
+                         'dst_buffer_slot_idx'):
+                assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (limit, sync, name)
+            assert np.array_equal(handle.recv_src_metadata.cpu().numpy()[:lay['num_recv_tokens']], lay['recv_src_metadata'])
+    finally:
+        deep_ep._C.set_layout_recount_limit(-1)
     buf.destroy()
 
 
