@@ -1507,7 +1507,8 @@ extern "C" int ep_dispatch_static_launch(const ep_dispatch_args_t* d, const ep_d
     ep_buffer* v = nullptr;
     rc = guarded([&] { v = static_view_of_current_device(); });
     if (rc != 0) return rc;
-    rc = ep_dispatch_begin(v, d);
+    // (an epilogue that pads for other experts or another alignment than the layout's comes behind a layout of its own)
+    rc = dispatch_launch(v, d, d->num_experts == e->num_experts and d->expert_alignment == e->expert_alignment);
     if (rc != 0) return rc;
     ep_dispatch_epilogue_args_t ee = *e;
     ee.dispatch_stamp = v->last.stamp;

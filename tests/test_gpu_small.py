@@ -244,3 +244,30 @@ def test_epilogue_of_other_experts_or_alignment_is_refused(field, value):
     torch.cuda.synchronize()
     d.check(x, topk, w, E, A)
     buf.destroy()
+
+
+@pytest.mark.parametrize('T', [64, 129])
+def test_static_dispatch_with_an_epilogue_of_its_own_alignment(T):
+    """The static entry point takes an epilogue that pads to another alignment than its layout's, at any size: the rows are
+    those of the layout, and alignment 1 leaves the padding as it was."""
+    import deep_ep
+    C = deep_ep._C
+    H, E, K, A = 128, 16, 4, 8
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    x = make_tokens(T, H, seed=8)
+    topk, w = make_routing(T, E, K, seed=43, masked=0.2)
+    d = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), topk.to(DEV), w.to(DEV))
+    d.e.expert_alignment = 1
+    d.a.stream = d.e.stream = torch.cuda.current_stream().cuda_stream
+    C._check(C._ep_dispatch_static(ctypes.byref(d.a), ctypes.byref(d.e)))
+    torch.cuda.synchronize()
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
+    n, ne = lay['num_recv_tokens'], lay['num_expanded_tokens']
+    ex, _, _ = O.rank_share_dispatch(bf16_bits(x), None, w.numpy(), lay)
+    assert np.array_equal(d.meta.cpu().numpy()[:n], lay['recv_src_metadata'])
+    slots = lay['recv_src_metadata'][:, :K]
+    real = np.zeros(ne, dtype=bool)
+    real[slots[slots >= 0]] = True
+    rows = bf16_bits(d.rows)[:ne]
+    assert np.array_equal(rows[real], ex[real]) and (rows[~real].view(np.int16) == 77).all() and not real.all()
+    buf.destroy()
