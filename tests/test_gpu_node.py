@@ -202,6 +202,7 @@ def test_node_dispatch_combine(R, max_tokens, H, E, K, A, masked, mode, do_cpu_s
     (16, 300, [300 - 9 * r for r in range(16)], 2048, 4),   # more count columns than the send side sums itself
     (3, 2500, [2500, 2049, 2304], 384, 7),  # more entries a workgroup than one round of four a thread
     (2, 70000, [300, 129], 40, 32),         # the rank box does not fit the workspace: counted and ranked on arrival
+    (129, 3, [3 - r % 4 for r in range(129)], 258, 3),          # more partitions than the header has host boxes for
 ])
 def test_node_receive_layout(R, max_tokens, Ts, E, K):
     """Slots out of the shipped counts and ranks, or counted on arrival: the handles of the oracle either way."""
@@ -559,13 +560,13 @@ def test_node_rejects_scaled_rows_that_would_overlap():
         b.destroy()
 
 
-def test_owner_side_whole_rows_shorter_than_a_wave_carry_all_their_weights():
-    """From 16384 metadata rows on the owner-side reduce takes whole rows per wave, and a row with a single local
-    slot is copied verbatim.  With rows of fewer 16-byte vectors than top-k positions (hidden 64, top-16) the
-    weight vector of such a row is wider than its payload: every position of it must still be written."""
-    R, max_tokens, H, E, K, A = 2, 8400, 64, 32, 16, 8
+def test_owner_side_long_parts_shorter_than_a_wave_carry_all_their_weights():
+    """From 16384 metadata rows on and with less than two selections a partition the owner-side reduce takes long parts, and a
+    row with a single local slot is copied verbatim.  With rows of fewer 16-byte vectors than top-k positions (hidden 64,
+    top-16) the weight vector of such a row is wider than its payload: every position of it must still be written."""
+    R, max_tokens, H, E, K, A = 9, 1830, 64, 36, 16, 8
     bufs = make_node(R, max_tokens, H, K, False)
-    Ts = [max_tokens, max_tokens - 100]
+    Ts = [200 - r for r in range(R)]
     xs = [make_tokens(T, H, seed=50 + r) for r, T in enumerate(Ts)]
     routing = [make_routing(T, E, K, seed=60 + r, masked=0.85) for r, T in enumerate(Ts)]     # mostly one local slot a row
     topks, ws = [t for t, _ in routing], [w for _, w in routing]
@@ -576,7 +577,7 @@ def test_owner_side_whole_rows_shorter_than_a_wave_carry_all_their_weights():
                         do_zero_padding=True, do_cpu_sync=False)
     torch.cuda.synchronize()
     handles = [o[3] for o in outs]
-    assert all(h.recv_src_metadata.size(0) >= 16384 for h in handles)          # the whole-row path is the one that runs
+    assert all(h.recv_src_metadata.size(0) >= 16384 for h in handles) and K < 2 * R and K > H // 8     # the long parts are what runs
     single = sum(int(((want[r]['lay']['recv_src_metadata'][:, :K] >= 0).sum(axis=1) == 1).sum()) for r in range(R))
     assert single > 1000                                                       # and verbatim rows are many
     g = torch.Generator().manual_seed(7)
