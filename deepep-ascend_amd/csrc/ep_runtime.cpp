@@ -353,7 +353,21 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
 unsigned small_lds(int E, int R) {
     return (unsigned)(2 * E + R * (EP_TOKENS_PER_BLOCK / 32) + EP_ROW_THREADS / 64) * sizeof(int) + EP_SMALL_ENTRIES * sizeof(short);
 }
-constexpr unsigned kSmallPadBlocks = 2048;
+// Workgroups that zero the padding of such a dispatch: each counts all ids first, in LDS that grows with the experts, so they
+// are no more than fit the chip at once with the row workgroups (1024), unless the padding may be more than 48 MiB.
+// us of a replayed dispatch, two launches / one with 1024 / with 2048 workgroups: 128 tokens top-1, 2048 experts, 7168 FP8
+// channels, alignment 16 14.9 / 13.2 / 17.3, 128 29.9 / 31.6 / 29.5; 4 tokens top-8, 1024 experts, 2048 BF16 channels, alignment 64
+// 15.2 / 9.6 / 11.6; 128 tokens top-8, 1024 experts, alignment 128 (0.9 GB at most) 126 / 124 / 111, 256 experts 53 / 45 / 47;
+// 32 tokens top-8, 512 experts, 2048 BF16 channels, alignment 64 (66 MB at most) 19.1 / 14.3 / 13.7.
+unsigned small_pad_blocks(unsigned pieces, int num_tokens, int K, int num_experts, int alignment, int64_t row_bytes) {
+    const int64_t most_padding = (int64_t)std::min(num_experts, num_tokens * K) * (alignment - 1) * row_bytes;
+    return std::min(pieces, most_padding > (48 << 20) ? 2048u : 1024u);
+}
+// Up to here one launch is the faster form (us of a replayed dispatch without padding, 7168 BF16 channels, two launches / one):
+// top-8 of 256, 1 token 10.4 / 6.0, 32 11.8 / 6.8, 96 12.9 / 9.9, 128 13.4 / 11.1; 128 tokens top-1 8.0 / 4.9, top-8 of 2048
+// 16.9 / 12.8, 16384 channels 15.6 / 14.9; top-16, 64 tokens 17.6 / 12.8; top-32, 32 tokens 27.9 / 20.1.  One of eight partitions
+// (FP8, top-8), 64 tokens 29.2 / 22.6, 128 30.6 / 25.4.  The line is one block of ids: a token's bit and its rank are kept for
+// that many.
 bool small_dispatch(int num_tokens, int K) {
     return num_tokens > 0 and num_tokens <= EP_TOKENS_PER_BLOCK and num_tokens * K <= EP_SMALL_ENTRIES;
 }
@@ -1273,7 +1287,8 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
             // the one launch sizes its LDS by the begin's experts and pads by the epilogue's
             EP_HOST_ASSERT(a.num_experts == b->last.num_experts and a.expert_alignment == b->last.alignment and
                            "the copy epilogue has the experts and the alignment of its ep_dispatch_begin");
-            launch_small(b->last.pending, sa, false, quantise_here, (int)std::min(pad_blocks, kSmallPadBlocks), a.stream);
+            launch_small(b->last.pending, sa, false, quantise_here,
+                         (int)small_pad_blocks(pad_blocks, num_tokens, K, El, a.expert_alignment, sa.out_row_bytes), a.stream);
             b->last.layout_pending = false;
             b->last.copied = true;
         } else if (grid > 0) {

@@ -23,6 +23,8 @@ CASES = [
     (127, 2064, 8, 3, 8, 0.5, None),
     (129, 256, 16, 2, 64, 0.0, None),       # one token beyond it
     (64, 256, 300, 16, 1, 0.0, None),       # more experts than threads
+    (128, 64, 2048, 1, 16, 0.0, None),      # more pieces of padding (4096) than workgroups that zero them (1024)
+    (128, 2080, 160, 8, 128, 0.0, None),    # the same with more than 48 MiB of padding in BF16 (2560 pieces, 2048 workgroups)
 ]
 
 
