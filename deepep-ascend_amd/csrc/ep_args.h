@@ -175,7 +175,7 @@ struct EpSmallArgs {
 #define EP_SF_COL_MAJOR 1
 #define EP_SF_COL_MAJOR_COUNTED 2
 #define EP_SF_TILE 64
-#define EP_SF_WIDE_ROW_BYTES 256        // scale rows up to this wide are turned 16 bytes at a time (8192 channels)
+#define EP_SF_WIDE_ROW_BYTES 256        // scale rows up to this wide (8192 channels) are turned 64 at a time, wider ones fewer
 
 // Row-major scale rows -> column-major, 64 x 64 tiles through LDS.
 struct EpSfTransposeArgs {

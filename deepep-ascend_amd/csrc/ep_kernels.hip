@@ -1551,17 +1551,21 @@ __device__ __forceinline__ void sf_transpose_body(const EpSfTransposeArgs& a, in
     }
 }
 
-// Rows of at most EP_SF_WIDE_ROW_BYTES from a 16-byte aligned source.  The 64 rows of a workgroup are one contiguous piece
-// of it: the piece goes to LDS in 16-byte loads, all of a thread's in flight, and leaves as V adjacent rows of a column a
-// store: 16 bytes where columns start on 16 bytes (128 or 256 bytes a column and workgroup), else 4, else one element.
+// Whole rows through LDS, from a 16-byte aligned source: 64 rows of at most EP_SF_WIDE_ROW_BYTES, half as many at a time per
+// doubling of the row (8 at the widest).  They are one contiguous piece of the source: the piece goes to LDS in 16-byte loads,
+// all of a thread's in flight, and leaves as V adjacent rows of a column a
+// store: 16 bytes where columns start on 16 bytes (16 to 256 bytes a column and piece), else 4, else one element.
 // 52 thousand rows of 112 2-byte packs: 11.2 us with pairs of packs and two barriers per 64 columns, 7.7 us so (fetching the
 // rows before the row count is known, to save its trip, measured 8.4: the workgroups beyond the rows then fetch as well).
+// Wider rows, whole calls (pairs of packs / element by element / so): 3000 tokens top-2, 192 packs 171 / 184 / 161 us; 2501 tokens
+// top-4, 256 packs 157 / 170 / 150; 2000 tokens top-8, 320 packs 535 / 557 / 527.
 template <typename E, int V>
-__device__ __forceinline__ void sf_columns_out(const EpSfTransposeArgs& a, int n, int rows, int pitch, const unsigned char* lds) {
+__device__ __forceinline__ void sf_columns_out(const EpSfTransposeArgs& a, int n, int r0, int log_rows, int rows, int pitch,
+                                               const unsigned char* lds) {
     typedef E vec_t __attribute__((ext_vector_type(V)));
-    constexpr int GROUPS = EP_SF_TILE / V;
-    const int r0 = blockIdx.x * EP_SF_TILE, rr = threadIdx.x % GROUPS * V;
-    for (int c = threadIdx.x / GROUPS; c < a.num_cols; c += EP_LAYOUT_THREADS / GROUPS) {
+    const int log_groups = log_rows - __builtin_ctz(V);                // 2^log_groups vectors of V rows a column
+    const int rr = ((int)threadIdx.x & ((1 << log_groups) - 1)) * V;
+    for (int c = (int)threadIdx.x >> log_groups; c < a.num_cols; c += EP_LAYOUT_THREADS >> log_groups) {
         E* out = (E*)a.dst + (int64_t)c * n + r0 + rr;
         vec_t x;
 #pragma unroll
@@ -1573,9 +1577,9 @@ __device__ __forceinline__ void sf_columns_out(const EpSfTransposeArgs& a, int n
     }
 }
 template <typename E>
-__device__ __forceinline__ void sf_transpose_wide(const EpSfTransposeArgs& a, int n, unsigned char* lds) {
+__device__ __forceinline__ void sf_transpose_wide(const EpSfTransposeArgs& a, int n, int r0, int log_rows, unsigned char* lds) {
     constexpr int VEC = 16 / (int)sizeof(E), MAXV = EP_SF_TILE * EP_SF_WIDE_ROW_BYTES / 16 / EP_LAYOUT_THREADS;
-    const int cols = a.num_cols, r0 = blockIdx.x * EP_SF_TILE, rows = min(EP_SF_TILE, n - r0);
+    const int cols = a.num_cols, rows = min(1 << log_rows, n - r0);
     // rows of an odd number of words: the rows that neighbouring lanes read spread over the banks
     const int pitch = ((cols * (int)sizeof(E) + 3) / 4 | 1) * 4;
     const int count = rows * cols, nvec = count / VEC;
@@ -1605,9 +1609,27 @@ __device__ __forceinline__ void sf_transpose_wide(const EpSfTransposeArgs& a, in
     }
     __syncthreads();
     const int step = n * (int)sizeof(E) | (int)((uintptr_t)a.dst & 15);
-    if ((step & 15) == 0) sf_columns_out<E, VEC>(a, n, rows, pitch, lds);
-    else if ((step & 3) == 0) sf_columns_out<E, 4 / (int)sizeof(E)>(a, n, rows, pitch, lds);
-    else sf_columns_out<E, 1>(a, n, rows, pitch, lds);
+    if ((step & 15) == 0) sf_columns_out<E, VEC>(a, n, r0, log_rows, rows, pitch, lds);
+    else if ((step & 3) == 0) sf_columns_out<E, 4 / (int)sizeof(E)>(a, n, r0, log_rows, rows, pitch, lds);
+    else sf_columns_out<E, 1>(a, n, r0, log_rows, rows, pitch, lds);
+}
+// The 64 rows of a workgroup: at once (a case of its own: with the number of rows in a register narrow rows lose 3 % of a
+// call, 160 thousand rows of 16 packs), or in pieces of fewer where the rows are wider.
+template <typename E>
+__device__ __forceinline__ void sf_transpose_pieces(const EpSfTransposeArgs& a, int n, unsigned char* lds) {
+    constexpr int LOG_TILE = __builtin_ctz(EP_SF_TILE);
+    const int r0 = blockIdx.x * EP_SF_TILE, row_bytes = a.num_cols * (int)sizeof(E);
+    if (row_bytes <= EP_SF_WIDE_ROW_BYTES) {
+        sf_transpose_wide<E>(a, n, r0, LOG_TILE, lds);
+        return;
+    }
+    int log_rows = LOG_TILE - 1;
+    while (row_bytes << log_rows > EP_SF_TILE * EP_SF_WIDE_ROW_BYTES) --log_rows;
+    const int end = min(r0 + EP_SF_TILE, n);
+    for (int r = r0; r < end; r += 1 << log_rows) {
+        if (r != r0) __syncthreads();                       // (the piece before has left the LDS)
+        sf_transpose_wide<E>(a, n, r, log_rows, lds);
+    }
 }
 
 extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_sf_transpose(EpSfTransposeArgs a) {
@@ -1615,12 +1637,14 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_sf_transpose(
     int n = a.num_rows;
     if (a.counted) n = min(n, align_up(a.psum_expert[a.num_local_experts - 1], a.expert_alignment));
     if ((int)blockIdx.x * EP_SF_TILE >= n) return;
-    const bool wide = a.num_cols * a.elem_bytes <= EP_SF_WIDE_ROW_BYTES && ((uintptr_t)a.src & 15) == 0;
+    // (8 rows: the fewest that still make a 16-byte store of 2-byte packs; wider rows, and a source that does not start on 16
+    // bytes, go element by element)
+    const bool wide = a.num_cols * a.elem_bytes <= EP_SF_WIDE_ROW_BYTES * EP_SF_TILE / 8 && ((uintptr_t)a.src & 15) == 0;
     if (a.elem_bytes == 4) {
-        if (wide) sf_transpose_wide<unsigned>(a, n, lds);
+        if (wide) sf_transpose_pieces<unsigned>(a, n, lds);
         else sf_transpose_body<unsigned>(a, n, (unsigned (*)[EP_SF_TILE + 1])lds);
     } else {
-        if (wide) sf_transpose_wide<unsigned short>(a, n, lds);
+        if (wide) sf_transpose_pieces<unsigned short>(a, n, lds);
         else sf_transpose_body<unsigned short>(a, n, (unsigned (*)[EP_SF_TILE + 1])lds);
     }
 }

@@ -554,11 +554,12 @@ def test_odd_topk_combine_of_small_launches(T, H, K):
     buf.destroy()
 
 
-@pytest.mark.parametrize('packs', [1, 2, 63, 64, 128, 130, 258])
+@pytest.mark.parametrize('packs', [1, 2, 63, 64, 128, 130, 256, 257, 258, 513, 1024, 1026])
 @pytest.mark.parametrize('alignment', [1, 2, 8])
 def test_scale_packs_of_any_count_and_stride(packs, alignment):
     """2-byte scale packs two at a time or one (odd counts, rows that start off 4 bytes, columns), more than a wave's
-    worth of pairs, and their columns with 16-byte, 4-byte and single stores, up to and beyond the widest rows in one go."""
+    worth of pairs, and their columns with 16-byte, 4-byte and single stores; rows turned 64, 32, 16 and 8 at a time, and
+    element by element beyond."""
     T, H, E, K = 73, 4096, 5, 3
     topk, w = make_routing(T, E, K, seed=alignment, masked=0.2)
     g = torch.Generator().manual_seed(packs)
@@ -581,9 +582,9 @@ def test_scale_packs_of_any_count_and_stride(packs, alignment):
     buf.destroy()
 
 
-@pytest.mark.parametrize('H', [8, 128, 520, 8192, 8200])
+@pytest.mark.parametrize('H', [8, 128, 520, 8192, 8200, 16384])
 def test_column_major_scales_of_the_fused_quantiser(H):
-    """4-byte scales as columns: one column, a partial group, rows as wide as one go takes and one column wider."""
+    """4-byte scales as columns: one column, a partial group, rows as wide as 64 a go takes, one column wider, the widest."""
     T, E, K = 130, 6, 2
     topk, w = make_routing(T, E, K, seed=H)
     x = make_tokens(T, H, seed=H)
