@@ -213,6 +213,7 @@ struct EpCombineArgs {
     // owner-side reduce: the partial of a row goes to the combine buffer of the partition its token came from
     char* const* peer_arenas;
     int64_t buffer_off;
+    int paced;                    // top-8: the first row's fetches go ahead of the others (launches that fill the chip several times)
     int long_parts;               // owner-side reduce: a task is EP_COMBINE_LONG_PART channels of a row, not 1024
 };
 

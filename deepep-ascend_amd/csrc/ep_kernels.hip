@@ -1951,8 +1951,8 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
                 d1[j] = __builtin_nontemporal_load(y + row + c1);
                 // sixteen and more fetches a wave are better sent in two goes, the first row ahead of the others
                 // (top-8 at 16384 / 32768 tokens: 354 / 707 us against 362 / 730 all at once; top-6 and below lose:
-                // 277 against 272)
-                if (KT >= 8 && j == 0) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                // 277 against 272), unless the launch waits for its trips to memory and not for their bandwidth
+                if (KT >= 8 && j == 0 && a.paced) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             }
         }
         // inputs in order: b0, b1, then the rows in ascending position; zero inputs -> zeros, one input -> verbatim

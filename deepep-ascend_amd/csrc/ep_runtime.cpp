@@ -153,6 +153,10 @@ unsigned combine_lds_cap(int num_topk, bool specialised, int num_row_blocks, int
     if (share <= 1024u) return 0;
     return std::min(64u * 1024u, share - 1024u);       // n of them fit a CU, n + 1 do not
 }
+// From here on the top-8 kernels send their first row's fetches ahead of the others.  Replayed combines of 7168 channels, us
+// first row ahead / all at once: 32 tokens (56 row blocks) 5.3 / 5.1, 64 6.2 / 5.9, 128 7.0 / 6.7, 256 9.3 / 9.2, 1024 25.4 / 25.2,
+// 2048 (3584 row blocks) 47.6 / 47.5, 4096 91.0 / 90.8, 6144 (10752) 136.5 / 137.1, 8192 181.7 / 183.3, 16384 354 / 362.
+constexpr int kPacedRowBlocks = 8192;
 std::atomic<int> g_recount_limit{-1};     // blocks x top-k up to which one partition's slot assignment counts all ids itself; negative: recount_pays
 std::atomic<int> g_fold_max_blocks{256};    // up to this many layout workgroups the slot assignment sums the block counts itself
 
@@ -1437,6 +1441,7 @@ int ep_combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase) {
             // odd top-k: a launch of less than a row block a CU waits for its trips to memory and takes the unrolled kernel;
             // at 765 blocks the two are level (top-3 / 5 / 7: 9.5 / 11.2 / 13.0 us against 9.6 / 11.3 / 13.1 of the general
             // one), beyond, the general one's shorter bursts win (1787 blocks: 14.9 / 19.7 / 23.8 us against 16.5 / 20.4 / 25.0)
+            ca.paced = ca.num_row_blocks >= kPacedRowBlocks ? 1 : 0;
             const bool odd = ca.num_row_blocks < 256 and (K == 3 or K == 5 or K == 7);
             const unsigned cap = combine_lds_cap(K + (ca.bias_0 != nullptr) + (ca.bias_1 != nullptr), kidx != 0, ca.num_row_blocks, hidden);
             launch(odd ? g_k.combine_odd[(K - 3) / 2] : g_k.combine[EP_COMBINE_FUSED][kidx], grid, EP_ROW_THREADS, cap, a.stream, ca);
@@ -1451,6 +1456,7 @@ int ep_combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase) {
             ca.num_rows_bound = num_combined_tokens;
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROW_THREADS / 64);
             if (ca.num_row_blocks == 0) return;
+            ca.paced = ca.num_row_blocks >= kPacedRowBlocks ? 1 : 0;
             launch(g_k.combine[EP_COMBINE_FINAL][kidx], (unsigned)ca.num_row_blocks, EP_ROW_THREADS, 0, a.stream, ca);
         }
     });

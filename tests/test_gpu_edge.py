@@ -434,3 +434,37 @@ def test_combine_on_non_finite_expert_outputs():
         assert ((got == want) | both_nan).all()
         assert both_nan.any() and ((want & 0x7fff) == 0x7f80).any()
     buf.destroy()
+
+
+@pytest.mark.parametrize('T,nodes', [(32764, 1), (32768, 1), (32768, 2)])
+def test_top8_combine_on_both_sides_of_the_paced_line(T, nodes):
+    """8191 and 8192 row blocks of one 64-channel part: the row sums are those of torch in the same order, bit for bit."""
+    import deep_ep
+    H, E, K = 64, 16, 8
+    node = None if nodes == 1 else deep_ep.LocalNode(nodes)
+    group = [deep_ep.LocalGroup() if node is None else node.group(r) for r in range(nodes)]
+    bufs = [deep_ep.EPBuffer(g, num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True) for g in group]
+    gen = torch.Generator(device=DEV).manual_seed(T + nodes)
+    topk = [torch.rand((T, E), generator=gen, device=DEV).topk(K, dim=-1).indices for _ in bufs]
+    x = [torch.randn((T, H), generator=gen, device=DEV, dtype=torch.bfloat16) for _ in bufs]
+    kw = dict(num_experts=E, num_max_tokens_per_rank=T, do_expand=True, async_with_compute_stream=True, defer_epilogue=True)
+    sent = [b.dispatch(v, topk_idx=t, **kw) for b, v, t in zip(bufs, x, topk)]
+    got = [e.current_stream_wait() for e in sent]
+    reduced = [b.combine(rows, h, async_with_compute_stream=True, defer_epilogue=True) for b, (rows, _, _, h) in zip(bufs, got)]
+    for v, t, e in zip(x, topk, reduced):
+        out = e.current_stream_wait()[0]
+        # a token's row comes back K times over; partition by partition, each partial rounded to BF16 (doublings and sums of
+        # equal terms in the same order as the kernels')
+        total = None
+        for r in range(nodes):
+            here = (t * nodes // E == r).sum(dim=-1)
+            acc = torch.zeros((T, H), device=DEV)
+            for j in range(K):
+                acc = torch.where((here > j)[:, None], acc + v.float(), acc)
+            part = acc.to(torch.bfloat16).float()
+            total = part if total is None else total + part
+        # (masters in ascending position: with two partitions the sum of two terms does not depend on their order)
+        assert torch.equal(out, total.to(torch.bfloat16))
+    torch.cuda.synchronize()
+    for b in bufs:
+        b.destroy()
