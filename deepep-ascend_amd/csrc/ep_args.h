@@ -159,11 +159,11 @@ struct EpScatterArgs {
     int rows_are_tokens;          // cached expand: every token was received, so row i of the receive stream is token i
 };
 
-// A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES (token, slot) entries in one launch: every
-// workgroup works the layout out for itself.
+// A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES (token, slot) entries in one launch, or the receive
+// side of a node that ships ranks: every workgroup works the layout out for itself.
 #define EP_SMALL_ENTRIES 1024
 struct EpSmallArgs {
-    EpLayoutArgs l;               // what ep_layout_assign would have been given
+    EpLayoutArgs l;               // what ep_layout_assign (ep_recv_copy: ep_layout_place) would have been given
     EpScatterArgs s;              // what the copy kernel would have been given
     int num_pad_blocks;           // workgroups behind the row workgroups, each zeroing every num_pad_blocks-th padding piece
 };

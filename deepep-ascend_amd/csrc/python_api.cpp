@@ -156,7 +156,7 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
         r.do_cpu_sync = s.do_cpu_sync ? 1 : 0;
         r.dispatch_stamp = s.stamp;
         r.stream = current_stream();
-        check(ep_dispatch_recv_launch(s.buf, &r));
+        check(ep_dispatch_recv_begin(s.buf, &r));
     }
 
     int num_recv = -1, num_expanded = -1;

@@ -108,6 +108,7 @@ _ep_dispatch_begin = _sig('ep_dispatch_begin', ctypes.c_int, ctypes.c_void_p, ct
 _ep_wait = _sig('ep_dispatch_wait_counts', ctypes.c_int, ctypes.c_void_p, _c_int_p, _c_int_p, _c_int_p)
 _ep_worst = _sig('ep_dispatch_worst_case_sizes', ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                  ctypes.c_int, ctypes.c_int, _c_int_p, _c_int_p)
+_ep_dispatch_recv_begin = _sig('ep_dispatch_recv_begin', ctypes.c_int, ctypes.c_void_p, ctypes.POINTER(_DispatchRecvArgs))
 _ep_dispatch_recv = _sig('ep_dispatch_recv_launch', ctypes.c_int, ctypes.c_void_p, ctypes.POINTER(_DispatchRecvArgs))
 _ep_connect = _sig('ep_buffer_connect', ctypes.c_int, ctypes.POINTER(ctypes.c_void_p), ctypes.c_int)
 _ep_set_peers = _sig('ep_buffer_set_peers', ctypes.c_int, ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p), ctypes.c_int)

@@ -202,6 +202,11 @@ void ep_set_combine_blocks_per_cu(int num_blocks);
  * ep_dispatch_launch (of every partition of a node) and before ep_dispatch_wait_counts /
  * ep_dispatch_epilogue_launch. */
 int ep_dispatch_recv_launch(ep_buffer_t* buf, const ep_dispatch_recv_args_t* args);
+/* The same for a caller whose next launch on this buffer is this dispatch's ep_dispatch_epilogue_launch: in a node whose send
+ * sides ship ranks the library may then leave the placing to the copy launch (one launch instead of two).  Everything this
+ * call would have enqueued is then enqueued by the epilogue, on the epilogue's stream; ep_dispatch_wait_counts may come
+ * between the two. */
+int ep_dispatch_recv_begin(ep_buffer_t* buf, const ep_dispatch_recv_args_t* args);
 
 /* Host wait for the counts of the last non-cached do_cpu_sync dispatch, with the buffer's CPU
  * timeout ("reduction timeout").  per_expert receives E/R aligned counts.  Replaces the

@@ -636,3 +636,95 @@ def test_owner_side_long_parts(H, K):
         assert torch.equal(res[s][1].cpu(), ow)
     for b in bufs:
         b.destroy()
+
+
+ONE_LAUNCH_CASES = [
+    # R, max_tokens, H, E, K, A, masked
+    (64, 9, 64, 64, 8, 1, 0.3),            # a source a lane, one expert a partition
+    (2, 300, 2112, 1024, 32, 4, 0.1),      # two experts a thread, the widest metadata rows, rows beyond one 4 KiB part
+    (2, 40, 64, 2048, 5, 8, 0.0),          # four experts a thread
+    (2, 4200, 16, 2048, 2, 1, 0.2),        # the same with more than 2048 row blocks: two launches
+    (3, 33, 256, 12, 5, 128, 1.0),         # nobody receives anything
+]
+
+
+@pytest.mark.parametrize('R,max_tokens,H,E,K,A,masked', ONE_LAUNCH_CASES)
+@pytest.mark.parametrize('do_cpu_sync', [True, False])
+def test_receive_side_in_one_launch(R, max_tokens, H, E, K, A, masked, do_cpu_sync):
+    """Received rows placed and copied in one launch, at the edges of what that takes."""
+    bufs = make_node(R, max_tokens, H, K, False)
+    Ts = [max(1, max_tokens - r) for r in range(R)]
+    xs = [make_tokens(T, H, seed=90 + r) for r, T in enumerate(Ts)]
+    routing = [make_routing(T, E, K, seed=95 + r, masked=masked) for r, T in enumerate(Ts)]
+    topks, ws = [t for t, _ in routing], [w for _, w in routing]
+    rows = [bf16_bits(x).view(np.uint8).reshape(x.size(0), -1) for x in xs]
+    _, want = oracle_dispatch(rows, [None] * R, [t.numpy() for t in topks], [w.numpy() for w in ws], E, R, A, max_tokens)
+    outs = dispatch_all(bufs, [x.to(DEV) for x in xs], [t.to(DEV) for t in topks], [w.to(DEV) for w in ws], num_experts=E,
+                        num_max_tokens_per_rank=max_tokens, expert_alignment=A, do_expand=True, do_zero_padding=True,
+                        do_cpu_sync=do_cpu_sync)
+    for r, (recv, _, rw, handle) in enumerate(outs):
+        lay = want[r]['lay']
+        n, ne = lay['num_recv_tokens'], lay['num_expanded_tokens']
+        for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert'):
+            assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
+        assert np.array_equal(handle.recv_src_metadata.cpu().numpy()[:n], lay['recv_src_metadata'])
+        assert np.array_equal(recv.view(torch.uint8).cpu().numpy().reshape(-1, 2 * H)[:ne], want[r]['x'])
+        assert np.array_equal(rw.cpu().numpy().view(np.uint32)[:ne], want[r]['w'].view(np.uint32))
+    for b in bufs:
+        b.destroy()
+
+
+@pytest.mark.parametrize('begin', [True, False])
+@pytest.mark.parametrize('alignment', [8, 1])
+def test_receive_side_through_the_abi(begin, alignment):
+    """ep_dispatch_recv_begin and ep_dispatch_recv_launch leave the same behind the epilogue, also with an epilogue of another
+    alignment than the receive side's (which pads by its own and copies as placed)."""
+    import ctypes
+    import deep_ep
+    C = deep_ep._C
+    R, T, H, E, K, A = 2, 50, 128, 12, 3, 8
+    bufs = make_node(R, T, H, K, False)
+    xs = [make_tokens(T, H, seed=33 + r) for r in range(R)]
+    routing = [make_routing(T, E, K, seed=44 + r, masked=0.2) for r in range(R)]
+    topks, ws = [t for t, _ in routing], [w for _, w in routing]
+    rows = [bf16_bits(x).view(np.uint8).reshape(x.size(0), -1) for x in xs]
+    _, want = oracle_dispatch(rows, [None] * R, [t.numpy() for t in topks], [w.numpy() for w in ws], E, R, A, T)
+    sent = [b.dispatch(x.to(DEV), topk_idx=t.to(DEV), topk_weights=w.to(DEV), num_experts=E, num_max_tokens_per_rank=T, expert_alignment=A,
+                       do_expand=True, do_cpu_sync=False, async_with_compute_stream=True, defer_epilogue=True)
+            for b, x, t, w in zip(bufs, xs, topks, ws)]
+    n_recv, n_exp = O.no_sync_sizes(R, T, K, E, A)
+    stream = torch.cuda.current_stream().cuda_stream
+    for r, b in enumerate(bufs):
+        lay = want[r]['lay']
+        n, ne = lay['num_recv_tokens'], lay['num_expanded_tokens']
+        x, w = xs[r].to(DEV), ws[r].to(DEV)
+        psum_r, psum_e, counts = (torch.full((m,), -7, dtype=torch.int32, device=DEV) for m in (R, E // R, E // R))
+        meta = torch.full((n_recv, K + 2), -7, dtype=torch.int32, device=DEV)
+        out = torch.full((n_exp, H), 77, dtype=torch.int16, device=DEV).view(torch.bfloat16)
+        gates = torch.full((n_exp,), -7.0, device=DEV)
+        a, e = C._DispatchRecvArgs(), C._DispatchEpilogueArgs()
+        for f in (a, e):
+            f.psum_num_recv_tokens_per_rank, f.psum_num_recv_tokens_per_expert = C._desc(psum_r), C._desc(psum_e)
+            f.recv_src_metadata = C._desc(meta)
+            f.num_topk, f.num_max_tokens_per_rank, f.num_experts, f.expert_alignment = K, T, E, A
+            f.stream, f.dispatch_stamp = stream, C._ep_stamp(b.runtime._h)
+        a.num_unaligned_recv_tokens_per_expert, a.hidden_bytes = C._desc(counts), 2 * H
+        e.x, e.topk_weights, e.recv_x, e.recv_topk_weights = C._desc(x), C._desc(w), C._desc(out), C._desc(gates)
+        e.do_zero_padding, e.expert_alignment = 1, alignment
+        torch.cuda.synchronize()
+        C._check((C._ep_dispatch_recv_begin if begin else C._ep_dispatch_recv)(b.runtime._h, ctypes.byref(a)))
+        C._check(C._ep_dispatch_epi(b.runtime._h, ctypes.byref(e)))
+        torch.cuda.synchronize()
+        assert np.array_equal(psum_r.cpu().numpy(), lay['psum_num_recv_tokens_per_rank'])
+        assert np.array_equal(psum_e.cpu().numpy(), lay['psum_num_recv_tokens_per_expert'])
+        assert np.array_equal(counts.cpu().numpy(), lay['num_unaligned_recv_tokens_per_expert'])
+        assert np.array_equal(meta.cpu().numpy()[:n], lay['recv_src_metadata'])
+        used = np.zeros(ne, dtype=bool)
+        used[lay['recv_src_metadata'][:, :K][lay['recv_src_metadata'][:, :K] >= 0]] = True
+        got = out.view(torch.uint8).cpu().numpy().reshape(n_exp, -1)
+        assert np.array_equal(got[:ne][used], want[r]['x'][used])
+        assert (got[:ne][~used] == (0 if alignment == A else np.tile([77, 0], H))).all()
+        assert np.array_equal(gates.cpu().numpy()[:ne][used].view(np.uint32), want[r]['w'][used].view(np.uint32))
+    del sent
+    for b in bufs:
+        b.destroy()
