@@ -93,6 +93,16 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
     return v;
 }
 
+// Counts for the host go to its pinned page (fine-grained memory) with stores that pass the L2, one by one; when a workgroup's have
+// arrived, one more says so.  A release at system scope would write the whole L2 back in front of it: two or three times 1 us
+// where nothing is dirty, and longer beside the stores of a copy in the same launch.  Whole host-synchronised cases (us): 128 tokens of a
+// toy layer 25.2 -> 23.8, a chunk of 1021 tokens 34.0 -> 33.3.
+__device__ __forceinline__ void host_store(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
+__device__ __forceinline__ void host_stores_arrived() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
 // Reads one word of every 64 bytes of the kernel's arguments, all in one trip.  The compiler fetches arguments where they are
 // first used, in some kernels four or five times in a row along the way to the first store, and each first touch of a
 // cache line is a trip to memory.  Whole cases (us): a replayed decode of 32 tokens 18.0 -> 17.3, prefill of 4096 tokens top-8
@@ -630,7 +640,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
                 a.unaligned_expert[e] = c;
                 a.psum_expert[e] = run + c;
                 if (a.cumulative_stats != nullptr) atomicAdd(&a.cumulative_stats[e], c);
-                if (a.notify_host) a.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
+                if (a.notify_host) host_store(&a.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
             }
             if (SEND) {
                 // slots are the receivers' business: ranks count from 0, and the receivers get the counts they need
@@ -638,7 +648,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
                 if (publisher && a.count_box_off != 0) {
                     const int r = e / a.experts_per_rank, at = a.rank_idx * a.experts_per_rank + (e - r * a.experts_per_rank);
                     ((int*)(a.peer_arenas[r] + a.count_box_off))[at] = c;
-                    if (a.host_boxes != nullptr) a.host_boxes[r][a.host_box_slot + at] = c;
+                    if (a.host_boxes != nullptr) host_store(&a.host_boxes[r][a.host_box_slot + at], c);
                 }
                 s_start[e] = 0;
                 continue;
@@ -659,12 +669,10 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
             // in a stream of phases comes behind the copies of the partitions before it (eight partitions of 2048 tokens:
             // 18-21 us of idle GPU a partition, all phases 1436 -> 1384 us)
             for (int r = tid; r < R; r += blockDim.x)
-                a.host_boxes[r][a.host_box_slot + EP_HOST_BOX_ROWS_OFF + a.rank_idx] = min(s_tot[El + r], a.max_tokens);
-            __threadfence_system();
-            __syncthreads();
+                host_store(&a.host_boxes[r][a.host_box_slot + EP_HOST_BOX_ROWS_OFF + a.rank_idx], min(s_tot[El + r], a.max_tokens));
+            host_stores_arrived();
             for (int r = tid; r < R; r += blockDim.x)
-                __hip_atomic_store(&a.host_boxes[r][a.host_box_slot + EP_HOST_BOX_SEQ_OFF + a.rank_idx], a.seq, __ATOMIC_RELEASE,
-                                   __HIP_MEMORY_SCOPE_SYSTEM);
+                host_store(&a.host_boxes[r][a.host_box_slot + EP_HOST_BOX_SEQ_OFF + a.rank_idx], a.seq);
         }
     }
     if (publisher && !SEND) {
@@ -675,17 +683,15 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
             const int upto = RECV ? s_psum[r] : n_recv;
             const int from = RECV && r ? s_psum[r - 1] : 0;
             a.psum_rank[r] = upto;
-            if (a.notify_host) a.host_page[EP_HOST_RANK_OFF + r] = upto - from;
+            if (a.notify_host) host_store(&a.host_page[EP_HOST_RANK_OFF + r], upto - from);
         }
         if (a.notify_host) {
-            __threadfence_system();
-            __syncthreads();
             if (tid == 0) {
-                a.host_page[1] = n_recv;
-                a.host_page[2] = grand;
-                __threadfence_system();
-                __hip_atomic_store(&a.host_page[0], a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                host_store(&a.host_page[1], n_recv);
+                host_store(&a.host_page[2], grand);
             }
+            host_stores_arrived();
+            if (tid == 0) host_store(&a.host_page[0], a.seq);
         }
     }
     if (!worker) return;
@@ -837,7 +843,7 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_place(
             a.unaligned_expert[e] = c;
             a.psum_expert[e] = run + c;
             if (a.cumulative_stats != nullptr) atomicAdd(&a.cumulative_stats[e], c);
-            if (a.notify_host) a.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
+            if (a.notify_host) host_store(&a.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
         }
         s_tot[e] = run;
         run += align_up(c, A);
@@ -846,17 +852,15 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_place(
         for (int r = tid; r < R; r += EP_LAYOUT_THREADS) {
             const int upto = s_psum[r], from = r ? s_psum[r - 1] : 0;
             a.psum_rank[r] = upto;
-            if (a.notify_host) a.host_page[EP_HOST_RANK_OFF + r] = upto - from;
+            if (a.notify_host) host_store(&a.host_page[EP_HOST_RANK_OFF + r], upto - from);
         }
         if (a.notify_host) {
-            __threadfence_system();
-            __syncthreads();
             if (tid == 0) {
-                a.host_page[1] = num_rows;
-                a.host_page[2] = grand;
-                __threadfence_system();
-                __hip_atomic_store(&a.host_page[0], a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                host_store(&a.host_page[1], num_rows);
+                host_store(&a.host_page[2], grand);
             }
+            host_stores_arrived();
+            if (tid == 0) host_store(&a.host_page[0], a.seq);
         }
         return;
     }
@@ -1410,36 +1414,35 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
             if (PACK) {
                 const int r = e / El, at = l.rank_idx * El + (e - r * El);
                 if (l.count_box_off != 0) ((int*)(l.peer_arenas[r] + l.count_box_off))[at] = c;
-                if (l.host_boxes != nullptr) l.host_boxes[r][l.host_box_slot + at] = c;
+                if (l.host_boxes != nullptr) host_store(&l.host_boxes[r][l.host_box_slot + at], c);
             } else {
                 l.unaligned_expert[e] = c;
                 l.psum_expert[e] = s_start[e] + c;
                 if (l.cumulative_stats != nullptr) atomicAdd(&l.cumulative_stats[e], c);
-                if (l.notify_host) l.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
+                if (l.notify_host) host_store(&l.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
             }
         }
         for (int r = tid; r < R; r += EP_ROW_THREADS) {
             const int rows = min(tokens_to(r, EP_TOKENS_PER_BLOCK), l.max_tokens);
             if (PACK) {
                 if (l.connected || r == l.rank_idx) ((int*)(l.peer_arenas[r] + EP_WS_INBOX_OFF))[l.rank_idx] = rows;
-                if (l.host_boxes != nullptr) l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_ROWS_OFF + l.rank_idx] = rows;
+                if (l.host_boxes != nullptr) host_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_ROWS_OFF + l.rank_idx], rows);
             } else {
                 l.psum_rank[r] = rows;
-                if (l.notify_host) l.host_page[EP_HOST_RANK_OFF + r] = rows;
+                if (l.notify_host) host_store(&l.host_page[EP_HOST_RANK_OFF + r], rows);
             }
         }
         if (PACK ? l.host_boxes != nullptr : l.notify_host != 0) {
-            __threadfence_system();
-            __syncthreads();
+            if (!PACK && tid == 0) {
+                host_store(&l.host_page[1], tokens_to(0, EP_TOKENS_PER_BLOCK));
+                host_store(&l.host_page[2], grand);
+            }
+            host_stores_arrived();
             if (PACK) {
                 for (int r = tid; r < R; r += EP_ROW_THREADS)
-                    __hip_atomic_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_SEQ_OFF + l.rank_idx], l.seq,
-                                       __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                    host_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_SEQ_OFF + l.rank_idx], l.seq);
             } else if (tid == 0) {
-                l.host_page[1] = tokens_to(0, EP_TOKENS_PER_BLOCK);
-                l.host_page[2] = grand;
-                __threadfence_system();
-                __hip_atomic_store(&l.host_page[0], l.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                host_store(&l.host_page[0], l.seq);
             }
         }
         return;
@@ -1616,21 +1619,19 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_recv_copy(EpSmal
             l.unaligned_expert[e] = c;
             l.psum_expert[e] = s_start[e] + c;
             if (l.cumulative_stats != nullptr) atomicAdd(&l.cumulative_stats[e], c);
-            if (l.notify_host) l.host_page[EP_HOST_EXPERT_OFF + e] = align_up(c, A);
+            if (l.notify_host) host_store(&l.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
         }
         if (tid < R) {                                   // (the first wave: R <= 64)
             l.psum_rank[tid] = upto;
-            if (l.notify_host) l.host_page[EP_HOST_RANK_OFF + tid] = mine;
+            if (l.notify_host) host_store(&l.host_page[EP_HOST_RANK_OFF + tid], mine);
         }
         if (l.notify_host) {
-            __threadfence_system();
-            __syncthreads();
             if (tid == 0) {
-                l.host_page[1] = num_rows;
-                l.host_page[2] = grand;
-                __threadfence_system();
-                __hip_atomic_store(&l.host_page[0], l.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+                host_store(&l.host_page[1], num_rows);
+                host_store(&l.host_page[2], grand);
             }
+            host_stores_arrived();
+            if (tid == 0) host_store(&l.host_page[0], l.seq);
         }
         return;
     }
