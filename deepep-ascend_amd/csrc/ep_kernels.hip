@@ -624,6 +624,13 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
     const int e0 = min(El, tid * per), e1 = min(El, e0 + per);
     int mine = 0;
     for (int e = e0; e < e1; ++e) mine += align_up(s_tot[e], A);
+    if (publisher && (SEND ? a.host_boxes != nullptr : a.notify_host != 0))
+        // (the host's copy, in adjacent words: every other word of a line is a transfer of its own, 384 experts 27 us later)
+        for (int e = tid; e < El; e += EP_LAYOUT_THREADS) {
+            const int r = SEND ? e / a.experts_per_rank : 0, at = a.rank_idx * a.experts_per_rank + (e - r * a.experts_per_rank);
+            if (SEND) host_store(&a.host_boxes[r][a.host_box_slot + at], s_tot[e]);
+            else host_store(&a.host_page[EP_HOST_EXPERT_OFF + e], align_up(s_tot[e], A));
+        }
     const int incl = wave_inclusive_sum(mine);
     if (lane == WAVE - 1) s_tmp[w] = incl;
     __syncthreads();
@@ -640,7 +647,6 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
                 a.unaligned_expert[e] = c;
                 a.psum_expert[e] = run + c;
                 if (a.cumulative_stats != nullptr) atomicAdd(&a.cumulative_stats[e], c);
-                if (a.notify_host) host_store(&a.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
             }
             if (SEND) {
                 // slots are the receivers' business: ranks count from 0, and the receivers get the counts they need
@@ -648,7 +654,6 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
                 if (publisher && a.count_box_off != 0) {
                     const int r = e / a.experts_per_rank, at = a.rank_idx * a.experts_per_rank + (e - r * a.experts_per_rank);
                     ((int*)(a.peer_arenas[r] + a.count_box_off))[at] = c;
-                    if (a.host_boxes != nullptr) host_store(&a.host_boxes[r][a.host_box_slot + at], c);
                 }
                 s_start[e] = 0;
                 continue;
@@ -829,6 +834,8 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_place(
     const int e0 = min(El, tid * per), e1 = min(El, e0 + per);
     int mine = 0;
     for (int e = e0; e < e1; ++e) mine += align_up(s_tot[e], A);
+    if (publisher && a.notify_host)                 // (in adjacent words, as in the slot assignment)
+        for (int e = tid; e < El; e += EP_LAYOUT_THREADS) host_store(&a.host_page[EP_HOST_EXPERT_OFF + e], align_up(s_tot[e], A));
     const int incl = wave_inclusive_sum(mine);
     if (lane == WAVE - 1) s_tmp[w] = incl;
     __syncthreads();
@@ -843,7 +850,6 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_place(
             a.unaligned_expert[e] = c;
             a.psum_expert[e] = run + c;
             if (a.cumulative_stats != nullptr) atomicAdd(&a.cumulative_stats[e], c);
-            if (a.notify_host) host_store(&a.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
         }
         s_tot[e] = run;
         run += align_up(c, A);
