@@ -166,7 +166,16 @@ struct EpSmallArgs {
     EpLayoutArgs l;               // what ep_layout_assign (ep_recv_copy: ep_layout_place) would have been given
     EpScatterArgs s;              // what the copy kernel would have been given
     int num_pad_blocks;           // workgroups behind the row workgroups, each zeroing every num_pad_blocks-th padding piece
+                                  //   (ep_dispatch_chunk_*: not 0 where there is padding to zero; every workgroup takes a share)
+    int tasks_per_block;          // ep_dispatch_chunk_*: (token, part) tasks of a workgroup
 };
+// ep_dispatch_chunk_*: workgroups of EP_CHUNK_THREADS, at most EP_CHUNK_BLOCKS of them (two a CU) beside the publishing one, each
+// with at most EP_CHUNK_OWN entries of its own; the counts of all entries fit 16 bits
+#define EP_CHUNK_THREADS 1024
+#define EP_CHUNK_BLOCKS 512
+#define EP_CHUNK_OWN 512
+#define EP_CHUNK_ENTRIES 16384
+#define EP_CHUNK_TOKENS 4096
 
 // recv_sf layouts: rows of scales, or columns of scales whose stride is the row count of recv_sf
 // (EP_SF_COL_MAJOR) or the expanded row count the layout pass produced (EP_SF_COL_MAJOR_COUNTED:

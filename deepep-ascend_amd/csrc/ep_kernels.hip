@@ -12,6 +12,7 @@
 //   ep_scatter_copy_pack / ep_scatter_quant_pack           token -> one packed row per destination partition
 //   ep_recv_copy                                           ep_layout_place and the copy of the received rows in one launch
 //   ep_dispatch_small_*                                    layout and copy (or pack) of a decode-size dispatch in one launch
+//   ep_dispatch_chunk_*                                    the same of a dispatch of up to a few thousand tokens
 //   ep_sf_transpose                                        scale rows -> scale columns
 //   ep_quant_rows                                          the quantiser alone (rows in place)
 //   ep_combine_k<K> / ep_combine_generic                   K-way gather + fp32 reduce back to token order
@@ -83,13 +84,15 @@ __device__ __forceinline__ uint64_t match_any(int key, int nbits) {
     return peers;
 }
 
+// Every lane must be active.  (DPP shifts inside a row of 16 lanes, then the rows' last lanes broadcast to the rows behind: six
+// dependent VALU operations, where shuffles are six trips through the LDS.)
 __device__ __forceinline__ int wave_inclusive_sum(int v) {
-    const int lane = lane_id();
-#pragma unroll
-    for (int off = 1; off < WAVE; off <<= 1) {
-        const int o = __shfl_up(v, off, WAVE);
-        if (lane >= off) v += o;
-    }
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);      // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);      // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);      // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // row_bcast:15 to rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);      // row_bcast:31 to rows 2 and 3
     return v;
 }
 
@@ -1117,7 +1120,7 @@ __device__ __forceinline__ int64_t scatter_guess_source_row(const EpScatterArgs&
 // (dispatch_copy_epilogue.hpp:547-620).
 __device__ __forceinline__ void zero_span(char* base, int64_t nbytes, int part, int nparts) {
     const u32x4 z = {0u, 0u, 0u, 0u};
-    const int64_t tid = (int64_t)part * EP_ROW_THREADS + threadIdx.x;     // among the threads sharing the span
+    const int64_t tid = (int64_t)part * EP_ROW_THREADS + (threadIdx.x & (EP_ROW_THREADS - 1));    // among the threads sharing the span
     const int64_t nthreads = (int64_t)nparts * EP_ROW_THREADS;
     // 16-byte stores over the aligned body; the ends in 2-byte units (every element here is 2 or 4 bytes wide)
     const int64_t head = min((int64_t)((16 - ((uintptr_t)base & 15)) & 15), nbytes);
@@ -1154,16 +1157,17 @@ __device__ __forceinline__ unsigned early_scales(const EpScatterArgs& a, int64_t
     if (!a.sf_pairs || part != 0 || lane >= (a.num_sf_packs >> 1)) return 0u;
     return *(const unsigned*)((const char*)a.sf + src_row * a.sf_token_stride_bytes + 4 * lane);
 }
-template <bool PACK>
-__device__ __forceinline__ void copy_row_out(const EpScatterArgs& a, const RowCtx& c, int part, const u32x4 (&d)[4], unsigned scales) {
-    const int lane = lane_id(), K = a.num_topk, U = a.vecs_per_lane;
+// (VECS: the most vectors a lane moves per task)
+template <bool PACK, int VECS>
+__device__ __forceinline__ void copy_row_out(const EpScatterArgs& a, const RowCtx& c, int part, const u32x4 (&d)[VECS], unsigned scales) {
+    const int lane = lane_id(), K = a.num_topk, U = VECS == 1 ? 1 : a.vecs_per_lane;
     const int nvec = (int)(a.copy_bytes >> 4);
     for (int j = 0; j < K; ++j) {
         const int s = readlane(c.myslot, j);
         if (s < 0) continue;
         u32x4* row = (u32x4*)(out_rows_of<PACK>(a, c, j) + (int64_t)s * a.out_row_bytes);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < VECS; ++u) {
             const int v = (part * U + u) * WAVE + lane;
             if (u < U && v < nvec) stream_store<EP_SCATTER_ST_POL>(row + v, d[u]);
         }
@@ -1321,6 +1325,49 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_scatter_quant_sw
     scatter_quant_body<false, true>(a);
 }
 
+// What the publishing workgroup of a one-launch dispatch (below) leaves: the handle tensors and the host count page, or
+// (several partitions) the counts in the receivers' inboxes and boxes.
+template <bool PACK, typename CountOf, typename TokensTo>
+__device__ __forceinline__ void publish_dispatch(const EpLayoutArgs& l, int grand, CountOf count_of, const int* s_start, TokensTo tokens_to) {
+    const int E = l.num_experts, R = l.num_ranks, A = l.expert_alignment, El = l.experts_per_rank, tid = threadIdx.x;
+    for (int e = tid; e < E; e += (int)blockDim.x) {
+        const int c = count_of(e);
+        if (PACK) {
+            const int r = e / El, at = l.rank_idx * El + (e - r * El);
+            if (l.count_box_off != 0) ((int*)(l.peer_arenas[r] + l.count_box_off))[at] = c;
+            if (l.host_boxes != nullptr) host_store(&l.host_boxes[r][l.host_box_slot + at], c);
+        } else {
+            l.unaligned_expert[e] = c;
+            l.psum_expert[e] = s_start[e] + c;
+            if (l.cumulative_stats != nullptr) atomicAdd(&l.cumulative_stats[e], c);
+            if (l.notify_host) host_store(&l.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
+        }
+    }
+    for (int r = tid; r < R; r += (int)blockDim.x) {
+        const int rows = min(tokens_to(r), l.max_tokens);
+        if (PACK) {
+            if (l.connected || r == l.rank_idx) ((int*)(l.peer_arenas[r] + EP_WS_INBOX_OFF))[l.rank_idx] = rows;
+            if (l.host_boxes != nullptr) host_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_ROWS_OFF + l.rank_idx], rows);
+        } else {
+            l.psum_rank[r] = rows;
+            if (l.notify_host) host_store(&l.host_page[EP_HOST_RANK_OFF + r], rows);
+        }
+    }
+    if (PACK ? l.host_boxes != nullptr : l.notify_host != 0) {
+        if (!PACK && tid == 0) {
+            host_store(&l.host_page[1], tokens_to(0));
+            host_store(&l.host_page[2], grand);
+        }
+        host_stores_arrived();
+        if (PACK) {
+            for (int r = tid; r < R; r += (int)blockDim.x)
+                host_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_SEQ_OFF + l.rank_idx], l.seq);
+        } else if (tid == 0) {
+            host_store(&l.host_page[0], l.seq);
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------------------
 // A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES entries in one launch.  Instead of a slot
 // assignment in front of the copy (a launch that one or two workgroups of the chip work at, bound by its own dependent
@@ -1361,8 +1408,7 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     const int nvec = QUANT ? s.hidden >> 3 : (int)(s.copy_bytes >> 4);
     const int v = part * WAVE + lane;
     const bool live = works && v < nvec;
-    u32x4 d[4];
-    d[0] = u32x4{0u, 0u, 0u, 0u};
+    u32x4 d[1] = {{0u, 0u, 0u, 0u}};
     if (live) d[0] = __builtin_nontemporal_load((const u32x4*)((const char*)s.x + (int64_t)t * s.x_row_bytes) + v);
     const unsigned scales = !QUANT && works ? early_scales(s, t, part) : 0u;
     float gate = 0.0f;
@@ -1415,42 +1461,8 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     };
 
     if (publisher) {
-        for (int e = tid; e < E; e += EP_ROW_THREADS) {
-            const int c = s_cnt[e];
-            if (PACK) {
-                const int r = e / El, at = l.rank_idx * El + (e - r * El);
-                if (l.count_box_off != 0) ((int*)(l.peer_arenas[r] + l.count_box_off))[at] = c;
-                if (l.host_boxes != nullptr) host_store(&l.host_boxes[r][l.host_box_slot + at], c);
-            } else {
-                l.unaligned_expert[e] = c;
-                l.psum_expert[e] = s_start[e] + c;
-                if (l.cumulative_stats != nullptr) atomicAdd(&l.cumulative_stats[e], c);
-                if (l.notify_host) host_store(&l.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
-            }
-        }
-        for (int r = tid; r < R; r += EP_ROW_THREADS) {
-            const int rows = min(tokens_to(r, EP_TOKENS_PER_BLOCK), l.max_tokens);
-            if (PACK) {
-                if (l.connected || r == l.rank_idx) ((int*)(l.peer_arenas[r] + EP_WS_INBOX_OFF))[l.rank_idx] = rows;
-                if (l.host_boxes != nullptr) host_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_ROWS_OFF + l.rank_idx], rows);
-            } else {
-                l.psum_rank[r] = rows;
-                if (l.notify_host) host_store(&l.host_page[EP_HOST_RANK_OFF + r], rows);
-            }
-        }
-        if (PACK ? l.host_boxes != nullptr : l.notify_host != 0) {
-            if (!PACK && tid == 0) {
-                host_store(&l.host_page[1], tokens_to(0, EP_TOKENS_PER_BLOCK));
-                host_store(&l.host_page[2], grand);
-            }
-            host_stores_arrived();
-            if (PACK) {
-                for (int r = tid; r < R; r += EP_ROW_THREADS)
-                    host_store(&l.host_boxes[r][l.host_box_slot + EP_HOST_BOX_SEQ_OFF + l.rank_idx], l.seq);
-            } else if (tid == 0) {
-                host_store(&l.host_page[0], l.seq);
-            }
-        }
+        publish_dispatch<PACK>(l, grand, [&](int e) { return s_cnt[e]; }, s_start,
+                               [&](int r) { return tokens_to(r, EP_TOKENS_PER_BLOCK); });
         return;
     }
     if (!copies) {
@@ -1532,6 +1544,242 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_q
 extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_copy_pack(EpSmallArgs a) { fetch_arguments<EpSmallArgs>(); dispatch_small_body<false, true, true>(a); }
 extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_quant_pack(EpSmallArgs a) { fetch_arguments<EpSmallArgs>(); dispatch_small_body<true, true, true>(a); }
 extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_quant_sw_pack(EpSmallArgs a) { fetch_arguments<EpSmallArgs>(); dispatch_small_body<true, false, true>(a); }
+
+// ------------------------------------------------------------------------------------------------
+// A dispatch of up to EP_CHUNK_ENTRIES entries in one launch.  Workgroups that fill the chip once, each with an equal share of the
+// (token, part) tasks of the copy: every one of them counts the ids of all tokens (all, and those of the tokens before its own
+// first, in the two halves of one counter an expert), ranks the entries of the few tokens it copies in one wave, and copies (or
+// packs) them.  The payload of a wave's first task is on its way meanwhile; the next one's is fetched ahead of each task's stores.
+// Bound by the copy's traffic behind the phases in front of it; those by the launch, a trip to memory for the ids and the
+// instructions a thread spends on each (1024 threads of a workgroup, eight waves a SIMD with two workgroups a CU).  At 2048 tokens top-8,
+// us from the kernel's start (stamps, 256 workgroups): ids on the way and LDS cleared 1.4, counted 3.0, scanned and ranked 1.8; with a
+// mark byte a token, quotients carried along and a token a wave ranked position by position 6.4 + 2.7 + 1.6 at 512 workgroups,
+// now 5.0 + 2.2.  A replayed dispatch, two launches / this one (us): 200 tokens x 7168 FP8, top-8, alignment 128 56.7 / 49.2; 512 tokens
+// without padding 19.6 / 13.0; 1021 x 2560 BF16, top-7 23.3 / 14.6; 1024 x 7168 BF16, top-8 41.1 / 30.4; 2048 x 7168 66.9 / 53.0; 4096 x
+// 1024 top-2 16.4 / 12.9; one of eight partitions, FP8, all of its dispatch: 256 tokens top-8 32.4 / 18.5, 2048 top-6 71.4 / 65.6.
+// (Padding as equal shares of all padding rows in place of pieces of experts: 256 tokens 50.8 -> 56.9; the ids of two goes in flight:
+// spills, or one workgroup a CU and level.)
+// ------------------------------------------------------------------------------------------------
+template <bool QUANT, bool HW, bool PACK>
+__device__ __forceinline__ void dispatch_chunk_body(const EpSmallArgs& a) {
+    extern __shared__ int smem[];
+    constexpr int NT = EP_CHUNK_THREADS, NW = NT / WAVE, GO = 8;
+    const EpLayoutArgs& l = a.l;
+    const EpScatterArgs& s = a.s;
+    const int E = l.num_experts, R = l.num_ranks, K = l.num_topk, A = l.expert_alignment, El = l.experts_per_rank;
+    const int T = l.num_tokens, n = T * K;
+    unsigned* s_cnt = (unsigned*)smem;                  // [E] entries per expert; high half: those before the ones being ranked
+    int* s_start = (int*)(s_cnt + E);                   // [E] first slot of each expert (one partition)
+    unsigned* s_rcnt = (unsigned*)(s_start + E);        // [R] tokens per partition; high half: those before this workgroup's
+    int* s_rown = (int*)(s_rcnt + R);                   // [R] of this workgroup's, those ranked so far
+    int* s_tmp = s_rown + R;                            // [NW]
+    int* s_rank = s_tmp + NW;                           // [EP_CHUNK_OWN] of an own entry: entries of the same expert before it
+    int* s_rslot = s_rank + EP_CHUNK_OWN;               // [EP_CHUNK_OWN] own tokens before its own in its partition (masters), or -1
+    short* s_key = (short*)(s_rslot + EP_CHUNK_OWN);    // [EP_CHUNK_OWN] its expert, -1: none
+    unsigned* s_mask = (unsigned*)(s_key + EP_CHUNK_OWN);              // [T] partitions a token goes to, a bit each (several), or
+                                                        // [entries / 32 + 2] entries with an expert, a bit each (one partition)
+    const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
+    const bool publisher = blockIdx.x == 0;
+    const int wg = (int)blockIdx.x - 1;
+    const int tasks = T * s.num_parts;
+    const int task0 = publisher ? 0 : min(tasks, wg * a.tasks_per_block), task1 = publisher ? 0 : min(tasks, task0 + a.tasks_per_block);
+    const int first = task0 / s.num_parts, own = task1 > task0 ? (task1 - 1) / s.num_parts - first + 1 : 0;
+    const int nvec = QUANT ? s.hidden >> 3 : (int)(s.copy_bytes >> 4);
+
+    u32x2 id[GO];
+    auto fetch_ids = [&](int i0) {
+#pragma unroll
+        for (int u = 0; u < GO; ++u) id[u] = *(const u32x2*)((const char*)l.topk_idx + 8u * (unsigned)min(i0 + tid + u * NT, n - 1));
+    };
+    fetch_ids(0);
+    u32x4 next = {0u, 0u, 0u, 0u};
+    unsigned next_scales = 0u;
+    float next_gate = 0.0f;
+    auto fetch_task = [&](int task) {
+        if (task >= task1) return;
+        const int t = task / s.num_parts, part = task - t * s.num_parts, v = part * WAVE + lane;
+        next = u32x4{0u, 0u, 0u, 0u};                   // (channels past the end of the row count as zeros in their group)
+        if (v < nvec) next = __builtin_nontemporal_load((const u32x4*)((const char*)s.x + (int64_t)t * s.x_row_bytes) + v);
+        if (!QUANT) next_scales = early_scales(s, t, part);
+        if (part == 0 && lane < K && s.topk_weights != nullptr) next_gate = s.topk_weights[(int64_t)t * K + lane];
+    };
+    fetch_task(task0 + w);
+
+    for (int i = tid; i < E; i += NT) s_cnt[i] = 0u;
+    if (PACK)
+        for (int i = tid; i < T; i += NT) s_mask[i] = 0u;
+    if (tid < R) {
+        s_rcnt[tid] = 0u;
+        s_rown[tid] = 0;
+    }
+    __syncthreads();
+    // (quotients of small integers: (x + 1/2) / y is at least 1 / 2y away from the next integer, far more than the products round)
+    const float per_token = 1.0f / (float)K, per_partition = 1.0f / (float)El;
+    auto partition_of = [&](int e) { return (int)(((float)e + 0.5f) * per_partition); };
+    {
+        const int own0 = first * K, nown = own * K, wave0 = __builtin_amdgcn_readfirstlane(w) * WAVE;
+        for (int i0 = 0; i0 < n; i0 += GO * NT) {
+            if (i0 > 0) fetch_ids(i0);
+#pragma unroll
+            for (int u = 0; u < GO; ++u) {
+                const int i = i0 + tid + u * NT;
+                if (i0 + u * NT + wave0 >= n) break;
+                const bool valid = id[u].y == 0u && id[u].x < (unsigned)E && i < n;
+                if (!PACK) {
+                    const uint64_t bits = __ballot(valid);
+                    if (lane == 0) ((uint64_t*)s_mask)[i >> 6] = bits;
+                }
+                if (valid) {
+                    atomicAdd(&s_cnt[id[u].x], i < own0 ? 0x10001u : 1u);
+                    if (PACK) atomicOr(&s_mask[(int)(((float)i + 0.5f) * per_token)], 1u << partition_of((int)id[u].x));
+                }
+                if ((unsigned)(i - own0) < (unsigned)nown) s_key[i - own0] = valid ? (short)id[u].x : (short)-1;
+            }
+        }
+    }
+    __syncthreads();
+    // ---- tokens per partition; aligned exclusive scan over the experts (one partition) ----
+    {
+        unsigned sum = 0u;                              // lane r < R: of partition r
+        for (int t0 = w * WAVE; t0 < T; t0 += NT) {
+            const int t = t0 + lane, at = t * K;
+            const uint64_t earlier = __ballot(t < first);
+            if (PACK) {
+                const unsigned m = t < T ? s_mask[t] : 0u;
+                for (int r = 0; r < R; ++r) {
+                    const uint64_t to = __ballot((m >> r) & 1u);
+                    if (lane == r) sum += (unsigned)__popcll(to) | (unsigned)__popcll(to & earlier) << 16;
+                }
+            } else {
+                const uint64_t bits = t < T ? ((uint64_t)s_mask[(at >> 5) + 1] << 32 | s_mask[at >> 5]) >> (at & 31) : 0ull;
+                const uint64_t to = __ballot((bits & ((1ull << K) - 1ull)) != 0ull);
+                if (lane == 0) sum += (unsigned)__popcll(to) | (unsigned)__popcll(to & earlier) << 16;
+            }
+        }
+        if (lane < R && sum != 0u) atomicAdd(&s_rcnt[lane], sum);
+    }
+    int grand = 0, mine = 0, incl = 0;
+    const int per = (E + NT - 1) / NT, e0 = min(E, tid * per), e1 = min(E, e0 + per);
+    if (!PACK) {
+        for (int e = e0; e < e1; ++e) mine += align_up((int)(s_cnt[e] & 0xffffu), A);
+        incl = wave_inclusive_sum(mine);
+        if (lane == WAVE - 1) s_tmp[w] = incl;
+    }
+    // ---- meanwhile one wave ranks the own entries, whole tokens at a time: earlier entries with the same expert, masters (the
+    //      last entry of a token for a partition), earlier masters of the same partition ----
+    if (w == NW - 1) {
+        const int ebits = 32 - __builtin_clz(E), rbits = 32 - __builtin_clz(R);
+        const int toks = WAVE / K, pos = lane - lane / K * K;
+        const uint64_t lt = (1ull << lane) - 1ull, later = (1ull << (K - 1 - pos)) - 1ull;
+        for (int c = 0; c < own; c += toks) {
+            const int at = c * K + lane;
+            const bool in = lane < toks * K && at < own * K;
+            const int e = in ? s_key[at] : -1, r = e < 0 ? -1 : PACK ? partition_of(e) : 0;
+            const uint64_t pe = match_any(e + 1, ebits), pr = PACK ? match_any(r + 1, rbits) : __ballot(r == 0);
+            const bool master = r >= 0 && (pr >> lane >> 1 & later) == 0ull;
+            const uint64_t pm = PACK ? match_any(master ? r + 1 : 0, rbits) : __ballot(master);
+            int rank = -1, rslot = -1;
+            if (e >= 0) {
+                const unsigned cnt = s_cnt[e];
+                rank = (int)(cnt >> 16) + __popcll(pe & lt);
+                if ((pe >> lane) == 1ull) s_cnt[e] = cnt + ((unsigned)__popcll(pe) << 16);      // highest peer
+            }
+            if (master) {
+                const int before = s_rown[r];
+                rslot = before + __popcll(pm & lt);
+                if ((pm >> lane) == 1ull) s_rown[r] = rslot + 1;
+            }
+            if (in) {
+                s_rank[at] = rank;
+                s_rslot[at] = rslot;
+            }
+            __builtin_amdgcn_wave_barrier();            // (the LDS operations of a wave complete in order)
+        }
+    }
+    if (!PACK) {
+        __syncthreads();
+        int run = incl - mine;
+        for (int i = 0; i < NW; ++i) {
+            if (i < w) run += s_tmp[i];
+            grand += s_tmp[i];
+        }
+        for (int e = e0; e < e1; ++e) {
+            s_start[e] = run;
+            run += align_up((int)(s_cnt[e] & 0xffffu), A);
+        }
+    }
+    __syncthreads();
+    if (publisher) {
+        publish_dispatch<PACK>(l, grand, [&](int e) { return (int)(s_cnt[e] & 0xffffu); }, s_start,
+                               [&](int r) { return (int)(s_rcnt[r] & 0xffffu); });
+        return;
+    }
+    // ---- the tasks ----
+    for (int task = task0 + w; task < task1; task += NW) {
+        const u32x4 d[1] = {next};
+        const unsigned scales = next_scales;
+        const float gate = next_gate;
+        fetch_task(task + NW);
+        const int t = task / s.num_parts, part = task - t * s.num_parts, at = (t - first) * K + lane;
+        const int e = lane < K ? s_key[at] : -1, r = PACK ? partition_of(e) : 0;
+        int rank = -1, rslot = -1, slot = -1;
+        if (e >= 0) {
+            rank = s_rank[at];
+            if (PACK || part == 0) {
+                rslot = s_rslot[at];
+                if (rslot >= 0) rslot += (int)(s_rcnt[r] >> 16);
+            }
+            if (!PACK) slot = s_start[e] + rank;
+            else if (rslot >= 0 && rslot < s.max_tokens) slot = (s.region_by_source ? s.rank_idx : r) * s.max_tokens + rslot;
+        }
+        RowCtx c;
+        c.t = t;
+        c.src_row = t;
+        c.mybase = PACK && slot >= 0 ? (uint64_t)(s.peer_arenas[r] + s.buffer_off) : 0;
+        c.myslot = slot;
+        if (part == 0) {
+            if (lane < K) {
+                l.dst_buffer_slot_idx[(int64_t)t * K + lane] = rslot;
+                l.dst_gsge_idx[(int64_t)t * K + lane] = -1;             // every copy is local: no transport descriptors
+            }
+            if (PACK) {
+                pack_row_metadata(s, c, lane < K && e < 0 ? l.topk_idx[(int64_t)t * K + lane] : e, gate, rank);
+            } else {
+                const uint64_t vm = __ballot(slot >= 0);
+                const int last = vm != 0 ? 63 - __builtin_clzll(vm) : 0;
+                const int row = readlane(rslot, last);
+                // [slot_0 .. slot_{K-1}, src_token_global_idx, last local j]  (dispatch_copy_epilogue.hpp:514-522)
+                const int mv = lane < K ? slot : (lane == K ? s.rank_idx * s.max_tokens + t : last);
+                if (vm != 0 && lane < K + 2 && row >= 0 && row < s.num_meta_rows) s.recv_src_metadata[(int64_t)row * (K + 2) + lane] = mv;
+            }
+        }
+        if (!PACK) {
+            c.myslot = slot < s.num_out_rows ? slot : -1;
+            if (part == 0 && s.recv_topk_weights != nullptr && c.myslot >= 0) s.recv_topk_weights[c.myslot] = gate;
+        }
+        const int v = part * WAVE + lane;
+        if (QUANT) quant_row_out<HW, PACK>(s, c, v, v < nvec, d[0]);
+        else copy_row_out<PACK>(s, c, part, d, scales);
+    }
+    // ---- padding, in pieces of a 256-thread workgroup ----
+    if (!PACK && a.num_pad_blocks > 0) {
+        constexpr int GROUPS = NT / EP_ROW_THREADS;
+        const int pieces = s.num_local_experts * s.pad_blocks_per_expert;
+        for (int p = wg * GROUPS + __builtin_amdgcn_readfirstlane(tid / EP_ROW_THREADS); p < pieces; p += ((int)gridDim.x - 1) * GROUPS) {
+            const int e = p / s.pad_blocks_per_expert;
+            const int end = __builtin_amdgcn_readfirstlane(s_start[e] + (int)(s_cnt[e] & 0xffffu));
+            zero_padding_piece(s, end, p - e * s.pad_blocks_per_expert);
+        }
+    }
+}
+#define EP_CHUNK_KERNEL(NAME, QUANT, HW, PACK) \
+    extern "C" __global__ __launch_bounds__(EP_CHUNK_THREADS, 8) void ep_dispatch_chunk_##NAME(EpSmallArgs a) { fetch_arguments<EpSmallArgs>(); dispatch_chunk_body<QUANT, HW, PACK>(a); }
+EP_CHUNK_KERNEL(copy, false, true, false)
+EP_CHUNK_KERNEL(quant, true, true, false)
+EP_CHUNK_KERNEL(quant_sw, true, false, false)
+EP_CHUNK_KERNEL(copy_pack, false, true, true)
+EP_CHUNK_KERNEL(quant_pack, true, true, true)
+EP_CHUNK_KERNEL(quant_sw_pack, true, false, true)
 
 // ------------------------------------------------------------------------------------------------
 // Receive side of a node whose send sides ship ranks, placing and copying in one launch: what ep_layout_place and the

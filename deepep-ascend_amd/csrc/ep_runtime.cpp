@@ -115,6 +115,7 @@ struct Kernels {
     hipFunction_t scatter_copy, scatter_quant, scatter_quant_sw, sf_transpose;
     hipFunction_t scatter_copy_pack, scatter_quant_pack, scatter_quant_sw_pack;
     hipFunction_t small[2][3];       // [packs][copy, quant, quant_sw]
+    hipFunction_t chunk[2][3];
     hipFunction_t recv_copy;
     hipFunction_t combine[3][5];     // [mode][generic, k2, k4, k6, k8]
     hipFunction_t combine_odd[3];    // single partition, small launches: k3, k5, k7
@@ -201,6 +202,8 @@ void load_kernels(const char* dir) {
     for (int i = 0; i < 3; ++i) {
         get(g_k.small[0][i], (std::string("ep_dispatch_small_") + small_names[i]).c_str());
         get(g_k.small[1][i], (std::string("ep_dispatch_small_") + small_names[i] + "_pack").c_str());
+        get(g_k.chunk[0][i], (std::string("ep_dispatch_chunk_") + small_names[i]).c_str());
+        get(g_k.chunk[1][i], (std::string("ep_dispatch_chunk_") + small_names[i] + "_pack").c_str());
     }
     get(g_k.recv_copy, "ep_recv_copy");
     get(g_k.sf_transpose, "ep_sf_transpose");
@@ -387,6 +390,45 @@ void launch_small(const EpLayoutArgs& la, const EpScatterArgs& sa, bool pack, bo
     EP_HOST_ASSERT(sa.vecs_per_lane == 1);
     launch(g_k.small[pack][quantise ? (g_fp8_hw ? 1 : 2) : 0], 1u + (unsigned)sa.num_row_blocks + (unsigned)num_pad_blocks, EP_ROW_THREADS,
            small_lds(la.num_experts, la.num_ranks), stream, args);
+}
+
+
+// Chunk sizes: layout and copy in one launch as well, by workgroups that all count every id (ep_dispatch_chunk_*).
+unsigned chunk_lds(int num_tokens, int K, int E, int R) {
+    const unsigned marks = R > 1 ? (unsigned)num_tokens : (unsigned)ceil_div((int64_t)num_tokens * K, 64) * 2u + 2u;
+    return (unsigned)(2 * E + 2 * R + EP_CHUNK_THREADS / 64 + 2 * EP_CHUNK_OWN) * sizeof(int) + EP_CHUNK_OWN * sizeof(short) + marks * sizeof(int);
+}
+// Up to here one launch is the faster form: what it costs is ids to every workgroup, what it saves is the launches and trips
+// of the layout in front.  us of a replayed dispatch, two launches / one: 129 tokens x 256, top-2 9.1 / 6.7; 512 x 4096 top-32
+// 60.4 / 34.6; 2048 x 7168 BF16 top-8 (16384 entries) 66.9 / 53.0, 108.6 / 105.2 with alignment 128; 2700 FP8 top-6 65.8 / 62.3;
+// 4096 x 512 top-4 16.8 / 14.5; beyond: 3000 tokens FP8 top-6 67.0 / 65.7, 4096 top-6 58.7 / 60.1, top-8 BF16 152 / 157, 8192 x 512 top-2 16.3 / 22.1.
+// Several partitions, all of a partition's dispatch: two of 2048 tokens x 2048 top-8 44.0 / 41.3, four of 1500 x 7168 top-8 94.3 / 86.4, 32 of 1024 top-6
+// 54.8 / 48.0; beyond, four of 4096 top-4 89.3 / 90.2, two of 4096 x 2048 top-2 38.7 / 38.7 (a word a token is kept in LDS).
+// (a partition is a bit of that word)
+bool chunk_dispatch(int num_tokens, int K, int E, int R) {
+    return num_tokens > 0 and num_tokens <= (R > 1 ? EP_CHUNK_TOKENS / 2 : EP_CHUNK_TOKENS) and num_tokens * K <= EP_CHUNK_ENTRIES and R <= 32 and
+           chunk_lds(num_tokens, K, E, R) <= 64 * 1024;
+}
+// Workgroups: no more than one task a wave needs.  Two a CU keep twice the rows on the way, one a CU counts the ids half as
+// often (us at 256 / 512 workgroups): 1024 x 7168 BF16 top-8 31.7 / 30.4, eight partitions of 1024 68.9 / 66.9; 2048 x 7168 top-8
+// 53.0 / 60.3, eight partitions of 2048 FP8 top-6 65.6 / 67.6; rows of fewer parts, 2048 x 4096 top-4 26.8 / 28.5, 4096 x 1024 top-2 12.9 / 15.3.
+// Padding is shared by all workgroups: as many as there is padding for.
+void launch_chunk(const EpLayoutArgs& la, const EpScatterArgs& sa, bool pack, bool quantise, unsigned pad_pieces, void* stream) {
+    EpSmallArgs args{};
+    args.l = la;
+    args.s = sa;
+    args.num_pad_blocks = pad_pieces > 0;
+    EP_HOST_ASSERT(sa.vecs_per_lane == 1 and sa.num_rows_bound == la.num_tokens);
+    const int64_t tasks = (int64_t)la.num_tokens * sa.num_parts;
+    const bool two_a_cu = sa.num_parts >= 10 and la.num_tokens * la.num_topk <= EP_CHUNK_ENTRIES / 2;
+    const int64_t most = two_a_cu ? EP_CHUNK_BLOCKS : EP_CHUNK_BLOCKS / 2;
+    const int64_t blocks = std::min<int64_t>(most, ceil_div(tasks, EP_CHUNK_THREADS / 64));
+    args.tasks_per_block = (int)ceil_div(tasks, blocks);
+    const int64_t own = (args.tasks_per_block + sa.num_parts - 2) / sa.num_parts + 1;      // tokens that so many tasks can touch
+    EP_HOST_ASSERT(own * la.num_topk <= EP_CHUNK_OWN);
+    const int64_t pads = std::min<int64_t>(most, ceil_div((int64_t)pad_pieces, EP_CHUNK_THREADS / EP_ROW_THREADS));
+    launch(g_k.chunk[pack][quantise ? (g_fp8_hw ? 1 : 2) : 0], 1u + (unsigned)std::max(blocks, pads), EP_CHUNK_THREADS,
+           chunk_lds(la.num_tokens, la.num_topk, la.num_experts, la.num_ranks), stream, args);
 }
 
 // Scale packs (2 bytes) can move two at a time: packs side by side, rows that start on 4 bytes where they are read and written.
@@ -793,7 +835,7 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
 
         const RankBoxes boxes = cached_mode ? RankBoxes{} : rank_boxes(b, a.num_max_tokens_per_rank, num_topk, a.num_experts);
         int* rank_map = nullptr;
-        const EpLayoutArgs* small_layout = nullptr;     // the pack launch works out the layout as well
+        const EpLayoutArgs* own_layout = nullptr;       // the pack launch works out the layout as well
         // geometry of the packed rows of the partition-major regions (only materialised when R > 1)
         const PackedToken pk = packed_token(hidden * packed_elem, packed_sf * 2, num_topk, not cached_mode);
         auto launch_pack = [&]() {
@@ -842,8 +884,9 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
             sa.num_parts = (int)std::max<int64_t>(1, a.fused_fp8_quant ? ceil_div(hidden, 512) : ceil_div(sa.copy_bytes, 1024));
             sa.num_row_blocks = (int)ceil_div((int64_t)num_tokens * sa.num_parts, EP_ROWS_PER_BLOCK);
             if (sa.num_row_blocks == 0) return;
-            if (small_layout != nullptr) {
-                launch_small(*small_layout, sa, true, a.fused_fp8_quant != 0, 0, a.stream);
+            if (own_layout != nullptr) {
+                if (small_dispatch(num_tokens, num_topk)) launch_small(*own_layout, sa, true, a.fused_fp8_quant != 0, 0, a.stream);
+                else launch_chunk(*own_layout, sa, true, a.fused_fp8_quant != 0, 0, a.stream);
                 return;
             }
             hipFunction_t fn = a.fused_fp8_quant ? (g_fp8_hw ? g_k.scatter_quant_pack : g_k.scatter_quant_sw_pack)
@@ -925,11 +968,11 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
         la.cumulative_stats = (int*)a.cumulative_local_expert_recv_stats.data;
         la.host_page = b->host_page_dev;
 
-        const bool small = small_dispatch(num_tokens, K);
+        const bool one_launch = small_dispatch(num_tokens, K) or chunk_dispatch(num_tokens, K, E, R);
         b->last.layout_pending = b->last.place_pending = b->last.copied = false;
-        if (small and num_ranks > 1) {
-            small_layout = &la;
-        } else if (small and epilogue_follows) {
+        if (one_launch and num_ranks > 1) {
+            own_layout = &la;
+        } else if (one_launch and epilogue_follows) {
             b->last.layout_pending = true;
             b->last.pending = la;
         } else {
@@ -1334,8 +1377,11 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
             // the one launch sizes its LDS by the begin's experts and pads by the epilogue's
             EP_HOST_ASSERT(a.num_experts == b->last.num_experts and a.expert_alignment == b->last.alignment and
                            "the copy epilogue has the experts and the alignment of its ep_dispatch_begin");
-            launch_small(b->last.pending, sa, false, quantise_here,
-                         (int)small_pad_blocks(pad_blocks, num_tokens, K, El, a.expert_alignment, sa.out_row_bytes), a.stream);
+            if (small_dispatch(num_tokens, K))
+                launch_small(b->last.pending, sa, false, quantise_here,
+                             (int)small_pad_blocks(pad_blocks, num_tokens, K, El, a.expert_alignment, sa.out_row_bytes), a.stream);
+            else
+                launch_chunk(b->last.pending, sa, false, quantise_here, pad_blocks, a.stream);
             b->last.layout_pending = false;
             b->last.copied = true;
         } else if (place_here) {

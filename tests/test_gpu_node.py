@@ -674,6 +674,27 @@ def test_receive_side_in_one_launch(R, max_tokens, H, E, K, A, masked, do_cpu_sy
         b.destroy()
 
 
+SEND_CASES = [
+    # R, max_tokens, H, E, K, A, masked
+    (32, 131, 64, 64, 8, 1, 0.3),          # a bit a partition, every one used
+    (3, 700, 1056, 93, 23, 4, 0.1),        # 31 experts a partition, two tokens a turn of the ranking wave
+    (2, 2049, 64, 16, 3, 8, 0.2),          # one partition beyond the tokens of one launch, the other at them
+    (2, 140, 160, 2046, 5, 1, 0.0),        # 1023 experts a partition
+    (4, 300, 5152, 16, 2, 16, 0.1),        # two workgroups a CU
+]
+
+
+@pytest.mark.parametrize('R,max_tokens,H,E,K,A,masked', SEND_CASES)
+def test_send_side_in_one_launch(R, max_tokens, H, E, K, A, masked):
+    """Layout and pack of the send side in one launch, at the edges of what that takes."""
+    test_receive_side_in_one_launch(R, max_tokens, H, E, K, A, masked, True)
+
+
+@pytest.mark.parametrize('mode', ['fp8_fused', 'fp8_prequant'])
+def test_send_side_in_one_launch_with_scales(mode):
+    test_node_dispatch_combine(4, 260, 1056, 32, 6, 16, 0.1, mode, True)
+
+
 @pytest.mark.parametrize('begin', [True, False])
 @pytest.mark.parametrize('alignment', [8, 1])
 def test_receive_side_through_the_abi(begin, alignment):

@@ -69,6 +69,27 @@ def test_small_dispatch(T, H, E, K, A, masked, zipf, mode):
     buf.destroy()
 
 
+CHUNK_CASES = [
+    # T, H, E, K, A, masked, zipf
+    (130, 16, 8, 1, 1, 0.0, None),          # one workgroup a wave's worth of tasks each
+    (200, 512, 2048, 32, 16, 0.1, None),    # most experts, most entries a token, 16 own tokens a workgroup (one part a row)
+    (512, 528, 40, 32, 3, 0.3, None),       # every entry of the limit
+    (2048, 272, 256, 8, 128, 0.1, 1.2),     # the same, hot and empty experts
+    (4096, 64, 5, 4, 64, 0.5, None),        # and every token
+    (1021, 2576, 64, 7, 32, 0.0, None),     # tokens shared by two workgroups
+    (300, 5136, 300, 5, 16, 0.2, None),     # two workgroups a CU
+    (1366, 64, 12, 12, 1, 0.0, None),       # beyond the entries: two launches
+    (4097, 64, 8, 2, 8, 0.0, None),         # beyond the tokens
+]
+
+
+@pytest.mark.parametrize('T,H,E,K,A,masked,zipf', CHUNK_CASES)
+@pytest.mark.parametrize('mode', ['bf16', 'fused', 'pair'])
+def test_chunk_dispatch(T, H, E, K, A, masked, zipf, mode):
+    """The same of dispatches beyond decode size that are one launch, at the edges of what that takes."""
+    test_small_dispatch(T, H, E, K, A, masked, zipf, mode)
+
+
 def test_small_dispatch_deferred_exact_and_replayed():
     """The same handles from the calls that keep the two launches (a deferred epilogue, exact sizes), and a cached
     dispatch behind the single launch."""
