@@ -89,6 +89,41 @@ py::object new_event() {
     return (*cls)();
 }
 
+// The event behind the launches of a deferred call, recorded by the library (as part of the last launch where it can be).
+class LaunchEvent {
+public:
+    LaunchEvent() { check_hip(hipEventCreateWithFlags(&event_, hipEventDisableTiming)); }
+    ~LaunchEvent() { (void)hipEventDestroy(event_); }
+    LaunchEvent(const LaunchEvent&) = delete;
+    LaunchEvent& operator=(const LaunchEvent&) = delete;
+    void* get() const { return (void*)event_; }
+    void current_stream_wait() { check_hip(hipStreamWaitEvent((hipStream_t)::current_stream(), event_, 0)); }
+    // what torch.cuda.Event offers of an event that is already recorded
+    void wait(const py::object& stream) {
+        if (stream.is_none()) return current_stream_wait();
+        check_hip(hipStreamWaitEvent((hipStream_t)stream.attr("cuda_stream").cast<uintptr_t>(), event_, 0));
+    }
+    bool query() {
+        const hipError_t rc = hipEventQuery(event_);
+        if (rc != hipErrorNotReady) check_hip(rc);
+        return rc == hipSuccess;
+    }
+    void synchronize() {
+        py::gil_scoped_release release;
+        check_hip(hipEventSynchronize(event_));
+    }
+
+private:
+    static void check_hip(hipError_t rc) {
+        if (rc != hipSuccess) throw EpPyError(hipGetErrorString(rc));
+    }
+    hipEvent_t event_ = nullptr;
+};
+py::object event_handle(std::unique_ptr<LaunchEvent> event) {
+    static auto* cls = new py::object(py::module_::import("deep_ep._C").attr("_LaunchEventHandle"));
+    return (*cls)(py::cast(std::move(event)));
+}
+
 // Uninitialised device tensors straight from torch's caching allocator (what at::empty reaches through its
 // dispatcher).
 at::Tensor alloc(at::IntArrayRef shape, at::ScalarType dtype, const at::Device& dev) {
@@ -398,14 +433,17 @@ public:
         a.stream = current_stream();
         // (the copy follows at once, unless it is deferred or the output sizes are waited for first)
         const bool copy_follows = num_ranks_ == 1 && !defer_epilogue && !(do_cpu_sync && exact_sync_sizes_);
-        check(copy_follows ? ep_dispatch_begin(buf_, &a) : ep_dispatch_launch(buf_, &a));
+        std::unique_ptr<LaunchEvent> event;
+        if (defer_epilogue && async_with_compute_stream) event = std::make_unique<LaunchEvent>();
+        check(event != nullptr ? ep_dispatch_launch_event(buf_, &a, event->get())
+                               : copy_follows ? ep_dispatch_begin(buf_, &a) : ep_dispatch_launch(buf_, &a));
         // the epilogue below belongs to this launch: the library refuses it once a later dispatch has taken over
         // the buffer's workspace
         s.stamp = ep_dispatch_stamp(buf_);
 
         if (defer_epilogue) {
             if (!async_with_compute_stream) throw EpPyError("Assertion exception (python_api.cpp): async_with_compute_stream");
-            py::object ev = new_event();
+            py::object ev = event_handle(std::move(event));
             py::cpp_function epilogue([st]() { return run_dispatch_epilogue(*st); });
             return py::make_tuple(py::none(), ev, epilogue);
         }
@@ -454,11 +492,14 @@ public:
         c.stream = current_stream();
         // owner side; with one partition it only validates, which the token side below repeats: then it is called
         // only where the token side is deferred, so that a bad argument still fails at the call
-        if (num_ranks_ > 1 || defer_epilogue) check(ep_combine_launch(buf_, &c, 0));
+        std::unique_ptr<LaunchEvent> event;
+        if (defer_epilogue && async_with_compute_stream) event = std::make_unique<LaunchEvent>();
+        if (event != nullptr) check(ep_combine_begin_event(buf_, &c, event->get()));
+        else if (num_ranks_ > 1 || defer_epilogue) check(ep_combine_launch(buf_, &c, 0));
 
         if (defer_epilogue) {
             if (!async_with_compute_stream) throw EpPyError("Assertion exception (python_api.cpp): async_with_compute_stream");
-            py::object ev = new_event();
+            py::object ev = event_handle(std::move(event));
             py::cpp_function epilogue([st]() { return run_combine_epilogue(*st); });
             return py::make_tuple(py::none(), ev, epilogue);
         }
@@ -483,6 +524,11 @@ PYBIND11_MODULE(_native, m) {
         const auto stream = c10::hip::getCurrentHIPStream();
         return py::make_tuple((int64_t)stream.id(), (int)stream.device_index(), (int)stream.unwrap().device_type());
     }, "(stream_id, device_index, device_type) of the current stream");
+    py::class_<LaunchEvent>(m, "LaunchEvent")
+        .def("current_stream_wait", &LaunchEvent::current_stream_wait)
+        .def("wait", &LaunchEvent::wait, py::arg("stream") = py::none())
+        .def("query", &LaunchEvent::query)
+        .def("synchronize", &LaunchEvent::synchronize);
     py::class_<NativeBuffer>(m, "Buffer")
         .def(py::init<uintptr_t, int, int>())
         .def("set_connected", &NativeBuffer::set_connected)

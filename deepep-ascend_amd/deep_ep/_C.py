@@ -311,6 +311,14 @@ class EventHandle:
         _current_stream().wait_event(self.event)
 
 
+class _LaunchEventHandle(EventHandle):
+    """An event that the library recorded behind the launches of a deferred call."""
+
+    def __init__(self, event):
+        self.event = event
+        self.current_stream_wait = event.current_stream_wait
+
+
 class Context:
     """The part of the reference's comm::Context the Python API reads."""
 

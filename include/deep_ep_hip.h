@@ -147,6 +147,9 @@ typedef struct ep_dispatch_args {
  * partition this is the send side (dst_buffer_slot_idx, dst_gsge_idx, packed rows, inbox counts)
  * and ep_dispatch_recv_launch writes the other handle tensors. */
 int ep_dispatch_launch(ep_buffer_t* buf, const ep_dispatch_args_t* args);
+/* The same, with an event (a hipEvent_t of the device, made by the caller) that is recorded behind everything the call has
+ * enqueued on its stream, as a hipEventRecord right after it would, but where that is possible as part of the last launch. */
+int ep_dispatch_launch_event(ep_buffer_t* buf, const ep_dispatch_args_t* args, void* event);
 /* The same for a caller whose next call on this buffer is this dispatch's ep_dispatch_epilogue_launch: the library may
  * then leave the layout to the copy launch (one partition, at most 128 tokens and 1024 (token, slot) entries: one
  * launch instead of two).  Everything this call would have enqueued is then enqueued by the epilogue, on the epilogue's
@@ -294,6 +297,8 @@ typedef struct ep_combine_args {
  * a partition used alone (not connected) holds only its own partials after phase 0, the caller
  * places the others (what a transport would deliver) before phase 1. */
 int ep_combine_launch(ep_buffer_t* buf, const ep_combine_args_t* args, int phase);
+/* Phase 0 with an event behind it (see ep_dispatch_launch_event). */
+int ep_combine_begin_event(ep_buffer_t* buf, const ep_combine_args_t* args, void* event);
 
 #ifdef __cplusplus
 }

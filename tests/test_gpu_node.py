@@ -749,3 +749,105 @@ def test_receive_side_through_the_abi(begin, alignment):
     del sent
     for b in bufs:
         b.destroy()
+
+
+def deferred_pass(bufs, xs, topks, ws, ys, wait, **kw):
+    """A dispatch and a combine, deferred; `wait` orders what follows behind the events of a phase."""
+    sent = [b.dispatch(x, topk_idx=t, topk_weights=w, do_expand=True, do_cpu_sync=False, do_zero_padding=True,
+                       async_with_compute_stream=True, defer_epilogue=True, **kw) for b, x, t, w in zip(bufs, xs, topks, ws)]
+    wait(sent)
+    got = [e.current_stream_wait() for e in sent]
+    reduced = [b.combine(y, h, topk_weights=w, async_with_compute_stream=True, defer_epilogue=True)
+               for b, y, (_, _, w, h) in zip(bufs, ys, got)]
+    wait(reduced)
+    results = [e.current_stream_wait() for e in reduced]
+    return [(h.psum_num_recv_tokens_per_expert, rows, w, out, out_w) for (rows, _, w, h), (out, out_w) in zip(got, results)]
+
+
+EVENT_CASES = [
+    # R, tokens, H, E, K, A
+    (1, 40, 256, 8, 2, 4),            # one partition: the event behind the layout alone, and behind nothing
+    (2, 40, 256, 8, 2, 4),            # layout and pack in one launch of decode size
+    (2, 700, 512, 16, 4, 8),          # of chunk size
+    (2, 2300, 512, 16, 4, 8),         # in launches of their own
+    (3, 0, 256, 12, 3, 4),            # nobody has anything to send
+]
+
+
+@pytest.mark.parametrize('R,T,H,E,K,A', EVENT_CASES)
+def test_events_of_deferred_calls_order_other_streams(R, T, H, E, K, A):
+    """The phases on streams of their own, ordered by the events of the deferred calls alone, behind work that takes a while;
+    and captured into a graph.  Both leave what one stream leaves."""
+    import deep_ep
+    max_tokens = max(T, 16)
+    bufs = [deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=max_tokens, hidden=H, num_topk=K,
+                             explicitly_destroy=True)] if R == 1 else make_node(R, max_tokens, H, K, False)
+    rows = [make_tokens(T, H, seed=r).to(DEV) for r in range(R)]
+    routing = [make_routing(T, E, K, seed=5 + r, masked=0.1) for r in range(R)]
+    topks, ws = [t.to(DEV) for t, _ in routing], [w.to(DEV) for _, w in routing]
+    kw = dict(num_experts=E, num_max_tokens_per_rank=max_tokens, expert_alignment=A)
+    gen = torch.Generator(device=DEV).manual_seed(3)
+    n = O.no_sync_sizes(R, max_tokens, K, E, A)[1]
+    y = [torch.randn((n, H), generator=gen, device=DEV, dtype=torch.bfloat16) for _ in bufs]
+
+    def seen(results):
+        out = []
+        for psum, recv, w, combined, weights in results:
+            used = int(psum[-1])                                             # (behind it nothing is written)
+            out += [psum.cpu(), bf16_bits(recv[:used]), w[:used].cpu(), bf16_bits(combined), weights.cpu()]
+        return [np.asarray(o) for o in out]
+
+    want = seen(deferred_pass(bufs, rows, topks, ws, y, lambda events: None, **kw))
+    xs, ys = [torch.zeros_like(x) for x in rows], [torch.zeros_like(v) for v in y]
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    torch.cuda.synchronize()
+    late = [list(zip(xs, rows)), list(zip(ys, y))]
+
+    def arrive():
+        torch.cuda._sleep(20_000_000)
+        for to, source in late.pop(0):
+            to.copy_(source)
+
+    def wait(events):
+        assert all(not e.event.event.query() for e in events)                # (the sleep in front of the phase)
+        torch.cuda.set_stream(streams.pop(0))
+        for e in events:
+            e.event.current_stream_wait()
+        if late:
+            arrive()
+
+    here = torch.cuda.current_stream()
+    try:
+        torch.cuda.set_stream(streams.pop(0))
+        arrive()
+        results = deferred_pass(bufs, xs, topks, ws, ys, wait, **kw)
+        torch.cuda.current_stream().synchronize()
+    finally:
+        torch.cuda.set_stream(here)
+    for a, b in zip(seen(results), want):
+        assert np.array_equal(a, b)
+    torch.cuda.synchronize()
+
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        deferred_pass(bufs, xs, topks, ws, ys, lambda events: None, **kw)
+    side.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = deferred_pass(bufs, xs, topks, ws, ys, lambda events: None, **kw)
+    for _ in range(3):
+        for _, recv, w, combined, weights in captured:
+            for t in (recv, w, combined, weights):
+                t.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(seen(captured), want):
+            assert np.array_equal(a, b)
+    ev = bufs[0].dispatch(xs[0], topk_idx=topks[0], topk_weights=ws[0], do_expand=True, do_cpu_sync=False,
+                          async_with_compute_stream=True, defer_epilogue=True, **kw)
+    ev.event.event.synchronize()
+    assert ev.event.event.query()
+    side.wait_event(ev.event.event)
+    for b in bufs:
+        b.destroy()
