@@ -627,7 +627,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
     const int e0 = min(El, tid * per), e1 = min(El, e0 + per);
     int mine = 0;
     for (int e = e0; e < e1; ++e) mine += align_up(s_tot[e], A);
-    if (publisher && (SEND ? a.host_boxes != nullptr : a.notify_host != 0))
+    if (publisher && !RECV && (SEND ? a.host_boxes != nullptr : a.notify_host != 0))
         // (the host's copy, in adjacent words: every other word of a line is a transfer of its own, 384 experts 27 us later)
         for (int e = tid; e < El; e += EP_LAYOUT_THREADS) {
             const int r = SEND ? e / a.experts_per_rank : 0, at = a.rank_idx * a.experts_per_rank + (e - r * a.experts_per_rank);
@@ -694,6 +694,11 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
             if (a.notify_host) host_store(&a.host_page[EP_HOST_RANK_OFF + r], upto - from);
         }
         if (a.notify_host) {
+            if (RECV) {                 // (from the first slots: ahead of the scan its registers spill)
+                __syncthreads();
+                for (int e = tid; e < El; e += EP_LAYOUT_THREADS)
+                    host_store(&a.host_page[EP_HOST_EXPERT_OFF + e], (e + 1 < El ? s_start[e + 1] : grand) - s_start[e]);
+            }
             if (tid == 0) {
                 host_store(&a.host_page[1], n_recv);
                 host_store(&a.host_page[2], grand);
