@@ -361,7 +361,7 @@ __device__ __forceinline__ void layout_assign_body(const EpLayoutArgs& a) {
 
     // The launch has one workgroup more than blocks of tokens.  It ranks nothing: it gets the totals like the others
     // (a single block: it counts that block's ids once more) and publishes them (handle tensors, inboxes, the host count
-    // page with its two system-scope fences), so that no ranking workgroup has that on its way.
+    // page and the wait for its stores), so that no ranking workgroup has that on its way.
     const bool single = !FOLD && a.scan_mode == EP_LAYOUT_SINGLE;     // (the summing instance never runs alone)
     const bool publisher = b == a.num_blocks, worker = !publisher;
     const int kb = single ? 0 : b;         // the block whose ids this workgroup stages

@@ -151,8 +151,8 @@ int ep_dispatch_launch(ep_buffer_t* buf, const ep_dispatch_args_t* args);
  * enqueued on its stream, as a hipEventRecord right after it would, but where that is possible as part of the last launch. */
 int ep_dispatch_launch_event(ep_buffer_t* buf, const ep_dispatch_args_t* args, void* event);
 /* The same for a caller whose next call on this buffer is this dispatch's ep_dispatch_epilogue_launch: the library may
- * then leave the layout to the copy launch (one partition, at most 128 tokens and 1024 (token, slot) entries: one
- * launch instead of two).  Everything this call would have enqueued is then enqueued by the epilogue, on the epilogue's
+ * then leave the layout to the copy launch (one partition, at most 4096 tokens and 16384 (token, slot) entries:
+ * one launch instead of two or three).  Everything this call would have enqueued is then enqueued by the epilogue, on the epilogue's
  * stream: the handle tensors, the running statistics and the host counts are complete behind the epilogue only, and the
  * inputs have to stay until then.  An epilogue on another stream is ordered behind what the begin is ordered behind by
  * the caller, as after ep_dispatch_launch (an event recorded after the begin, waited for on the other stream). */
