@@ -92,17 +92,19 @@ py::object new_event() {
 // The event behind the launches of a deferred call, recorded by the library (as part of the last launch where it can be).
 class LaunchEvent {
 public:
-    LaunchEvent() { check_hip(hipEventCreateWithFlags(&event_, hipEventDisableTiming)); }
+    LaunchEvent() {
+        check_hip(hipGetDevice(&device_));
+        check_hip(hipEventCreateWithFlags(&event_, hipEventDisableTiming));
+    }
     ~LaunchEvent() { (void)hipEventDestroy(event_); }
     LaunchEvent(const LaunchEvent&) = delete;
     LaunchEvent& operator=(const LaunchEvent&) = delete;
     void* get() const { return (void*)event_; }
+    uintptr_t handle() const { return (uintptr_t)event_; }
+    int device() const { return device_; }
     void current_stream_wait() { check_hip(hipStreamWaitEvent((hipStream_t)::current_stream(), event_, 0)); }
-    // what torch.cuda.Event offers of an event that is already recorded
-    void wait(const py::object& stream) {
-        if (stream.is_none()) return current_stream_wait();
-        check_hip(hipStreamWaitEvent((hipStream_t)stream.attr("cuda_stream").cast<uintptr_t>(), event_, 0));
-    }
+    void wait(uintptr_t stream) { check_hip(hipStreamWaitEvent((hipStream_t)stream, event_, 0)); }
+    void record(uintptr_t stream) { check_hip(hipEventRecord(event_, (hipStream_t)stream)); }
     bool query() {
         const hipError_t rc = hipEventQuery(event_);
         if (rc != hipErrorNotReady) check_hip(rc);
@@ -118,6 +120,7 @@ private:
         if (rc != hipSuccess) throw EpPyError(hipGetErrorString(rc));
     }
     hipEvent_t event_ = nullptr;
+    int device_ = 0;
 };
 py::object event_handle(std::unique_ptr<LaunchEvent> event) {
     static auto* cls = new py::object(py::module_::import("deep_ep._C").attr("_LaunchEventHandle"));
@@ -526,7 +529,10 @@ PYBIND11_MODULE(_native, m) {
     }, "(stream_id, device_index, device_type) of the current stream");
     py::class_<LaunchEvent>(m, "LaunchEvent")
         .def("current_stream_wait", &LaunchEvent::current_stream_wait)
-        .def("wait", &LaunchEvent::wait, py::arg("stream") = py::none())
+        .def_property_readonly("handle", &LaunchEvent::handle)
+        .def_property_readonly("device", &LaunchEvent::device)
+        .def("wait", &LaunchEvent::wait, py::arg("stream"))
+        .def("record", &LaunchEvent::record, py::arg("stream"))
         .def("query", &LaunchEvent::query)
         .def("synchronize", &LaunchEvent::synchronize);
     py::class_<NativeBuffer>(m, "Buffer")

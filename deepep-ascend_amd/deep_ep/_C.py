@@ -311,12 +311,51 @@ class EventHandle:
         _current_stream().wait_event(self.event)
 
 
+class _LaunchEvent(torch.cuda.Event):
+    """The `torch.cuda.Event` of an event that the library recorded: everything that refers to the event goes to that one
+    (the base class keeps none of its own; its rest, timing and sharing between processes, needs flags that the events of
+    these calls never had)."""
+
+    def __new__(cls, native):
+        return super().__new__(cls)
+
+    def __init__(self, native):
+        self._event = native
+
+    @property
+    def cuda_event(self) -> int:
+        return self._event.handle
+
+    @property
+    def device(self) -> torch.device:
+        return torch.device('cuda', self._event.device)
+
+    def record(self, stream=None) -> None:
+        self._event.record((_current_stream() if stream is None else stream).cuda_stream)
+
+    def wait(self, stream=None) -> None:
+        self._event.wait((_current_stream() if stream is None else stream).cuda_stream)
+
+    def query(self) -> bool:
+        return self._event.query()
+
+    def synchronize(self) -> None:
+        self._event.synchronize()
+
+
 class _LaunchEventHandle(EventHandle):
     """An event that the library recorded behind the launches of a deferred call."""
 
-    def __init__(self, event):
-        self.event = event
-        self.current_stream_wait = event.current_stream_wait
+    def __init__(self, native):
+        self._event = native
+        self.current_stream_wait = native.current_stream_wait
+
+    def __getattr__(self, name):
+        # (made for those who ask: most wait through the handle)
+        if name != 'event':
+            raise AttributeError(name)
+        self.event = _LaunchEvent(self._event)
+        return self.event
 
 
 class Context:

@@ -851,3 +851,47 @@ def test_events_of_deferred_calls_order_other_streams(R, T, H, E, K, A):
     side.wait_event(ev.event.event)
     for b in bufs:
         b.destroy()
+
+
+@pytest.mark.parametrize('R', [1, 2])
+def test_event_of_a_deferred_call_is_a_torch_event(R):
+    """`EventHandle.event` of a deferred call serves whoever takes a `torch.cuda.Event`: by type, by its handle in another
+    library, and recorded again."""
+    import ctypes
+    import deep_ep
+    T, H, E, K = 32, 256, 8, 2
+    bufs = [deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K,
+                             explicitly_destroy=True)] if R == 1 else make_node(R, T, H, K, False)
+    x = make_tokens(T, H).to(DEV)
+    topk, w = make_routing(T, E, K)
+    sent = [b.dispatch(x, topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E, num_max_tokens_per_rank=T, do_expand=True,
+                       do_cpu_sync=False, async_with_compute_stream=True, defer_epilogue=True) for b in bufs]
+    got = [e.current_stream_wait() for e in sent]
+    reduced = [b.combine(rows, h, topk_weights=rw, async_with_compute_stream=True, defer_epilogue=True)
+               for b, (rows, _, rw, h) in zip(bufs, got)]
+    hip = ctypes.CDLL('libamdhip64.so')
+    side = torch.cuda.Stream()
+    for overlap in sent + reduced:
+        handle, event = overlap.event, overlap.event.event
+        assert isinstance(event, torch.cuda.Event) and handle.event is event
+        event.synchronize()
+        assert event.query() and event.device == x.device
+        assert hip.hipEventQuery(ctypes.c_void_p(event.cuda_event)) == 0
+        assert hex(event.cuda_event) in repr(event)
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(20_000_000)
+            event.record()
+        assert not event.query()
+        handle.current_stream_wait()             # behind what it is recorded behind now
+        here = torch.cuda.current_stream().record_event()
+        assert not here.query()
+        here.synchronize()
+        assert event.query()
+        assert side.record_event(event) is event
+        event.wait(side)
+        event.wait()
+    for overlap in reduced:
+        overlap.current_stream_wait()
+    torch.cuda.synchronize()
+    for b in bufs:
+        b.destroy()
