@@ -223,13 +223,13 @@ void load_kernels(const char* dir) {
 
 // The event that a call leaves behind its launches.  Recorded by itself it is a packet of its own in the queue, with fences
 // (2.7 us of the GPU behind a kernel that writes 16 MiB); as the stop event of the call's last kernel it is that kernel's
-// completion signal and costs nothing there.  Under capture, where the call launches nothing, or where it stores into arenas given
-// by address (another GPU's, for which the stores are released at system scope), it is recorded as usual.
+// completion signal and costs nothing there.  It rides where what the call stored is read by this process on this GPU: one
+// partition, or all of a node's in this process.  What a partition alone or with arenas given by address has stored is read from outside
+// (by a transport, by another GPU) behind the event: there, under capture, and where the call launches nothing, it is recorded.
 // A pass of eight partitions, two deferred calls each: of 2048 tokens 1290 -> 1249 us; of 64 (bound by the host) a tenth less.
 class DoneEvent {
 public:
-    DoneEvent(void* event, void* stream, bool foreign_arenas)
-        : event_((hipEvent_t)event), stream_((hipStream_t)stream), rides_(not foreign_arenas) {}
+    DoneEvent(void* event, void* stream, const ep_buffer* b);
     // for the last launch of the call: the event to ride on it, or none
     hipEvent_t take(uint64_t threads) {
         if (event_ == nullptr or not rides_ or threads > UINT32_MAX) return nullptr;      // (that launch takes threads, not workgroups)
@@ -338,6 +338,9 @@ struct ep_buffer {
     char* buffer() const { return arena + workspace_bytes; }
     char* lb() const { return arena + workspace_bytes + num_buffer_bytes; }
 };
+
+DoneEvent::DoneEvent(void* event, void* stream, const ep_buffer* b)
+    : event_((hipEvent_t)event), stream_((hipStream_t)stream), rides_(b->num_ranks == 1 or not b->peers.empty()) {}
 
 namespace {
 // LDS of the layout kernels: histograms / per-wave counters, the staged keys, the per-source row counts
@@ -783,7 +786,7 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
         EP_HOST_ASSERT(pa != nullptr);
         check_buffer(b);
         const ep_dispatch_args_t& a = *pa;
-        DoneEvent done(event, a.stream, b->connected and b->peers.empty());
+        DoneEvent done(event, a.stream, b);
         const bool cached_mode = a.cached_mode != 0;
         const bool do_cpu_sync = a.do_cpu_sync != 0;
         EP_HOST_ASSERT(not b->is_static or (not cached_mode and not do_cpu_sync and b->num_ranks == 1));
@@ -1461,7 +1464,7 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
         EP_HOST_ASSERT(pa != nullptr);
         check_buffer(b);
         const ep_combine_args_t& a = *pa;
-        DoneEvent done(event, a.stream, b->connected and b->peers.empty());
+        DoneEvent done(event, a.stream, b);
         const int R = b->num_ranks;
         EP_HOST_ASSERT(a.num_experts > 0 and a.num_experts % R == 0);
 

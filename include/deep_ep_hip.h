@@ -148,7 +148,9 @@ typedef struct ep_dispatch_args {
  * and ep_dispatch_recv_launch writes the other handle tensors. */
 int ep_dispatch_launch(ep_buffer_t* buf, const ep_dispatch_args_t* args);
 /* The same, with an event (a hipEvent_t of the device, made by the caller) that is recorded behind everything the call has
- * enqueued on its stream, as a hipEventRecord right after it would, but where that is possible as part of the last launch. */
+ * enqueued on its stream.  With one partition, or all partitions of the node in this process (ep_buffer_connect), it may be
+ * part of the last launch (complete when that kernel is: whoever waits for it on this GPU finds what the call has stored);
+ * otherwise, and under capture, it is a hipEventRecord right after the call's launches. */
 int ep_dispatch_launch_event(ep_buffer_t* buf, const ep_dispatch_args_t* args, void* event);
 /* The same for a caller whose next call on this buffer is this dispatch's ep_dispatch_epilogue_launch: the library may
  * then leave the layout to the copy launch (one partition, at most 4096 tokens and 16384 (token, slot) entries:

@@ -270,3 +270,41 @@ def test_calibration_rig_is_a_library_of_its_own(de):
     for k in (b'ep_calib_fill', b'ep_calib_fronts', b'ep_calib_mixed', b'ep_calib_scatter_stores_only', b'ep_calib_read_rows',
               b'ep_calib_ordered_steered', b'ep_calib_copy_ordered_flat', b'gfx950'):
         assert k in cblob, k
+
+
+@pytest.fixture(scope='module')
+def host_calls(de, tmp_path_factory):
+    """Runs `tests/host_calls.c`: what the library launches, without a GPU."""
+    import subprocess
+    from deep_ep import _build
+    exe = tmp_path_factory.mktemp('host_calls') / 'host_calls'
+    lib = os.path.dirname(LIB)
+    subprocess.run(['gcc', *_build.C_CLIENT_FLAGS, '-o', str(exe), os.path.join(ROOT, 'tests', 'host_calls.c'), f'-L{lib}', '-ldeep_ep_hip',
+                    f'-Wl,-rpath,{lib}', f'-Wl,-rpath,{_build.ROCM}/lib', f'-Wl,-rpath-link,{_build.ROCM}/lib'], check=True)
+
+    def run(*args):
+        r = subprocess.run([str(exe), *map(str, args)], capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0, r.stdout + r.stderr
+        assert 'refused' not in r.stdout or args[0] != 'event', r.stdout
+        return r.stdout.splitlines()
+    return run
+
+
+@pytest.mark.parametrize('form,rides', [('node', True), ('alone', False), ('mapped', False)])
+@pytest.mark.parametrize('tokens', [40, 700, 3000])
+def test_event_rides_only_where_this_process_reads_what_the_call_stored(host_calls, form, rides, tokens):
+    """The event behind a deferred call is part of its last launch where the partitions live in this process.  A partition
+    whose packed rows and partials somebody else takes (one alone, whose rows a transport ships; arenas given by address)
+    gets an event of its own behind the launch, and so does a call under capture."""
+    lines = host_calls('event', tokens, 2, form)
+    at = lines.index('combine')
+    count = 2 if form == 'node' else 1
+    for phase, kernel in ((lines[:at], '_pack'), (lines[at:], 'ep_combine_partial_k4')):
+        last = [line for line in phase if kernel in line]
+        assert len(last) == count, lines
+        assert all(line.endswith('on 1 + event') == rides for line in last), lines
+        assert phase.count('event on 1') == (0 if rides else count), lines
+        if not rides:
+            assert phase.index('event on 1') == phase.index(last[0]) + 1, lines
+    captured = host_calls('event', tokens, 2, form, 'capture')
+    assert not any('+ event' in line for line in captured) and captured.count('event on 1') == 2 * count
