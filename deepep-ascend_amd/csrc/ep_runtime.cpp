@@ -781,7 +781,12 @@ int ep_buffer_print_memory_usage(ep_buffer_t* b) {
 }
 
 // ---- dispatch ---------------------------------------------------------------------------------
-static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool epilogue_follows, void* event = nullptr) {
+// What the caller says of the copy epilogue: nothing (the layout is enqueued at once), that it is the next call (a decode-size layout
+// is left to it), or that it is the only one, of the same experts and alignment, with no wait for counts in front (every
+// layout that a copy launch can make is).
+enum class Epilogue { any, next, only };
+
+static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, Epilogue epilogue, void* event = nullptr) {
     return guarded([&] {
         EP_HOST_ASSERT(pa != nullptr);
         check_buffer(b);
@@ -1013,11 +1018,11 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
         la.cumulative_stats = (int*)a.cumulative_local_expert_recv_stats.data;
         la.host_page = b->host_page_dev;
 
-        const bool one_launch = small_dispatch(num_tokens, K) or chunk_dispatch(num_tokens, K, E, R);
+        const bool small = small_dispatch(num_tokens, K), one_launch = small or chunk_dispatch(num_tokens, K, E, R);
         b->last.layout_pending = b->last.place_pending = b->last.copied = false;
         if (one_launch and num_ranks > 1) {
             own_layout = &la;
-        } else if (one_launch and epilogue_follows) {
+        } else if ((small and epilogue == Epilogue::next) or (one_launch and epilogue == Epilogue::only)) {
             b->last.layout_pending = true;
             b->last.pending = la;
         } else {
@@ -1047,9 +1052,10 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, bool ep
     });
 }
 
-int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) { return dispatch_launch(b, pa, false); }
-int ep_dispatch_launch_event(ep_buffer_t* b, const ep_dispatch_args_t* pa, void* event) { return dispatch_launch(b, pa, false, event); }
-int ep_dispatch_begin(ep_buffer_t* b, const ep_dispatch_args_t* pa) { return dispatch_launch(b, pa, true); }
+int ep_dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa) { return dispatch_launch(b, pa, Epilogue::any); }
+int ep_dispatch_launch_event(ep_buffer_t* b, const ep_dispatch_args_t* pa, void* event) { return dispatch_launch(b, pa, Epilogue::any, event); }
+int ep_dispatch_begin(ep_buffer_t* b, const ep_dispatch_args_t* pa) { return dispatch_launch(b, pa, Epilogue::next); }
+int ep_dispatch_begin_only(ep_buffer_t* b, const ep_dispatch_args_t* pa) { return dispatch_launch(b, pa, Epilogue::only); }
 
 int64_t ep_dispatch_stamp(ep_buffer_t* b) {
     return (b == nullptr || b->destroyed || !b->last.valid) ? 0 : b->last.stamp;
@@ -1676,7 +1682,7 @@ extern "C" int ep_dispatch_static_launch(const ep_dispatch_args_t* d, const ep_d
     rc = guarded([&] { v = static_view_of_current_device(); });
     if (rc != 0) return rc;
     // (an epilogue that pads for other experts or another alignment than the layout's comes behind a layout of its own)
-    rc = dispatch_launch(v, d, d->num_experts == e->num_experts and d->expert_alignment == e->expert_alignment);
+    rc = dispatch_launch(v, d, d->num_experts == e->num_experts and d->expert_alignment == e->expert_alignment ? Epilogue::only : Epilogue::any);
     if (rc != 0) return rc;
     ep_dispatch_epilogue_args_t ee = *e;
     ee.dispatch_stamp = v->last.stamp;

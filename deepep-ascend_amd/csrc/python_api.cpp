@@ -439,7 +439,7 @@ public:
         std::unique_ptr<LaunchEvent> event;
         if (defer_epilogue && async_with_compute_stream) event = std::make_unique<LaunchEvent>();
         check(event != nullptr ? ep_dispatch_launch_event(buf_, &a, event->get())
-                               : copy_follows ? ep_dispatch_begin(buf_, &a) : ep_dispatch_launch(buf_, &a));
+                               : copy_follows ? ep_dispatch_begin_only(buf_, &a) : ep_dispatch_launch(buf_, &a));
         // the epilogue below belongs to this launch: the library refuses it once a later dispatch has taken over
         // the buffer's workspace
         s.stamp = ep_dispatch_stamp(buf_);

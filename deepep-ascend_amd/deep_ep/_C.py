@@ -105,6 +105,7 @@ _ep_region = _sig('ep_buffer_region', ctypes.c_void_p, ctypes.c_void_p, ctypes.c
 _ep_print_mem = _sig('ep_buffer_print_memory_usage', ctypes.c_int, ctypes.c_void_p)
 _ep_dispatch = _sig('ep_dispatch_launch', ctypes.c_int, ctypes.c_void_p, ctypes.POINTER(_DispatchArgs))
 _ep_dispatch_begin = _sig('ep_dispatch_begin', ctypes.c_int, ctypes.c_void_p, ctypes.POINTER(_DispatchArgs))
+_ep_dispatch_begin_only = _sig('ep_dispatch_begin_only', ctypes.c_int, ctypes.c_void_p, ctypes.POINTER(_DispatchArgs))
 _ep_wait = _sig('ep_dispatch_wait_counts', ctypes.c_int, ctypes.c_void_p, _c_int_p, _c_int_p, _c_int_p)
 _ep_worst = _sig('ep_dispatch_worst_case_sizes', ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_int,
                  ctypes.c_int, ctypes.c_int, _c_int_p, _c_int_p)

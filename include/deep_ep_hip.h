@@ -153,12 +153,17 @@ int ep_dispatch_launch(ep_buffer_t* buf, const ep_dispatch_args_t* args);
  * otherwise, and under capture, it is a hipEventRecord right after the call's launches. */
 int ep_dispatch_launch_event(ep_buffer_t* buf, const ep_dispatch_args_t* args, void* event);
 /* The same for a caller whose next call on this buffer is this dispatch's ep_dispatch_epilogue_launch: the library may
- * then leave the layout to the copy launch (one partition, at most 4096 tokens and 16384 (token, slot) entries:
- * one launch instead of two or three).  Everything this call would have enqueued is then enqueued by the epilogue, on the epilogue's
+ * then leave the layout to the copy launch (one partition, at most 128 tokens and 1024 (token, slot) entries: one
+ * launch instead of two).  Everything this call would have enqueued is then enqueued by the epilogue, on the epilogue's
  * stream: the handle tensors, the running statistics and the host counts are complete behind the epilogue only, and the
- * inputs have to stay until then.  An epilogue on another stream is ordered behind what the begin is ordered behind by
+ * inputs and handle tensors have to stay until then; ep_dispatch_wait_counts in between, a second epilogue and one of other
+ * experts or another alignment are refused.  An epilogue on another stream is ordered behind what the begin is ordered behind by
  * the caller, as after ep_dispatch_launch (an event recorded after the begin, waited for on the other stream). */
 int ep_dispatch_begin(ep_buffer_t* buf, const ep_dispatch_args_t* args);
+/* The same for a caller who keeps to those rules at every size: exactly one epilogue, of the same experts and alignment, and no
+ * wait for the counts before it.  The layout may then be left to the copy launch up to 4096 tokens and 16384 entries (one launch
+ * instead of two or three), with what is said above about streams, inputs and refusals. */
+int ep_dispatch_begin_only(ep_buffer_t* buf, const ep_dispatch_args_t* args);
 
 typedef struct ep_dispatch_recv_args {
     /* handle tensors, written here (csrc/buffers/ep.hpp:205-246) */

@@ -148,6 +148,16 @@ static void event_behind_calls(int T, int R, const char* form) {
     for (int i = 0; i < n; ++i) said("combine", ep_combine_begin_event(b[i], &c, (void*)7));
 }
 
+/* begin T next|only: a dispatch of one partition on stream 1 and its copy epilogue on stream 2 */
+static void begin_and_epilogue(int T, const char* form) {
+    ep_buffer_t* b;
+    said("create", ep_buffer_create(0, 1, ep_calculate_buffer_size(1, T, H, K, 0), 0, 1, 1, &b));
+    ep_dispatch_args_t a = dispatch_args(T, 1);
+    said("begin", strcmp(form, "only") == 0 ? ep_dispatch_begin_only(b, &a) : ep_dispatch_begin(b, &a));
+    ep_dispatch_epilogue_args_t e = epilogue_args(T, 1, b);
+    said("epilogue", ep_dispatch_epilogue_launch(b, &e));
+}
+
 int main(int argc, char** argv) {
     const int T = argc > 2 ? atoi(argv[2]) : 0, R = argc > 3 ? atoi(argv[3]) : 1;
     if (ep_init(NULL) != 0) {
@@ -156,6 +166,7 @@ int main(int argc, char** argv) {
     }
     capturing = argc > 5;
     if (argc > 4 && strcmp(argv[1], "event") == 0) event_behind_calls(T, R, argv[4]);
+    if (argc > 3 && strcmp(argv[1], "begin") == 0) begin_and_epilogue(T, argv[3]);
     fflush(stdout);
     return 0;
 }

@@ -168,9 +168,10 @@ class AbiDispatch:
         self.e.num_topk, self.e.do_zero_padding = K, 1
         torch.cuda.synchronize()
 
-    def begin(self, stream):
+    def begin(self, stream, call='begin'):
         self.a.stream = stream.cuda_stream
-        self.C._check(self.C._ep_dispatch_begin(self.buf.runtime._h, ctypes.byref(self.a)))
+        begin = {'begin': self.C._ep_dispatch_begin, 'begin_only': self.C._ep_dispatch_begin_only}[call]
+        self.C._check(begin(self.buf.runtime._h, ctypes.byref(self.a)))
         self.e.dispatch_stamp = self.C._ep_stamp(self.buf.runtime._h)
 
     def epilogue(self, stream):
@@ -189,12 +190,16 @@ class AbiDispatch:
         assert np.array_equal(self.gates.cpu().numpy().view(np.uint32)[:ne], ew.view(np.uint32))
 
 
-def test_begin_and_epilogue_on_two_streams():
+BEGINS = [(96, 'begin'), (64, 'begin_only'), (700, 'begin_only'), (4096, 'begin_only')]       # the last two in a launch of chunk size
+
+
+@pytest.mark.parametrize('T,call', BEGINS)
+def test_begin_and_epilogue_on_two_streams(T, call):
     """The epilogue of an ep_dispatch_begin on another stream, ordered behind the begin by an event only: the ids arrive
     late on the first stream, and every pass routes differently, so that a layout of the pass before would show."""
     import deep_ep
     C = deep_ep._C
-    T, H, E, K, A = 96, 256, 16, 4, 8
+    H, E, K, A = 256, 16, 4, 8
     buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
     x = make_tokens(T, H, seed=4)
     first, second = torch.cuda.Stream(), torch.cuda.Stream()
@@ -206,7 +211,7 @@ def test_begin_and_epilogue_on_two_streams():
             for _ in range(4):
                 junk = torch.randn((1024, 1024), device=DEV) @ torch.randn((1024, 1024), device=DEV)
             late.copy_(source)
-        d.begin(first)
+        d.begin(first, call)
         second.wait_event(first.record_event())
         d.epilogue(second)
         torch.cuda.synchronize()
@@ -215,21 +220,22 @@ def test_begin_and_epilogue_on_two_streams():
     buf.destroy()
 
 
-def test_cached_epilogue_between_begin_and_its_epilogue():
+@pytest.mark.parametrize('T,call', BEGINS)
+def test_cached_epilogue_between_begin_and_its_epilogue(T, call):
     """A replay of another handle between the two calls leaves the waiting layout where it is."""
     import deep_ep
     C = deep_ep._C
-    T, H, E, K, A = 96, 256, 16, 4, 8
+    H, E, K, A = 256, 16, 4, 8
     buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
     x = make_tokens(T, H, seed=6)
     stream = torch.cuda.current_stream()
     old_topk, old_w = make_routing(T, E, K, seed=40)
     old = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), old_topk.to(DEV), old_w.to(DEV))
-    old.begin(stream)
+    old.begin(stream, call)
     old.epilogue(stream)
     topk, w = make_routing(T, E, K, seed=41, masked=0.2)
     d = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), topk.to(DEV), w.to(DEV))
-    d.begin(stream)
+    d.begin(stream, call)
     old.rows.zero_()
     old.e.cached_mode = 1
     old.epilogue(stream)
@@ -242,19 +248,62 @@ def test_cached_epilogue_between_begin_and_its_epilogue():
     buf.destroy()
 
 
-@pytest.mark.parametrize('field,value', [('experts', 64), ('experts', 8), ('alignment', 16)])
-def test_epilogue_of_other_experts_or_alignment_is_refused(field, value):
-    """The one launch counts in LDS sized by the begin's experts: an epilogue that names others is refused on the host,
-    and the right one still runs."""
+@pytest.mark.parametrize('T', [129, 700, 2049])
+def test_begin_beyond_decode_size_enqueues_its_layout(T):
+    """What an ep_dispatch_begin of more than 128 tokens serves: the ids may change behind it on its stream, the counts can be
+    waited for before the epilogue, and epilogues may come again, padded otherwise too."""
     import deep_ep
     C = deep_ep._C
-    T, H, E, K, A = 64, 128, 16, 4, 8
+    H, E, K, A = 128, 16, 4, 8
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    x = make_tokens(T, H, seed=9)
+    topk, w = make_routing(T, E, K, seed=44, masked=0.2)
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
+    ids = topk.to(DEV)
+    d = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), ids, w.to(DEV))
+    d.a.do_cpu_sync = 1
+    stream = torch.cuda.current_stream()
+    d.begin(stream)
+    ids.fill_(-1)
+    n, ne, per_expert = ctypes.c_int(), ctypes.c_int(), (ctypes.c_int * E)()
+    C._check(C._ep_wait(buf.runtime._h, ctypes.byref(n), ctypes.byref(ne), per_expert))
+    assert (n.value, ne.value) == (lay['num_recv_tokens'], lay['num_expanded_tokens'])
+    assert list(per_expert) == lay['num_recv_tokens_per_expert_list']
+    d.epilogue(stream)
+    torch.cuda.synchronize()
+    d.check(x, topk, w, E, A)
+    d.rows.view(torch.int16).fill_(77)
+    d.e.expert_alignment = 1
+    d.epilogue(stream)
+    torch.cuda.synchronize()
+    slots = lay['recv_src_metadata'][:, :K]
+    real = np.zeros(ne.value, dtype=bool)
+    real[slots[slots >= 0]] = True
+    rows, ex = bf16_bits(d.rows)[:ne.value], O.rank_share_dispatch(bf16_bits(x), None, w.numpy(), lay)[0]
+    assert np.array_equal(rows[real], ex[real]) and (rows[~real].view(np.int16) == 77).all() and not real.all()
+    d.e.expert_alignment = A
+    d.epilogue(stream)
+    torch.cuda.synchronize()
+    d.check(x, topk, w, E, A)
+    buf.destroy()
+
+
+@pytest.mark.parametrize('T,call', BEGINS)
+@pytest.mark.parametrize('field,value', [('experts', 64), ('experts', 8), ('alignment', 16)])
+def test_epilogue_of_other_experts_or_alignment_is_refused(field, value, T, call):
+    """The one launch counts in LDS sized by the begin's experts: an epilogue that names others is refused on the host,
+    and the right one still runs; so is a wait for the counts in between."""
+    import deep_ep
+    C = deep_ep._C
+    H, E, K, A = 128, 16, 4, 8
     buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
     x = make_tokens(T, H, seed=7)
     topk, w = make_routing(T, E, K, seed=42, masked=0.2)
     d = AbiDispatch(C, buf, T, H, E, K, A, x.to(DEV), topk.to(DEV), w.to(DEV))
     stream = torch.cuda.current_stream()
-    d.begin(stream)
+    d.begin(stream, call)
+    with pytest.raises(C.EPException, match='comes before the counts'):
+        C._check(C._ep_wait(buf.runtime._h, None, None, None))
     if field == 'experts':
         other = torch.zeros(value, dtype=torch.int32, device=DEV)
         d.e.num_experts, d.e.psum_num_recv_tokens_per_expert = value, C._desc(other)

@@ -308,3 +308,16 @@ def test_event_rides_only_where_this_process_reads_what_the_call_stored(host_cal
             assert phase.index('event on 1') == phase.index(last[0]) + 1, lines
     captured = host_calls('event', tokens, 2, form, 'capture')
     assert not any('+ event' in line for line in captured) and captured.count('event on 1') == 2 * count
+
+
+def test_which_begins_leave_the_layout_to_the_copy_launch(host_calls):
+    """ep_dispatch_begin up to 128 tokens, ep_dispatch_begin_only up to 4096; beyond, the layout is on the begin's stream."""
+    for form in ('next', 'only'):
+        for tokens in (1, 128, 129, 700, 4096, 4097):
+            launches = [line for line in host_calls('begin', tokens, form) if line.startswith('ep_')]
+            kind = 'small' if tokens <= 128 else 'chunk' if form == 'only' and tokens <= 4096 else None
+            if kind is not None:
+                assert launches == [f'ep_dispatch_{kind}_copy on 2'], (form, tokens, launches)
+            else:
+                assert launches[-1] == 'ep_scatter_copy on 2' and len(launches) >= 2, (form, tokens, launches)
+                assert all(line.startswith('ep_layout_') and line.endswith(' on 1') for line in launches[:-1]), (form, tokens, launches)
