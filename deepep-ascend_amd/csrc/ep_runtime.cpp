@@ -679,7 +679,9 @@ int ep_buffer_create(int rank_idx, int num_ranks, int64_t num_bytes, int64_t num
             HIP_CHECK(hipMalloc((void**)&b->arena, (size_t)total));
             HIP_CHECK(hipMemset(b->arena, 0, (size_t)total));
             const size_t page_bytes = (EP_HOST_PAGE_INTS + (num_ranks > 1 ? 2 * EP_HOST_BOX_INTS : 0)) * sizeof(int);
-            HIP_CHECK(hipHostMalloc((void**)&b->host_page, page_bytes, hipHostMallocMapped));
+            // (coherent: the kernels' stores to it are announced by one more store behind them, with no release of a cache in front.
+            //  That is the runtime's default too, unless its environment says otherwise)
+            HIP_CHECK(hipHostMalloc((void**)&b->host_page, page_bytes, hipHostMallocMapped | hipHostMallocCoherent));
             memset(b->host_page, 0, page_bytes);
             HIP_CHECK(hipHostGetDevicePointer((void**)&b->host_page_dev, b->host_page, 0));
             write_peer_table(b, std::vector<char*>(num_ranks, b->arena));    // not connected: every peer is this arena

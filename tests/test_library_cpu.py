@@ -321,3 +321,9 @@ def test_which_begins_leave_the_layout_to_the_copy_launch(host_calls):
             else:
                 assert launches[-1] == 'ep_scatter_copy on 2' and len(launches) >= 2, (form, tokens, launches)
                 assert all(line.startswith('ep_layout_') and line.endswith(' on 1') for line in launches[:-1]), (form, tokens, launches)
+
+
+def test_count_pages_are_coherent_memory(host_calls):
+    """The kernels announce counts with plain stores to the pinned page: it has to be asked for as fine-grained memory."""
+    pages = [line for line in host_calls('event', 40, 2, 'node') if line.startswith('pinned')]
+    assert pages == ['pinned mapped coherent'] * 2
