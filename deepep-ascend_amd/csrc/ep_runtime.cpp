@@ -447,9 +447,19 @@ unsigned chunk_lds(int num_tokens, int K, int E, int R) {
 // Several partitions, all of a partition's dispatch: two of 2048 tokens x 2048 top-8 44.0 / 41.3, four of 1500 x 7168 top-8 94.3 / 86.4, 32 of 1024 top-6
 // 54.8 / 48.0; beyond, four of 4096 top-4 89.3 / 90.2, two of 4096 x 2048 top-2 38.7 / 38.7 (a word a token is kept in LDS).
 // (a partition is a bit of that word)
-bool chunk_dispatch(int num_tokens, int K, int E, int R) {
-    return num_tokens > 0 and num_tokens <= (R > 1 ? EP_CHUNK_TOKENS / 2 : EP_CHUNK_TOKENS) and num_tokens * K <= EP_CHUNK_ENTRIES and R <= 32 and
-           chunk_lds(num_tokens, K, E, R) <= 64 * 1024;
+// Wide rows of many tokens are a copy long enough for its fixed shares a workgroup to cost more than the launch saved, most with hot
+// experts.  Mean of BF16 and FP8, alignment 1, 16 and 128, uniform and Zipf (1.2) routing, two launches / one: 7168 channels, 2700 top-6
+// 73.5 / 72.7, 2900 top-5 70.8 / 70.5, 3200 top-5 73.8 / 74.8, 3800 top-4 73.0 / 74.5, 4096 top-3 68.9 / 70.0, top-4 75.4 / 77.6 (Zipf, alignment
+// 16, FP8 51.2 / 55.3), but 4096 top-2 56.7 / 53.1; 10240, 2400 top-6 91.5 / 92.0, 2700 96.5 / 99.6; 16384, 2048 top-6 112.5 / 108.4, 2700 134.0 /
+// 136.1.  5120 channels are level at 4096 top-4 (59.1 / 59.5), 4096 gain (51.1 / 50.5).
+bool chunk_dispatch(int num_tokens, int K, int E, int R, int num_parts) {
+    if (num_tokens <= 0 or num_tokens > (R > 1 ? EP_CHUNK_TOKENS / 2 : EP_CHUNK_TOKENS) or num_tokens * K > EP_CHUNK_ENTRIES or R > 32) return false;
+    const bool long_copy = num_parts >= 12 and num_tokens > (num_parts <= 16 ? 3072 : 2560) and num_tokens * K > 12000;
+    return not long_copy and chunk_lds(num_tokens, K, E, R) <= 64 * 1024;
+}
+// (token, part) tasks a row of a dispatch falls into: 512 channels of a row being quantised, 1 KiB of any other
+int row_parts(int64_t hidden, int64_t row_bytes, bool quantise) {
+    return (int)std::max<int64_t>(1, quantise ? ceil_div(hidden, 512) : ceil_div(row_bytes, 1024));
 }
 // Workgroups: no more than one task a wave needs.  Two a CU keep twice the rows on the way, one a CU counts the ids half as
 // often (us at 256 / 512 workgroups): 1024 x 7168 BF16 top-8 31.7 / 30.4, eight partitions of 1024 68.9 / 66.9; 2048 x 7168 top-8
@@ -932,7 +942,7 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, Epilogu
             sa.slot_map = rank_map;
             sa.rank_box_off = boxes.used ? boxes.rank_off : 0;
             sa.vecs_per_lane = 1;
-            sa.num_parts = (int)std::max<int64_t>(1, a.fused_fp8_quant ? ceil_div(hidden, 512) : ceil_div(sa.copy_bytes, 1024));
+            sa.num_parts = row_parts(hidden, sa.copy_bytes, a.fused_fp8_quant != 0);
             sa.num_row_blocks = (int)ceil_div((int64_t)num_tokens * sa.num_parts, EP_ROWS_PER_BLOCK);
             if (sa.num_row_blocks == 0) return;
             if (own_layout != nullptr) {
@@ -1020,7 +1030,8 @@ static int dispatch_launch(ep_buffer_t* b, const ep_dispatch_args_t* pa, Epilogu
         la.cumulative_stats = (int*)a.cumulative_local_expert_recv_stats.data;
         la.host_page = b->host_page_dev;
 
-        const bool small = small_dispatch(num_tokens, K), one_launch = small or chunk_dispatch(num_tokens, K, E, R);
+        const bool small = small_dispatch(num_tokens, K);
+        const bool one_launch = small or chunk_dispatch(num_tokens, K, E, R, row_parts(hidden, (int64_t)hidden * x_elem, a.fused_fp8_quant != 0));
         b->last.layout_pending = b->last.place_pending = b->last.copied = false;
         if (one_launch and num_ranks > 1) {
             own_layout = &la;
@@ -1394,8 +1405,7 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
         // a wave task covers 1 KiB of a verbatim row (4 KiB of a packed row, which mostly has one destination
         // among this partition's few experts), or 512 channels of a row being quantised
         sa.vecs_per_lane = sa.mode == EP_SCATTER_REGION ? 4 : 1;
-        sa.num_parts = (int)std::max<int64_t>(
-            1, quantise_here ? ceil_div(hidden, 512) : ceil_div(sa.copy_bytes, 1024 * sa.vecs_per_lane));
+        sa.num_parts = row_parts(hidden, ceil_div(sa.copy_bytes, sa.vecs_per_lane), quantise_here);
         const int64_t row_blocks = ceil_div((int64_t)sa.num_rows_bound * sa.num_parts, EP_ROWS_PER_BLOCK);
         EP_HOST_ASSERT(row_blocks <= INT32_MAX / 2);
         sa.num_row_blocks = (int)row_blocks;

@@ -69,7 +69,8 @@ static void said(const char* what, int rc) {
     if (rc != 0) printf("%s refused: %s\n", what, ep_last_error());
 }
 
-enum { K = 4, E = 32, H = 256, A = 8 };
+enum { K = 4, E = 32, A = 8 };
+static int64_t H = 256;
 
 static ep_dispatch_args_t dispatch_args(int T, int R) {
     ep_dispatch_args_t a;
@@ -148,7 +149,7 @@ static void event_behind_calls(int T, int R, const char* form) {
     for (int i = 0; i < n; ++i) said("combine", ep_combine_begin_event(b[i], &c, (void*)7));
 }
 
-/* begin T next|only: a dispatch of one partition on stream 1 and its copy epilogue on stream 2 */
+/* begin T next|only [H]: a dispatch of one partition on stream 1 and its copy epilogue on stream 2 */
 static void begin_and_epilogue(int T, const char* form) {
     ep_buffer_t* b;
     said("create", ep_buffer_create(0, 1, ep_calculate_buffer_size(1, T, H, K, 0), 0, 1, 1, &b));
@@ -164,8 +165,8 @@ int main(int argc, char** argv) {
         said("init", 1);
         return 1;
     }
-    capturing = argc > 5;
-    if (argc > 4 && strcmp(argv[1], "event") == 0) event_behind_calls(T, R, argv[4]);
+    if (argc > 4 && strcmp(argv[1], "event") == 0) capturing = argc > 5, event_behind_calls(T, R, argv[4]);
+    if (argc > 4 && strcmp(argv[1], "begin") == 0) H = atoi(argv[4]);
     if (argc > 3 && strcmp(argv[1], "begin") == 0) begin_and_epilogue(T, argv[3]);
     fflush(stdout);
     return 0;

@@ -323,6 +323,17 @@ def test_which_begins_leave_the_layout_to_the_copy_launch(host_calls):
                 assert all(line.startswith('ep_layout_') and line.endswith(' on 1') for line in launches[:-1]), (form, tokens, launches)
 
 
+@pytest.mark.parametrize('hidden,tokens', [(256, 4096), (5632, 4096), (6144, 3072), (7168, 3072), (8192, 3072), (8704, 2560), (10240, 2560), (10240, 2900)])
+def test_wide_rows_of_many_tokens_keep_the_launch_in_front(host_calls, hidden, tokens):
+    """Four entries a token: from 12 parts a row (6144 BF16 channels) on, beyond 3072 tokens, and with more than 16 parts beyond 2560,
+    where that is more than 12000 entries, the layout is not left to the copy launch."""
+    for t in (tokens, tokens + 1, 3001):
+        launches = [line for line in host_calls('begin', t, 'only', hidden) if line.startswith('ep_')]
+        parts = hidden // 512
+        narrow = t <= 4096 and (parts < 12 or t <= (3072 if parts <= 16 else 2560) or 4 * t <= 12000)
+        assert (launches == ['ep_dispatch_chunk_copy on 2']) == narrow, (hidden, t, launches)
+
+
 def test_count_pages_are_coherent_memory(host_calls):
     """The kernels announce counts with plain stores to the pinned page: it has to be asked for as fine-grained memory."""
     pages = [line for line in host_calls('event', 40, 2, 'node') if line.startswith('pinned')]
