@@ -108,8 +108,9 @@ __device__ __forceinline__ void host_stores_arrived() {
 
 // Reads one word of every 64 bytes of the kernel's arguments, all in one trip.  The compiler fetches arguments where they are
 // first used, in some kernels four or five times in a row along the way to the first store, and each first touch of a
-// cache line is a trip to memory.  Whole cases (us): a replayed decode of 32 tokens 18.0 -> 17.3, prefill of 4096 tokens top-8
-// 248.2 -> 246.0, of 32768 1206.2 -> 1199.9, a training step of 8192 268.9 -> 266.9.
+// cache line is a trip to memory.  Whole cases, three pairs of processes, without / with (us): prefill of 4096 tokens top-8 246.4 / 244.6, a
+// training step of 8192 269.1 / 267.2, prefill of 32768 1202.4 / 1201.5, a replayed decode of 32 17.5 / 17.5.  Not in the combine kernels of
+// several partitions, where it loses (eight partitions of 2048 tokens 1241.4 / 1247.8, with it in these kernels alone).
 template <typename Args>
 __device__ __forceinline__ void fetch_arguments() {
     typedef const unsigned __attribute__((address_space(4)))* words_t;
@@ -2495,11 +2496,11 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
 }
 
 #define EP_COMBINE_KERNELS(SUFFIX, MODE)                                                                                   \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_generic(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<0, MODE>(a); } \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k2(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<2, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k4(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<4, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k6(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<6, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k8(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<8, MODE>(a); }
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_generic(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<0, MODE>(a); } \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k2(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<2, MODE>(a); }     \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k4(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<4, MODE>(a); }     \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k6(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<6, MODE>(a); }     \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k8(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<8, MODE>(a); }
 
 EP_COMBINE_KERNELS(, EP_COMBINE_FUSED)
 EP_COMBINE_KERNELS(_partial, EP_COMBINE_PARTIAL)
