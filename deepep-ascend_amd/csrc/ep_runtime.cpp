@@ -419,7 +419,10 @@ unsigned small_pad_blocks(unsigned pieces, int num_tokens, int K, int num_expert
 // top-8 of 256, 1 token 10.4 / 6.0, 32 11.8 / 6.8, 96 12.9 / 9.9, 128 13.4 / 11.1; 128 tokens top-1 8.0 / 4.9, top-8 of 2048
 // 16.9 / 12.8, 16384 channels 15.6 / 14.9; top-16, 64 tokens 17.6 / 12.8; top-32, 32 tokens 27.9 / 20.1.  One of eight partitions
 // (FP8, top-8), 64 tokens 29.2 / 22.6, 128 30.6 / 25.4.  The line is one block of ids: a token's bit and its rank are kept for
-// that many.
+// that many.  The form beyond (ep_dispatch_chunk_*) at these sizes is slower nearly everywhere (us, that form / this one): whole passes of a
+// synchronised dispatch and a combine, 8 experts, 8 / 128 tokens 27.5 / 26.3, 27.6 / 26.7, 256 experts 28.9 / 27.8, 29.1 / 28.7; replayed passes of
+// eight partitions top-2, 8 / 64 / 128 tokens 84.3 / 72.3, 92.5 / 78.5, 94.4 / 80.7, top-8 100.9 / 95.2, 114.2 / 106.4, 119.9 / 120.9; of two, 128
+// tokens top-8 33.1 / 35.1.
 bool small_dispatch(int num_tokens, int K) {
     return num_tokens > 0 and num_tokens <= EP_TOKENS_PER_BLOCK and num_tokens * K <= EP_SMALL_ENTRIES;
 }
@@ -462,9 +465,13 @@ int row_parts(int64_t hidden, int64_t row_bytes, bool quantise) {
     return (int)std::max<int64_t>(1, quantise ? ceil_div(hidden, 512) : ceil_div(row_bytes, 1024));
 }
 // Workgroups: no more than one task a wave needs.  Two a CU keep twice the rows on the way, one a CU counts the ids half as
-// often (us at 256 / 512 workgroups): 1024 x 7168 BF16 top-8 31.7 / 30.4, eight partitions of 1024 68.9 / 66.9; 2048 x 7168 top-8
-// 53.0 / 60.3, eight partitions of 2048 FP8 top-6 65.6 / 67.6; rows of fewer parts, 2048 x 4096 top-4 26.8 / 28.5, 4096 x 1024 top-2 12.9 / 15.3.
-// Padding is shared by all workgroups: as many as there is padding for.
+// often (us at 256 / 512 workgroups): 14 parts a row, 1021 tokens top-8 35.6 / 34.5, 2048 top-4 39.9 / 38.1, but 2048 top-8 53.0 / 60.3 and eight
+// partitions of 2048 FP8 top-6 65.6 / 67.6; 10 parts, 1021 top-8 27.8 / 27.0; 8 parts, 2048 top-4 27.2 / 26.3, 1021 top-8 23.6 / 23.7, one of two
+// partitions, all of a pass, 1021 top-8 59.7 / 62.4; 9 parts, 2048 top-4 28.6 / 28.8, eight partitions of 500 top-8 198.0 / 208.6; 5 parts, 1021 top-6
+// 17.6 / 18.4; 2 parts, 4096 top-2 12.9 / 15.3.  (The publishing workgroup beside 512 costs nothing: with 511, 1021 x 7168 top-8 34.4 / 34.4.)
+// Padding is shared by all workgroups: as many as there is padding for.  (Two a CU for it alone: 2048 experts at alignment 128 2 % faster, 64
+// to 256 experts 0 to 15 % slower.  That much padding beside few tokens is the one case left where two launches were faster: 2048 experts, 2560
+// channels, 500 tokens top-4 124.8 / 138.2, 200 top-8 112.5 / 115.4, 1000 top-8 205.6 / 199.7; whether padding is zeroed is not known at the begin.)
 void launch_chunk(const EpLayoutArgs& la, const EpScatterArgs& sa, bool pack, bool quantise, unsigned pad_pieces, void* stream,
                   DoneEvent* done = nullptr) {
     EpSmallArgs args{};
@@ -499,7 +506,10 @@ unsigned layout_place_lds(int E, int R, int K) {
 // wave has lanes.  It saves a launch and its trips; each workgroup adds up the counts of all experts instead.  us of all phases of a
 // node (host included), two launches / one: 8 partitions of 64 tokens 409 / 401, of 2048 1378 / 1332; 32 of 16384 1243 / 1198
 // a partition; 16 of 2048 with 2048 experts 1438 / 1385; 2 partitions, 2048 experts, 512 channels: 2048 tokens top-8 155 / 153, 4096 top-2
-// 148 / 147, 8192 top-2 (3300 row blocks) 154 / 165, with 1024 experts 148 / 145.
+// 148 / 147, 8192 top-2 (3300 row blocks) 154 / 165, with 1024 experts 148 / 145.  Means over 512 to 7168 channels, top-2 and 8, replayed: two
+// partitions, 64 experts, 64 / 4096 / 16384 tokens 34.4 / 26.6, 146 / 136, 401 / 408; eight, 64 experts 124 / 89, 487 / 459, 742 / 720, 512 experts
+// 133 / 96, 497 / 478, 767 / 761, 1024 experts 144 / 106, 530 / 516, 807 / 828 (with a host sync, whose row blocks are those of rows that came, there too
+// 786 / 763).
 constexpr int kRecvCopyMaxRanks = 64;
 unsigned recv_copy_lds(int E, int R) { return (unsigned)(E + 2 * (E / R) + EP_ROW_THREADS / 64) * sizeof(int); }
 bool recv_copy_pays(int num_experts, int row_blocks) { return num_experts <= 1024 or row_blocks <= 2048; }
