@@ -1791,8 +1791,8 @@ EP_CHUNK_KERNEL(quant_sw_pack, true, false, true)
 // Receive side of a node whose send sides ship ranks, placing and copying in one launch: what ep_layout_place and the
 // copy kernel of received rows do, for at most 64 partitions.  Every workgroup adds the counts up itself: the row counts of
 // the sources in registers (a lane a source), the counts per source and expert in LDS; a wave then knows the slots of its
-// row's entries from their ids and shipped ranks.  The row's payload is fetched with its ids.  Workgroup 0 publishes, the next
-// ones copy, the last zero the padding.
+// row's entries from their ids and shipped ranks.  The row's payload is fetched with its ids.  Workgroup 0 writes the handle tensors (no
+// host waits for counts of this launch), the next ones copy, the last zero the padding.
 // Bound by two trips to memory (counts; ids, ranks and payload) and the launch at decode sizes, by the copy's traffic beyond.
 // Eight partitions of 2048 tokens, all phases 1372 -> 1325 us; of 64 tokens (bound by the host's calls) 409 -> 383 us.
 // ------------------------------------------------------------------------------------------------
@@ -1862,11 +1862,9 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_recv_copy(EpSmal
     const int incl = wave_inclusive_sum(aligned);
     if (lane == WAVE - 1) s_tmp[w] = incl;
     __syncthreads();
-    int run = incl - aligned, grand = 0;
-    for (int k = 0; k < NW; ++k) {
+    int run = incl - aligned;
+    for (int k = 0; k < NW; ++k)
         if (k < w) run += s_tmp[k];
-        grand += s_tmp[k];
-    }
     for (int e = e0; e < e1; ++e) {
         s_start[e] = run;
         run += align_up(s_cnt[e], A);
@@ -1879,20 +1877,8 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_recv_copy(EpSmal
             l.unaligned_expert[e] = c;
             l.psum_expert[e] = s_start[e] + c;
             if (l.cumulative_stats != nullptr) atomicAdd(&l.cumulative_stats[e], c);
-            if (l.notify_host) host_store(&l.host_page[EP_HOST_EXPERT_OFF + e], align_up(c, A));
         }
-        if (tid < R) {                                   // (the first wave: R <= 64)
-            l.psum_rank[tid] = upto;
-            if (l.notify_host) host_store(&l.host_page[EP_HOST_RANK_OFF + tid], mine);
-        }
-        if (l.notify_host) {
-            if (tid == 0) {
-                host_store(&l.host_page[1], num_rows);
-                host_store(&l.host_page[2], grand);
-            }
-            host_stores_arrived();
-            if (tid == 0) host_store(&l.host_page[0], l.seq);
-        }
+        if (tid < R) l.psum_rank[tid] = upto;            // (the first wave: R <= 64)
         return;
     }
     if (!copies) {

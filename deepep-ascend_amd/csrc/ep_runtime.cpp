@@ -1464,6 +1464,7 @@ int ep_dispatch_epilogue_launch(ep_buffer_t* b, const ep_dispatch_epilogue_args_
             args.l = b->last.pending;
             args.s = sa;
             args.num_pad_blocks = (int)pad_blocks;
+            EP_HOST_ASSERT(args.l.notify_host == 0);       // (that kernel announces nothing)
             launch(g_k.recv_copy, 1u + grid, EP_ROW_THREADS, recv_copy_lds(a.num_experts, R), a.stream, args);
             b->last.place_pending = false;
         } else if (grid > 0) {
