@@ -165,9 +165,11 @@ struct EpScatterArgs {
 struct EpSmallArgs {
     EpLayoutArgs l;               // what ep_layout_assign (ep_recv_copy: ep_layout_place) would have been given
     EpScatterArgs s;              // what the copy kernel would have been given
+    // ep_dispatch_small_*, ep_recv_copy
     int num_pad_blocks;           // workgroups behind the row workgroups, each zeroing every num_pad_blocks-th padding piece
-                                  //   (ep_dispatch_chunk_*: not 0 where there is padding to zero; every workgroup takes a share)
-    int tasks_per_block;          // ep_dispatch_chunk_*: (token, part) tasks of a workgroup
+    // ep_dispatch_chunk_*
+    int zero_padding;             // there is padding to zero: every copying workgroup takes a share
+    int tasks_per_block;          // (token, part) tasks of a workgroup
 };
 // ep_dispatch_chunk_*: workgroups of EP_CHUNK_THREADS, at most EP_CHUNK_BLOCKS of them (two a CU) beside the publishing one, each
 // with at most EP_CHUNK_OWN entries of its own; the counts of all entries fit 16 bits

@@ -1768,7 +1768,7 @@ __device__ __forceinline__ void dispatch_chunk_body(const EpSmallArgs& a) {
         else copy_row_out<PACK>(s, c, part, d, scales);
     }
     // ---- padding, in pieces of a 256-thread workgroup ----
-    if (!PACK && a.num_pad_blocks > 0) {
+    if (!PACK && a.zero_padding) {
         constexpr int GROUPS = NT / EP_ROW_THREADS;
         const int pieces = s.num_local_experts * s.pad_blocks_per_expert;
         for (int p = wg * GROUPS + __builtin_amdgcn_readfirstlane(tid / EP_ROW_THREADS); p < pieces; p += ((int)gridDim.x - 1) * GROUPS) {

@@ -477,7 +477,7 @@ void launch_chunk(const EpLayoutArgs& la, const EpScatterArgs& sa, bool pack, bo
     EpSmallArgs args{};
     args.l = la;
     args.s = sa;
-    args.num_pad_blocks = pad_pieces > 0;
+    args.zero_padding = pad_pieces > 0;
     EP_HOST_ASSERT(sa.vecs_per_lane == 1 and sa.num_rows_bound == la.num_tokens);
     const int64_t tasks = (int64_t)la.num_tokens * sa.num_parts;
     const bool two_a_cu = sa.num_parts >= 10 and la.num_tokens * la.num_topk <= EP_CHUNK_ENTRIES / 2;
