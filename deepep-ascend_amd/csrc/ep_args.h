@@ -37,7 +37,8 @@
 #define EP_COMBINE_LONG_PART 2048
 
 // Host-visible count page (pinned, mapped).  Written once per non-cached dispatch.
-//   [0] ready sequence number (written last, release at system scope)
+//   [0] ready sequence number: a relaxed store behind the arrival of the page's other words, which it orders and nothing else that the
+//       kernel wrote (that is complete in stream order)
 //   [1] number of received tokens   [2] number of expanded tokens (aligned)
 //   [16 .. 16+R)                 received tokens per source rank
 //   [16+EP_MAX_RANKS .. +El)     aligned received tokens per local expert
@@ -57,7 +58,7 @@
 #define EP_HOST_PAGE_INTS (16 + EP_MAX_RANKS + EP_MAX_EXPERTS)
 // Behind it, with several partitions: two slots (dispatches alternate) that the send sides of a node fill:
 //   [source][El] entries per local expert, then per source the rows it sent here, then per source its sequence number
-//   (written last, release at system scope)
+//   (behind the arrival of that source's other words, as above)
 #define EP_HOST_BOX_ROWS_OFF EP_MAX_EXPERTS
 #define EP_HOST_BOX_SEQ_OFF (EP_HOST_BOX_ROWS_OFF + EP_MAX_RANKS)
 #define EP_HOST_BOX_INTS (EP_HOST_BOX_SEQ_OFF + EP_MAX_RANKS)
@@ -171,8 +172,8 @@ struct EpSmallArgs {
     int zero_padding;             // there is padding to zero: every copying workgroup takes a share
     int tasks_per_block;          // (token, part) tasks of a workgroup
 };
-// ep_dispatch_chunk_*: workgroups of EP_CHUNK_THREADS, at most EP_CHUNK_BLOCKS of them (two a CU) beside the publishing one, each
-// with at most EP_CHUNK_OWN entries of its own; the counts of all entries fit 16 bits
+// ep_dispatch_chunk_*: workgroups of EP_CHUNK_THREADS, at most EP_CHUNK_BLOCKS of them (two a CU; the last one takes the place of the
+// publishing one, which ends early), each with at most EP_CHUNK_OWN entries of its own; the counts of all entries fit 16 bits
 #define EP_CHUNK_THREADS 1024
 #define EP_CHUNK_BLOCKS 512
 #define EP_CHUNK_OWN 512

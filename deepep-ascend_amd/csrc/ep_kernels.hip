@@ -85,7 +85,8 @@ __device__ __forceinline__ uint64_t match_any(int key, int nbits) {
 }
 
 // Every lane must be active.  (DPP shifts inside a row of 16 lanes, then the rows' last lanes broadcast to the rows behind: six
-// dependent VALU operations, where shuffles are six trips through the LDS.)
+// dependent VALU operations, where shuffles are six trips through the LDS: a replayed decode of 32 tokens 17.7 -> 17.5 us, larger calls
+// level.)
 __device__ __forceinline__ int wave_inclusive_sum(int v) {
     v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr:1
     v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);      // row_shr:2
@@ -97,9 +98,9 @@ __device__ __forceinline__ int wave_inclusive_sum(int v) {
 }
 
 // Counts for the host go to its pinned page (fine-grained memory) with stores that pass the L2, one by one; when a workgroup's have
-// arrived, one more says so.  A release at system scope would write the whole L2 back in front of it: two or three times 1 us
-// where nothing is dirty, and longer beside the stores of a copy in the same launch.  Whole host-synchronised cases (us): 128 tokens of a
-// toy layer 25.2 -> 23.8, a chunk of 1021 tokens 34.0 -> 33.3.
+// arrived, one more says so; it orders them and nothing else.  A release at system scope would write the whole L2 back in front of
+// it: 1 us where nothing is dirty, and far longer beside the stores of a copy in the same launch.  Whole host-synchronised cases, three pairs of
+// processes, release / this (us): 128 tokens of a toy layer 25.0 / 24.9, a chunk of 1021 tokens 35.4 / 28.2, eight partitions of 2048 1293 / 1252.
 __device__ __forceinline__ void host_store(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); }
 __device__ __forceinline__ void host_stores_arrived() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
