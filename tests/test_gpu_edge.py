@@ -17,6 +17,14 @@ def _buffer(maxT, H, K, R=1, rank=0, **kw):
                             explicitly_destroy=True, **kw)
 
 
+def _dispatched(buf, deferred, *args, **kw):
+    """The handle of a dispatch: of calls that one launch may serve whole, or (deferred: one partition; several: never) laid out by
+    launches of its own."""
+    if not deferred:
+        return buf.dispatch(*args, **kw)[3]
+    return buf.dispatch(*args, async_with_compute_stream=True, defer_epilogue=True, **kw).current_stream_wait()[3]
+
+
 def _roundtrip(T, maxT, H, E, K, A, topk, w, x, R=1, rank=0, fused=False, seed=0):
     lay = O.rank_share_layout(topk.numpy(), E, R, rank, A, maxT)
     buf = _buffer(maxT, H, K, R, rank, use_fp8_dispatch=fused)
@@ -218,22 +226,24 @@ def test_deterministic_flag_gives_the_same_layout():
 
 
 @pytest.mark.parametrize('T,E,K,R,rank', [(700, 64, 6, 1, 0), (1500, 256, 8, 8, 3), (300, 2048, 4, 1, 0), (128, 256, 8, 1, 0),
-                                         (129, 256, 8, 4, 2), (300, 2048, 8, 1, 0), (300, 2048, 32, 1, 0)])
+                                         (129, 256, 8, 4, 2), (300, 2048, 8, 1, 0), (300, 2048, 32, 1, 0), (2049, 256, 8, 4, 2)])
 def test_single_and_multi_block_layouts_agree_with_oracle(T, E, K, R, rank):
-    """128 tokens fit one layout block (no counting pass runs); 129 need the counting pass.  2048 experts of one
-    partition are more count columns than the slot assignment that sums the counts itself has threads for: the scan
-    kernel runs at any size."""
+    """In launches of their own (deferred calls of one partition, several partitions beyond 2048 tokens), 128 tokens fit one
+    layout block (no counting pass runs); more need the counting pass.  2048 experts of one partition are more count columns
+    than the slot assignment that sums the counts itself has threads for: the scan kernel runs at any size.  The other calls
+    are laid out by the copy or pack launch."""
     H, A = 128, 16
     topk, w = make_routing(T, E, K, seed=T, masked=0.1)
     lay = O.rank_share_layout(topk.numpy(), E, R, rank, A, T)
     buf = _buffer(T, H, K, R, rank)
-    _, _, _, handle, _ = buf.dispatch(make_tokens(T, H).to(DEV), topk_idx=topk.to(DEV), topk_weights=w.to(DEV),
-                                      num_experts=E, expert_alignment=A, do_expand=True)
-    torch.cuda.synchronize()
-    for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert',
-                 'num_unaligned_recv_tokens_per_expert', 'dst_buffer_slot_idx', 'recv_src_metadata'):
-        assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
-    assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
+    for deferred in (False, True):
+        handle = _dispatched(buf, deferred, make_tokens(T, H).to(DEV), topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E,
+                             expert_alignment=A, do_expand=True)
+        torch.cuda.synchronize()
+        for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert',
+                     'num_unaligned_recv_tokens_per_expert', 'dst_buffer_slot_idx', 'recv_src_metadata'):
+            assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (deferred, name)
+        assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
     buf.destroy()
 
 
@@ -257,12 +267,13 @@ def test_block_counts_at_their_16_bit_bound():
 
 
 @pytest.mark.parametrize('T,E,K,R,rank', [(1500, 256, 8, 1, 0), (700, 64, 6, 4, 1), (700, 64, 6, 1, 0), (257, 256, 8, 1, 0),
-                                         (1000, 2048, 2, 1, 0), (40000, 64, 2, 8, 3)])
+                                         (1000, 2048, 2, 1, 0), (40000, 64, 2, 8, 3), (2100, 64, 6, 4, 1), (2100, 2048, 8, 1, 0)])
 def test_layout_paths_agree(T, E, K, R, rank):
     """Several layout workgroups, four ways to the counts of the workgroups before one: the slot assignment sums the
-    histograms itself, or reads the prefixes a scan kernel left, or (one partition, few blocks: the last three shapes) no
-    histogram kernel runs and it counts the ids of all blocks itself.  Same handle tensors every way.  (The last shape:
-    313 blocks of a partition with 16 count columns, which the slot assignment still sums itself.)"""
+    histograms itself, or reads the prefixes a scan kernel left, or (few blocks of one partition: 700, 257 and 1000 tokens) no
+    histogram kernel runs and it counts the ids of all blocks itself, or the copy or pack launch of up to 16384 entries does.
+    Same handle tensors every way.  (One partition takes the first three where the epilogue is deferred, several beyond 2048 tokens.
+    40000 tokens: 313 blocks of a partition with 16 count columns, which the slot assignment still sums itself.)"""
     import deep_ep
     H, A = 128, 16
     topk, w = make_routing(T, E, K, seed=T + 1, masked=0.1)
@@ -274,12 +285,14 @@ def test_layout_paths_agree(T, E, K, R, rank):
             deep_ep._C.set_layout_fold_max_blocks(fold_max)
             deep_ep._C.set_layout_recount_limit(recount)
             buf = _buffer(T, H, K, R, rank)
-            _, _, _, handle, _ = buf.dispatch(make_tokens(T, H).to(DEV), topk_idx=topk.to(DEV), topk_weights=w.to(DEV),
-                                              num_experts=E, expert_alignment=A, do_expand=True)
-            torch.cuda.synchronize()
-            for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert',
-                         'num_unaligned_recv_tokens_per_expert', 'dst_buffer_slot_idx', 'recv_src_metadata'):
-                assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (fold_max, recount, name)
+            for deferred in (False, True):
+                handle = _dispatched(buf, deferred, make_tokens(T, H).to(DEV), topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E,
+                                     expert_alignment=A, do_expand=True)
+                torch.cuda.synchronize()
+                for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert',
+                             'num_unaligned_recv_tokens_per_expert', 'dst_buffer_slot_idx', 'recv_src_metadata'):
+                    assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (fold_max, recount, deferred, name)
+                assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
             buf.destroy()
     finally:
         deep_ep._C.set_layout_fold_max_blocks(256)

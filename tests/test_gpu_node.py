@@ -199,7 +199,8 @@ def test_node_dispatch_combine(R, max_tokens, H, E, K, A, masked, mode, do_cpu_s
     (2, 128, [128, 127], 16, 8),            # one block of tokens a partition, receive streams of one block and a row
     (4, 129, [129, 1, 128, 0], 8, 3),       # sources of one and of no token
     (2, 600, [600, 511], 12, 1),            # a single selection: several blocks on both sides
-    (16, 300, [300 - 9 * r for r in range(16)], 2048, 4),   # more count columns than the send side sums itself
+    (16, 300, [300 - 9 * r for r in range(16)], 2048, 4),   # the most experts, laid out by the pack launch
+    (2, 2100, [2100, 2050], 2048, 4),       # more count columns than the send side sums itself, in launches of its own
     (3, 2500, [2500, 2049, 2304], 384, 7),  # more entries a workgroup than one round of four a thread
     (2, 70000, [300, 129], 40, 32),         # the rank box does not fit the workspace: counted and ranked on arrival
     (129, 3, [3 - r % 4 for r in range(129)], 258, 3),          # more partitions than the header has host boxes for

@@ -119,7 +119,8 @@ def test_small_dispatch_deferred_exact_and_replayed():
                                    (2049, 32, 2), (1281, 64, 5)])
 def test_ids_of_all_blocks_counted_in_place(T, E, K):
     """Around the most blocks x top-k (64) for which the histogram kernel can be left out (every workgroup then reads all ids
-    itself), and around the library's own limits: the same handles whichever launches run."""
+    itself), and around the library's own limits: the same handles whichever launches run.  (The layout has launches of its own where
+    the epilogue is deferred, and beyond 4096 tokens or 16384 entries.)"""
     import deep_ep
     H, A = 64, 4
     x = make_tokens(T, H, seed=T).to(DEV)
@@ -130,13 +131,17 @@ def test_ids_of_all_blocks_counted_in_place(T, E, K):
     try:
         for limit, sync in ((64, True), (-1, True), (-1, False)):
             deep_ep._C.set_layout_recount_limit(limit)
-            _, _, _, handle, _ = buf.dispatch(x, topk_idx=topk.to(DEV), num_experts=E, expert_alignment=A, do_expand=True,
-                                              do_cpu_sync=sync)
+            args = dict(topk_idx=topk.to(DEV), num_experts=E, expert_alignment=A, do_expand=True, do_cpu_sync=sync)
+            handles = [buf.dispatch(x, **args)[3],
+                       buf.dispatch(x, async_with_compute_stream=True, defer_epilogue=True, **args).current_stream_wait()[3]]
             torch.cuda.synchronize()
-            for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
-                         'dst_buffer_slot_idx'):
-                assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (limit, sync, name)
-            assert np.array_equal(handle.recv_src_metadata.cpu().numpy()[:lay['num_recv_tokens']], lay['recv_src_metadata'])
+            for handle in handles:
+                for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
+                             'dst_buffer_slot_idx'):
+                    assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), (limit, sync, name)
+                assert np.array_equal(handle.recv_src_metadata.cpu().numpy()[:lay['num_recv_tokens']], lay['recv_src_metadata'])
+                if sync:
+                    assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
     finally:
         deep_ep._C.set_layout_recount_limit(-1)
     buf.destroy()

@@ -323,6 +323,17 @@ def test_which_begins_leave_the_layout_to_the_copy_launch(host_calls):
                 assert all(line.startswith('ep_layout_') and line.endswith(' on 1') for line in launches[:-1]), (form, tokens, launches)
 
 
+@pytest.mark.parametrize('tokens,partitions,own', [(2, 1, True), (129, 1, True), (700, 1, True), (4096, 1, True), (9000, 1, True), (129, 2, False),
+                                                   (2048, 2, False), (2049, 2, True)])
+def test_which_deferred_calls_have_their_layout_in_launches_of_its_own(host_calls, tokens, partitions, own):
+    """What the GPU tests of the layout kernels rest on: one partition's deferred dispatch always has, a send side beyond 2048
+    tokens."""
+    lines = host_calls('event', tokens, partitions, 'alone')
+    sent = [line.split()[0] for line in lines[:lines.index('event on 1')] if line.startswith('ep_')]
+    assert any(name.startswith('ep_layout_assign') for name in sent) == own, lines
+    assert any(name.startswith('ep_dispatch_') for name in sent) != own, lines
+
+
 @pytest.mark.parametrize('hidden,tokens', [(256, 4096), (5632, 4096), (6144, 3072), (7168, 3072), (8192, 3072), (8704, 2560), (10240, 2560), (10240, 2900)])
 def test_wide_rows_of_many_tokens_keep_the_launch_in_front(host_calls, hidden, tokens):
     """Four entries a token: from 12 parts a row (6144 BF16 channels) on, beyond 3072 tokens, and with more than 16 parts beyond 2560,
