@@ -214,8 +214,11 @@ void ep_set_combine_blocks_per_cu(int num_blocks);
 int ep_dispatch_recv_launch(ep_buffer_t* buf, const ep_dispatch_recv_args_t* args);
 /* The same for a caller whose next launch on this buffer is this dispatch's ep_dispatch_epilogue_launch: in a node whose send
  * sides ship ranks the library may then leave the placing to the copy launch (one launch instead of two).  Everything this
- * call would have enqueued is then enqueued by the epilogue, on the epilogue's stream; ep_dispatch_wait_counts may come
- * between the two. */
+ * call would have enqueued is then enqueued by the epilogue, on the epilogue's stream: every tensor given here (the handle
+ * tensors, num_unaligned..., the running statistics, the metadata rows) has to stay until the epilogue and is complete
+ * behind it only, also where ep_dispatch_wait_counts, which may come between the two, has returned before.  An epilogue on another
+ * stream is ordered behind what this call is ordered behind by the caller, as after ep_dispatch_recv_launch.  A dispatch that
+ * comes first takes its place. */
 int ep_dispatch_recv_begin(ep_buffer_t* buf, const ep_dispatch_recv_args_t* args);
 
 /* Host wait for the counts of the last non-cached do_cpu_sync dispatch, with the buffer's CPU
