@@ -110,8 +110,8 @@ __device__ __forceinline__ void host_stores_arrived() {
 // Reads one word of every 64 bytes of the kernel's arguments, all in one trip.  The compiler fetches arguments where they are
 // first used, in some kernels four or five times in a row along the way to the first store, and each first touch of a
 // cache line is a trip to memory.  Whole cases, three pairs of processes, without / with (us): prefill of 4096 tokens top-8 246.4 / 244.6, a
-// training step of 8192 269.1 / 267.2, prefill of 32768 1202.4 / 1201.5, a replayed decode of 32 17.5 / 17.5.  Not in the combine kernels of
-// several partitions, where it loses (eight partitions of 2048 tokens 1241.4 / 1247.8, with it in these kernels alone).
+// training step of 8192 269.1 / 267.2, prefill of 32768 1202.4 / 1201.5, a replayed decode of 32 17.5 / 17.5; in the combine kernels
+// of eight partitions of 2048 tokens 1242.7 / 1239.0, replayed, 600 tokens 473.0 / 468.8.
 template <typename Args>
 __device__ __forceinline__ void fetch_arguments() {
     typedef const unsigned __attribute__((address_space(4)))* words_t;
@@ -122,6 +122,15 @@ __device__ __forceinline__ void fetch_arguments() {
 #pragma unroll
     for (int i = 0; i < 10; ++i) v[i] = words[16 * i <= LAST ? 16 * i : LAST];
     asm volatile("" ::"s"(v[0]), "s"(v[1]), "s"(v[2]), "s"(v[3]), "s"(v[4]), "s"(v[5]), "s"(v[6]), "s"(v[7]), "s"(v[8]), "s"(v[9]));
+}
+
+// A word that every lane reads alike and nothing of the launch writes, by way of the scalar cache.  The compiler takes the asm of
+// fetch_arguments for a store and reads such words behind it with a vector load: two trips in a row in the owner-side reduce (eight
+// partitions of 2048 tokens, three pairs of processes, 1252.0 -> 1241.7 us).  Not in the copy kernels, where the one word comes back no later than
+// the metadata row beside it (a training step 264.6 -> 266.2).
+template <typename T>
+__device__ __forceinline__ T uniform_load(const T* p) {
+    return *(const T __attribute__((address_space(4)))*)p;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -2207,7 +2216,8 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
         if (master) myslot = (a.num_ranks < K ? r : lane) * a.max_tokens + t;
     } else {
         const int mv = lane < K + 2 ? a.recv_src_metadata[(int64_t)i * (K + 2) + lane] : -1;
-        if (i >= *a.num_recv_ptr) return;                // (checked after the row's own load has been issued)
+        const int num_recv = MODE == EP_COMBINE_PARTIAL ? uniform_load(a.num_recv_ptr) : *a.num_recv_ptr;
+        if (i >= num_recv) return;                       // (checked after the row's own load has been issued)
         if (lane < K && mv >= 0 && mv < a.num_in_rows) myslot = mv;
         const int src = readlane(mv, K);                        // source partition * max_tokens + its token
         if (MODE == EP_COMBINE_PARTIAL) {
@@ -2231,7 +2241,7 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
     const u32x4* y = (const u32x4*)a.y;
     // a partial goes to the combine buffer of the partition its token came from (impls/ep/combine.hpp:291-324)
     char* out_row = MODE == EP_COMBINE_PARTIAL
-        ? a.peer_arenas[src_rank] + a.buffer_off + ((int64_t)group * a.max_tokens + t) * a.out_row_bytes
+        ? uniform_load(&a.peer_arenas[src_rank]) + a.buffer_off + ((int64_t)group * a.max_tokens + t) * a.out_row_bytes
         : (char*)a.combined_x + (int64_t)t * a.out_row_bytes;
 
     // ---- gate weights ----
@@ -2483,11 +2493,11 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
 }
 
 #define EP_COMBINE_KERNELS(SUFFIX, MODE)                                                                                   \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_generic(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<0, MODE>(a); } \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k2(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<2, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k4(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<4, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k6(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<6, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k8(EpCombineArgs a) { if (MODE == EP_COMBINE_FUSED) fetch_arguments<EpCombineArgs>(); combine_body<8, MODE>(a); }
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_generic(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<0, MODE>(a); } \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k2(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<2, MODE>(a); }     \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k4(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<4, MODE>(a); }     \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k6(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<6, MODE>(a); }     \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k8(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<8, MODE>(a); }
 
 EP_COMBINE_KERNELS(, EP_COMBINE_FUSED)
 EP_COMBINE_KERNELS(_partial, EP_COMBINE_PARTIAL)
