@@ -163,6 +163,7 @@ struct EpScatterArgs {
 // A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES (token, slot) entries in one launch, or the receive
 // side of a node that ships ranks: every workgroup works the layout out for itself.
 #define EP_SMALL_ENTRIES 1024
+#define EP_SMALL_MASK_EXPERTS 1024    // ep_dispatch_small_*: up to here a bit a token and expert is kept in LDS (16 bytes an expert)
 struct EpSmallArgs {
     EpLayoutArgs l;               // what ep_layout_assign (ep_recv_copy: ep_layout_place) would have been given
     EpScatterArgs s;              // what the copy kernel would have been given

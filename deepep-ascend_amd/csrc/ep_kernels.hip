@@ -1015,20 +1015,27 @@ __device__ __forceinline__ char* out_sf_of(const EpScatterArgs& a, char* rows) {
 }
 
 // Part 0 of a packed row's task: the metadata of the row and its ranks, in every destination.  Lane j < K holds the
-// expert id, the gate weight and the rank of entry (t, j).
+// expert id, the gate weight and the rank of entry (t, j).  Lane l of a round stores item l % K of destination l / K: as many
+// destinations a round as fit a wave.  (A destination after the other is K times the address arithmetic and the store queue's turns, which
+// the other parts of the row do not have: 64 tokens x 7168 top-8, each of eight partitions, dispatches of all
+// 93.4 -> 88.3 us; 200 to 2048 tokens 2 % of a dispatch.)
 __device__ __forceinline__ void pack_row_metadata(const EpScatterArgs& a, const RowCtx& c, int64_t e, float w, int rank) {
     const int lane = lane_id(), K = a.num_topk;
-    for (int j = 0; j < K; ++j) {
-        const int g = readlane(c.myslot, j);
-        if (g < 0) continue;
-        char* rows = out_rows_of<true>(a, c, j);
+    const int at_once = WAVE / K, jj = lane / K, k = lane - jj * K;
+    const unsigned e_lo = (unsigned)__shfl((int)(unsigned)e, k), e_hi = (unsigned)__shfl((int)(e >> 32), k);
+    const int rank_k = __shfl(rank, k);
+    const float w_k = __shfl(w, k);
+    for (int j0 = 0; j0 < K; j0 += at_once) {
+        const int j = j0 + jj;
+        const int g = __shfl(c.myslot, j);
+        const unsigned lo = (unsigned)__shfl((int)(unsigned)c.mybase, j), hi = (unsigned)__shfl((int)(unsigned)(c.mybase >> 32), j);
+        if (jj >= at_once || j >= K || g < 0) continue;
+        char* rows = (char*)((uint64_t)hi << 32 | lo);
         char* row = rows + (int64_t)g * a.out_row_bytes;
-        if (a.rank_box_off != 0 && lane < K) ((int*)(rows - a.buffer_off + a.rank_box_off))[(int64_t)g * K + lane] = rank;
-        if (lane < K) {
-            if (a.with_metadata) ((int64_t*)(row + a.idx_off))[lane] = e;
-            ((float*)(row + a.w_off))[lane] = w;
-        }
-        if (a.with_metadata && lane == 0) *(int*)(row + a.src_off) = a.rank_idx * a.max_tokens + c.t;
+        if (a.rank_box_off != 0) ((int*)(rows - a.buffer_off + a.rank_box_off))[(int64_t)g * K + k] = rank_k;
+        if (a.with_metadata) ((int64_t*)(row + a.idx_off))[k] = (int64_t)((uint64_t)e_hi << 32 | e_lo);
+        ((float*)(row + a.w_off))[k] = w_k;
+        if (a.with_metadata && k == 0) *(int*)(row + a.src_off) = a.rank_idx * a.max_tokens + c.t;
     }
 }
 
@@ -1387,40 +1394,48 @@ __device__ __forceinline__ void publish_dispatch(const EpLayoutArgs& l, int gran
 // ------------------------------------------------------------------------------------------------
 // A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES entries in one launch.  Instead of a slot
 // assignment in front of the copy (a launch that one or two workgroups of the chip work at, bound by its own dependent
-// phases), every workgroup stages all ids in LDS, counts them per expert, and its waves rank the one token each of
-// them copies: the number of earlier entries with the same expert, sixteen compare-and-count steps an expert at most.
+// phases), every workgroup counts all ids in LDS and leaves a bit a token and expert there; its waves rank the one token each of
+// them copies by the bits below it, a position a lane.  (A token that selects an expert twice has one bit for both: then, and beyond
+// EP_SMALL_MASK_EXPERTS, whose masks would leave a CU too few workgroups, the ids in front of the token are compared expert by expert.)
 // The payload is fetched before the ids are looked at.  Workgroup 0 publishes what the assignment's publishing workgroup
 // does, the next ones copy (or, with several partitions, pack) as the kernels above, the last zero the padding.
-// Bound by the launch, two trips to memory and the phases in LDS between them.  Assignment + copy -> this kernel (us): 32 tokens,
+// Bound by the launch, two trips to memory and the phases in LDS between them.  Assignment + copy -> this kernel with ids compared (us): 32 tokens,
 // top-8 of 256, FP8 8.8 + 6.2 -> 9.0; 61 tokens x 5120, top-6 of 160, BF16 7.5 + 4.2 -> 8.2; 128 tokens, top-8, 230 MB of
 // padding 10.0 + 31.2 -> 35.3; one of eight partitions of 64 tokens 11.2 + 5.6 -> 10.1.
+// Ids compared -> masks, and a scan that each wave makes alone (us a dispatch, several in a captured graph; stamps had the ranking at 2.4 of
+// 6.3): 256 experts, BF16, top-8, 7168 channels 1 / 32 / 61 tokens 5.7 / 6.4 / 7.5 -> 4.3 / 4.9 / 5.7, 256 channels 128 tokens 8.2 -> 5.8; top-6, FP8,
+// alignment 16, 96 tokens 8.0 -> 6.5; 1024 experts, 61 tokens top-8 7.4 -> 5.8; top-1 level; all of a dispatch of eight partitions of 64 tokens
+// top-8, metadata above included, 110.0 -> 88.3.  Masks at 2048 experts: 1 token top-1 with padding 8.3 -> 10.8, compared so 8.2.
 // ------------------------------------------------------------------------------------------------
 template <bool QUANT, bool HW, bool PACK>
 __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     extern __shared__ int smem[];
-    constexpr int NW = EP_ROW_THREADS / WAVE, CH = EP_SMALL_ENTRIES / WAVE, PER = EP_SMALL_ENTRIES / EP_ROW_THREADS;
+    constexpr int CH = EP_SMALL_ENTRIES / WAVE, PER = EP_SMALL_ENTRIES / EP_ROW_THREADS, TW = EP_TOKENS_PER_BLOCK / 32;
     const EpLayoutArgs& l = a.l;
     const EpScatterArgs& s = a.s;
     const int E = l.num_experts, R = l.num_ranks, K = l.num_topk, A = l.expert_alignment, El = l.experts_per_rank;
-    int* s_cnt = smem;                                  // [E] entries per expert
-    int* s_start = s_cnt + E;                           // [E] first slot of each expert (one partition)
-    unsigned* s_tok = (unsigned*)(s_start + E);         // [R][EP_TOKENS_PER_BLOCK / 32] tokens that go to a partition, a bit each
-    int* s_tmp = (int*)(s_tok + R * (EP_TOKENS_PER_BLOCK / 32));       // [NW]
-    short* s_key = (short*)(s_tmp + NW);                // [EP_SMALL_ENTRIES] expert of every entry, -1: none
-    constexpr int TW = EP_TOKENS_PER_BLOCK / 32;
-    const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
-    const int n = l.num_tokens * K;
+    const int Ep = (E + 7) & ~7;
     const bool publisher = blockIdx.x == 0;
     const int rb = (int)blockIdx.x - 1;
     const bool copies = !publisher && rb < s.num_row_blocks;
+    const bool masks = copies && E <= EP_SMALL_MASK_EXPERTS;            // (who ranks nothing needs none)
+    u32x4* s_tok = (u32x4*)smem;                        // [R] tokens that go to a partition, a bit each
+    u32x4* s_mask = s_tok + R;                          // [E] tokens that selected an expert, a bit each (E <= EP_SMALL_MASK_EXPERTS)
+    int* s_cnt = (int*)(s_mask + (masks ? E : 0));      // [Ep] entries per expert
+    int* s_twice = s_cnt + Ep;                          // [4] a token selected an expert twice: the masks do not say how often
+    int* s_start = s_twice + 4;                         // [Ep] first slot of each expert (one partition)
+    short* s_key = (short*)(s_start + Ep);              // [EP_SMALL_ENTRIES] expert of every entry, -1: none
+    const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
+    const int n = l.num_tokens * K;
 
-    // ids, then the payload of this wave's task, all in flight together
+    // all ids, the ids of this wave's own token, then the payload of its task, all in flight together
     int64_t id[PER];
 #pragma unroll
     for (int u = 0; u < PER; ++u) id[u] = l.topk_idx[min(tid + u * EP_ROW_THREADS, n - 1)];
     const int task = copies ? rb * EP_ROWS_PER_BLOCK + w : 0;
     const int t = task / s.num_parts, part = task - t * s.num_parts;
     const bool works = copies && t < s.num_rows_bound;
+    const int64_t own = l.topk_idx[works ? t * K + min(lane, K - 1) : 0];
     const int nvec = QUANT ? s.hidden >> 3 : (int)(s.copy_bytes >> 4);
     const int v = part * WAVE + lane;
     const bool live = works && v < nvec;
@@ -1430,55 +1445,72 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     float gate = 0.0f;
     if (works && part == 0 && lane < K && s.topk_weights != nullptr) gate = s.topk_weights[(int64_t)t * K + lane];
 
-    for (int i = tid; i < E; i += EP_ROW_THREADS) s_cnt[i] = 0;
-    for (int i = tid; i < R * TW; i += EP_ROW_THREADS) s_tok[i] = 0u;
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    for (int i = tid; i < R + (masks ? E : 0) + (Ep >> 2) + 1; i += EP_ROW_THREADS) s_tok[i] = zero;
     __syncthreads();
+    // (quotients of small integers: (x + 1/2) / y is at least 1 / 2y away from the next integer, far more than the products round)
+    const float per_token = 1.0f / (float)K, per_partition = 1.0f / (float)El;
+    auto partition_of = [&](int e) { return (int)(((float)e + 0.5f) * per_partition); };
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
+        if (u * EP_ROW_THREADS >= n) break;
         const int i = tid + u * EP_ROW_THREADS;
         const bool valid = i < n && id[u] >= 0 && id[u] < E;
         const int e = valid ? (int)id[u] : -1;
         s_key[i] = (short)e;
         if (valid) {
-            const int tok = i / K;
+            const int tok = (int)(((float)i + 0.5f) * per_token);
+            const unsigned bit = 1u << (tok & 31);
             atomicAdd(&s_cnt[e], 1);
-            atomicOr(&s_tok[(PACK ? e / El : 0) * TW + (tok >> 5)], 1u << (tok & 31));
+            atomicOr((unsigned*)&s_tok[PACK ? partition_of(e) : 0] + (tok >> 5), bit);
+            if (masks && (atomicOr((unsigned*)&s_mask[e] + (tok >> 5), bit) & bit)) *s_twice = 1;
         }
     }
+    // (own ids are here by now, and with them the arenas of the token's partitions, which are a trip of their own)
+    const int e = (works && lane < K && own >= 0 && own < E) ? (int)own : -1;
+    const int r = e < 0 ? -1 : PACK ? partition_of(e) : 0;
+    char* peer = nullptr;
+    if (PACK && works) peer = s.peer_arenas[max(r, 0)];
     __syncthreads();
     int grand = 0;
     if (!PACK) {
-        // aligned exclusive scan over the experts
-        const int per = (E + EP_ROW_THREADS - 1) / EP_ROW_THREADS;
-        const int e0 = min(E, tid * per), e1 = min(E, e0 + per);
-        int mine = 0;
-        for (int e = e0; e < e1; ++e) mine += align_up(s_cnt[e], A);
-        const int incl = wave_inclusive_sum(mine);
-        if (lane == WAVE - 1) s_tmp[w] = incl;
-        __syncthreads();
-        int run = incl - mine;
-        for (int i = 0; i < NW; ++i) {
-            if (i < w) run += s_tmp[i];
-            grand += s_tmp[i];
+        // aligned exclusive scan over the experts, eight a lane: every wave makes all of it (and writes the same words), which
+        // costs less than meeting twice
+        const bool pow2 = (A & (A - 1)) == 0;
+        for (int e0 = 8 * lane; e0 - 8 * lane < E; e0 += 8 * WAVE) {
+            u32x4 c[2] = {zero, zero};
+            if (e0 < E) {
+                c[0] = *(const u32x4*)(s_cnt + e0);
+                c[1] = *(const u32x4*)(s_cnt + e0 + 4);
+            }
+            int before[8], sum = 0;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const int x = (int)c[q >> 2][q & 3];
+                before[q] = sum;
+                sum += pow2 ? (x + A - 1) & -A : align_up(x, A);
+            }
+            const int incl = wave_inclusive_sum(sum), run = grand + incl - sum;
+            if (e0 < E) {
+                *(u32x4*)(s_start + e0) = u32x4{(unsigned)run, (unsigned)(run + before[1]), (unsigned)(run + before[2]), (unsigned)(run + before[3])};
+                *(u32x4*)(s_start + e0 + 4) = u32x4{(unsigned)(run + before[4]), (unsigned)(run + before[5]), (unsigned)(run + before[6]), (unsigned)(run + before[7])};
+            }
+            grand += readlane(incl, WAVE - 1);
         }
-        for (int e = e0; e < e1; ++e) {
-            s_start[e] = run;
-            run += align_up(s_cnt[e], A);
-        }
-        __syncthreads();
     }
-    auto tokens_to = [&](int r, int before) -> int {     // tokens below `before` that go to partition r
+    auto below = [&](const u32x4& m, int before) -> int {      // bits of m below `before`
         int c = 0;
+#pragma unroll
         for (int q = 0; q < TW; ++q) {
             const int bits = min(max(before - 32 * q, 0), 32);
-            c += __popc(bits == 32 ? s_tok[r * TW + q] : s_tok[r * TW + q] & ((1u << bits) - 1u));
+            c += __popc(m[q] & (bits == 32 ? ~0u : (1u << bits) - 1u));
         }
         return c;
     };
 
     if (publisher) {
         publish_dispatch<PACK>(l, grand, [&](int e) { return s_cnt[e]; }, s_start,
-                               [&](int r) { return tokens_to(r, EP_TOKENS_PER_BLOCK); });
+                               [&](int r) { return below(s_tok[r], EP_TOKENS_PER_BLOCK); });
         return;
     }
     if (!copies) {
@@ -1492,36 +1524,34 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     if (!works) return;
 
     // ---- rank of the token's entries: earlier entries with the same expert ----
-    const int e = lane < K ? s_key[t * K + lane] : -1;
-    const int before = t * K, chunks = (before + WAVE - 1) / WAVE;
-    int key[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int i = c * WAVE + lane;
-        key[c] = i < before ? s_key[i] : -2;            // (-2 equals no expert and no missing selection)
-    }
     int rank = 0;
-    for (int j = 0; j < K; ++j) {
-        const int ej = readlane(e, j);
-        if (ej < 0) continue;
-        // (the same expert twice in one token: the earlier one counts too)
-        int c0 = __popcll(__ballot(e == ej) & ((1ull << j) - 1ull));
+    if (masks && __builtin_amdgcn_readfirstlane(*s_twice) == 0) {
+        rank = below(s_mask[max(e, 0)], t);             // earlier tokens, each of which selected it once
+    } else {
+        const int before = t * K, chunks = (before + WAVE - 1) / WAVE;
+        int key[CH];
 #pragma unroll
-        for (int c = 0; c < CH; c += 4)                 // (four chunks a branch; a break would keep the loop from being unrolled)
-            if (c < chunks) {
+        for (int c = 0; c < CH; ++c) {
+            const int i = c * WAVE + lane;
+            key[c] = i < before ? s_key[i] : -2;        // (-2 equals no expert and no missing selection)
+        }
+        for (int j = 0; j < K; ++j) {
+            const int ej = readlane(e, j);
+            if (ej < 0) continue;
+            // (the same expert twice in one token: the earlier one counts too)
+            int c0 = __popcll(__ballot(e == ej) & ((1ull << j) - 1ull));
 #pragma unroll
-                for (int q = 0; q < 4; ++q) c0 += __popcll(__ballot(key[c + q] == ej));
-            }
-        if (lane == j) rank = c0;
+            for (int c = 0; c < CH; c += 4)             // (four chunks a branch; a break would keep the loop from being unrolled)
+                if (c < chunks) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) c0 += __popcll(__ballot(key[c + q] == ej));
+                }
+            if (lane == j) rank = c0;
+        }
     }
     // ---- masters: the last entry of the token for a partition; its slot there ----
-    const int r = e < 0 ? -1 : PACK ? e / El : 0;
-    bool master = r >= 0;
-    for (int jj = 1; jj < K; ++jj) {
-        const int rj = readlane(r, jj);
-        if (lane < jj && rj == r) master = false;
-    }
-    const int rslot = master ? tokens_to(r, t) : -1;
+    const uint64_t peers = PACK ? match_any(r + 1, 32 - __builtin_clz(R)) : __ballot(r == 0);
+    const int rslot = r >= 0 && (peers >> lane) == 1ull ? below(s_tok[r], t) : -1;
     if (part == 0 && lane < K) {
         l.dst_buffer_slot_idx[(int64_t)t * K + lane] = rslot;
         l.dst_gsge_idx[(int64_t)t * K + lane] = -1;     // every copy is local: no transport descriptors
@@ -1532,11 +1562,11 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     c.mybase = 0;
     c.myslot = -1;
     if (PACK) {
-        if (master && rslot < s.max_tokens) {
+        if (rslot >= 0 && rslot < s.max_tokens) {
             c.myslot = (s.region_by_source ? s.rank_idx : r) * s.max_tokens + rslot;
-            c.mybase = (uint64_t)(s.peer_arenas[r] + s.buffer_off);
+            c.mybase = (uint64_t)(peer + s.buffer_off);
         }
-        if (part == 0) pack_row_metadata(s, c, (lane < K && e >= 0) ? e : (lane < K ? l.topk_idx[(int64_t)t * K + lane] : 0), gate, e >= 0 ? rank : -1);
+        if (part == 0) pack_row_metadata(s, c, lane < K ? own : 0, gate, e >= 0 ? rank : -1);
     } else {
         const uint64_t vm = __ballot(e >= 0);
         if (vm == 0) return;                            // a token nobody receives

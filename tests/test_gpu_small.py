@@ -69,6 +69,65 @@ def test_small_dispatch(T, H, E, K, A, masked, zipf, mode):
     buf.destroy()
 
 
+@pytest.mark.parametrize('T,E,K,A,masked', [(1, 8, 8, 1, 0.0), (32, 9, 3, 4, 0.3), (33, 255, 8, 1, 0.0), (64, 1024, 16, 128, 0.0),
+                                            (65, 1025, 15, 3, 0.1), (96, 4, 4, 7, 0.0), (128, 1024, 8, 1, 0.2), (128, 2048, 8, 96, 0.0)])
+@pytest.mark.parametrize('R', [1, 2])
+def test_small_dispatch_each_expert_once(T, E, K, A, masked, R):
+    """No token selects an expert twice: ranks are counted in the bits of the tokens below (up to 1024 experts), at the edges of
+    the words that hold them and of the groups of experts that are scanned."""
+    import deep_ep
+    H, E = 64, E + E % R
+    x = [make_tokens(T, H, seed=T + r) for r in range(R)]
+    rt = [make_routing(T, E, K, seed=T + K + r, masked=masked) for r in range(R)]
+    assert all(len(set(row[row >= 0])) == (row >= 0).sum() for topk, _ in rt for row in topk.numpy())
+    node = deep_ep.LocalNode(R) if R > 1 else None
+    bufs = [deep_ep.EPBuffer(node.group(r) if R > 1 else deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K,
+                             explicitly_destroy=True) for r in range(R)]
+    args = dict(num_experts=E, num_max_tokens_per_rank=T, expert_alignment=A, do_expand=True, do_zero_padding=True, do_cpu_sync=False)
+    if R == 1:
+        got = [bufs[0].dispatch(x[0].to(DEV), topk_idx=rt[0][0].to(DEV), topk_weights=rt[0][1].to(DEV), **args)]
+    else:
+        events = [b.dispatch(xx.to(DEV), topk_idx=t.to(DEV), topk_weights=w.to(DEV), async_with_compute_stream=True, defer_epilogue=True, **args)
+                  for b, xx, (t, w) in zip(bufs, x, rt)]
+        got = [e.current_stream_wait() for e in events]
+    torch.cuda.synchronize()
+    El = E // R
+    for r in range(R):
+        rows, _, weights, handle = got[r][:4]
+        # the stable order: sources in turn, their tokens ascending, positions ascending inside a token
+        entries = [[] for _ in range(El)]
+        for s in range(R):
+            for t in range(T):
+                for j in range(K):
+                    e = int(rt[s][0][t, j]) - r * El
+                    if 0 <= e < El:
+                        entries[e].append((s, t, j))
+        assert [len(e) for e in entries] == handle.num_unaligned_recv_tokens_per_expert.cpu().tolist()
+        start, want, want_w = 0, [], []
+        rows, weights = bf16_bits(rows), weights.cpu().numpy()
+        for e in entries:
+            for i, (s, t, j) in enumerate(e):
+                want.append((start + i, bf16_bits(x[s])[t]))
+                want_w.append((start + i, rt[s][1][t, j].item()))
+            n = -(-len(e) // A) * A
+            assert not rows[start + len(e):start + n].any() and not weights[start + len(e):start + n].any()
+            start += n
+        at = [i for i, _ in want]
+        assert np.array_equal(rows[at], np.stack([v for _, v in want])) and np.array_equal(weights[at], np.float32([v for _, v in want_w]))
+        masters = (rt[r][0].numpy() >= 0) & (rt[r][0].numpy() < E)
+        slots = handle.dst_buffer_slot_idx.cpu().numpy()
+        for p in range(R):          # a token's last selection of a partition has its place among the tokens that go there
+            seen = 0
+            for t in range(T):
+                js = [j for j in range(K) if masters[t, j] and int(rt[r][0][t, j]) // El == p]
+                assert all(slots[t, j] == -1 for j in js[:-1])
+                if js:
+                    assert slots[t, js[-1]] == seen
+                    seen += 1
+    for b in bufs:
+        b.destroy()
+
+
 CHUNK_CASES = [
     # T, H, E, K, A, masked, zipf
     (130, 16, 8, 1, 1, 0.0, None),          # one workgroup a wave's worth of tasks each
