@@ -1603,8 +1603,13 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_q
 // now 5.0 + 2.2.  A replayed dispatch, two launches / this one (us): 200 tokens x 7168 FP8, top-8, alignment 128 56.7 / 49.2; 512 tokens
 // without padding 19.6 / 13.0; 1021 x 2560 BF16, top-7 23.3 / 14.6; 1024 x 7168 BF16, top-8 41.1 / 30.4; 2048 x 7168 66.9 / 53.0; 4096 x
 // 1024 top-2 16.4 / 12.9; one of eight partitions, FP8, all of its dispatch: 256 tokens top-8 32.4 / 18.5, 2048 top-6 71.4 / 65.6.
+// With several partitions a workgroup counts the ids up to its own tokens' and no further (ranks and places in a partition
+// count what is before), so that half of the chip's share of that work falls away and the first workgroups copy meanwhile.  us a
+// dispatch and its receive side, all partitions in a captured graph, before / after: eight of 2048 tokens FP8 top-6 532 / 518, of 512 185.7 / 182.7,
+// of 256 125.9 / 125.2; four of 1024 x 4096 top-8 148.1 / 147.3, top-4 106.5 / 106.7.
 // (Padding as equal shares of all padding rows in place of pieces of experts: 256 tokens 50.8 -> 56.9; the ids of two goes in flight:
-// spills, or one workgroup a CU and level.)
+// spills, or one workgroup a CU and level; each id of the next go asked for as one of this go is used: 2048 x 2560 19.8 -> 18.7, but one go
+// 1 to 2 % slower.)
 // ------------------------------------------------------------------------------------------------
 template <bool QUANT, bool HW, bool PACK>
 __device__ __forceinline__ void dispatch_chunk_body(const EpSmallArgs& a) {
@@ -1630,6 +1635,8 @@ __device__ __forceinline__ void dispatch_chunk_body(const EpSmallArgs& a) {
     const int tasks = T * s.num_parts;
     const int task0 = publisher ? 0 : min(tasks, wg * a.tasks_per_block), task1 = publisher ? 0 : min(tasks, task0 + a.tasks_per_block);
     const int first = task0 / s.num_parts, own = task1 > task0 ? (task1 - 1) / s.num_parts - first + 1 : 0;
+    // who packs needs the ids up to its own and no further (the slots are the receivers' business)
+    const int upto = PACK && !publisher ? (first + own) * K : n;
     const int nvec = QUANT ? s.hidden >> 3 : (int)(s.copy_bytes >> 4);
 
     u32x2 id[GO];
@@ -1664,13 +1671,13 @@ __device__ __forceinline__ void dispatch_chunk_body(const EpSmallArgs& a) {
     auto partition_of = [&](int e) { return (int)(((float)e + 0.5f) * per_partition); };
     {
         const int own0 = first * K, nown = own * K, wave0 = __builtin_amdgcn_readfirstlane(w) * WAVE;
-        for (int i0 = 0; i0 < n; i0 += GO * NT) {
+        for (int i0 = 0; i0 < upto; i0 += GO * NT) {
             if (i0 > 0) fetch_ids(i0);
 #pragma unroll
             for (int u = 0; u < GO; ++u) {
                 const int i = i0 + tid + u * NT;
-                if (i0 + u * NT + wave0 >= n) break;
-                const bool valid = id[u].y == 0u && id[u].x < (unsigned)E && i < n;
+                if (i0 + u * NT + wave0 >= upto) break;
+                const bool valid = id[u].y == 0u && id[u].x < (unsigned)E && i < upto;
                 if (!PACK) {
                     const uint64_t bits = __ballot(valid);
                     if (lane == 0) ((uint64_t*)s_mask)[i >> 6] = bits;
@@ -1687,7 +1694,7 @@ __device__ __forceinline__ void dispatch_chunk_body(const EpSmallArgs& a) {
     // ---- tokens per partition; aligned exclusive scan over the experts (one partition) ----
     {
         unsigned sum = 0u;                              // lane r < R: of partition r
-        for (int t0 = w * WAVE; t0 < T; t0 += NT) {
+        for (int t0 = w * WAVE; t0 < (PACK && !publisher ? first : T); t0 += NT) {
             const int t = t0 + lane, at = t * K;
             const uint64_t earlier = __ballot(t < first);
             if (PACK) {
