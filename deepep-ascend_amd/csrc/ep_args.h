@@ -18,6 +18,7 @@
 #define EP_LAYOUT_FOLDED 1
 #define EP_LAYOUT_SINGLE 2
 #define EP_LAYOUT_RECOUNTED 3     // no kernel in front: every workgroup counts the ids of all (few) blocks itself
+#define EP_BITS_TOPK 8            // ep_layout_*_bits: most selections of a token (1024 entries a block)
 #define EP_RECOUNT_DEPTH 32       // ids a thread of the slot assignment holds in flight for that (blocks x top-k <= 2 x this)
 
 // Instances of the slot assignment: one partition; of several, the send side (dst_buffer_slot_idx, dst_gsge_idx, the peers'
@@ -163,7 +164,7 @@ struct EpScatterArgs {
 // A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES (token, slot) entries in one launch, or the receive
 // side of a node that ships ranks: every workgroup works the layout out for itself.
 #define EP_SMALL_ENTRIES 1024
-#define EP_SMALL_MASK_EXPERTS 1024    // ep_dispatch_small_*: up to here a bit a token and expert is kept in LDS (16 bytes an expert)
+#define EP_SMALL_MASK_EXPERTS 1024    // ep_dispatch_small_*, ep_layout_assign_bits: up to here a bit a token and expert is kept in LDS (16 bytes an expert)
 struct EpSmallArgs {
     EpLayoutArgs l;               // what ep_layout_assign (ep_recv_copy: ep_layout_place) would have been given
     EpScatterArgs s;              // what the copy kernel would have been given

@@ -7,6 +7,7 @@
 //       partitions once on the send side (slots in the destinations' regions) and, where the send sides
 //       ship no ranks, once on the receive side (slots of the rows that arrived).  Two launches up to a few hundred workgroups (the
 //       assignment sums the histograms of the workgroups before it itself), three beyond.
+//   ep_layout_count_bits / ep_layout_assign_bits           the same two launches for one partition, up to top-8
 //   ep_layout_place                                        receive side of a node out of the shipped counts and ranks
 //   ep_scatter_copy / ep_scatter_quant                     token (or receive-stream row) -> its expanded slots
 //   ep_scatter_copy_pack / ep_scatter_quant_pack           token -> one packed row per destination partition
@@ -1388,6 +1389,217 @@ __device__ __forceinline__ void publish_dispatch(const EpLayoutArgs& l, int gran
         } else if (tid == 0) {
             host_store(&l.host_page[0], l.seq);
         }
+    }
+}
+
+// A block's entries that have an expert, a bit each: those of the token whose first entry is `at`.
+__device__ __forceinline__ unsigned entry_marks(const uint64_t* s_mark, int at, int K) {
+    const uint64_t lo = s_mark[at >> 6] >> (at & 63), hi = (at & 63) ? s_mark[(at >> 6) + 1] << (64 - (at & 63)) : 0ull;
+    return (unsigned)(lo | hi) & ((1u << K) - 1u);
+}
+
+// ------------------------------------------------------------------------------------------------
+// The histograms in front of ep_layout_assign_bits: what ep_layout_count leaves for EP_LAYOUT_FOLDED, of one partition and up to top-8: a
+// token is received where one of its entries has an expert, which a bit an entry tells without a look at its neighbours.
+// Bound by the launch and the trip for the ids.  us of a layout (both launches, several in a captured graph) of 256 experts behind ep_layout_count
+// and this one: 4096 tokens top-8 11.7 / 10.7, top-4 10.4 / 9.9, 16384 top-4 11.2 / 10.6, 32768 top-2 14.0 / 13.7.
+// ------------------------------------------------------------------------------------------------
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_count_bits(EpLayoutArgs a) {
+    fetch_arguments<EpLayoutArgs>();
+    extern __shared__ int smem[];
+    constexpr int NT = EP_LAYOUT_THREADS, PER = EP_TOKENS_PER_BLOCK * EP_BITS_TOPK / NT;
+    const int E = a.num_experts, K = a.num_topk, n = EP_TOKENS_PER_BLOCK * K, W = a.cnt_stride, tid = threadIdx.x, lane = lane_id();
+    int* s_cnt = smem;                                  // [W]
+    uint64_t* s_mark = (uint64_t*)(s_cnt + W);          // [n / 64 + 1] entries with an expert, a bit each
+    const int64_t base = (int64_t)blockIdx.x * n, total = (int64_t)a.num_tokens * K;
+    int64_t id[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) id[u] = a.topk_idx[min(base + tid + u * NT, total - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    for (int i = tid; i < W; i += NT) s_cnt[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * NT;
+        const bool valid = i < n && base + i < total && id[u] >= 0 && id[u] < E;
+        const uint64_t bits = __ballot(valid);
+        if (lane == 0 && i < n) s_mark[i >> 6] = bits;
+        if (valid) atomicAdd(&s_cnt[(int)id[u]], 1);
+    }
+    __syncthreads();
+    const int rows = __popcll(__ballot(entry_marks(s_mark, lane * K, K) != 0u)) + __popcll(__ballot(entry_marks(s_mark, (lane + WAVE) * K, K) != 0u));
+    auto count_of = [&](int c) -> unsigned { return c < E ? (unsigned)s_cnt[c] : c == E ? (unsigned)rows : 0u; };
+    unsigned* row = (unsigned*)a.blk_cnt + (int64_t)blockIdx.x * (W >> 1);
+    for (int i = tid; i < (W >> 1); i += NT) row[i] = count_of(2 * i) | count_of(2 * i + 1) << 16;
+}
+
+// ------------------------------------------------------------------------------------------------
+// The slot assignment of one partition behind ep_layout_count, up to top-8 and EP_SMALL_MASK_EXPERTS experts: what
+// ep_layout_assign_fold does, with ranks from bit masks.  A block's ids leave a bit a token and expert in LDS, and an entry's rank is
+// the number of bits below its token (a token that selects an expert twice leaves one bit and an entry in a list that is looked
+// through where there is one); the last valid position of a token and the tokens with one come from a bit an entry.  Neither counts per
+// wave nor rounds of match-any, and two barriers: one behind the clearing of the LDS, one behind bits and sums of the count rows.
+// Each wave makes the scan over the experts alone.
+// Bound by the launch and its trips to memory (ids and count rows, asked for together).  us of a layout (both launches, several in a
+// captured graph), ep_layout_count + ep_layout_assign_fold / ep_layout_count_bits + this one: 256 experts, 2048 tokens top-8 14.6 / 10.6, 4096
+// top-8 14.6 / 10.7, top-6 13.4 / 10.2, 8192 top-4 12.1 / 10.0, 16384 top-2 11.4 / 10.3; 64 experts 4096 top-8 14.2 / 10.7, 32768 top-2
+// 11.0 / 10.9.  (Every workgroup counting all ids in one launch, as ep_dispatch_chunk_* does: 1024 top-8 7.8, 2048 9.6, 4096 13.1, 8192 top-4
+// 13.7: better only where that launch copies as well.)
+// ------------------------------------------------------------------------------------------------
+extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_bits(EpLayoutArgs a) {
+    fetch_arguments<EpLayoutArgs>();
+    extern __shared__ int smem[];
+    constexpr int NT = EP_LAYOUT_THREADS, PER = EP_TOKENS_PER_BLOCK * EP_BITS_TOPK / NT, TW = EP_TOKENS_PER_BLOCK / 32;
+    const int E = a.num_experts, K = a.num_topk, A = a.expert_alignment, b = blockIdx.x, nb = a.num_blocks;
+    const bool publisher = b == nb;
+    const int n = EP_TOKENS_PER_BLOCK * K, W = a.cnt_stride, FG = W >> 3;      // W: the experts, the partition, up to 8 columns
+    u32x4* s_mask = (u32x4*)smem;                       // [E] tokens of the block that selected an expert, a bit each
+    int* s_pre = (int*)(s_mask + E);                    // [W] entries in the blocks before, columns rotated as below
+    int* s_tot = s_pre + W;                             // [W] entries in all blocks
+    int* s_start = s_tot + W;                           // [W] first slot of an expert
+    uint64_t* s_mark = (uint64_t*)(s_start + W);        // [n / 64 + 1] entries with an expert, a bit each
+    int* s_extra = (int*)(s_mark + EP_TOKENS_PER_BLOCK * EP_BITS_TOPK / WAVE + 1);     // [1] entries in
+    unsigned* s_list = (unsigned*)(s_extra + 2);        // [n] (token, expert) pairs met once more
+    short* s_key = (short*)(s_list + EP_TOKENS_PER_BLOCK * EP_BITS_TOPK);              // [n] expert of an entry, -1: none
+    const int tid = threadIdx.x, lane = lane_id();
+
+    // ---- ids first, count rows behind them: a thread takes 8 adjacent columns of every S-th row (see ep_layout_assign_fold) ----
+    const int64_t base = (int64_t)min(b, nb - 1) * n, total = (int64_t)a.num_tokens * K;
+    int64_t id[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) id[u] = a.topk_idx[min(base + tid + u * NT, total - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+    const int S = FG >= NT ? 1 : NT / FG, s0 = FG >= NT ? 0 : tid / FG, g0 = FG >= NT ? tid : tid - s0 * FG;
+    const unsigned row_bytes = (unsigned)W * 2u, step = (unsigned)S * row_bytes;
+    u32x4 v[EP_FOLD_DEPTH];
+    auto fold_loads = [&](int r) {
+        const unsigned off = (unsigned)r * row_bytes + 16u * min(g0, FG - 1), last = (unsigned)(nb - 1) * row_bytes + 16u * min(g0, FG - 1);
+#pragma unroll
+        for (int u = 0; u < EP_FOLD_DEPTH; ++u) v[u] = *(const u32x4*)((const char*)a.blk_cnt + min(off + u * step, last));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    fold_loads(s0);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    for (int i = tid; i < E + (W >> 1); i += NT) s_mask[i] = zero;      // masks and both rows of sums
+    if (tid == 0) *s_extra = 0;
+    __syncthreads();
+
+    // ---- a bit a token and expert, a bit an entry ----
+    const float per_token = 1.0f / (float)K;            // (as in the one-launch kernels: exact for these quotients)
+    int tok[PER], key[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * NT;
+        const bool valid = i < n && base + i < total && id[u] >= 0 && id[u] < E;
+        tok[u] = (int)(((float)i + 0.5f) * per_token);
+        key[u] = valid ? (int)id[u] : -1;
+        const uint64_t bits = __ballot(valid);
+        if (lane == 0 && i < n) s_mark[i >> 6] = bits;
+        if (i < n) s_key[i] = (short)key[u];
+        if (valid && !publisher) {
+            const unsigned bit = 1u << (tok[u] & 31);
+            if (atomicOr((unsigned*)&s_mask[key[u]] + (tok[u] >> 5), bit) & bit) s_list[atomicAdd(s_extra, 1)] = (unsigned)(tok[u] << 16 | key[u]);
+        }
+    }
+    // ---- sums of the count rows: blocks before this one, and all ----
+    if (s0 < S && g0 < FG) {
+        int p[8], t[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) p[q] = t[q] = 0;
+        for (int r = s0;;) {
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {               // (11 rows of at most 128 top-k entries stay below 2^16)
+                if (h == 1 && r + (EP_FOLD_DEPTH / 2) * S >= nb) break;
+                u16x2 ts[4], ps[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) ts[q] = ps[q] = u16x2{0, 0};
+#pragma unroll
+                for (int u = h * (EP_FOLD_DEPTH / 2); u < (h + 1) * (EP_FOLD_DEPTH / 2); ++u) {
+                    const int rr = r + u * S;
+                    const unsigned mt = rr < nb ? ~0u : 0u, mp = rr < min(b, nb) ? ~0u : 0u;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        ts[q] += __builtin_bit_cast(u16x2, v[u][q] & mt);
+                        ps[q] += __builtin_bit_cast(u16x2, v[u][q] & mp);
+                    }
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    t[2 * q] += (int)ts[q].x;
+                    t[2 * q + 1] += (int)ts[q].y;
+                    p[2 * q] += (int)ps[q].x;
+                    p[2 * q + 1] += (int)ps[q].y;
+                }
+            }
+            r += EP_FOLD_DEPTH * S;
+            if (r >= nb) break;
+            fold_loads(r);
+        }
+        // (the lanes of an add are 8 columns apart: column 8 g + q lives at 8 g + ((q + g / 4) & 7), which spreads them over the banks)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int at = 8 * g0 + ((q + (g0 >> 2)) & 7);
+            atomicAdd(&s_pre[at], p[q]);
+            atomicAdd(&s_tot[at], t[q]);
+        }
+    }
+    __syncthreads();
+    auto at_of = [](int c) { return (c & ~7) | ((c + (c >> 5)) & 7); };
+
+    // ---- aligned exclusive scan over the experts, eight a lane ----
+    const bool pow2 = (A & (A - 1)) == 0;
+    int grand = 0;
+    for (int e0 = 0; e0 < E; e0 += 8 * WAVE) {
+        const int e = e0 + 8 * lane;
+        int before[8], sum = 0;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const int x = e + q < E ? s_tot[at_of(e + q)] : 0;
+            before[q] = sum;
+            sum += pow2 ? (x + A - 1) & -A : align_up(x, A);
+        }
+        const int incl = wave_inclusive_sum(sum), run = grand + incl - sum;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            if (e + q < E) s_start[e + q] = run + before[q];
+        grand += readlane(incl, WAVE - 1);
+    }
+    __builtin_amdgcn_wave_barrier();                    // (the LDS operations of a wave complete in order)
+    if (publisher) {
+        publish_dispatch<false>(a, grand, [&](int e) { return s_tot[at_of(e)]; }, s_start, [&](int) { return s_tot[at_of(E)]; });
+        return;
+    }
+    // ---- tokens with an expert, a bit each (a wave has 128 tokens in two ballots) ----
+    auto marks_of = [&](int t) { return entry_marks(s_mark, t * K, K); };
+    const uint64_t any_lo = __ballot(marks_of(lane) != 0u), any_hi = __ballot(marks_of(lane + WAVE) != 0u);
+    const int rows_before = s_pre[at_of(E)], extras = *s_extra;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = tid + u * NT, t = tok[u], e = key[u];
+        if (i >= n || base + i >= total) continue;
+        const int pos = i - t * K;
+        int slot = -1, rslot = -1;
+        if (e >= 0) {
+            const u32x4 m = s_mask[e];
+            int rank = 0;
+#pragma unroll
+            for (int q = 0; q < TW; ++q) {
+                const int bits = min(max(t - 32 * q, 0), 32);
+                rank += __popc(m[q] & (bits == 32 ? ~0u : (1u << bits) - 1u));
+            }
+            if (extras > 0) {
+                for (int x = 0; x < extras; ++x) rank += (int)(s_list[x] & 0xffffu) == e && (int)(s_list[x] >> 16) < t ? 1 : 0;
+                for (int j = 0; j < pos; ++j) rank += s_key[t * K + j] == e ? 1 : 0;
+            }
+            slot = s_start[e] + s_pre[at_of(e)] + rank;
+            if ((marks_of(t) >> pos) == 1u)             // the last one of its token
+                rslot = rows_before + (t < WAVE ? __popcll(any_lo & ((1ull << t) - 1ull))
+                                                : __popcll(any_lo) + __popcll(any_hi & ((1ull << (t - WAVE)) - 1ull)));
+        }
+        a.dst_buffer_slot_idx[base + i] = rslot;
+        a.dst_gsge_idx[base + i] = -1;                  // every copy is local: no transport descriptors
+        a.slot_map[base + i] = slot;
+        if (rslot >= 0) a.tok_row[b * EP_TOKENS_PER_BLOCK + t] = rslot;
     }
 }
 

@@ -117,6 +117,7 @@ struct Kernels {
     hipFunction_t scatter_copy_pack, scatter_quant_pack, scatter_quant_sw_pack;
     hipFunction_t small[2][3];       // [packs][copy, quant, quant_sw]
     hipFunction_t chunk[2][3];
+    hipFunction_t layout_count_bits, layout_assign_bits;        // one partition, up to top-8: instead of layout_count and layout_assign
     hipFunction_t recv_copy;
     hipFunction_t combine[3][5];     // [mode][generic, k2, k4, k6, k8]
     hipFunction_t combine_odd[3];    // single partition, small launches: k3, k5, k7
@@ -187,6 +188,8 @@ void load_kernels(const char* dir) {
     auto get = [&](hipFunction_t& fn, const char* name) { HIP_CHECK(hipModuleGetFunction(&fn, m, name)); };
     get(g_k.layout_count, "ep_layout_count");
     get(g_k.layout_scan, "ep_layout_scan");
+    get(g_k.layout_count_bits, "ep_layout_count_bits");
+    get(g_k.layout_assign_bits, "ep_layout_assign_bits");
     get(g_k.layout_place, "ep_layout_place");
     const char* sides[3] = {"", "_send", "_recv"};      // EP_LAYOUT_SIDE_*
     for (int side = 0; side < 3; ++side) {
@@ -354,16 +357,31 @@ unsigned layout_assign_lds(int E, int R, int K, int count_experts, int cnt_strid
     return (unsigned)(count_experts + R + nw * (E + R) + nw + 1 + R + nw + 2 * cnt_stride) * sizeof(int) + layout_key_bytes(K);
 }
 
+unsigned layout_count_bits_lds(int cnt_stride) { return 4u * (unsigned)cnt_stride + 8u * (EP_TOKENS_PER_BLOCK * EP_BITS_TOPK / 64 + 1); }
+unsigned layout_assign_bits_lds(int E, int cnt_stride) {
+    constexpr unsigned entries = EP_TOKENS_PER_BLOCK * EP_BITS_TOPK;
+    return 16u * (unsigned)E + 12u * (unsigned)cnt_stride + 8u * (entries / 64 + 1) + 8u + 4u * entries + 2u * entries;
+}
+
+// Up to here one partition ranks in bit masks, behind histograms of its own: never the slower of the two forms (figures at the kernel;
+// beyond top-8 a thread would hold more than four ids, and the masks of more experts leave a CU too few workgroups).
+bool bits_layout(int K, int E) { return K <= EP_BITS_TOPK and E <= EP_SMALL_MASK_EXPERTS; }
+
 // Where one launch that counts the ids of all blocks in every workgroup beats a histogram launch in front of the slot
 // assignment.  It saves a launch; each further block is more ids to every workgroup, and one more of these.  us of a replayed
 // dispatch of 16 channels, 256 experts, two launches / one: top-1, 16 blocks 12.8 / 11.6, 24 12.9 / 13.9, 64 14.4 / 21.9; top-2,
 // 12 13.0 / 12.5, 16 13.0 / 13.1, 32 13.6 / 17.8; top-3, 10 14.4 / 13.4, 16 14.6 / 15.6; top-4, 8 14.5 / 13.3, 16 14.8 / 17.0; top-6, 8
 // 16.1 / 15.7, 10 16.3 / 17.3; top-8, 6 17.5 / 16.7, 8 17.6 / 18.3; top-12, 4 21.1 / 18.9; top-32, 2 37.3 / 31.5.  To a host that waits for
 // the counts the saved launch is worth more (wall clock, 8 blocks, top-7 24.3 / 23.7, top-8 25.3 / 25.0).
-bool recount_pays(int num_blocks, int K, bool host_waits) {
+// Against the two launches that rank in bit masks the line lies lower where no host waits, and stays where one does.  us, two
+// launches / one, 256 experts: top-1, 16 blocks 9.4 / 8.9; top-2, 8 9.3 / 8.2, 16 9.4 / 10.3; top-4, 4 9.7 / 8.8, 6 9.8 / 10.1; top-8, 2 10.3 / 10.5,
+// 3 10.1 / 11.8; 32 experts top-4, 4 10.0 / 8.1, 6 10.2 / 9.5; 1024 experts 10.7 / 10.3, 10.8 / 11.6.  Wall clock of a dispatch of exact
+// sizes: top-2, 12 blocks 27.5 / 26.0; top-4, 12 27.5 / 27.3; top-8, 4 27.1 / 25.7, 6 27.4 / 27.0.
+bool recount_pays(int num_blocks, int K, int E, bool host_waits) {
     const int most = 2 * EP_RECOUNT_DEPTH;
-    const int limit = K > 8 ? most : std::min(8 * K, host_waits ? most : 48);
-    return num_blocks <= 16 and num_blocks * K <= std::max(limit, 32);
+    const int limit = bits_layout(K, E) ? (host_waits ? 48 : 16)
+                                        : std::max(K > 8 ? most : std::min(8 * K, host_waits ? most : 48), 32);
+    return num_blocks <= 16 and num_blocks * K <= limit;
 }
 
 // The layout pass: per-block histograms, then the slot assignment.  One block needs no histogram pass; up
@@ -383,7 +401,7 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
     const int side = la.recv_mode ? EP_LAYOUT_SIDE_RECV : R > 1 ? EP_LAYOUT_SIDE_SEND : EP_LAYOUT_SIDE_SINGLE;
     const int limit = g_recount_limit.load();
     const bool recount = side == EP_LAYOUT_SIDE_SINGLE and num_blocks >= 2 and
-                         (limit < 0 ? recount_pays(num_blocks, K, la.notify_host != 0) : num_blocks <= std::min(limit, 2 * EP_RECOUNT_DEPTH) / K) and
+                         (limit < 0 ? recount_pays(num_blocks, K, E, la.notify_host != 0) : num_blocks <= std::min(limit, 2 * EP_RECOUNT_DEPTH) / K) and
                          layout_assign_lds(E, R, K, C, 0) + recount_extra <= 64 * 1024;
     la.scan_mode = num_blocks == 1 ? EP_LAYOUT_SINGLE
                    : recount       ? EP_LAYOUT_RECOUNTED
@@ -392,6 +410,11 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
     const unsigned smem_assign = layout_assign_lds(E, R, K, C, la.scan_mode == EP_LAYOUT_FOLDED ? la.cnt_stride : 0) +
                                  (la.scan_mode == EP_LAYOUT_RECOUNTED ? recount_extra : 0u);
     EP_HOST_ASSERT(smem_assign <= 64 * 1024);
+    if (la.scan_mode == EP_LAYOUT_FOLDED and side == EP_LAYOUT_SIDE_SINGLE and bits_layout(K, E)) {
+        launch(g_k.layout_count_bits, num_blocks, EP_LAYOUT_THREADS, layout_count_bits_lds(la.cnt_stride), stream, la);
+        launch(g_k.layout_assign_bits, (unsigned)num_blocks + 1u, EP_LAYOUT_THREADS, layout_assign_bits_lds(E, la.cnt_stride), stream, la);
+        return;
+    }
     if (la.scan_mode == EP_LAYOUT_FOLDED or la.scan_mode == EP_LAYOUT_SCANNED)
         launch(g_k.layout_count, num_blocks, EP_LAYOUT_THREADS, layout_count_lds(E, R, K), stream, la);
     if (la.scan_mode == EP_LAYOUT_SCANNED)

@@ -206,6 +206,39 @@ def test_ids_of_all_blocks_counted_in_place(T, E, K):
     buf.destroy()
 
 
+@pytest.mark.parametrize('T,E,K,how', [(2049, 9, 7, ''), (1153, 256, 8, ''), (3001, 1024, 8, ''), (20001, 8, 1, ''), (4224, 130, 3, ''), (2100, 256, 8, 'twice'),
+                                       (1400, 8, 8, 'one'), (2305, 257, 5, 'few'), (3000, 1025, 8, ''), (2200, 64, 9, '')])
+def test_slots_from_bits(T, E, K, how):
+    """The two layout launches of one partition that rank in bit masks (up to top-8 and 1024 experts; the last two cases are beyond), at
+    the edges of blocks, words and groups of experts, in more count rows than one go holds (3001 tokens, 1024 experts), with
+    experts selected twice (every entry on one expert: the longest list), and with most selections missing."""
+    import deep_ep
+    H, A = 16, 4
+    x = make_tokens(T, H, seed=T).to(DEV)
+    topk, _ = make_routing(T, E, K, seed=K, masked=0.95 if how == 'few' else 0.1)
+    if how == 'twice':
+        topk[::3, K - 1] = topk[::3, 0]
+        topk[1::7, 2] = topk[1::7, 1]
+    if how == 'one':
+        topk[:] = 3
+    topk[130] = -1
+    topk[T - 1, :] = E + 1                      # (no such expert)
+    lay = O.rank_share_layout(np.where(topk.numpy() < E, topk.numpy(), -1), E, 1, 0, A, T)
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    try:
+        deep_ep._C.set_layout_recount_limit(0)
+        handle = buf.dispatch(x, topk_idx=topk.to(DEV), num_experts=E, expert_alignment=A, do_expand=True, async_with_compute_stream=True,
+                              defer_epilogue=True).current_stream_wait()[3]
+        torch.cuda.synchronize()
+    finally:
+        deep_ep._C.set_layout_recount_limit(-1)
+    for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
+                 'dst_buffer_slot_idx', 'recv_src_metadata'):
+        assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
+    assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
+    buf.destroy()
+
+
 class AbiDispatch:
     """One BF16 dispatch through the C ABI: descriptors and outputs of the two calls it is made of."""
 
