@@ -299,6 +299,32 @@ def test_layout_paths_agree(T, E, K, R, rank):
         deep_ep._C.set_layout_recount_limit(-1)
 
 
+@pytest.mark.parametrize('wrong', [dict(expert_alignment=0), dict(expert_alignment=-3), dict(num_max_tokens_per_rank=5), dict(num_max_tokens_per_rank=-1),
+                                   dict(num_experts=-8), dict(num_experts=2049)])
+@pytest.mark.parametrize('sync', [False, True])
+def test_arguments_that_no_output_can_be_sized_by_are_refused(wrong, sync):
+    """Outputs that share an allocation are sized ahead of the library's checks: what it refuses is still refused by it, and the
+    buffer serves the next call."""
+    import deep_ep
+    T, H, E, K = 40, 64, 8, 2
+    topk, w = make_routing(T, E, K, seed=5)
+    buf = _buffer(T, H, K)
+    args = dict(topk_idx=topk.to(DEV), topk_weights=w.to(DEV), num_experts=E, expert_alignment=4, num_max_tokens_per_rank=T, do_expand=True,
+                do_cpu_sync=sync)
+    with pytest.raises(deep_ep._C.EPException, match='Assertion'):
+        buf.dispatch(make_tokens(T, H).to(DEV), **dict(args, **wrong))
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, 4, T)
+    _, _, weights, handle, _ = buf.dispatch(make_tokens(T, H).to(DEV), **args)
+    torch.cuda.synchronize()
+    assert np.array_equal(handle.recv_src_metadata.cpu().numpy()[:T], lay['recv_src_metadata'])
+    # the pieces of one allocation: none reaches into another
+    parts = [weights, handle.recv_src_metadata, handle.dst_buffer_slot_idx, handle.dst_gsge_idx, handle.psum_num_recv_tokens_per_rank,
+             handle.psum_num_recv_tokens_per_expert, handle.num_unaligned_recv_tokens_per_expert]
+    spans = sorted((p.data_ptr(), p.data_ptr() + 4 * p.numel()) for p in parts)
+    assert all(p.is_contiguous() for p in parts) and all(a[1] <= b[0] for a, b in zip(spans, spans[1:]))
+    buf.destroy()
+
+
 @pytest.mark.parametrize('fused', [False, True])
 def test_exact_sync_sizes_allocate_what_the_results_show(fused):
     """A host-synchronised dispatch returns views of bound-sized storage by default; with `set_exact_sync_sizes()` the
