@@ -2751,7 +2751,7 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
 EP_COMBINE_KERNELS(, EP_COMBINE_FUSED)
 EP_COMBINE_KERNELS(_partial, EP_COMBINE_PARTIAL)
 EP_COMBINE_KERNELS(_final, EP_COMBINE_FINAL)
-// odd top-k, launches of the single partition that wait for one trip to memory and not for its bandwidth: all rows in one
+// odd top-k, the smallest and the largest launches of the single partition (the host has the lines): all rows in one
 // trip instead of one trip a row (61 tokens x 5120, flushed: top-3 8.0 -> 7.3 us, top-5 9.2 -> 7.6, top-7 10.7 -> 8.2)
 extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine_k3(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<3, EP_COMBINE_FUSED>(a); }
 extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine_k5(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<5, EP_COMBINE_FUSED>(a); }

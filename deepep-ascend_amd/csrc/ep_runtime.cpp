@@ -139,7 +139,9 @@ std::atomic<bool> g_fp8_hw{true};
 // The two-phase kernels of the partitioned path do not react to it.
 std::atomic<int> g_combine_blocks_per_cu{-1};
 constexpr unsigned kLdsBytesPerCu = 160 * 1024;
-unsigned combine_lds_cap(int num_topk, bool specialised, int num_row_blocks, int hidden) {     // num_topk: rows a wave fetches, biases included
+// The unrolled kernels of odd top-k at 3/4/5/6 and uncapped: top-3 - 158 153 153 153, top-5 233 234 241 244 -, at 8192 tokens 123 119 120 122 -;
+// top-7 314 329 335 - -, of 2560 channels at 8192 tokens 62.1 60.6 60.8 - -.
+unsigned combine_lds_cap(int num_topk, bool specialised, bool odd, int num_row_blocks, int hidden) {     // num_topk: rows a wave fetches, biases included
     int n = g_combine_blocks_per_cu;
     if (n < 0) {
         // a launch that fills the machine less than about twice over wants every wave it can get
@@ -148,6 +150,7 @@ unsigned combine_lds_cap(int num_topk, bool specialised, int num_row_blocks, int
         // cap wins)
         if (num_row_blocks < 4096 or hidden < 2048) n = 0;
         else if (specialised) n = num_topk <= 2 ? 0 : num_topk <= 4 ? 4 : 3;
+        else if (odd) n = num_topk <= 3 ? 6 : num_topk <= 5 or hidden < 4096 ? 4 : 3;
         else n = num_topk <= 2 ? 0 : num_topk == 3 ? 6 : num_topk <= 5 ? 5 : 4;
     }
     // a workgroup can ask for 64 KiB at most, which lets two of them into a CU: a cap of one cannot be enforced this
@@ -1635,12 +1638,14 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROWS_PER_BLOCK);
             const unsigned grid = (unsigned)ca.num_row_blocks + (unsigned)ceil_div(num_combined_tokens, EP_ROW_THREADS);
             if (grid == 0) return;
-            // odd top-k: a launch of less than a row block a CU waits for its trips to memory and takes the unrolled kernel;
-            // at 765 blocks the two are level (top-3 / 5 / 7: 9.5 / 11.2 / 13.0 us against 9.6 / 11.3 / 13.1 of the general
-            // one), beyond, the general one's shorter bursts win (1787 blocks: 14.9 / 19.7 / 23.8 us against 16.5 / 20.4 / 25.0)
+            // odd top-k: a launch of few row blocks a CU waits for its trips to memory and takes the unrolled kernel, and so does one that fills
+            // the chip several times over; between the two the general one's shorter bursts win.  us, general / unrolled, four outputs in
+            // turn, top-3 / 5 / 7: 384 blocks 6.5 / 6.1, 8.2 / 7.1, 9.9 / 8.4; 766 7.6 / 7.3, 9.5 / 9.0, 11.6 / 11.1; 896 8.7 / 9.0, 10.5 / 10.9, 13.0 /
+            // 13.7; 1787 13.2 / 14.0, 18.4 / 18.8, 22.8 / 23.5; 3584 24.1 / 24.3, 33.4 / 33.7, 43.2 / 43.7; 5376 33.3 / 32.9, 50.6 / 47.9, 68.2 / 66.0;
+            // 28672 155 / 153, 233 / 234, 319 / 314; 6144 (2560 channels) 34.3 / 32.3, 49.6 / 45.6, 67.6 / 60.6
             ca.paced = ca.num_row_blocks >= kPacedRowBlocks ? 1 : 0;
-            const bool odd = ca.num_row_blocks < 256 and (K == 3 or K == 5 or K == 7);
-            const unsigned cap = combine_lds_cap(K + (ca.bias_0 != nullptr) + (ca.bias_1 != nullptr), kidx != 0, ca.num_row_blocks, hidden);
+            const bool odd = (ca.num_row_blocks < 800 or ca.num_row_blocks >= 4096) and (K == 3 or K == 5 or K == 7);
+            const unsigned cap = combine_lds_cap(K + (ca.bias_0 != nullptr) + (ca.bias_1 != nullptr), kidx != 0, odd, ca.num_row_blocks, hidden);
             launch(odd ? g_k.combine_odd[(K - 3) / 2] : g_k.combine[EP_COMBINE_FUSED][kidx], grid, EP_ROW_THREADS, cap, a.stream, ca);
         } else {
             check_peers(b, [&](const ep_buffer& p) { return p.num_partials >= b->num_partials; },

@@ -507,3 +507,41 @@ def test_top8_combine_on_both_sides_of_the_paced_line(T, nodes):
     torch.cuda.synchronize()
     for b in bufs:
         b.destroy()
+
+
+@pytest.mark.parametrize('K', [3, 5, 7])
+@pytest.mark.parametrize('T,bias', [(3196, 0), (3200, 1), (16380, 1), (16384, 0), (16387, 2)])
+def test_odd_topk_combine_on_both_sides_of_its_lines(T, bias, K):
+    """799, 800, 4095, 4096 and 4097 row blocks of one part (H = 1000: the second vector of a lane is partly past the end): torch's float32 sums in the same
+    order, rounded once, then once with the biases; weights carried back."""
+    import deep_ep
+    H, E = 1000, 16
+    gen = torch.Generator(device=DEV).manual_seed(T + K)
+    topk = torch.rand((T, E), generator=gen, device=DEV).topk(K, dim=-1).indices
+    topk[torch.rand((T, K), generator=gen, device=DEV) < 0.1] = -1
+    topk[0] = -1
+    w = torch.rand((T, K), generator=gen, device=DEV).masked_fill(topk < 0, 0.0)
+    buf = _buffer(T, H, K)
+    x = torch.randn((T, H), generator=gen, device=DEV, dtype=torch.bfloat16)
+    rows, _, weights, handle, _ = buf.dispatch(x, topk_idx=topk, topk_weights=w, num_experts=E, num_max_tokens_per_rank=T, do_expand=True)
+    y = torch.randn(rows.shape, generator=gen, device=DEV, dtype=torch.bfloat16)
+    biases = [torch.randn((T, H), generator=gen, device=DEV, dtype=torch.bfloat16) for _ in range(bias)]
+    out, out_w, _ = buf.combine(y, handle, topk_weights=weights, bias=None if not bias else biases[0] if bias == 1 else tuple(biases))
+    meta = handle.recv_src_metadata.long()
+    slots = torch.full((T, K), -1, dtype=torch.long, device=DEV)
+    slots[meta[:, K]] = meta[:, :K]
+    assert torch.equal(slots >= 0, topk >= 0)
+    acc, seen = torch.zeros((T, H), device=DEV), torch.zeros((T, 1), dtype=torch.bool, device=DEV)
+    for j in range(K):
+        here = (slots[:, j] >= 0)[:, None]
+        acc = torch.where(here, torch.where(seen, acc + y[slots[:, j].clamp(min=0)].float(), y[slots[:, j].clamp(min=0)].float()), acc)
+        seen |= here
+    want = acc.to(torch.bfloat16)
+    if bias:
+        total = biases[0].float()
+        for b in biases[1:]:
+            total = total + b.float()
+        want = torch.where(seen, (total + want.float()).to(torch.bfloat16), total.to(torch.bfloat16))
+    assert torch.equal(out, want) and torch.equal(out_w, w)
+    torch.cuda.synchronize()
+    buf.destroy()
