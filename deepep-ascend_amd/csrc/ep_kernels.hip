@@ -2741,21 +2741,24 @@ __device__ __forceinline__ void combine_body(const EpCombineArgs& a) {
     }
 }
 
-#define EP_COMBINE_KERNELS(SUFFIX, MODE)                                                                                   \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_generic(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<0, MODE>(a); } \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k2(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<2, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k4(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<4, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k6(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<6, MODE>(a); }     \
-    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##SUFFIX##_k8(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<8, MODE>(a); }
+// Unrolled for top-2 to top-8, and one for any top-k; which of the two a launch takes is the host's rule.  (Odd top-k, all rows in one trip
+// instead of one trip a row: 61 tokens x 5120, flushed, top-3 / 5 / 7 8.0 / 9.2 / 10.7 -> 7.3 / 7.6 / 8.2 us; both reduces of eight partitions
+// of 64 tokens x 7168, top-3 / 5 / 7 81.8 / 104 / 125 -> 70.7 / 75.8 / 85.8.)
+#define EP_COMBINE_KERNEL(NAME, KT, MODE) \
+    extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine##NAME(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<KT, MODE>(a); }
+#define EP_COMBINE_KERNELS(SUFFIX, MODE)           \
+    EP_COMBINE_KERNEL(SUFFIX##_generic, 0, MODE)   \
+    EP_COMBINE_KERNEL(SUFFIX##_k2, 2, MODE)        \
+    EP_COMBINE_KERNEL(SUFFIX##_k3, 3, MODE)        \
+    EP_COMBINE_KERNEL(SUFFIX##_k4, 4, MODE)        \
+    EP_COMBINE_KERNEL(SUFFIX##_k5, 5, MODE)        \
+    EP_COMBINE_KERNEL(SUFFIX##_k6, 6, MODE)        \
+    EP_COMBINE_KERNEL(SUFFIX##_k7, 7, MODE)        \
+    EP_COMBINE_KERNEL(SUFFIX##_k8, 8, MODE)
 
 EP_COMBINE_KERNELS(, EP_COMBINE_FUSED)
 EP_COMBINE_KERNELS(_partial, EP_COMBINE_PARTIAL)
 EP_COMBINE_KERNELS(_final, EP_COMBINE_FINAL)
-// odd top-k, the smallest and the largest launches of the single partition (the host has the lines): all rows in one
-// trip instead of one trip a row (61 tokens x 5120, flushed: top-3 8.0 -> 7.3 us, top-5 9.2 -> 7.6, top-7 10.7 -> 8.2)
-extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine_k3(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<3, EP_COMBINE_FUSED>(a); }
-extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine_k5(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<5, EP_COMBINE_FUSED>(a); }
-extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_combine_k7(EpCombineArgs a) { fetch_arguments<EpCombineArgs>(); combine_body<7, EP_COMBINE_FUSED>(a); }
 
 // ------------------------------------------------------------------------------------------------
 // Self-test: hardware e4m3fn conversion against the integer conversion over a range of fp32 bit

@@ -119,8 +119,7 @@ struct Kernels {
     hipFunction_t chunk[2][3];
     hipFunction_t layout_count_bits, layout_assign_bits;        // one partition, up to top-8: instead of layout_count and layout_assign
     hipFunction_t recv_copy;
-    hipFunction_t combine[3][5];     // [mode][generic, k2, k4, k6, k8]
-    hipFunction_t combine_odd[3];    // single partition, small launches: k3, k5, k7
+    hipFunction_t combine[3][8];     // [mode][generic, k2 .. k8]
     hipFunction_t fp8_selftest, quant_rows;
     int device = -1;
 };
@@ -149,8 +148,8 @@ unsigned combine_lds_cap(int num_topk, bool specialised, bool odd, int num_row_b
         // and so do short rows (hidden 512 / 1536, top-8: 113 / 160 us uncapped, 124 / 170 at three; from 2048 on the
         // cap wins)
         if (num_row_blocks < 4096 or hidden < 2048) n = 0;
+        else if (specialised and odd) n = num_topk <= 3 ? 6 : num_topk <= 5 or hidden < 4096 ? 4 : 3;
         else if (specialised) n = num_topk <= 2 ? 0 : num_topk <= 4 ? 4 : 3;
-        else if (odd) n = num_topk <= 3 ? 6 : num_topk <= 5 or hidden < 4096 ? 4 : 3;
         else n = num_topk <= 2 ? 0 : num_topk == 3 ? 6 : num_topk <= 5 ? 5 : 4;
     }
     // a workgroup can ask for 64 KiB at most, which lets two of them into a CU: a cap of one cannot be enforced this
@@ -215,13 +214,10 @@ void load_kernels(const char* dir) {
     get(g_k.recv_copy, "ep_recv_copy");
     get(g_k.sf_transpose, "ep_sf_transpose");
     const char* modes[3] = {"", "_partial", "_final"};
-    const char* ks[5] = {"_generic", "_k2", "_k4", "_k6", "_k8"};
+    const char* ks[8] = {"_generic", "_k2", "_k3", "_k4", "_k5", "_k6", "_k7", "_k8"};
     for (int mode = 0; mode < 3; ++mode)
-        for (int k = 0; k < 5; ++k)
+        for (int k = 0; k < 8; ++k)
             get(g_k.combine[mode][k], (std::string("ep_combine") + modes[mode] + ks[k]).c_str());
-    get(g_k.combine_odd[0], "ep_combine_k3");
-    get(g_k.combine_odd[1], "ep_combine_k5");
-    get(g_k.combine_odd[2], "ep_combine_k7");
     get(g_k.fp8_selftest, "ep_fp8_selftest");
     get(g_k.quant_rows, "ep_quant_rows");
     g_k.module = m;
@@ -1566,7 +1562,7 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
         EP_HOST_ASSERT(combine_buffer_size(R, a.num_max_tokens_per_rank, hidden, K) <= b->num_buffer_bytes);
         EP_HOST_ASSERT(phase == 0 or phase == 1);
         EP_HOST_ASSERT(not a.apply_weights or R == 1);
-        const int kidx = K == 2 ? 1 : K == 4 ? 2 : K == 6 ? 3 : K == 8 ? 4 : 0;
+        const int unrolled = K >= 2 and K <= 8 ? K - 1 : 0;      // (0: the kernel for any top-k)
         const int64_t combine_token = token_bytes(hidden * 2, 0, K, false);
 
         EpCombineArgs ca{};
@@ -1610,8 +1606,10 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
                 ca.num_parts = (int)std::max<int64_t>(1, ceil_div(hidden, EP_COMBINE_LONG_PART));
             }
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROWS_PER_BLOCK);
+            // (odd top-k, kernel for any / unrolled, both reduces: eight of 64 tokens x 7168 top-3 / 7 81.8 / 76.4, 125 / 121, with the token side 70.7,
+            // 85.8; two of 1024 top-7 75.1 / 71.4, top-3 51.2 / 51.9)
             if (ca.num_row_blocks > 0)
-                launch(g_k.combine[EP_COMBINE_PARTIAL][kidx], (unsigned)ca.num_row_blocks, EP_ROW_THREADS, 0, a.stream, ca, &done);
+                launch(g_k.combine[EP_COMBINE_PARTIAL][unrolled], (unsigned)ca.num_row_blocks, EP_ROW_THREADS, 0, a.stream, ca, &done);
             return done.record();
         }
 
@@ -1644,9 +1642,10 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
             // 13.7; 1787 13.2 / 14.0, 18.4 / 18.8, 22.8 / 23.5; 3584 24.1 / 24.3, 33.4 / 33.7, 43.2 / 43.7; 5376 33.3 / 32.9, 50.6 / 47.9, 68.2 / 66.0;
             // 28672 155 / 153, 233 / 234, 319 / 314; 6144 (2560 channels) 34.3 / 32.3, 49.6 / 45.6, 67.6 / 60.6
             ca.paced = ca.num_row_blocks >= kPacedRowBlocks ? 1 : 0;
-            const bool odd = (ca.num_row_blocks < 800 or ca.num_row_blocks >= 4096) and (K == 3 or K == 5 or K == 7);
+            const bool odd = unrolled != 0 and K % 2 != 0;
+            const int kidx = odd and ca.num_row_blocks >= 800 and ca.num_row_blocks < 4096 ? 0 : unrolled;
             const unsigned cap = combine_lds_cap(K + (ca.bias_0 != nullptr) + (ca.bias_1 != nullptr), kidx != 0, odd, ca.num_row_blocks, hidden);
-            launch(odd ? g_k.combine_odd[(K - 3) / 2] : g_k.combine[EP_COMBINE_FUSED][kidx], grid, EP_ROW_THREADS, cap, a.stream, ca);
+            launch(g_k.combine[EP_COMBINE_FUSED][kidx], grid, EP_ROW_THREADS, cap, a.stream, ca);
         } else {
             check_peers(b, [&](const ep_buffer& p) { return p.num_partials >= b->num_partials; },
                         "its owner-side reduce (phase 0) comes before any token-side reduce");
@@ -1659,7 +1658,14 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROW_THREADS / 64);
             if (ca.num_row_blocks == 0) return;
             ca.paced = ca.num_row_blocks >= kPacedRowBlocks ? 1 : 0;
-            launch(g_k.combine[EP_COMBINE_FINAL][kidx], (unsigned)ca.num_row_blocks, EP_ROW_THREADS, 0, a.stream, ca);
+            // The unrolled kernels fetch a row for every position, a master's again where a position is none: most of them with few
+            // partitions.  Launches that have more than a trip to wait for take the kernel that goes master by master there, and for
+            // top-2 and 3, where it has the more waves.  us of both reduces of all partitions (7168 channels, captured), unrolled / that: two of 64 /
+            // 256 / 1024 / 2048 tokens top-8 21.3 / 21.2, 32.6 / 31.3, 90.5 / 79.3, 164 / 143, of 256 top-4 24.5 / 24.0, top-2 21.1 / 21.4; four of 256
+            // / 512 / 2048 top-8 77.1 / 79.6, 122 / 117, 379 / 358, of 512 top-4 87.6 / 87.0, of 2048 258 / 258; eight of 256 / 800 / 2048 top-3 101.5 /
+            // 105.9, 228 / 210, 476 / 463, top-6 146 / 163, 346 / 348, a pass of them with a host sync 1234 / 1243.
+            const bool master_by_master = ca.num_row_blocks >= (R == 2 ? 448 : 896) and (R <= 4 ? K > 2 : K <= 3);
+            launch(g_k.combine[EP_COMBINE_FINAL][master_by_master ? 0 : unrolled], (unsigned)ca.num_row_blocks, EP_ROW_THREADS, 0, a.stream, ca);
         }
     });
 }

@@ -475,11 +475,22 @@ def test_combine_on_non_finite_expert_outputs():
     buf.destroy()
 
 
+@pytest.mark.parametrize('T,nodes,K', [(64, 2, 3), (1788, 2, 8), (1792, 2, 8), (1792, 2, 2), (1793, 2, 5), (3580, 4, 6), (3584, 4, 7), (3584, 4, 2), (3584, 8, 3),
+                                       (3584, 8, 7), (100, 8, 5), (97, 16, 7)])
+def test_reduces_of_a_node_by_partitions_topk_and_size(T, nodes, K):
+    """Owner side and token side at both sides of the lines between their kernels (448 and 896 row blocks of one part)."""
+    _reduce_rows_that_come_back(T, nodes, K)
+
+
 @pytest.mark.parametrize('T,nodes', [(32764, 1), (32768, 1), (32768, 2)])
 def test_top8_combine_on_both_sides_of_the_paced_line(T, nodes):
     """8191 and 8192 row blocks of one 64-channel part: the row sums are those of torch in the same order, bit for bit."""
+    _reduce_rows_that_come_back(T, nodes, 8)
+
+
+def _reduce_rows_that_come_back(T, nodes, K):
     import deep_ep
-    H, E, K = 64, 16, 8
+    H, E = 64, 16
     node = None if nodes == 1 else deep_ep.LocalNode(nodes)
     group = [deep_ep.LocalGroup() if node is None else node.group(r) for r in range(nodes)]
     bufs = [deep_ep.EPBuffer(g, num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True) for g in group]
