@@ -475,22 +475,11 @@ def test_combine_on_non_finite_expert_outputs():
     buf.destroy()
 
 
-@pytest.mark.parametrize('T,nodes,K', [(64, 2, 3), (1788, 2, 8), (1792, 2, 8), (1792, 2, 2), (1793, 2, 5), (3580, 4, 6), (3584, 4, 7), (3584, 4, 2), (3584, 8, 3),
-                                       (3584, 8, 7), (100, 8, 5), (97, 16, 7)])
-def test_reduces_of_a_node_by_partitions_topk_and_size(T, nodes, K):
-    """Owner side and token side at both sides of the lines between their kernels (448 and 896 row blocks of one part)."""
-    _reduce_rows_that_come_back(T, nodes, K)
-
-
 @pytest.mark.parametrize('T,nodes', [(32764, 1), (32768, 1), (32768, 2)])
 def test_top8_combine_on_both_sides_of_the_paced_line(T, nodes):
     """8191 and 8192 row blocks of one 64-channel part: the row sums are those of torch in the same order, bit for bit."""
-    _reduce_rows_that_come_back(T, nodes, 8)
-
-
-def _reduce_rows_that_come_back(T, nodes, K):
     import deep_ep
-    H, E = 64, 16
+    H, E, K = 64, 16, 8
     node = None if nodes == 1 else deep_ep.LocalNode(nodes)
     group = [deep_ep.LocalGroup() if node is None else node.group(r) for r in range(nodes)]
     bufs = [deep_ep.EPBuffer(g, num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True) for g in group]
@@ -515,6 +504,33 @@ def _reduce_rows_that_come_back(T, nodes, K):
             total = part if total is None else total + part
         # (masters in ascending position: with two partitions the sum of two terms does not depend on their order)
         assert torch.equal(out, total.to(torch.bfloat16))
+    torch.cuda.synchronize()
+    for b in bufs:
+        b.destroy()
+
+
+@pytest.mark.parametrize('T,nodes,K', [(64, 2, 3), (1788, 2, 8), (1792, 2, 8), (1792, 2, 2), (1793, 2, 5), (3580, 4, 6), (3584, 4, 7), (3584, 4, 2), (3584, 8, 3),
+                                       (3584, 8, 7), (100, 8, 5), (97, 16, 7)])
+def test_reduces_of_a_node_by_partitions_topk_and_size(T, nodes, K):
+    """Owner side and token side at both sides of the lines between their kernels (448 and 896 row blocks of one part).  A token's row
+    comes back once a selection: a partial is a multiple of it, rounded once, and sums of at most eight of those are exact in float32."""
+    import deep_ep
+    H, E = 64, 16
+    node = deep_ep.LocalNode(nodes)
+    bufs = [deep_ep.EPBuffer(node.group(r), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True) for r in range(nodes)]
+    gen = torch.Generator(device=DEV).manual_seed(T + nodes)
+    topk = [torch.rand((T, E), generator=gen, device=DEV).topk(K, dim=-1).indices for _ in bufs]
+    x = [torch.randn((T, H), generator=gen, device=DEV, dtype=torch.bfloat16) for _ in bufs]
+    w = [torch.rand((T, K), generator=gen, device=DEV) for _ in bufs]
+    kw = dict(async_with_compute_stream=True, defer_epilogue=True)
+    sent = [b.dispatch(v, topk_idx=t, topk_weights=g, num_experts=E, num_max_tokens_per_rank=T, do_expand=True, **kw)
+            for b, v, t, g in zip(bufs, x, topk, w)]
+    got = [e.current_stream_wait() for e in sent]
+    reduced = [b.combine(rows, h, topk_weights=g, **kw) for b, (rows, _, g, h) in zip(bufs, got)]
+    for v, t, g, e in zip(x, topk, w, reduced):
+        out, out_w = e.current_stream_wait()
+        total = sum(((t * nodes // E == r).sum(dim=-1, keepdim=True) * v.float()).to(torch.bfloat16).float() for r in range(nodes))
+        assert torch.equal(out, total.to(torch.bfloat16)) and torch.equal(out_w, g)
     torch.cuda.synchronize()
     for b in bufs:
         b.destroy()
