@@ -144,9 +144,10 @@ at::Tensor view_of(const at::Tensor& base, at::IntArrayRef sizes, at::IntArrayRe
 at::Tensor first_rows(const at::Tensor& t, int64_t rows) {
     return t.dim() == 1 ? view_of(t, {rows}, {1}, 0) : view_of(t, {rows, t.size(1)}, {t.size(1), 1}, 0);
 }
-// 4-byte tensors of one call, out of one allocation (each starts on a multiple of 256 bytes): one of the caching allocator's costs
-// 0.5 us and its release about 0.3, a view 0.1.  A dispatch without a host sync, host time: 61 tokens 11.6 -> 9.8 us, one of eight partitions
-// of 64 tokens 12.9 -> 11.9, its receive side 11.1 -> 10.0; whole passes of a toy layer 25.2 -> 23.9, of 61 tokens 19.8 -> 18.4.
+// Contiguous int32 tensors out of one allocation (each starts on a multiple of 256 bytes): an allocation of the caching allocator's costs
+// 0.5 us and its release about 0.3, a view 0.1.  Host time of the native dispatch with the counts' and slots' three allocations as one: 61 tokens
+// 8.5 -> 7.6 us, one of eight partitions of 64 tokens 8.7 -> 7.9.  (Metadata rows and received weights in it as well: 6.6, and 8.5 -> 7.7 for the
+// receive side; but the weights are the caller's, to save or to free without the handle.)
 class Together {
 public:
     // where the next `n` elements will be
@@ -156,17 +157,15 @@ public:
         return at;
     }
     void allocate(const at::Device& dev) { base_ = alloc({size_}, at::kInt, dev); }
-    at::Tensor ints(int64_t at, at::IntArrayRef sizes) const { return part(at, sizes, at::kInt); }
-    at::Tensor floats(int64_t at, at::IntArrayRef sizes) const { return part(at, sizes, at::kFloat); }
-
-private:
-    at::Tensor part(int64_t at, at::IntArrayRef sizes, at::ScalarType dtype) const {
+    at::Tensor part(int64_t at, at::IntArrayRef sizes) const {
         at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(base_.storage()), base_.key_set(),
-                                                                at::scalarTypeToTypeMeta(dtype));
+                                                                base_.dtype());
         t.unsafeGetTensorImpl()->set_storage_offset(at);
         t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
         return t;
     }
+
+private:
     int64_t size_ = 0;
     at::Tensor base_;
 };
@@ -182,7 +181,6 @@ struct DispatchState {
     OptTensor sf, topk_weights, stats;
     at::Tensor psum_rank, psum_expert, unaligned, dst_slot, dst_gsge;
     OptTensor cached_meta;
-    OptTensor meta, recv_w;     // allocated with the handle tensors, where the copy follows at once
     py::object cached_list;
     int64_t cached_num_recv = 0, cached_num_expanded = 0;
     ep_dispatch_args_t a{};
@@ -192,12 +190,6 @@ struct DispatchState {
     bool cached_mode, do_cpu_sync, do_zero_padding, use_col_major_sf, fused;
     bool exact_sync_sizes = false;
 };
-
-// Rows that T tokens of one partition expand to at most.
-int64_t expanded_bound(int64_t T, int K, int El, int A) {
-    const int64_t rows = T * std::min(K, El) + (int64_t)(A - 1) * El;
-    return (rows + A - 1) / A * A;
-}
 
 py::tuple run_dispatch_epilogue(DispatchState& s) {
     const at::Device dev = s.x.device();
@@ -210,16 +202,7 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
         // receive side: count and rank the rows that arrived in this partition's regions
         int c_recv = 0, c_exp = 0;
         check(ep_dispatch_worst_case_sizes(s.buf, s.num_max_tokens_per_rank, K, s.num_experts, A, &c_recv, &c_exp));
-        if (s.do_cpu_sync) {
-            meta = empty_i32({rows_bound, K + 2}, dev);
-        } else {
-            const bool weights = s.topk_weights.has_value() && s.topk_weights->scalar_type() == at::kFloat;
-            Together t;
-            const int64_t meta_at = t.add((int64_t)c_recv * (K + 2)), weights_at = weights ? t.add(c_exp) : 0;
-            t.allocate(dev);
-            meta = t.ints(meta_at, {c_recv, K + 2});
-            if (weights) s.recv_w = t.floats(weights_at, {c_exp});
-        }
+        meta = empty_i32({s.do_cpu_sync ? rows_bound : (int64_t)c_recv, K + 2}, dev);
         have_meta = true;
         ep_dispatch_recv_args_t r{};
         r.psum_num_recv_tokens_per_rank = s.a.psum_num_recv_tokens_per_rank;
@@ -270,7 +253,8 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
         // layout kernels and the copy.  Allocate for this call's upper bound, enqueue the copy, and read the counts
         // while it runs; the results are narrowed below.
         alloc_recv = T;
-        alloc_expanded = expanded_bound(T, K, El, A);
+        alloc_expanded = (int64_t)T * std::min(K, El) + (int64_t)(A - 1) * El;
+        alloc_expanded = (alloc_expanded + A - 1) / A * A;
         counts_known = false;
     } else {
         int c_recv = 0, c_exp = 0;
@@ -297,14 +281,11 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
             recv_sf = alloc({alloc_expanded, sf_cols}, sf_type, dev);
         }
     }
-    if (s.recv_w.has_value()) recv_w = std::move(s.recv_w);
-    else if (s.topk_weights.has_value()) recv_w = alloc({alloc_expanded}, s.topk_weights->scalar_type(), dev);
+    if (s.topk_weights.has_value()) recv_w = alloc({alloc_expanded}, s.topk_weights->scalar_type(), dev);
     if (s.cached_mode) {
         meta = *s.cached_meta;
         if (meta.dim() != 2 || meta.size(0) != num_recv)
             throw EpPyError("Assertion exception (python_api.cpp): recv_src_metadata.size(0) == num_recv_tokens");
-    } else if (s.meta.has_value()) {
-        meta = *std::move(s.meta);
     } else if (!have_meta) {
         meta = empty_i32({alloc_recv, K + 2}, dev);
     }
@@ -442,7 +423,6 @@ public:
         const at::Device dev = x.device();
         // (the copy follows at once, unless it is deferred or the output sizes are waited for first)
         const bool copy_follows = num_ranks_ == 1 && !defer_epilogue && !(do_cpu_sync && exact_sync_sizes_);
-        const bool weights_here = topk_weights.has_value() && topk_weights->scalar_type() == at::kFloat;
         if (cached_mode) {
             s.psum_rank = *cached_psum_rank;
             s.psum_expert = *cached_psum_expert;
@@ -454,35 +434,18 @@ public:
             s.cached_num_recv = *cached_num_recv_tokens;
             s.cached_num_expanded = *cached_num_expanded_tokens;
         } else {
-            // the handle tensors share one allocation; where the copy follows on the same stream, its metadata rows and weights too
+            // the counts and slots of the handle share one allocation, sized by the arguments' shapes; what has worst-case size or
+            // belongs to the caller alone (metadata rows, received weights) has storage of its own, allocated once the library
+            // has accepted the call
             const int64_t El = std::max(0, s.num_local_experts), TK = (int64_t)s.num_tokens * s.num_topk;
             Together t;
             const int64_t rank_at = t.add(num_ranks_), expert_at = t.add(El), unaligned_at = t.add(El), slot_at = t.add(TK), gsge_at = t.add(TK);
-            int64_t meta_at = 0, weights_at = 0, recv_rows = 0, expanded_rows = 0;
-            // (sizes only out of arguments that make sense: the library refuses the others below)
-            const bool copy_sizes = copy_follows && s.num_topk > 0 && El > 0 && expert_alignment > 0 && s.num_tokens <= num_max_tokens_per_rank;
-            if (copy_sizes) {
-                recv_rows = s.num_tokens;
-                expanded_rows = expanded_bound(s.num_tokens, s.num_topk, (int)El, expert_alignment);
-                if (!do_cpu_sync) {
-                    int c_recv = 0, c_exp = 0;
-                    check(ep_dispatch_worst_case_sizes(buf_, num_max_tokens_per_rank, s.num_topk, num_experts, expert_alignment, &c_recv, &c_exp));
-                    recv_rows = c_recv;
-                    expanded_rows = c_exp;
-                }
-                meta_at = t.add(recv_rows * (s.num_topk + 2));
-                if (weights_here) weights_at = t.add(expanded_rows);
-            }
             t.allocate(dev);
-            s.psum_rank = t.ints(rank_at, {(int64_t)num_ranks_});
-            s.psum_expert = t.ints(expert_at, {El});
-            s.unaligned = t.ints(unaligned_at, {El});
-            s.dst_slot = t.ints(slot_at, {s.num_tokens, s.num_topk});
-            s.dst_gsge = t.ints(gsge_at, {s.num_tokens, s.num_topk});
-            if (copy_sizes) {
-                s.meta = t.ints(meta_at, {recv_rows, s.num_topk + 2});
-                if (weights_here) s.recv_w = t.floats(weights_at, {expanded_rows});
-            }
+            s.psum_rank = t.part(rank_at, {(int64_t)num_ranks_});
+            s.psum_expert = t.part(expert_at, {El});
+            s.unaligned = t.part(unaligned_at, {El});
+            s.dst_slot = t.part(slot_at, {s.num_tokens, s.num_topk});
+            s.dst_gsge = t.part(gsge_at, {s.num_tokens, s.num_topk});
         }
         ep_dispatch_args_t& a = s.a;
         a.x = desc(x);

@@ -325,6 +325,70 @@ def test_arguments_that_no_output_can_be_sized_by_are_refused(wrong, sync):
     buf.destroy()
 
 
+@pytest.mark.parametrize('sync', [False, True])
+def test_a_refused_call_allocates_nothing_of_worst_case_size(sync):
+    """A token bound far beyond what the buffer was made for is refused by the library, and before anything is sized by it."""
+    import deep_ep
+    T, H, E, K = 40, 64, 8, 2
+    topk, w = make_routing(T, E, K, seed=5)
+    topk, w, x = topk.to(DEV), w.to(DEV), make_tokens(T, H).to(DEV)
+    buf = _buffer(T, H, K)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    with pytest.raises(deep_ep._C.EPException, match='Assertion'):
+        buf.dispatch(x, topk_idx=topk, topk_weights=w, num_experts=E, expert_alignment=4, num_max_tokens_per_rank=1 << 26, do_expand=True,
+                     do_cpu_sync=sync)
+    assert torch.cuda.max_memory_allocated() - before < 1 << 20
+    buf.destroy()
+
+
+@pytest.mark.parametrize('nodes', [1, 2])
+@pytest.mark.parametrize('sync', [False, True])
+@pytest.mark.parametrize('deferred', [False, True])
+def test_received_weights_and_metadata_have_storage_of_their_own(nodes, sync, deferred):
+    """The received weights are the caller's alone: they can be written to a file beside the handle, and their memory can be given up
+    while the handle serves a replay and a combine."""
+    import io
+    import deep_ep
+    if nodes > 1 and not deferred:
+        pytest.skip('the partitions of a node dispatch phase by phase')
+    T, H, E, K = 40, 64, 8, 2
+    node = deep_ep.LocalNode(nodes) if nodes > 1 else None
+    bufs = [deep_ep.EPBuffer(node.group(r) if node else deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K,
+                             explicitly_destroy=True) for r in range(nodes)]
+    # (two experts of different partitions a token: a row a partition that holds the token as it is, and a sum of two equal rows)
+    topk = torch.stack([torch.arange(T) % 4, 4 + torch.arange(T) % 4], dim=1).to(DEV)
+    xs = [make_tokens(T, H, seed=r).to(DEV) for r in range(nodes)]
+    w = torch.rand((T, K), device=DEV)
+    options = dict(async_with_compute_stream=True, defer_epilogue=True) if deferred else {}
+    sent = [b.dispatch(x, topk_idx=topk, topk_weights=w, num_experts=E, expert_alignment=4, num_max_tokens_per_rank=T, do_expand=True,
+                       do_cpu_sync=sync, do_zero_padding=True, **options) for b, x in zip(bufs, xs)]
+    got = [s.current_stream_wait() if deferred else (s[0], s[1], s[2], s[3]) for s in sent]
+    for rows, _, weights, handle in got:
+        of_handle = [handle.recv_src_metadata, handle.dst_buffer_slot_idx, handle.dst_gsge_idx, handle.psum_num_recv_tokens_per_rank,
+                     handle.psum_num_recv_tokens_per_expert, handle.num_unaligned_recv_tokens_per_expert]
+        storages = [t.untyped_storage().data_ptr() for t in of_handle]
+        assert weights.untyped_storage().data_ptr() not in storages
+        assert handle.recv_src_metadata.untyped_storage().data_ptr() not in storages[1:]
+        assert rows.untyped_storage().data_ptr() not in storages + [weights.untyped_storage().data_ptr()]
+        torch.save([weights, *of_handle], io.BytesIO())
+        weights.untyped_storage().resize_(0)
+    if deferred:
+        reduced = [b.combine(rows, handle, **options) for b, (rows, _, _, handle) in zip(bufs, got)]
+        outs = [event.current_stream_wait()[0] for event in reduced]
+    else:
+        outs = [b.combine(rows, handle)[0] for b, (rows, _, _, handle) in zip(bufs, got)]
+    for x, out in zip(xs, outs):
+        assert torch.equal(out, x + x)
+    if nodes == 1 and sync:
+        again = bufs[0].dispatch(xs[0], handle=got[0][3], do_expand=True, do_zero_padding=True)[0]
+        assert torch.equal(again, got[0][0])
+    torch.cuda.synchronize()
+    for b in bufs:
+        b.destroy()
+
+
 @pytest.mark.parametrize('fused', [False, True])
 def test_exact_sync_sizes_allocate_what_the_results_show(fused):
     """A host-synchronised dispatch returns views of bound-sized storage by default; with `set_exact_sync_sizes()` the
