@@ -1436,14 +1436,17 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_count_
 // ------------------------------------------------------------------------------------------------
 // The slot assignment of one partition behind ep_layout_count, up to top-8 and EP_SMALL_MASK_EXPERTS experts: what
 // ep_layout_assign_fold does, with ranks from bit masks.  A block's ids leave a bit a token and expert in LDS, and an entry's rank is
-// the number of bits below its token (a token that selects an expert twice leaves one bit and an entry in a list that is looked
-// through where there is one); the last valid position of a token and the tokens with one come from a bit an entry.  Neither counts per
+// the number of bits below its token (where tokens select an expert more than once, the second, third, .. selections leave their bits
+// one after the other in passes of their own); the last valid position of a token and the tokens with one come from a bit an entry.  Neither counts per
 // wave nor rounds of match-any, and two barriers: one behind the clearing of the LDS, one behind bits and sums of the count rows.
 // Each wave makes the scan over the experts alone.
 // Bound by the launch and its trips to memory (ids and count rows, asked for together).  us of a layout (both launches, several in a
 // captured graph), ep_layout_count + ep_layout_assign_fold / ep_layout_count_bits + this one: 256 experts, 2048 tokens top-8 14.6 / 10.6, 4096
 // top-8 14.6 / 10.7, top-6 13.4 / 10.2, 8192 top-4 12.1 / 10.0, 16384 top-2 11.4 / 10.3; 64 experts 4096 top-8 14.2 / 10.7, 32768 top-2
-// 11.0 / 10.9.  (Every workgroup counting all ids in one launch, as ep_dispatch_chunk_* does: 1024 top-8 7.8, 2048 9.6, 4096 13.1, 8192 top-4
+// 11.0 / 10.9.  With repeated selections, 4096 tokens top-8 of 256 experts, ids of one repeated once 14.6 / 12.7, of all 14.6 / 12.8, drawn with
+// repetitions 14.6 / 13.1, every token on one expert 14.8 / 15.8 (up to 64 experts 14.3 / 15.9), every entry on one 15.9 / 16.4; top-4 12.1 /
+// 11.0, 11.0, 11.0, 12.0, 12.4.  (The repetitions in a list that every entry looks through: 12.6, 22.4, 15.1, 80, 81; passes that take bits
+// away instead of setting them, a barrier less each but all of a token's ids to compare in front: 13.2, 13.2, 13.6, 17.0, 17.5.)  (Every workgroup counting all ids in one launch, as ep_dispatch_chunk_* does: 1024 top-8 7.8, 2048 9.6, 4096 13.1, 8192 top-4
 // 13.7: better only where that launch copies as well.)
 // ------------------------------------------------------------------------------------------------
 extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign_bits(EpLayoutArgs a) {
@@ -1458,9 +1461,8 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
     int* s_tot = s_pre + W;                             // [W] entries in all blocks
     int* s_start = s_tot + W;                           // [W] first slot of an expert
     uint64_t* s_mark = (uint64_t*)(s_start + W);        // [n / 64 + 1] entries with an expert, a bit each
-    int* s_extra = (int*)(s_mark + EP_TOKENS_PER_BLOCK * EP_BITS_TOPK / WAVE + 1);     // [1] entries in
-    unsigned* s_list = (unsigned*)(s_extra + 2);        // [n] (token, expert) pairs met once more
-    short* s_key = (short*)(s_list + EP_TOKENS_PER_BLOCK * EP_BITS_TOPK);              // [n] expert of an entry, -1: none
+    int* s_last = (int*)(s_mark + EP_TOKENS_PER_BLOCK * EP_BITS_TOPK / WAVE + 1);      // [2] last pass over repeated selections, 0: there are none
+    short* s_key = (short*)(s_last + 2);                // [n] expert of an entry, -1: none
     const int tid = threadIdx.x, lane = lane_id();
 
     // ---- ids first, count rows behind them: a thread takes 8 adjacent columns of every S-th row (see ep_layout_assign_fold) ----
@@ -1481,7 +1483,7 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
     fold_loads(s0);
     const u32x4 zero = {0u, 0u, 0u, 0u};
     for (int i = tid; i < E + (W >> 1); i += NT) s_mask[i] = zero;      // masks and both rows of sums
-    if (tid == 0) *s_extra = 0;
+    if (tid == 0) *s_last = 0;
     __syncthreads();
 
     // ---- a bit a token and expert, a bit an entry ----
@@ -1498,7 +1500,7 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
         if (i < n) s_key[i] = (short)key[u];
         if (valid && !publisher) {
             const unsigned bit = 1u << (tok[u] & 31);
-            if (atomicOr((unsigned*)&s_mask[key[u]] + (tok[u] >> 5), bit) & bit) s_list[atomicAdd(s_extra, 1)] = (unsigned)(tok[u] << 16 | key[u]);
+            if (atomicOr((unsigned*)&s_mask[key[u]] + (tok[u] >> 5), bit) & bit) *s_last = 1;
         }
     }
     // ---- sums of the count rows: blocks before this one, and all ----
@@ -1572,7 +1574,46 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
     // ---- tokens with an expert, a bit each (a wave has 128 tokens in two ballots) ----
     auto marks_of = [&](int t) { return entry_marks(s_mark, t * K, K); };
     const uint64_t any_lo = __ballot(marks_of(lane) != 0u), any_hi = __ballot(marks_of(lane + WAVE) != 0u);
-    const int rows_before = s_pre[at_of(E)], extras = *s_extra;
+    const int rows_before = s_pre[at_of(E)];
+    // ---- rank: the bits of the expert below the token ----
+    auto below = [&](int e, int t) -> int {
+        const u32x4 m = s_mask[e];
+        int c = 0;
+#pragma unroll
+        for (int q = 0; q < TW; ++q) {
+            const int bits = min(max(t - 32 * q, 0), 32);
+            c += __popc(m[q] & (bits == 32 ? ~0u : (1u << bits) - 1u));
+        }
+        return c;
+    };
+    int rank[PER];                                      // (where a token selects an expert more than once)
+    const bool repeats = __builtin_amdgcn_readfirstlane(*s_last) != 0;
+    if (repeats) {
+        // entries with as many equal ones in front of them in their token leave their bits together, a pass each
+        int met[PER];
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            rank[u] = below(max(key[u], 0), tok[u]);
+            met[u] = 0;
+            if (key[u] < 0) continue;
+            for (int at = tok[u] * K; at < tid + u * NT; ++at) met[u] += s_key[at] == key[u] ? 1 : 0;
+            rank[u] += met[u];
+        }
+        for (int pass = 1, last = pass; pass <= last; ++pass) {
+            __syncthreads();                            // (masks and last pass have been read)
+            for (int i = tid; i < E; i += NT) s_mask[i] = zero;
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                if (met[u] == pass) atomicOr((unsigned*)&s_mask[key[u]] + (tok[u] >> 5), 1u << (tok[u] & 31));
+                if (met[u] > pass) *s_last = pass + 1;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < PER; ++u) rank[u] += below(max(key[u], 0), tok[u]);
+            last = __builtin_amdgcn_readfirstlane(*s_last);
+        }
+    }
 #pragma unroll
     for (int u = 0; u < PER; ++u) {
         const int i = tid + u * NT, t = tok[u], e = key[u];
@@ -1580,18 +1621,7 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
         const int pos = i - t * K;
         int slot = -1, rslot = -1;
         if (e >= 0) {
-            const u32x4 m = s_mask[e];
-            int rank = 0;
-#pragma unroll
-            for (int q = 0; q < TW; ++q) {
-                const int bits = min(max(t - 32 * q, 0), 32);
-                rank += __popc(m[q] & (bits == 32 ? ~0u : (1u << bits) - 1u));
-            }
-            if (extras > 0) {
-                for (int x = 0; x < extras; ++x) rank += (int)(s_list[x] & 0xffffu) == e && (int)(s_list[x] >> 16) < t ? 1 : 0;
-                for (int j = 0; j < pos; ++j) rank += s_key[t * K + j] == e ? 1 : 0;
-            }
-            slot = s_start[e] + s_pre[at_of(e)] + rank;
+            slot = s_start[e] + s_pre[at_of(e)] + (repeats ? rank[u] : below(e, t));
             if ((marks_of(t) >> pos) == 1u)             // the last one of its token
                 rslot = rows_before + (t < WAVE ? __popcll(any_lo & ((1ull << t) - 1ull))
                                                 : __popcll(any_lo) + __popcll(any_hi & ((1ull << (t - WAVE)) - 1ull)));

@@ -359,7 +359,7 @@ unsigned layout_assign_lds(int E, int R, int K, int count_experts, int cnt_strid
 unsigned layout_count_bits_lds(int cnt_stride) { return 4u * (unsigned)cnt_stride + 8u * (EP_TOKENS_PER_BLOCK * EP_BITS_TOPK / 64 + 1); }
 unsigned layout_assign_bits_lds(int E, int cnt_stride) {
     constexpr unsigned entries = EP_TOKENS_PER_BLOCK * EP_BITS_TOPK;
-    return 16u * (unsigned)E + 12u * (unsigned)cnt_stride + 8u * (entries / 64 + 1) + 8u + 4u * entries + 2u * entries;
+    return 16u * (unsigned)E + 12u * (unsigned)cnt_stride + 8u * (entries / 64 + 1) + 8u + 2u * entries;
 }
 
 // Up to here one partition ranks in bit masks, behind histograms of its own: never the slower of the two forms (figures at the kernel;

@@ -211,7 +211,7 @@ def test_ids_of_all_blocks_counted_in_place(T, E, K):
 def test_slots_from_bits(T, E, K, how):
     """The two layout launches of one partition that rank in bit masks (up to top-8 and 1024 experts; the last two cases are beyond), at
     the edges of blocks, words and groups of experts, in more count rows than one go holds (3001 tokens, 1024 experts), with
-    experts selected twice (every entry on one expert: the longest list), and with most selections missing."""
+    experts selected twice (every entry on one expert: the most passes), and with most selections missing."""
     import deep_ep
     H, A = 16, 4
     x = make_tokens(T, H, seed=T).to(DEV)
@@ -236,6 +236,87 @@ def test_slots_from_bits(T, E, K, how):
                  'dst_buffer_slot_idx', 'recv_src_metadata'):
         assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
     assert handle.num_recv_tokens_per_expert_list == lay['num_recv_tokens_per_expert_list']
+    buf.destroy()
+
+
+def _repeated(T, E, K, how, seed):
+    """Selections in which tokens select an expert more than once."""
+    g = torch.Generator().manual_seed(seed)
+    topk = torch.randint(0, E, (T, K), generator=g)
+    if how == 'stairs':                         # 1, 2, .. K times, at any place of the token, beside distinct ones
+        topk, _ = make_routing(T, E, K, seed=seed)
+        for t in range(T):
+            topk[t, torch.randperm(K, generator=g)[:t % K + 1]] = topk[t, 0].item()
+    if how == 'last':                           # the last token's last two entries and no other
+        topk, _ = make_routing(T, E, K, seed=seed)
+        topk[T - 1, K - 1] = topk[T - 1, K - 2]
+    if how == 'same':                           # all of a token, the first and the last expert most
+        topk = torch.tensor([0, E - 1, E // 2])[torch.randint(0, 3, (T, 1), generator=g)].expand(T, K).contiguous()
+    return topk
+
+
+@pytest.mark.parametrize('T,E,K,how', [(1153, 8, 8, 'any'), (200, 9, 8, 'any'), (2049, 64, 8, 'stairs'), (1400, 1024, 7, 'stairs'), (1283, 256, 5, 'stairs'),
+                                       (1793, 256, 8, 'last'), (3000, 32, 2, 'last'), (2177, 1024, 8, 'same'), (1500, 48, 3, 'same'), (4100, 8, 4, 'any')])
+@pytest.mark.parametrize('masked', [False, True])
+def test_slots_from_bits_of_repeated_selections(T, E, K, how, masked):
+    """The second, third, .. selections of an expert by a token leave their bits a pass each: up to top-k passes, an entry alone in the
+    last one, missing selections in between."""
+    import deep_ep
+    H, A = 16, 4
+    x = make_tokens(T, H, seed=T).to(DEV)
+    topk = _repeated(T, E, K, how, seed=T + K)
+    if masked:
+        topk[torch.rand((T, K), generator=torch.Generator().manual_seed(3)) < 0.2] = -1
+    lay = O.rank_share_layout(topk.numpy(), E, 1, 0, A, T)
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    try:
+        deep_ep._C.set_layout_recount_limit(0)
+        handle = buf.dispatch(x, topk_idx=topk.to(DEV), num_experts=E, expert_alignment=A, do_expand=True, async_with_compute_stream=True,
+                              defer_epilogue=True).current_stream_wait()[3]
+        torch.cuda.synchronize()
+    finally:
+        deep_ep._C.set_layout_recount_limit(-1)
+    for name in ('psum_num_recv_tokens_per_rank', 'psum_num_recv_tokens_per_expert', 'num_unaligned_recv_tokens_per_expert',
+                 'dst_buffer_slot_idx', 'recv_src_metadata'):
+        assert np.array_equal(getattr(handle, name).cpu().numpy(), lay[name]), name
+    buf.destroy()
+
+
+def test_a_layout_of_repeated_selections_takes_no_multiple_of_one_without():
+    """A layout of several blocks behind the histograms, timed as replays of a captured graph: every selection of a token on one expert costs
+    up to seven passes over a block's masks (half as much again), not a look through all of its repetitions (eight times)."""
+    import deep_ep
+    T, H, E, K, calls = 4096, 16, 256, 8, 8
+    buf = deep_ep.EPBuffer(deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K, explicitly_destroy=True)
+    x = make_tokens(T, H).to(DEV)
+    distinct, _ = make_routing(T, E, K, seed=1)
+
+    def shortest(topk):
+        topk = topk.to(DEV)
+
+        def dispatches():
+            return [buf.dispatch(x, topk_idx=topk, num_experts=E, num_max_tokens_per_rank=T, expert_alignment=1, do_expand=True, do_cpu_sync=False,
+                                 async_with_compute_stream=True, defer_epilogue=True) for _ in range(calls)]
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            dispatches()
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            kept = dispatches()
+        times = []
+        for _ in range(20):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        del kept
+        return min(times)
+
+    assert shortest(distinct[:, :1].expand(T, K).contiguous()) < 3 * shortest(distinct)
     buf.destroy()
 
 
