@@ -1739,6 +1739,7 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
             }
             grand += readlane(incl, WAVE - 1);
         }
+        __builtin_amdgcn_wave_barrier();                // (a wave's lanes read each other's words: its LDS operations complete in order)
     }
     auto below = [&](const u32x4& m, int before) -> int {      // bits of m below `before`
         int c = 0;
