@@ -165,6 +165,7 @@ struct EpScatterArgs {
 // side of a node that ships ranks: every workgroup works the layout out for itself.
 #define EP_SMALL_ENTRIES 1024
 #define EP_SMALL_MASK_EXPERTS 1024    // ep_dispatch_small_*, ep_layout_assign_bits: up to here a bit a token and expert is kept in LDS (16 bytes an expert)
+#define EP_SMALL_REPEATS 128          // ep_dispatch_small_*: entries beyond the first of a token for an expert that are listed
 struct EpSmallArgs {
     EpLayoutArgs l;               // what ep_layout_assign (ep_recv_copy: ep_layout_place) would have been given
     EpScatterArgs s;              // what the copy kernel would have been given

@@ -1637,8 +1637,9 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
 // A dispatch of at most EP_TOKENS_PER_BLOCK tokens and EP_SMALL_ENTRIES entries in one launch.  Instead of a slot
 // assignment in front of the copy (a launch that one or two workgroups of the chip work at, bound by its own dependent
 // phases), every workgroup counts all ids in LDS and leaves a bit a token and expert there; its waves rank the one token each of
-// them copies by the bits below it, a position a lane.  (A token that selects an expert twice has one bit for both: then, and beyond
-// EP_SMALL_MASK_EXPERTS, whose masks would leave a CU too few workgroups, the ids in front of the token are compared expert by expert.)
+// them copies by the bits below it, a position a lane.  (A token that selects an expert twice has one bit for both and an entry in a
+// list, which is looked through 64 entries at a time.  With more than EP_SMALL_REPEATS of them, and beyond EP_SMALL_MASK_EXPERTS, whose masks
+// would leave a CU too few workgroups, the ids in front of the token are compared expert by expert.)
 // The payload is fetched before the ids are looked at.  Workgroup 0 publishes what the assignment's publishing workgroup
 // does, the next ones copy (or, with several partitions, pack) as the kernels above, the last zero the padding.
 // Bound by the launch, two trips to memory and the phases in LDS between them.  Assignment + copy -> this kernel with ids compared (us): 32 tokens,
@@ -1648,6 +1649,10 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
 // 6.3): 256 experts, BF16, top-8, 7168 channels 1 / 32 / 61 tokens 5.7 / 6.4 / 7.5 -> 4.3 / 4.9 / 5.7, 256 channels 128 tokens 8.2 -> 5.8; top-6, FP8,
 // alignment 16, 96 tokens 8.0 -> 6.5; 1024 experts, 61 tokens top-8 7.4 -> 5.8; top-1 level; all of a dispatch of eight partitions of 64 tokens
 // top-8, metadata above included, 110.0 -> 88.3.  Masks at 2048 experts: 1 token top-1 with padding 8.3 -> 10.8, compared so 8.2.
+// Repeated selections, ids compared without masks / compared behind masks / listed: 128 tokens x 7168 top-8 of 256, one repeated once
+// 10.9 / 11.1 / 9.2, ids drawn with repetitions 11.0 / 11.2 / 9.7, one repeated by every token 11.2 / 11.4 / 10.5; 61 tokens x 5120, top-6 7.1 / 7.2 / 6.5; beyond the
+// list (that form compares) every token on one expert 11.4 / 11.9 / 12.4, every entry on one 12.5 / 14.1 / 14.5, of 256 channels 9.6 / 10.2 / 10.6:
+// the masks' and the list's words are contended.  (A list of 256, level at 128 tokens with every one of them: 32 tokens on one expert each 8.0 -> 8.8.)
 // ------------------------------------------------------------------------------------------------
 template <bool QUANT, bool HW, bool PACK>
 __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
@@ -1664,9 +1669,10 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     u32x4* s_tok = (u32x4*)smem;                        // [R] tokens that go to a partition, a bit each
     u32x4* s_mask = s_tok + R;                          // [E] tokens that selected an expert, a bit each (E <= EP_SMALL_MASK_EXPERTS)
     int* s_cnt = (int*)(s_mask + (masks ? E : 0));      // [Ep] entries per expert
-    int* s_twice = s_cnt + Ep;                          // [4] a token selected an expert twice: the masks do not say how often
-    int* s_start = s_twice + 4;                         // [Ep] first slot of each expert (one partition)
+    int* s_more = s_cnt + Ep;                           // [4] entries that s_list has, or would have
+    int* s_start = s_more + 4;                          // [Ep] first slot of each expert (one partition)
     short* s_key = (short*)(s_start + Ep);              // [EP_SMALL_ENTRIES] expert of every entry, -1: none
+    unsigned* s_list = (unsigned*)(s_key + EP_SMALL_ENTRIES);           // [EP_SMALL_REPEATS] (token, expert) pairs beyond their first entry (masks)
     const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
     const int n = l.num_tokens * K;
 
@@ -1705,7 +1711,10 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
             const unsigned bit = 1u << (tok & 31);
             atomicAdd(&s_cnt[e], 1);
             atomicOr((unsigned*)&s_tok[PACK ? partition_of(e) : 0] + (tok >> 5), bit);
-            if (masks && (atomicOr((unsigned*)&s_mask[e] + (tok >> 5), bit) & bit)) *s_twice = 1;
+            if (masks && (atomicOr((unsigned*)&s_mask[e] + (tok >> 5), bit) & bit)) {
+                const int x = atomicAdd(s_more, 1);
+                if (x < EP_SMALL_REPEATS) s_list[x] = (unsigned)(tok << 16 | e);
+            }
         }
     }
     // (own ids are here by now, and with them the arenas of the token's partitions, which are a trip of their own)
@@ -1768,8 +1777,22 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
 
     // ---- rank of the token's entries: earlier entries with the same expert ----
     int rank = 0;
-    if (masks && __builtin_amdgcn_readfirstlane(*s_twice) == 0) {
-        rank = below(s_mask[max(e, 0)], t);             // earlier tokens, each of which selected it once
+    const int more = __builtin_amdgcn_readfirstlane(*s_more);
+    if (masks && more <= EP_SMALL_REPEATS) {
+        rank = below(s_mask[max(e, 0)], t);             // earlier tokens that selected it, and beyond that their repetitions
+        for (int x0 = 0; x0 < more; x0 += WAVE) {
+            const unsigned pair = x0 + lane < more ? s_list[x0 + lane] : ~0u;
+            const int earlier = (int)(pair >> 16) < t ? (int)(pair & 0xffffu) : -2;
+            for (int j = 0; j < K; ++j) {
+                const int c0 = __popcll(__ballot(earlier == readlane(e, j)));
+                if (lane == j) rank += c0;
+            }
+        }
+        if (more > 0)                                   // (and the same expert earlier in the own token)
+            for (int j = 1; j < K; ++j) {
+                const int c0 = __popcll(__ballot(e == readlane(e, j)) & ((1ull << j) - 1ull));
+                if (lane == j) rank += c0;
+            }
     } else {
         const int before = t * K, chunks = (before + WAVE - 1) / WAVE;
         int key[CH];

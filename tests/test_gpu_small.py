@@ -282,6 +282,46 @@ def test_slots_from_bits_of_repeated_selections(T, E, K, how, masked):
     buf.destroy()
 
 
+@pytest.mark.parametrize('T,E,K,how', [(128, 16, 8, 'stairs'), (128, 1024, 8, 'same'), (127, 256, 8, 'stairs'), (65, 64, 3, 'any'), (17, 1025, 5, 'stairs'),
+                                       (2, 24, 8, 'same'), (1, 16, 8, 'same'), (31, 64, 32, 'stairs'), (128, 160, 6, 'last')])
+@pytest.mark.parametrize('R', [1, 2])
+def test_small_dispatch_of_repeated_selections(T, E, K, how, R):
+    """Decode sizes: none, a wave's worth (64) and many more entries beyond the first of a token for an expert, in the order of sources,
+    tokens and positions (1025 experts: without masks)."""
+    import deep_ep
+    H, A, El = 32, 4, (E + E % R) // R
+    x = [make_tokens(T, H, seed=T + r).to(DEV) for r in range(R)]
+    topk = [_repeated(T, E, K, how, seed=T + K + r) for r in range(R)]
+    gates = [torch.rand((T, K), generator=torch.Generator().manual_seed(r)) for r in range(R)]
+    node = deep_ep.LocalNode(R) if R > 1 else None
+    bufs = [deep_ep.EPBuffer(node.group(r) if R > 1 else deep_ep.LocalGroup(), num_max_tokens_per_rank=T, hidden=H, num_topk=K,
+                             explicitly_destroy=True) for r in range(R)]
+    args = dict(num_experts=El * R, num_max_tokens_per_rank=T, expert_alignment=A, do_expand=True, do_cpu_sync=False)
+    if R == 1:
+        got = [bufs[0].dispatch(x[0], topk_idx=topk[0].to(DEV), topk_weights=gates[0].to(DEV), **args)]
+    else:
+        events = [b.dispatch(xx, topk_idx=t.to(DEV), topk_weights=g.to(DEV), async_with_compute_stream=True, defer_epilogue=True, **args)
+                  for b, xx, t, g in zip(bufs, x, topk, gates)]
+        got = [e.current_stream_wait() for e in events]
+    torch.cuda.synchronize()
+    every = torch.cat([t.reshape(-1) for t in topk])
+    rows_of = torch.cat([xx.cpu().repeat_interleave(K, dim=0) for xx in x])
+    gate_of = torch.cat([g.reshape(-1) for g in gates])
+    for r in range(R):
+        rows, _, weights, handle = got[r][:4]
+        local = torch.where((every >= r * El) & (every < (r + 1) * El), every - r * El, El)
+        counts = torch.bincount(local, minlength=El + 1)[:El]
+        assert torch.equal(handle.num_unaligned_recv_tokens_per_expert.cpu().long(), counts)
+        order = torch.argsort(local, stable=True)[:int(counts.sum())]
+        aligned = (counts + A - 1) // A * A
+        starts = torch.cumsum(aligned, 0) - aligned
+        slots = starts[local[order]] + torch.arange(len(order)) - (torch.cumsum(counts, 0) - counts)[local[order]]
+        assert torch.equal(rows.cpu()[slots].view(torch.int16), rows_of[order].view(torch.int16))
+        assert torch.equal(weights.cpu()[slots], gate_of[order])
+    for b in bufs:
+        b.destroy()
+
+
 def test_a_layout_of_repeated_selections_takes_no_multiple_of_one_without():
     """A layout of several blocks behind the histograms, timed as replays of a captured graph: every selection of a token on one expert costs
     up to seven passes over a block's masks (half as much again), not a look through all of its repetitions (eight times)."""
