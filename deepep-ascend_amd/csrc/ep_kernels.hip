@@ -1402,7 +1402,9 @@ __device__ __forceinline__ unsigned entry_marks(const uint64_t* s_mark, int at, 
 // The histograms in front of ep_layout_assign_bits: what ep_layout_count leaves for EP_LAYOUT_FOLDED, of one partition and up to top-8: a
 // token is received where one of its entries has an expert, which a bit an entry tells without a look at its neighbours.
 // Bound by the launch and the trip for the ids.  us of a layout (both launches, several in a captured graph) of 256 experts behind ep_layout_count
-// and this one: 4096 tokens top-8 11.7 / 10.7, top-4 10.4 / 9.9, 16384 top-4 11.2 / 10.6, 32768 top-2 14.0 / 13.7.
+// and this one: 4096 tokens top-8 11.7 / 10.7, top-4 10.4 / 9.9, 16384 top-4 11.2 / 10.6, 32768 top-2 14.0 / 13.7.  A thread asks for four ids
+// whatever the top-k, no further than its block's own: beyond those, the next blocks' ids came along, two to eight times the bytes at top-4
+// to top-1 (both kernels, 32768 tokens of 64 experts top-1 10.70 -> 10.59, 40960 of 32 experts top-2 11.64 -> 11.47, level at top-4).
 // ------------------------------------------------------------------------------------------------
 extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_count_bits(EpLayoutArgs a) {
     fetch_arguments<EpLayoutArgs>();
@@ -1414,7 +1416,7 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_count_
     const int64_t base = (int64_t)blockIdx.x * n, total = (int64_t)a.num_tokens * K;
     int64_t id[PER];
 #pragma unroll
-    for (int u = 0; u < PER; ++u) id[u] = a.topk_idx[min(base + tid + u * NT, total - 1)];
+    for (int u = 0; u < PER; ++u) id[u] = a.topk_idx[min(base + min(tid + u * NT, n - 1), total - 1)];
     __builtin_amdgcn_sched_barrier(0);
     for (int i = tid; i < W; i += NT) s_cnt[i] = 0;
     __syncthreads();
@@ -1434,7 +1436,7 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_count_
 }
 
 // ------------------------------------------------------------------------------------------------
-// The slot assignment of one partition behind ep_layout_count, up to top-8 and EP_SMALL_MASK_EXPERTS experts: what
+// The slot assignment of one partition behind ep_layout_count_bits, up to top-8 and EP_SMALL_MASK_EXPERTS experts: what
 // ep_layout_assign_fold does, with ranks from bit masks.  A block's ids leave a bit a token and expert in LDS, and an entry's rank is
 // the number of bits below its token (where tokens select an expert more than once, the second, third, .. selections leave their bits
 // one after the other in passes of their own); the last valid position of a token and the tokens with one come from a bit an entry.  Neither counts per
@@ -1469,7 +1471,7 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
     const int64_t base = (int64_t)min(b, nb - 1) * n, total = (int64_t)a.num_tokens * K;
     int64_t id[PER];
 #pragma unroll
-    for (int u = 0; u < PER; ++u) id[u] = a.topk_idx[min(base + tid + u * NT, total - 1)];
+    for (int u = 0; u < PER; ++u) id[u] = a.topk_idx[min(base + min(tid + u * NT, n - 1), total - 1)];
     __builtin_amdgcn_sched_barrier(0);
     const int S = FG >= NT ? 1 : NT / FG, s0 = FG >= NT ? 0 : tid / FG, g0 = FG >= NT ? tid : tid - s0 * FG;
     const unsigned row_bytes = (unsigned)W * 2u, step = (unsigned)S * row_bytes;

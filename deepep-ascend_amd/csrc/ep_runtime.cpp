@@ -362,8 +362,11 @@ unsigned layout_assign_bits_lds(int E, int cnt_stride) {
     return 16u * (unsigned)E + 12u * (unsigned)cnt_stride + 8u * (entries / 64 + 1) + 8u + 2u * entries;
 }
 
-// Up to here one partition ranks in bit masks, behind histograms of its own: never the slower of the two forms (figures at the kernel;
-// beyond top-8 a thread would hold more than four ids, and the masks of more experts leave a CU too few workgroups).
+// Up to here one partition ranks in bit masks, behind histograms of its own (figures at the kernel; beyond top-8 a thread would hold more
+// than four ids, and the masks of more experts leave a CU too few workgroups).  It is the faster form or level but for top-1 and top-2 of few
+// experts at some multiples of 256 blocks, between which it gains.  us of a layout, ids ranked by match-any / in masks: top-1, 64 experts,
+// 24576 tokens 10.3 / 9.7, 32768 10.6 / 10.6, 49152 12.6 / 12.0, 65536 12.9 / 13.1, 98304 18.9 / 18.8; 32 experts, 49152 12.3 / 11.8, 98304 16.3 / 16.8;
+// top-2 17.0 / 17.4; top-3 18.4 / 17.5.
 bool bits_layout(int K, int E) { return K <= EP_BITS_TOPK and E <= EP_SMALL_MASK_EXPERTS; }
 
 // Where one launch that counts the ids of all blocks in every workgroup beats a histogram launch in front of the slot
