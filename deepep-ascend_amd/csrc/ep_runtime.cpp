@@ -370,15 +370,20 @@ unsigned layout_assign_bits_lds(int E, int cnt_stride) {
 bool bits_layout(int K, int E) { return K <= EP_BITS_TOPK and E <= EP_SMALL_MASK_EXPERTS; }
 
 // Where one launch that counts the ids of all blocks in every workgroup beats a histogram launch in front of the slot
-// assignment.  It saves a launch; each further block is more ids to every workgroup, and one more of these.  us of a replayed
-// dispatch of 16 channels, 256 experts, two launches / one: top-1, 16 blocks 12.8 / 11.6, 24 12.9 / 13.9, 64 14.4 / 21.9; top-2,
-// 12 13.0 / 12.5, 16 13.0 / 13.1, 32 13.6 / 17.8; top-3, 10 14.4 / 13.4, 16 14.6 / 15.6; top-4, 8 14.5 / 13.3, 16 14.8 / 17.0; top-6, 8
-// 16.1 / 15.7, 10 16.3 / 17.3; top-8, 6 17.5 / 16.7, 8 17.6 / 18.3; top-12, 4 21.1 / 18.9; top-32, 2 37.3 / 31.5.  To a host that waits for
-// the counts the saved launch is worth more (wall clock, 8 blocks, top-7 24.3 / 23.7, top-8 25.3 / 25.0).
-// Against the two launches that rank in bit masks the line lies lower where no host waits, and stays where one does.  us, two
-// launches / one, 256 experts: top-1, 16 blocks 9.4 / 8.9; top-2, 8 9.3 / 8.2, 16 9.4 / 10.3; top-4, 4 9.7 / 8.8, 6 9.8 / 10.1; top-8, 2 10.3 / 10.5,
-// 3 10.1 / 11.8; 32 experts top-4, 4 10.0 / 8.1, 6 10.2 / 9.5; 1024 experts 10.7 / 10.3, 10.8 / 11.6.  Wall clock of a dispatch of exact
-// sizes: top-2, 12 blocks 27.5 / 26.0; top-4, 12 27.5 / 27.3; top-8, 4 27.1 / 25.7, 6 27.4 / 27.0.
+// assignment.  It saves a launch; each further block is more ids to every workgroup, and one more of these.
+// Against ep_layout_count + ep_layout_assign_fold (beyond top-8 or EP_SMALL_MASK_EXPERTS now), us of a replayed dispatch of 16 channels, 256 experts,
+// two launches / one: top-1, 16 blocks 12.8 / 11.6, 24 12.9 / 13.9, 64 14.4 / 21.9; top-2, 12 13.0 / 12.5, 16 13.0 / 13.1, 32 13.6 / 17.8; top-3, 10 14.4 /
+// 13.4, 16 14.6 / 15.6; top-4, 8 14.5 / 13.3, 16 14.8 / 17.0; top-6, 8 16.1 / 15.7, 10 16.3 / 17.3; top-8, 6 17.5 / 16.7, 8 17.6 / 18.3; top-12, 4 21.1 /
+// 18.9; top-32, 2 37.3 / 31.5.  To a host that waits for the counts the saved launch was worth more (wall clock, 8 blocks, top-7 24.3 / 23.7,
+// top-8 25.3 / 25.0).
+// Against the two launches that rank in bit masks the line lies lower where no host waits.  us, two launches / one, 256 experts: top-1,
+// 16 blocks 9.4 / 8.9; top-2, 8 9.3 / 8.2, 16 9.4 / 10.3; top-4, 4 9.7 / 8.8, 6 9.8 / 10.1; top-8, 2 10.3 / 10.5, 3 10.1 / 11.8; 32 experts top-4, 4
+// 10.0 / 8.1, 6 10.2 / 9.5; 1024 experts 10.7 / 10.3, 10.8 / 11.6.
+// Where a host waits it is 48 blocks x top-k for every top-k: higher than against the other two for top-3 to top-5 (32 to 40 there), lower for top-7
+// and top-8 (56, 64).  The ids come 16 a thread and trip: wall clock of a dispatch of exact sizes is level up to 48 and falls off beyond.  us, two
+// launches / one: 256 experts, top-3, 10 blocks 26.2 / 25.0, 12 26.8 / 27.2, 16 26.7 / 26.8; top-4, 8 26.6 / 25.0, 10 26.3 / 26.1, 12 26.7 / 27.0, 14 26.6 / 28.4; top-5, 9
+// 26.2 / 26.4, 10 26.2 / 27.2; top-6, 8 26.1 / 26.0, 9 26.3 / 27.3; top-7, 4 26.2 / 25.3, 6 26.5 / 26.7, 7 26.4 / 27.7, 8 26.3 / 27.3; top-8, 4 26.2 / 25.5, 6
+// 26.3 / 26.5, 7 26.5 / 27.8, 8 26.3 / 27.5; 32 experts, top-8, 6 26.5 / 25.9, 7 26.4 / 27.0; 1024, 4 30.3 / 30.0, 6 30.1 / 30.7.
 bool recount_pays(int num_blocks, int K, int E, bool host_waits) {
     const int most = 2 * EP_RECOUNT_DEPTH;
     const int limit = bits_layout(K, E) ? (host_waits ? 48 : 16)
