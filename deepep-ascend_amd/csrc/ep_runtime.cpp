@@ -1645,14 +1645,18 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROWS_PER_BLOCK);
             const unsigned grid = (unsigned)ca.num_row_blocks + (unsigned)ceil_div(num_combined_tokens, EP_ROW_THREADS);
             if (grid == 0) return;
-            // odd top-k: a launch of few row blocks a CU waits for its trips to memory and takes the unrolled kernel, and so does one that fills
-            // the chip several times over; between the two the general one's shorter bursts win.  us, general / unrolled, four outputs in
-            // turn, top-3 / 5 / 7: 384 blocks 6.5 / 6.1, 8.2 / 7.1, 9.9 / 8.4; 766 7.6 / 7.3, 9.5 / 9.0, 11.6 / 11.1; 896 8.7 / 9.0, 10.5 / 10.9, 13.0 /
-            // 13.7; 1787 13.2 / 14.0, 18.4 / 18.8, 22.8 / 23.5; 3584 24.1 / 24.3, 33.4 / 33.7, 43.2 / 43.7; 5376 33.3 / 32.9, 50.6 / 47.9, 68.2 / 66.0;
+            // odd top-k: a launch of up to three row blocks a CU, all on their way at once, waits for its trips to memory and takes the unrolled
+            // kernel, and so does one that fills the chip several times over; between the two the general one's shorter bursts win.
+            // us, general / unrolled, four outputs in turn, top-3 / 5 / 7, 2560 channels unless noted: 384 blocks 6.5 / 6.1, 8.2 / 7.1, 9.9 / 8.4; 766 7.6 /
+            // 7.3, 9.5 / 9.0, 11.6 / 11.1; 7168 channels 764 8.2 / 7.8, 10.0 / 9.9, 11.9 / 12.2; 776 8.0 / 7.8, 10.1 / 10.6, 11.8 / 12.8; 800 8.4 / 8.5, 10.3 / 11.0,
+            // 12.3 / 13.4 (the same of 1024 to 5120 channels; the third, half part of 2560 puts the line at 860, 790 and 770; top-7 loses from 720 full
+            // blocks on: 720 11.7 / 11.7, 750 11.8 / 12.0); 896 8.7 / 9.0, 10.5 / 10.9,
+            // 13.0 / 13.7; 1787 13.2 / 14.0, 18.4 / 18.8, 22.8 / 23.5; 3584 24.1 / 24.3, 33.4 / 33.7, 43.2 / 43.7; 5376 33.3 / 32.9, 50.6 / 47.9, 68.2 / 66.0;
             // 28672 155 / 153, 233 / 234, 319 / 314; 6144 (2560 channels) 34.3 / 32.3, 49.6 / 45.6, 67.6 / 60.6
             ca.paced = ca.num_row_blocks >= kPacedRowBlocks ? 1 : 0;
             const bool odd = unrolled != 0 and K % 2 != 0;
-            const int kidx = odd and ca.num_row_blocks >= 800 and ca.num_row_blocks < 4096 ? 0 : unrolled;
+            const bool once = ca.num_row_blocks <= 3 * 256 and (K < 7 or (int64_t)ca.num_rows_bound * hidden <= 720 * 4096);
+            const int kidx = odd and not once and ca.num_row_blocks < 4096 ? 0 : unrolled;
             const unsigned cap = combine_lds_cap(K + (ca.bias_0 != nullptr) + (ca.bias_1 != nullptr), kidx != 0, odd, ca.num_row_blocks, hidden);
             launch(g_k.combine[EP_COMBINE_FUSED][kidx], grid, EP_ROW_THREADS, cap, a.stream, ca);
         } else {

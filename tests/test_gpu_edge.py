@@ -601,12 +601,14 @@ def test_reduces_of_a_node_by_partitions_topk_and_size(T, nodes, K):
 
 
 @pytest.mark.parametrize('K', [3, 5, 7])
-@pytest.mark.parametrize('T,bias', [(3196, 0), (3200, 1), (16380, 1), (16384, 0), (16387, 2)])
-def test_odd_topk_combine_on_both_sides_of_its_lines(T, bias, K):
-    """799, 800, 4095, 4096 and 4097 row blocks of one part (H = 1000: the second vector of a lane is partly past the end): torch's float32 sums in the same
+@pytest.mark.parametrize('T,H,bias', [(2948, 1000, 0), (2950, 1000, 0), (3068, 1000, 1), (3072, 1000, 1), (3076, 1000, 0), (3200, 1000, 1), (16380, 1000, 1), (16384, 1000, 0), (16387, 1000, 2),
+                                      (8192, 2048, 0), (8191, 2056, 1), (4096, 4096, 0), (4099, 4104, 2)])
+def test_odd_topk_combine_on_both_sides_of_its_lines(T, H, bias, K):
+    """737 and 738 (top-7), 767 to 769, 800, 4095, 4096 and 4097 row blocks of one part (H = 1000: the second vector of a lane is partly past the end), and 4096 and a
+    few more of several parts, whose launches are held to fewer workgroups a CU: torch's float32 sums in the same
     order, rounded once, then once with the biases; weights carried back."""
     import deep_ep
-    H, E = 1000, 16
+    E = 16
     gen = torch.Generator(device=DEV).manual_seed(T + K)
     topk = torch.rand((T, E), generator=gen, device=DEV).topk(K, dim=-1).indices
     topk[torch.rand((T, K), generator=gen, device=DEV) < 0.1] = -1
