@@ -133,13 +133,16 @@ std::atomic<bool> g_fp8_hw{true};
 // than the memory keeps open.  Measured at 16384 tokens x 7168 (microseconds at 2/3/4/5 workgroups and uncapped):
 //   top-2  175 140 126 120 120      top-4  233 201 194 199 200
 //   top-6  297 272 286 289 291      top-8  385 354 377 378 376
-// and for the kernel that takes any top-k: top-1 best uncapped, top-3 at 6, top-5 at 5, top-7 to top-16 at 4.
+// and for the kernel that takes any top-k, which launches of this size take for top-1 and from top-9 on: top-1 best uncapped, with two
+// biases (three rows) at 6, from top-9 to top-16 at 4.
 // A bias row is one more row a wave fetches: top-6 with one / two biases 326 311 329 336 / 358 350 373 377 at 2/3/4/5.
 // The two-phase kernels of the partitioned path do not react to it.
 std::atomic<int> g_combine_blocks_per_cu{-1};
 constexpr unsigned kLdsBytesPerCu = 160 * 1024;
 // The unrolled kernels of odd top-k at 3/4/5/6 and uncapped: top-3 - 158 153 153 153, top-5 233 234 241 244 -, at 8192 tokens 123 119 120 122 -;
-// top-7 314 329 335 - -, of 2560 channels at 8192 tokens 62.1 60.6 60.8 - -.
+// top-7 314 329 335 - -, of 2560 channels at 8192 tokens 62.1 60.6 60.8 - -.  With one / two biases at 2/3/4/5/6 and uncapped, 16384 tokens: top-3 235 198
+// 188 191 195 196 / 260 228 229 235 239 240; top-5 287 268 277 284 288 288 / 316 309 323 331 331 334; top-7 357 354 372 377 377 379 / 388 399 415 421 420
+// 419 (the kernel for any top-k, at 4: 190 / 226, 272 / 308, 350 / 394); of 2560 channels top-7 137 127 128 130 131 130 / 149 140 142 145 145 145 (137 / 146).
 unsigned combine_lds_cap(int num_topk, bool specialised, bool odd, int num_row_blocks, int hidden) {     // num_topk: rows a wave fetches, biases included
     int n = g_combine_blocks_per_cu;
     if (n < 0) {
@@ -150,7 +153,7 @@ unsigned combine_lds_cap(int num_topk, bool specialised, bool odd, int num_row_b
         if (num_row_blocks < 4096 or hidden < 2048) n = 0;
         else if (specialised and odd) n = num_topk <= 3 ? 6 : num_topk <= 5 or hidden < 4096 ? 4 : 3;
         else if (specialised) n = num_topk <= 2 ? 0 : num_topk <= 4 ? 4 : 3;
-        else n = num_topk <= 2 ? 0 : num_topk == 3 ? 6 : num_topk <= 5 ? 5 : 4;
+        else n = num_topk <= 2 ? 0 : num_topk == 3 ? 6 : 4;
     }
     // a workgroup can ask for 64 KiB at most, which lets two of them into a CU: a cap of one cannot be enforced this
     // way (it is served as two), and from 160 workgroups on a share of the LDS is too small to mean anything (no cap)
