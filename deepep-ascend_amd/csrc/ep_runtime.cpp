@@ -1618,13 +1618,14 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
                 ca.num_parts = (int)std::max<int64_t>(1, ceil_div(hidden, EP_COMBINE_LONG_PART));
             }
             ca.num_row_blocks = (int)ceil_div((int64_t)ca.num_rows_bound * ca.num_parts, EP_ROWS_PER_BLOCK);
-            // Odd top-k: the unrolled kernels fetch a row for every position and save trips to memory; where rows are wide and many and most of
-            // their positions are none, the kernel for any top-k moves less.  us of both reduces of all partitions, that one / unrolled: eight of 64 tokens
-            // x 7168 top-3 / 7 81.8 / 76.4, 125 / 121; 1024 x 2560 top-3 / 5 / 7 137 / 131, 176 / 171, 214 / 210, 4096 x 1024 186 / 183, 242 / 240, 306 / 301; but
-            // 2048 x 7168 460 / 471, 666 / 681, 849 / 852, 4096 x 4096 526 / 548, 752 / 768, of 7168 851 / 888, 1254 / 1286; whole rows a wave (long_parts) 1029 /
-            // 1010, 1682 / 1657 (top-7).  Four of 1024 x 7168 125 / 125, 160 / 160, 188 / 187, 4096 394 / 409, 521 / 528, 627 / 633; 16 of 2048 x 2560 433 / 434, 600 / 610, 782 /
-            // 813.  Two of 2048 x 7168 93 / 94, 117 / 116, 140 / 137, 8192 x 4096 192 / 200, 245 / 250, 301 / 300, 16384 379 / 388, 469 / 491, 578 / 593, x 7168 632 /
-            // 640, 789 / 798, 980 / 963.
+            // Odd top-k: the unrolled kernels ask for all slots of a row at once and save trips to memory (top-3 with as many registers: 63
+            // against 62).  Launches of many wide rows wait for bandwidth, and where most positions are none the shorter bursts of the kernel for any
+            // top-k win, as they do for one partition.  us of both reduces of all partitions, that one / unrolled, top-3 / 5 / 7: eight of 64 tokens x
+            // 7168 (top-3, top-7) 81.8 / 76.4, 125 / 121; 1024 x 2560 137 / 131, 176 / 171, 214 / 210; 4096 x 1024 186 / 183, 242 / 240, 306 / 301; but 2048 x
+            // 7168 460 / 471, 666 / 681, 849 / 852; 4096 x 4096 526 / 548, 752 / 768, in long parts (top-7) 1029 / 1010; 4096 x 7168 851 / 888, 1254 / 1286,
+            // in long parts 1682 / 1657.  Four of 1024 x 7168 125 / 125, 160 / 160, 188 / 187; of 4096 394 / 409, 521 / 528, 627 / 633.  16 of 2048 x 2560
+            // 433 / 434, 600 / 610, 782 / 813; three and four of 4096 x 2560 top-3 123 / 122, 168 / 168.  Two of 2048 x 7168 93 / 94, 117 / 116, 140 / 137; 8192 x
+            // 4096 192 / 200, 245 / 250, 301 / 300; 16384 x 4096 379 / 388, 469 / 491, 578 / 593; x 7168 632 / 640, 789 / 798, 980 / 963.
             const bool few = K < 2 * R, wide = hidden >= 4096;
             const bool one_by_one = K % 2 != 0 and not ca.long_parts and
                                     (few ? ca.num_row_blocks >= 4000 and (wide or (K > 3 and K <= R)) : ca.num_row_blocks >= 12000 and wide and K <= 2 * R + 1);
