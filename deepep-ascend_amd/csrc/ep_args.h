@@ -165,7 +165,9 @@ struct EpScatterArgs {
 // side of a node that ships ranks: every workgroup works the layout out for itself.
 #define EP_SMALL_ENTRIES 1024
 #define EP_SMALL_MASK_EXPERTS 1024    // ep_dispatch_small_*, ep_layout_assign_bits: up to here a bit a token and expert is kept in LDS (16 bytes an expert)
-#define EP_SMALL_REPEATS 128          // ep_dispatch_small_*: entries beyond the first of a token for an expert that are listed
+// ep_dispatch_small_*: entries beyond the first of a token for an expert that are listed.  (No more: with 26880 bytes at 1024 experts six workgroups
+// share the LDS of a CU; 288 more, and 128 tokens x 7168 top-1 with padding took 11.1 us instead of 9.9.)
+#define EP_SMALL_REPEATS 112
 struct EpSmallArgs {
     EpLayoutArgs l;               // what ep_layout_assign (ep_recv_copy: ep_layout_place) would have been given
     EpScatterArgs s;              // what the copy kernel would have been given

@@ -1652,9 +1652,9 @@ extern "C" __global__ __launch_bounds__(EP_LAYOUT_THREADS) void ep_layout_assign
 // alignment 16, 96 tokens 8.0 -> 6.5; 1024 experts, 61 tokens top-8 7.4 -> 5.8; top-1 level; all of a dispatch of eight partitions of 64 tokens
 // top-8, metadata above included, 110.0 -> 88.3.  Masks at 2048 experts: 1 token top-1 with padding 8.3 -> 10.8, compared so 8.2.
 // Repeated selections, ids compared without masks / compared behind masks / listed: 128 tokens x 7168 top-8 of 256, one repeated once
-// 10.9 / 11.1 / 9.2, ids drawn with repetitions 11.0 / 11.2 / 9.7, one repeated by every token 11.2 / 11.4 / 10.5; 61 tokens x 5120, top-6 7.1 / 7.2 / 6.5; beyond the
-// list (that form compares) every token on one expert 11.4 / 11.9 / 12.4, every entry on one 12.5 / 14.1 / 14.5, of 256 channels 9.6 / 10.2 / 10.6:
-// the masks' and the list's words are contended.  (A list of 256, level at 128 tokens with every one of them: 32 tokens on one expert each 8.0 -> 8.8.)
+// 10.9 / 11.1 / 9.2, ids drawn with repetitions 11.0 / 11.2 / 9.7; one repeated by every token, 61 tokens x 5120 top-6 7.1 / 7.2 / 6.7, 100 x 2048 7.9 /
+// 7.8 / 7.4; beyond the list (that form compares) 128 tokens x 7168, one repeated by every token 11.2 / 11.4 / 11.9, every token on one expert 11.4 / 11.9 /
+// 12.4, every entry on one 12.5 / 14.1 / 14.5, of 256 channels 9.6 / 10.2 / 10.6: the masks' and the list's words are contended.
 // ------------------------------------------------------------------------------------------------
 template <bool QUANT, bool HW, bool PACK>
 __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
@@ -1674,7 +1674,7 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     int* s_more = s_cnt + Ep;                           // [4] entries that s_list has, or would have
     int* s_start = s_more + 4;                          // [Ep] first slot of each expert (one partition)
     short* s_key = (short*)(s_start + Ep);              // [EP_SMALL_ENTRIES] expert of every entry, -1: none
-    unsigned* s_list = (unsigned*)(s_key + EP_SMALL_ENTRIES);           // [EP_SMALL_REPEATS] (token, expert) pairs beyond their first entry (masks)
+    short* s_list = s_key + EP_SMALL_ENTRIES;           // [EP_SMALL_REPEATS] entries beyond the first of a token for an expert (masks)
     const int tid = threadIdx.x, lane = lane_id(), w = __builtin_amdgcn_readfirstlane(wave_id());
     const int n = l.num_tokens * K;
 
@@ -1715,7 +1715,7 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
             atomicOr((unsigned*)&s_tok[PACK ? partition_of(e) : 0] + (tok >> 5), bit);
             if (masks && (atomicOr((unsigned*)&s_mask[e] + (tok >> 5), bit) & bit)) {
                 const int x = atomicAdd(s_more, 1);
-                if (x < EP_SMALL_REPEATS) s_list[x] = (unsigned)(tok << 16 | e);
+                if (x < EP_SMALL_REPEATS) s_list[x] = (short)i;
             }
         }
     }
@@ -1783,8 +1783,8 @@ __device__ __forceinline__ void dispatch_small_body(const EpSmallArgs& a) {
     if (masks && more <= EP_SMALL_REPEATS) {
         rank = below(s_mask[max(e, 0)], t);             // earlier tokens that selected it, and beyond that their repetitions
         for (int x0 = 0; x0 < more; x0 += WAVE) {
-            const unsigned pair = x0 + lane < more ? s_list[x0 + lane] : ~0u;
-            const int earlier = (int)(pair >> 16) < t ? (int)(pair & 0xffffu) : -2;
+            const int at = s_list[min(x0 + lane, more - 1)];
+            const int earlier = x0 + lane < more && at < t * K ? s_key[at] : -2;
             for (int j = 0; j < K; ++j) {
                 const int c0 = __popcll(__ballot(earlier == readlane(e, j)));
                 if (lane == j) rank += c0;

@@ -438,7 +438,7 @@ void launch_layout(EpLayoutArgs& la, int num_blocks, void* stream) {
 unsigned small_lds(int E, int R) {
     const unsigned tokens = EP_TOKENS_PER_BLOCK / 8, masks = E <= EP_SMALL_MASK_EXPERTS ? (unsigned)E : 0u;
     return ((unsigned)R + masks) * tokens + (2u * (unsigned)align_up(E, 8) + 4u) * sizeof(int) +
-           EP_SMALL_ENTRIES * sizeof(short) + (masks > 0 ? EP_SMALL_REPEATS * sizeof(int) : 0u);
+           (EP_SMALL_ENTRIES + (masks > 0 ? EP_SMALL_REPEATS : 0)) * sizeof(short);
 }
 // Workgroups that zero the padding of such a dispatch: each counts all ids first, in LDS that grows with the experts, so they
 // are no more than fit the chip at once with the row workgroups (1024), unless the padding may be more than 48 MiB.
