@@ -379,9 +379,11 @@ bool bits_layout(int K, int E) { return K <= EP_BITS_TOPK and E <= EP_SMALL_MASK
 // 13.4, 16 14.6 / 15.6; top-4, 8 14.5 / 13.3, 16 14.8 / 17.0; top-6, 8 16.1 / 15.7, 10 16.3 / 17.3; top-8, 6 17.5 / 16.7, 8 17.6 / 18.3; top-12, 4 21.1 /
 // 18.9; top-32, 2 37.3 / 31.5.  To a host that waits for the counts the saved launch was worth more (wall clock, 8 blocks, top-7 24.3 / 23.7,
 // top-8 25.3 / 25.0).
-// Against the two launches that rank in bit masks the line lies lower where no host waits.  us, two launches / one, 256 experts: top-1,
-// 16 blocks 9.4 / 8.9; top-2, 8 9.3 / 8.2, 16 9.4 / 10.3; top-4, 4 9.7 / 8.8, 6 9.8 / 10.1; top-8, 2 10.3 / 10.5, 3 10.1 / 11.8; 32 experts top-4, 4
-// 10.0 / 8.1, 6 10.2 / 9.5; 1024 experts 10.7 / 10.3, 10.8 / 11.6.
+// Against the two launches that rank in bit masks the line lies lower where no host waits, and lower still with more than a few experts, whose
+// histograms every workgroup clears and scans.  us, two launches / one, 256 experts: top-1,
+// 16 blocks 9.4 / 8.9; top-2, 8 9.3 / 8.2, 16 9.4 / 10.3; top-4, 4 9.7 / 8.8, 6 9.8 / 10.1; top-8, 2 10.3 / 10.5, 3 10.1 / 11.8; 1024 experts top-4
+// 10.7 / 10.3, 10.8 / 11.6.  What one launch takes more, at 12 to 16, 18 to 24, 25 to 32 and 35 to 40 blocks x top-k, top-2 to 4 / top-5 to 8: 8 experts -3.2 / -2.7,
+// -1.7 / -1.4, -1.3 / -1.2, 0 / 0.2; 32 -2.0 / -1.4, -0.6 / -0.2, -0.3 / 0 (top-7 and 8 0.2, 0.2), 1.1 / 1.3; 64 -1.6 / -0.9, -0.2 / 0.3, 0.1 / 0.5, 1.5 / 1.8; 128 -1.3 / -0.6, 0.1 / 0.7, 0.4 / 0.8.
 // Where a host waits it is 48 blocks x top-k for every top-k: higher than against the other two for top-3 to top-5 (32 to 40 there), lower for top-7
 // and top-8 (56, 64).  The ids come 16 a thread and trip: wall clock of a dispatch of exact sizes is level up to 48 and falls off beyond.  us, two
 // launches / one: 256 experts, top-3, 10 blocks 26.2 / 25.0, 12 26.8 / 27.2, 16 26.7 / 26.8; top-4, 8 26.6 / 25.0, 10 26.3 / 26.1, 12 26.7 / 27.0, 14 26.6 / 28.4; top-5, 9
@@ -389,7 +391,7 @@ bool bits_layout(int K, int E) { return K <= EP_BITS_TOPK and E <= EP_SMALL_MASK
 // 26.3 / 26.5, 7 26.5 / 27.8, 8 26.3 / 27.5; 32 experts, top-8, 6 26.5 / 25.9, 7 26.4 / 27.0; 1024, 4 30.3 / 30.0, 6 30.1 / 30.7.
 bool recount_pays(int num_blocks, int K, int E, bool host_waits) {
     const int most = 2 * EP_RECOUNT_DEPTH;
-    const int limit = bits_layout(K, E) ? (host_waits ? 48 : 16)
+    const int limit = bits_layout(K, E) ? (host_waits ? 48 : E <= 32 and E * K <= 192 ? 32 : 16)
                                         : std::max(K > 8 ? most : std::min(8 * K, host_waits ? most : 48), 32);
     return num_blocks <= 16 and num_blocks * K <= limit;
 }

@@ -176,11 +176,12 @@ def test_small_dispatch_deferred_exact_and_replayed():
 
 @pytest.mark.parametrize('T,E,K', [(1021, 64, 7), (1024, 256, 8), (1025, 256, 8), (257, 48, 21), (900, 16, 6), (8192, 8, 1), (2048, 32, 2),
                                    (2049, 32, 2), (1281, 64, 5), (256, 256, 8), (257, 256, 8), (512, 64, 4), (513, 64, 4), (2048, 8, 1),
-                                   (2049, 8, 1), (2048, 64, 3), (2049, 64, 3), (1536, 64, 4), (1537, 64, 4), (768, 256, 8), (769, 256, 8),
+                                   (2049, 8, 1), (2048, 64, 3), (2049, 64, 3), (1536, 64, 4), (1537, 64, 4), (768, 256, 8), (769, 256, 8), (512, 16, 8),
+                                   (513, 16, 8), (640, 32, 6), (641, 32, 6), (257, 32, 7), (1024, 8, 4), (1025, 8, 4), (512, 33, 4), (513, 33, 4),
                                    (512, 64, 16), (513, 64, 16)])
 def test_ids_of_all_blocks_counted_in_place(T, E, K):
     """Around the most blocks x top-k (64) for which the histogram kernel can be left out (every workgroup then reads all ids
-    itself), and around the library's own limits: 16 without and 48 with a host that waits, 16 blocks, and 64 where the layout
+    itself), and around the library's own limits: 16 (of few experts, up to 32 for top-6: 32) without and 48 with a host that waits, 16 blocks, and 64 where the layout
     does not rank in bit masks (top-16).  The same handles whichever launches run.  (The layout has launches of its own where
     the epilogue is deferred, and beyond 4096 tokens or 16384 entries.)"""
     import deep_ep
