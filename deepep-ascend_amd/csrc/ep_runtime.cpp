@@ -1690,11 +1690,11 @@ static int combine_launch(ep_buffer_t* b, const ep_combine_args_t* pa, int phase
             // top-2 and 3, where it has the more waves.  us of both reduces of all partitions (7168 channels, captured), unrolled / that: two of 64 /
             // 256 / 1024 / 2048 tokens top-8 21.3 / 21.2, 32.6 / 31.3, 90.5 / 79.3, 164 / 143, of 256 top-4 24.5 / 24.0, top-2 21.1 / 21.4; four of 256
             // / 512 / 2048 top-8 77.1 / 79.6, 122 / 117, 379 / 358; eight of 256 / 800 / 2048 top-3 101.5 / 105.9, 228 / 210, 476 / 463, top-6 146 / 163,
-            // 346 / 348, a pass of them with a host sync 1234 / 1243; two, three and four of 640 to 2048 tokens top-3 0 to 6 % less; top-2 of five to 16 partitions
-            // level (1 % either way).  That against unrolled in % over 1024 to 7168 channels, at 900 / 1000 / 1100 / 1400 / 2000 row blocks: three partitions
+            // 346 / 348, a pass of them with a host sync 1234 / 1243; two, three and four of 640 to 2048 tokens top-3 0 to 6 % less; top-2 of five to eight
+            // partitions, 960 row blocks of 2560 channels 1 to 2 % more, 1120 of 7168 1 % less.  That against unrolled in % over 1024 to 7168 channels, at 900 / 1000 / 1100 / 1400 / 2000 row blocks: three partitions
             // top-4 0 / 0 / -2 / -2 / -2, top-5 -2 / -1 / -3 / -4 / -4, top-8 -6 / -5 / -9 / -9 / -8; four top-6 -1 / -1 / -2 / -4 / -3, top-8 -3 / -3 / -6 / -6 / -5, but top-5
             // +2 / +2 / 0 / -1 / -1, top-4 +3 / +3 / +1 / 0 / 0 (2560 channels +5 / +4 / +3 / +1 / -3).  Two, at 448 / 520 / 760: top-4 -1 / -2 / -2, top-8 -4 / -7 / -6.
-            const int from = R == 2 ? 448 : R == 4 and K == 4 ? 1500 : R == 4 and K == 5 ? 1100 : 896;
+            const int from = R == 2 ? 448 : R == 4 and K == 4 ? 1500 : R == 4 and K == 5 ? 1100 : K == 2 ? 1024 : 896;
             const bool master_by_master = ca.num_row_blocks >= from and (R <= 4 ? K > 2 : K <= 3);
             launch(g_k.combine[EP_COMBINE_FINAL][master_by_master ? 0 : unrolled], (unsigned)ca.num_row_blocks, EP_ROW_THREADS, 0, a.stream, ca);
         }

@@ -575,10 +575,10 @@ def test_top8_combine_on_both_sides_of_the_paced_line(T, nodes):
 
 @pytest.mark.parametrize('T,nodes,K,H', [(64, 2, 3, 64), (1788, 2, 8, 64), (1792, 2, 8, 64), (1792, 2, 2, 64), (1793, 2, 5, 64), (3580, 4, 6, 64), (3584, 4, 7, 64),
                                          (3584, 4, 2, 64), (3584, 4, 4, 64), (5996, 4, 4, 64), (6000, 4, 4, 64), (4396, 4, 5, 64),
-                                         (4400, 4, 5, 64), (3584, 8, 3, 64), (3584, 8, 7, 64), (100, 8, 5, 64), (97, 16, 7, 64), (2200, 2, 3, 4096),
+                                         (4400, 4, 5, 64), (3584, 8, 3, 64), (4092, 8, 2, 64), (4096, 8, 2, 64), (3584, 8, 7, 64), (100, 8, 5, 64), (97, 16, 7, 64), (2200, 2, 3, 4096),
                                          (2400, 2, 3, 4096), (1800, 4, 5, 4096), (6300, 2, 5, 4096), (700, 8, 7, 4104), (2000, 8, 5, 2056), (2000, 4, 7, 2056)])
 def test_reduces_of_a_node_by_partitions_topk_and_size(T, nodes, K, H):
-    """Owner side and token side at both sides of the lines between their kernels (448, 896 and, four partitions top-4 and top-5, 1500 and 1100 row blocks of one part; on the owner side 4000 and
+    """Owner side and token side at both sides of the lines between their kernels (448, 896, top-2 1024 and, four partitions top-4 and top-5, 1500 and 1100 row blocks of one part; on the owner side 4000 and
     12000 of wide and less wide rows).  A token's row
     comes back once a selection: a partial is a multiple of it, rounded once, and sums of at most eight of those are exact in float32."""
     import deep_ep
