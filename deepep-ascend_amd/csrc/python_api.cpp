@@ -145,9 +145,10 @@ at::Tensor first_rows(const at::Tensor& t, int64_t rows) {
     return t.dim() == 1 ? view_of(t, {rows}, {1}, 0) : view_of(t, {rows, t.size(1)}, {t.size(1), 1}, 0);
 }
 // Contiguous int32 tensors out of one allocation (each starts on a multiple of 256 bytes): an allocation of the caching allocator's costs
-// 0.5 us and its release about 0.3, a view 0.1.  Host time of the native dispatch with the counts' and slots' three allocations as one: 61 tokens
-// 8.5 -> 7.6 us, one of eight partitions of 64 tokens 8.7 -> 7.9.  (Metadata rows and received weights in it as well: 6.6, and 8.5 -> 7.7 for the
-// receive side; but the weights are the caller's, to save or to free without the handle.)
+// 0.5 us and its release about 0.3, a view 0.1.  Host time of the native dispatch, all apart / the handle's tensors out of one: 61 tokens
+// 8.7 / 7.3 us, one of eight partitions of 64 tokens 8.8 / 7.9.  (Received weights in it as well 6.8; but they are the caller's, to save or to
+// free without the handle.)
+constexpr int64_t kSharedMetadataWords = 1 << 20;        // metadata rows up to here: 4 MiB
 class Together {
 public:
     // where the next `n` elements will be
@@ -181,6 +182,7 @@ struct DispatchState {
     OptTensor sf, topk_weights, stats;
     at::Tensor psum_rank, psum_expert, unaligned, dst_slot, dst_gsge;
     OptTensor cached_meta;
+    OptTensor meta;             // allocated with the counts and slots
     py::object cached_list;
     int64_t cached_num_recv = 0, cached_num_expanded = 0;
     ep_dispatch_args_t a{};
@@ -286,6 +288,8 @@ py::tuple run_dispatch_epilogue(DispatchState& s) {
         meta = *s.cached_meta;
         if (meta.dim() != 2 || meta.size(0) != num_recv)
             throw EpPyError("Assertion exception (python_api.cpp): recv_src_metadata.size(0) == num_recv_tokens");
+    } else if (s.meta.has_value()) {
+        meta = *std::move(s.meta);
     } else if (!have_meta) {
         meta = empty_i32({alloc_recv, K + 2}, dev);
     }
@@ -434,13 +438,23 @@ public:
             s.cached_num_recv = *cached_num_recv_tokens;
             s.cached_num_expanded = *cached_num_expanded_tokens;
         } else {
-            // the counts and slots of the handle share one allocation, sized by the arguments' shapes; what has worst-case size or
-            // belongs to the caller alone (metadata rows, received weights) has storage of its own, allocated once the library
-            // has accepted the call
+            // the tensors of the handle share one allocation: counts and slots, sized by the arguments' shapes, and, where the copy follows at
+            // once, the metadata rows unless they are many (a call that is refused below should not have allocated them).  What the
+            // caller alone owns (received rows, scales and weights) has storage of its own.
             const int64_t El = std::max(0, s.num_local_experts), TK = (int64_t)s.num_tokens * s.num_topk;
+            int64_t meta_rows = -1, meta_at = 0;
+            if (copy_follows) {
+                int c_recv = 0, c_exp = 0;
+                if (do_cpu_sync) meta_rows = s.num_tokens;
+                else if (ep_dispatch_worst_case_sizes(buf_, num_max_tokens_per_rank, s.num_topk, num_experts, expert_alignment, &c_recv, &c_exp) == 0)
+                    meta_rows = c_recv;
+                if (meta_rows > kSharedMetadataWords / (s.num_topk + 2)) meta_rows = -1;
+            }
             Together t;
             const int64_t rank_at = t.add(num_ranks_), expert_at = t.add(El), unaligned_at = t.add(El), slot_at = t.add(TK), gsge_at = t.add(TK);
+            if (meta_rows >= 0) meta_at = t.add(meta_rows * (s.num_topk + 2));
             t.allocate(dev);
+            if (meta_rows >= 0) s.meta = t.part(meta_at, {meta_rows, s.num_topk + 2});
             s.psum_rank = t.part(rank_at, {(int64_t)num_ranks_});
             s.psum_expert = t.part(expert_at, {El});
             s.unaligned = t.part(unaligned_at, {El});
