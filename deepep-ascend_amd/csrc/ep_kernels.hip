@@ -1878,8 +1878,8 @@ extern "C" __global__ __launch_bounds__(EP_ROW_THREADS) void ep_dispatch_small_q
 // 1024 top-2 16.4 / 12.9; one of eight partitions, FP8, all of its dispatch: 256 tokens top-8 32.4 / 18.5, 2048 top-6 71.4 / 65.6.
 // With several partitions a workgroup counts the ids up to its own tokens' and no further (ranks and places in a partition
 // count what is before), so that half of the chip's share of that work falls away and the first workgroups copy meanwhile.  us a
-// dispatch and its receive side, all partitions in a captured graph, before / after: eight of 2048 tokens FP8 top-6 532 / 518, of 512 185.7 / 182.7,
-// of 256 125.9 / 125.2; four of 1024 x 4096 top-8 148.1 / 147.3, top-4 106.5 / 106.7.
+// dispatch and its receive side, all partitions in a captured graph, before / after: eight of 2048 tokens FP8 top-6 532 / 518 (a whole pass with
+// both reduces, 1235, is level), of 512 185.7 / 182.7, of 256 125.9 / 125.2; four of 1024 x 4096 top-8 148.1 / 147.3, top-4 106.5 / 106.7.
 // (Padding as equal shares of all padding rows in place of pieces of experts: 256 tokens 50.8 -> 56.9; the ids of two goes in flight:
 // spills, or one workgroup a CU and level; each id of the next go asked for as one of this go is used: 2048 x 2560 19.8 -> 18.7, but one go
 // 1 to 2 % slower.)
